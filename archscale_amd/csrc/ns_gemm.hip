@@ -14,14 +14,16 @@
 // the tile sizes, so the main loop has no bounds checks; only the FINAL epilogue
 // (which writes the caller's tensor) is bounds-checked.
 //
-// Data path: global -> LDS with direct 16-byte loads (no VGPR round trip), two
-// LDS stages, XOR-swizzled 16-byte chunks so the 128-bit MFMA operand reads are
-// bank-conflict free; v_mfma_f32_32x32x16_bf16 with fp32 accumulation.
+// Data path: global -> LDS with direct 16-byte loads (no VGPR round trip) into two or
+// more LDS stages, XOR-swizzled 16-byte chunks so the 128-bit MFMA operand reads are
+// bank-conflict free; v_mfma_f32_16x16x32 (bf16 or half) with fp32 accumulation.  Four
+// waves in a 2 x 2 arrangement, each with a quarter of the block tile.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <atomic>
 #include <type_traits>
+#include <utility>
 
 #include "ns_gemm.h"
 
@@ -36,7 +38,8 @@ namespace archscale {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
@@ -74,25 +77,88 @@ __device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
 // 16-byte bank groups (rows alternate between the two 128-byte halves of the 64 banks).
 __device__ __forceinline__ int lds_chunk_off(int r, int c) { return r * ROW_BYTES + ((c ^ ((r >> 1) & 7)) << 4); }
 
+// K-major tile in LDS: 64 k-rows of ROWS * 2 bytes.  The 16-byte chunk c of row k sits at chunk c ^ kmaj_swz<ROWS>(k), so
+// that what the 32 lanes of a half-wave touch with one transpose read (eight k-rows: k0..k0+3 and k0+8..k0+11, 32 bytes
+// each) covers all 64 banks.
+template <int ROWS>
+__device__ __forceinline__ int kmaj_swz(int k) {
+  return ROWS >= 128 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (((k >> 1) & 1) << 2) | (((k >> 3) & 1) << 1);
+}
+
+// f(0), f(1), ... f(N - 1) with the index as a compile-time constant
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+
+// counted wait for this wave's vector-memory operations and for its LDS operations (N: how many of the former may still
+// be in flight; vmcnt has six bits)
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// acc += a * b on the matrix cores.  Inline assembly with the accumulator as a read-write operand: the builtin leaves the
+// destination free, and over a software-pipelined loop the register allocator then rotates the accumulators with
+// register moves between the MFMAs (measured: half the issue rate).  What the assembler statement hides from the compiler
+// is kept by hand: an empty statement after the zero-initialisation keeps it away from the first MFMA, and acc_settle()
+// stands between the last MFMA and the first read of a result.
+template <bool HALF, bool AGPR>
+__device__ __forceinline__ void mfma16(f32x4& acc, const u32x4& a, const u32x4& b) {
+  if constexpr (AGPR) {
+    if constexpr (HALF) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  } else {
+    if constexpr (HALF) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  }
+}
+template <bool AGPR>
+__device__ __forceinline__ void acc_touch(f32x4& acc) {
+  if constexpr (AGPR) asm volatile("" : "+a"(acc));
+  else asm volatile("" : "+v"(acc));
+}
+// 16-bit transpose read of four k-values of one column per lane; the result arrives later (see the kernel)
+template <int OFF>
+__device__ __forceinline__ void lds_tr_read(uint32_t addr, unsigned long long& raw) {
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(raw) : "v"(addr), "n"(OFF));
+}
+__device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+
 // F16 = 1: the workspace matrices (operands, addend, non-final outputs) are IEEE half instead of bfloat16 (the caller's
 // tensors stay bfloat16); the host keeps them in range with power-of-two factors folded into alpha / beta / out_shift.
 // F16 = 2: bfloat16 operands and addend, IEEE-half output (the step from a bfloat16 iteration to a half one).
 // SK: problems of the launch may carry a K-split (GemmParams::ksplit; symmetric products, 128x128 configuration): the
 // blocks that share a tile leave their fp32 accumulators in the workspace and the last one to arrive adds them up in
 // the order of the parts and runs the epilogue.
-template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
-__global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
-ns_gemm_kernel(const GroupedGemmParams gp) {
+//
+// One block is four waves (one per SIMD of a compute unit), wave (r, c) of the 2 x 2 arrangement computes rows
+// r BT/2 .., columns c BT/2 .. of the BT x BT tile.  What bounds the 256 configuration is the LDS port and, at the power
+// limit, the energy of operand movement: four waves of 128 x 128 read 128 KB of LDS per k-tile where eight waves of
+// 128 x 64 read 192 KB, which with the 64 KB of copies is 2048 clk of LDS time per 2048 clk of matrix-core time.
+// Measured on 16 x (2048 x 5632 x 2048), Gaussian operands: 1145 TFLOP/s with eight waves and 32x32x16 MFMAs, 1215 to 1240
+// with four waves and 16x16x32 MFMAs, 1280 to 1300 with a third LDS stage for Q (zero operands, where power does not
+// limit: 1320 / 1330 / 1525).  A persistent form whose copies run on into the next tile measured the same (1300).
+//
+// LDS: SP stages of the P tile and SQ of the Q tile (SQ = SP or SP + 1).  The 256 configuration has room for 2 + 3: the
+// operand that streams from memory (Q = X^T) gets two k-tiles of time to arrive, P, which the caches hold, gets one.
+template <int BT, int SP, int SQ, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+__device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
+#if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know the buffer descriptor type)
+  static_assert(BT == 256 || BT == 128 || BT == 64, "block tiles");
   static_assert(!(F16 && SPLIT), "the hi+lo pair is a bfloat16 device");
-  static_assert(!SK || (BM == 128 && !SPLIT && !FINAL && MODE != MODE_BX), "the K-split serves symmetric products in the small configuration");
+  static_assert(!SK || (BT == 128 && !SPLIT && !FINAL && MODE != MODE_BX), "the K-split serves symmetric products in the 128 configuration");
   static_assert(F16 != 2 || (MODE == MODE_BX && !FINAL), "only X' changes its storage type");
   constexpr bool IN16 = F16 == 1, OUT16 = F16 != 0;
-  constexpr int NW = (BM / WM) * (BN / WN);
-  constexpr int WAVES_N = BN / WN;
-  constexpr int FM = WM / 32, FN = WN / 32;
-  constexpr int PBYTES = BM * ROW_BYTES, QBYTES = BN * ROW_BYTES, STAGE = PBYTES + QBYTES;
-  constexpr int JP = BM / 8 / NW, JQ = BN / 8 / NW;  // 8-row slabs (1 KiB) per wave
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile rows must split over waves");
+  constexpr int NW = 4, NT = 256;
+  constexpr int WT = BT / 2;            // side of a wave's sub-tile
+  constexpr int FR = WT / 16;           // 16x16 fragments along a side of it
+  constexpr bool AGPR = FR == 8;        // 256 accumulator registers per lane: they live in the accumulation half of the file
+  constexpr int OPBYTES = BT * ROW_BYTES;   // one stage of one operand
+  constexpr int NC = BT / 8 / NW;       // copies (1 KiB: 8 rows x 128 B) per wave, operand and k-tile
+  static_assert(BT % (8 * NW) == 0, "tile rows must split over waves");
+  static_assert(SP >= 2 && (SQ == SP || SQ == SP + 1), "stages");
   // MODE_SYRKT is MODE_SYRK with the operand given K-major: P = Q = X^T stored [K][M] (leading dimension ldp), so the
   // iteration needs no row-major copy of X at all; the MFMA fragments then come from LDS transpose reads
   constexpr bool KMAJ = (MODE == MODE_SYRKT);
@@ -115,7 +181,7 @@ ns_gemm_kernel(const GroupedGemmParams gp) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hi = lane >> 5;
+  const int l16 = lane & 15, lg = lane >> 4;
 
   // ---- block -> (problem, matrix, tile).  Workgroups are dealt round-robin to the 8 XCDs; runs of 32
   // consecutive logical tiles (neighbouring tiles of one matrix: shared operand panels) are kept on ONE
@@ -200,11 +266,10 @@ ns_gemm_kernel(const GroupedGemmParams gp) {
     tj = 2 * tj + (quadrant & 1);
     if (SYM && ti > tj) return;   // lower quadrant of a diagonal tile: its mirror image covers it
   }
-  const int R0 = ti * BM, C0 = tj * BN;
+  const int R0 = ti * BT, C0 = tj * BT;
 
   const char* Pb = KMAJ ? (const char*)(p.P + (size_t)b * p.strideP + R0)
                         : (const char*)(p.P + (size_t)b * p.strideP + (size_t)R0 * p.ldp);
-  const char* P2b = KSPLIT ? (const char*)(p.P2 + (size_t)b * p.strideP + (size_t)R0 * p.ldp) : nullptr;
   const char* Qb = KMAJ ? (const char*)(p.Q + (size_t)b * p.strideQ + C0)
                         : (const char*)(p.Q + (size_t)b * p.strideQ + (size_t)C0 * p.ldq);
   int KT = p.K / BK;
@@ -215,257 +280,253 @@ ns_gemm_kernel(const GroupedGemmParams gp) {
     Qb += KMAJ ? (size_t)kt0 * BK * p.ldq * 2 : (size_t)kt0 * ROW_BYTES;
     KT = kt1 - kt0;
   }
-
-  // per-lane byte offsets of the global chunks this lane copies (k-tile 0)
-  uint32_t offP[JP], offQ[JQ];
-  if constexpr (!KMAJ) {
-#pragma unroll
-    for (int j = 0; j < JP; ++j) {
-      const int r = (wave * JP + j) * 8 + (lane >> 3);
-      const int src = (lane & 7) ^ ((r >> 1) & 7);
-      offP[j] = (uint32_t)r * (uint32_t)p.ldp * 2u + (uint32_t)src * 16u;
-    }
-#pragma unroll
-    for (int j = 0; j < JQ; ++j) {
-      const int r = (wave * JQ + j) * 8 + (lane >> 3);
-      const int src = (lane & 7) ^ ((r >> 1) & 7);
-      offQ[j] = (uint32_t)r * (uint32_t)p.ldq * 2u + (uint32_t)src * 16u;
-    }
-  } else {
-    // K-major tile in LDS: 64 k-rows of BM*2 bytes; the 16-byte chunk c of row k sits at chunk c ^ ((k & 3) << 2), so
-    // that four consecutive k-rows of one 64-byte column segment cover all 64 banks (what a transpose read touches)
-    constexpr int CPRK = BM / 8;   // chunks per k-row
-#pragma unroll
-    for (int j = 0; j < JP; ++j) {
-      const int pidx = (wave * JP + j) * 64 + lane, k = pidx / CPRK, cpos = pidx % CPRK;
-      offP[j] = (uint32_t)k * (uint32_t)p.ldp * 2u + (uint32_t)((cpos ^ ((k & 3) << 2)) * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < JQ; ++j) {
-      const int pidx = (wave * JQ + j) * 64 + lane, k = pidx / CPRK, cpos = pidx % CPRK;
-      offQ[j] = (uint32_t)k * (uint32_t)p.ldq * 2u + (uint32_t)((cpos ^ ((k & 3) << 2)) * 16);
-    }
-  }
-
   const int KT_ALL = KSPLIT ? 2 * KT : KT;
 
-  // copy j (of JP + JQ per wave) of k-tile kt: one 1 KiB slab (8 rows x 128 B) straight into stage kt & 1
-  constexpr int NGL = JP + JQ;
-  auto gload = [&](int kt, int j) {
-    const char* pb = Pb;
-    int kk = kt;
-    if (KSPLIT && kt >= KT) { pb = P2b; kk = kt - KT; }
-    const size_t koffP = KMAJ ? (size_t)kk * BK * p.ldp * 2 : (size_t)kk * ROW_BYTES;
-    const size_t koffQ = KMAJ ? (size_t)kk * BK * p.ldq * 2 : (size_t)kk * ROW_BYTES;
-    char* sP = smem + (kt & 1) * STAGE;
-    char* sQ = sP + PBYTES;
-    if (j < JP) __builtin_amdgcn_global_load_lds((gptr_t)(pb + offP[j] + koffP), (lptr_t)(sP + (wave * JP + j) * 1024), 16, 0, 0);
-    else __builtin_amdgcn_global_load_lds((gptr_t)(Qb + offQ[j - JP] + koffQ), (lptr_t)(sQ + (wave * JQ + (j - JP)) * 1024), 16, 0, 0);
+  // ---- copies.  Buffer loads with a descriptor over the operand panel: the lane's place in the tile is a constant 32-bit
+  // offset per copy, the k-tile a scalar one (the host keeps panels below 4 GiB), so a copy is one instruction and the
+  // setting of M0.  The swizzle is folded into the SOURCE address of each lane, the LDS side is linear.
+  uint32_t offP[NC], offQ[NC];
+  auto lane_off = [&](int j, int ld) -> uint32_t {
+    if constexpr (!KMAJ) {
+      const int r = (wave * NC + j) * 8 + (lane >> 3);
+      return (uint32_t)r * (uint32_t)ld * 2u + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+    } else {
+      constexpr int CPRK = BT / 8;   // chunks per k-row
+      const int pidx = (wave * NC + j) * 64 + lane, k = pidx / CPRK, cpos = pidx % CPRK;
+      return (uint32_t)k * (uint32_t)ld * 2u + (uint32_t)((cpos ^ kmaj_swz<BT>(k)) * 16);
+    }
   };
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    offP[j] = lane_off(j, p.ldp);
+    offQ[j] = lane_off(j, p.ldq);
+  }
+  const uint32_t kstepP = KMAJ ? (uint32_t)BK * (uint32_t)p.ldp * 2u : (uint32_t)ROW_BYTES;
+  const uint32_t kstepQ = KMAJ ? (uint32_t)BK * (uint32_t)p.ldq * 2u : (uint32_t)ROW_BYTES;
+  const char* P2b = KSPLIT ? (const char*)(p.P2 + (size_t)b * p.strideP + (size_t)R0 * p.ldp) : Pb;
+  // (the descriptors have to be seen to be uniform: each is a loop over the lanes otherwise)
+  auto uniform = [](const char* q) {
+    const uint64_t v = (uint64_t)q;
+    return (void*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
+  };
+  void* const uP = uniform(Pb);
+  void* const uQ = uniform(Qb);
+  void* const uP2 = uniform(P2b);
+  // What the copies of k-tile kt use.  Past the last k-tile the descriptor has no records: the load touches no memory, and
+  // the main loop needs no tail without copies (three copies of its body cost registers where they meet).
+  struct Source { __amdgpu_buffer_rsrc_t P, Q; uint32_t atP, atQ; };
+  auto source = [&](int kt) __attribute__((always_inline)) {
+    const int records = __builtin_amdgcn_readfirstlane(kt < KT_ALL ? -1 : 0);
+    const int second = KSPLIT ? __builtin_amdgcn_readfirstlane(kt >= KT ? 1 : 0) : 0;
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane(second ? kt - KT : kt);
+    Source s = {__builtin_amdgcn_make_buffer_rsrc(second ? uP2 : uP, 0, records, 0x00027000),
+                __builtin_amdgcn_make_buffer_rsrc(uQ, 0, records, 0x00027000), k * kstepP, k * kstepQ};
+    return s;
+  };
+  // copy j of this wave of the P / Q tile into a stage (byte offset in LDS)
+  auto copyP = [&](const Source& s, int stage, int j) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.P, (lptr_t)(smem + stage + (wave * NC + j) * 1024), 16, (int)offP[j], (int)s.atP, 0, 0);
+  };
+  auto copyQ = [&](const Source& s, int stage, int j) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.Q, (lptr_t)(smem + stage + (wave * NC + j) * 1024), 16, (int)offQ[j], (int)s.atQ, 0, 0);
+  };
+  constexpr int QBASE = SP * OPBYTES;   // the Q stages follow the P stages
 
-  f32x16 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  const int wr0 = (wave / WAVES_N) * WM;  // wave origin inside the block tile
-  const int wc0 = (wave % WAVES_N) * WN;
-  // Diagonal tile of a symmetric product: a wave whose sub-tile lies wholly BELOW the diagonal computes nothing (it
-  // only takes part in the copies and the barriers); its part of the tile is the mirror image of the sub-tiles that
-  // lie wholly ABOVE the diagonal, and those waves write it (two of eight waves idle in the 256x256 configuration, one
-  // of four in the 128x128 one: a quarter of the tile's matrix-core work).
-  static_assert((BM == 256 && BN == 256 && WM == 128 && WN == 64) || (BM == 128 && BN == 128 && WM == 64 && WN == 64),
-                "checked for these two: the idle sub-tiles together are exactly the mirror image of the sub-tiles above the diagonal");
+  const int wr0 = (wave >> 1) * WT;     // wave origin inside the block tile
+  const int wc0 = (wave & 1) * WT;
+  // Diagonal tile of a symmetric product: wave (1, 0), whose sub-tile lies wholly BELOW the diagonal, computes nothing (it
+  // only takes part in the copies and the barriers); its part of the tile is the mirror image of the sub-tile of wave
+  // (0, 1), which writes it (a quarter of the tile's matrix-core work is saved).
   const bool diag = SYM && (ti == tj);
-  const bool idle = diag && (wc0 + WN <= wr0);
-  const bool above = diag && (wr0 + WM <= wc0);
-  // operand read offsets: row (w0 + i*32 + l32), chunk (2*kk + hi)
-  int rdP[4], rdQ[4];
+  const bool idle = diag && wave == 2;
+  const bool above = diag && wave == 1;
+
+  f32x4 acc[FR][FR];
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    rdP[kk] = lds_chunk_off(wr0 + l32, 2 * kk + hi);
-    rdQ[kk] = lds_chunk_off(wc0 + l32, 2 * kk + hi);
+  for (int i = 0; i < FR; ++i)
+#pragma unroll
+    for (int j = 0; j < FR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < FR; ++i)
+#pragma unroll
+    for (int j = 0; j < FR; ++j) acc_touch<AGPR>(acc[i][j]);
+
+  // ---- operand fragments.  A k-tile is two k-steps of 32.  Fragment f of a wave in k-step kk holds, in lane l16 + 16 lg, the
+  // eight k-values 32 kk + 8 lg .. + 7 of row (column) 16 f + l16 of the wave's sub-tile: one 16-byte read.
+  u32x4 af[2][FR], bq[2][FR];
+  int rdP[2], rdQ[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    rdP[kk] = lds_chunk_off(wr0 + l16, 4 * kk + lg);
+    rdQ[kk] = lds_chunk_off(wc0 + l16, 4 * kk + lg);
   }
   // K-major operands: a 16-lane group reads 4 k-rows x 16 columns with one LDS transpose read; lane s = 4e + a of the
   // group points at columns 4a..4a+3 of row k0 + e and receives, as lane 4a' + b', the 4 k-values of column 4a' + b'.
-  // Two such reads (k0, k0 + 4) make the 8 k-values of an MFMA operand; k0 = 16*kk + 8*(lane/32) is added below.
-  int trP[FM], trQ[FN];
+  // Two such reads (k0, k0 + 4) make the 8 k-values of a fragment; k0 = 32 kk + 8 lg.
+  int trP[KMAJ ? FR : 1], trQ[KMAJ ? FR : 1];
   if constexpr (KMAJ) {
-    const int g = lane >> 4, s16 = lane & 15, e = s16 >> 2, a = s16 & 3;
-    const int krow = 8 * (g >> 1) + e;
+    const int e = l16 >> 2, a = l16 & 3, k = 8 * lg + e;   // kmaj_swz takes the same value for k + 4 and k + 32
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      const int m = wr0 + i * 32 + (g & 1) * 16 + 4 * a;
-      trP[i] = krow * (BM * 2) + (((m >> 3) ^ (e << 2)) << 4) + ((m & 7) << 1);
-    }
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int n = wc0 + j * 32 + (g & 1) * 16 + 4 * a;
-      trQ[j] = krow * (BN * 2) + (((n >> 3) ^ (e << 2)) << 4) + ((n & 7) << 1);
+    for (int f = 0; f < FR; ++f) {
+      const int m = wr0 + f * 16 + 4 * a, n = wc0 + f * 16 + 4 * a;
+      trP[f] = k * (BT * 2) + (((m >> 3) ^ kmaj_swz<BT>(k)) << 4) + ((m & 7) << 1);
+      trQ[f] = k * (BT * 2) + (((n >> 3) ^ kmaj_swz<BT>(k)) << 4) + ((n & 7) << 1);
     }
   }
-
-  // ---- main loop.  A k-tile is four k-steps of FM*FN MFMAs; the operand fragments of a k-step are
-  // double-buffered in registers.  Every memory instruction is pinned behind an MFMA of its own:
-  //   * an LDS fragment read of the NEXT k-step after each of the first FM+FN MFMAs of a k-step;
-  //   * the global->LDS copies of a k-tile spread over the MFMAs of COPY_PHASES k-steps.  Issued back to
-  //     back, the copies hold the wave until the texture unit has accepted all of them (about as long as
-  //     the MFMAs of half a k-tile), and nothing overlaps.
-  // The loop is rotated by one k-step: the barrier that publishes k-tile kt+1 sits between k-steps 2 and 3
-  // of k-tile kt, so the MFMAs of k-step 3 run over the first fragment reads of the new tile and over the
-  // first copies of k-tile kt+2 into the stage that the barrier has just freed.
-  constexpr int NMF = FM * FN, NRD = FM + FN;
-  constexpr int COPY_PHASES = 2;
-  constexpr int GPP = (NGL + COPY_PHASES - 1) / COPY_PHASES;
-  constexpr int G1 = GPP < NGL ? GPP : NGL, G2 = 2 * GPP < NGL ? 2 * GPP : NGL, G3 = 3 * GPP < NGL ? 3 * GPP : NGL;
-  static_assert(G1 == 4 || G1 == 8 || G1 == 16, "the first wait below is written for these counts");
-  bf16x8 af[2][FM], bq[2][FN];
   // The transpose reads are inline assembly: the compiler makes the builtin wait for every outstanding global->LDS
   // copy (vmcnt(0)) before each read.  The compiler therefore does not know that their results arrive late.  The raw
   // results stay in variables of their own (afr / bqr, one 64-bit pair per read) that nothing touches until the explicit
-  // s_waitcnt lgkmcnt(0) before the first MFMA of the k-step; that wait is followed by empty asm statements that take
-  // every raw result as a read-write operand, so each use (the packing into an MFMA operand included) depends on a
-  // statement that comes after the wait.
+  // s_waitcnt lgkmcnt(0) at the end of the k-step that reads them (the last read is a quarter of a k-step old by then); that
+  // wait is followed by empty asm statements that take every raw result as a read-write operand, so each use (the
+  // packing into an MFMA operand included) depends on a statement that comes after the wait, and none is in flight
+  // where the loop closes.
   typedef unsigned long long u64;
-  u64 afr[2][KMAJ ? FM : 1][2], bqr[2][KMAJ ? FN : 1][2];
-  auto tr8 = [&](const char* base, int pitch, int kk, u64 (&raw)[2]) {
-    const uint32_t a0 = (uint32_t)(uintptr_t)base + (uint32_t)(16 * kk * pitch);
-    const uint32_t a1 = a0 + (uint32_t)(4 * pitch);
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(raw[0]) : "v"(a0));
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(raw[1]) : "v"(a1));
-  };
-  auto fread = [&](int buf, const char* sP, const char* sQ, int kk, int r) {
+  u64 afr[2][KMAJ ? FR : 1][2], bqr[2][KMAJ ? FR : 1][2];
+  // LDS reads of a k-step into fragment set BUF: NRD of them (Q operand first: the first row of MFMAs needs all of it)
+  constexpr int NRD = KMAJ ? 4 * FR : 2 * FR;
+  auto fread = [&](auto buf_, int sP, int sQ, auto kk_, auto r_) __attribute__((always_inline)) {
+    constexpr int buf = decltype(buf_)::value, kk = decltype(kk_)::value, r = decltype(r_)::value;
     if constexpr (!KMAJ) {
-      if (r < FM) af[buf][r] = *(const bf16x8*)(sP + rdP[kk] + r * 32 * ROW_BYTES);
-      else bq[buf][r - FM] = *(const bf16x8*)(sQ + rdQ[kk] + (r - FM) * 32 * ROW_BYTES);
+      if constexpr (r < FR) bq[buf][r] = *(const u32x4*)(smem + sQ + rdQ[kk] + r * 16 * ROW_BYTES);
+      else af[buf][r - FR] = *(const u32x4*)(smem + sP + rdP[kk] + (r - FR) * 16 * ROW_BYTES);
     } else {
-      if (r < FM) tr8(sP + trP[r], BM * 2, kk, afr[buf][r]);
-      else tr8(sQ + trQ[r - FM], BN * 2, kk, bqr[buf][r - FM]);
+      constexpr int f = (r >> 1) % FR, h = r & 1, off = (32 * kk + 4 * h) * (BT * 2);
+      if constexpr (r < 2 * FR) {
+        const uint32_t addr = (uint32_t)(uintptr_t)(smem + sQ) + (uint32_t)trQ[f];
+        lds_tr_read<off>(addr, bqr[buf][f][h]);
+      } else {
+        const uint32_t addr = (uint32_t)(uintptr_t)(smem + sP) + (uint32_t)trP[f];
+        lds_tr_read<off>(addr, afr[buf][f][h]);
+      }
     }
   };
-  // K-major operands: wait for the transpose reads of fragment buffer `buf`, then pack them
-  auto land = [&](int buf) {
+  // K-major operands: wait for the transpose reads of fragment set BUF, then make fragments of them
+  auto land = [&](auto buf_) __attribute__((always_inline)) {
     if constexpr (KMAJ) {
-      typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+      constexpr int buf = decltype(buf_)::value;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-      for (int i = 0; i < FM; ++i) asm volatile("" : "+v"(afr[buf][i][0]), "+v"(afr[buf][i][1]));
+      for (int f = 0; f < FR; ++f) {
+        asm volatile("" : "+v"(bqr[buf][f][0]), "+v"(bqr[buf][f][1]));
+        asm volatile("" : "+v"(afr[buf][f][0]), "+v"(afr[buf][f][1]));
+      }
 #pragma unroll
-      for (int j = 0; j < FN; ++j) asm volatile("" : "+v"(bqr[buf][j][0]), "+v"(bqr[buf][j][1]));
-#pragma unroll
-      for (int i = 0; i < FM; ++i) { const u64x2 v = {afr[buf][i][0], afr[buf][i][1]}; af[buf][i] = __builtin_bit_cast(bf16x8, v); }
-#pragma unroll
-      for (int j = 0; j < FN; ++j) { const u64x2 v = {bqr[buf][j][0], bqr[buf][j][1]}; bq[buf][j] = __builtin_bit_cast(bf16x8, v); }
+      for (int f = 0; f < FR; ++f) {
+        typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+        const u64x2 vb = {bqr[buf][f][0], bqr[buf][f][1]}, va = {afr[buf][f][0], afr[buf][f][1]};
+        bq[buf][f] = __builtin_bit_cast(u32x4, vb);
+        af[buf][f] = __builtin_bit_cast(u32x4, va);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // one k-step: MFMAs on fragment buffer CBUF (when COMPUTE), reads of k-step RKK of the stage at (rP, rQ)
-  // into buffer RBUF (when READ), copies [G0, G1) of k-tile gt
-  auto phase = [&](auto compute, auto read, auto cbuf_, auto rbuf_, const char* rP, const char* rQ, auto rkk_, int gt,
-                   auto g0_, auto g1_) {
-    constexpr bool COMPUTE = decltype(compute)::value, READ = decltype(read)::value;
-    constexpr int cbuf = decltype(cbuf_)::value, rbuf = decltype(rbuf_)::value, rkk = decltype(rkk_)::value;
-    constexpr int g0 = decltype(g0_)::value, g1 = decltype(g1_)::value;
-    if constexpr (COMPUTE) land(cbuf);
-#pragma unroll
-    for (int q = 0; q < NMF; ++q) {
-      if (COMPUTE)
-        acc[q / FN][q % FN] = IN16 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[cbuf][q / FN]), __builtin_bit_cast(f16x8, bq[cbuf][q % FN]), acc[q / FN][q % FN], 0, 0, 0)
-                                  : __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cbuf][q / FN], bq[cbuf][q % FN], acc[q / FN][q % FN], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      const int g_lo = g0 + (q * (g1 - g0) + NMF - 1) / NMF, g_hi = g0 + ((q + 1) * (g1 - g0) + NMF - 1) / NMF;
-      if (READ && q < NRD) fread(rbuf, rP, rQ, rkk, q);
-#pragma unroll
-      for (int g = 0; g < NGL; ++g)
-        if (g >= g_lo && g < g_hi) gload(gt, g);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
+
+  // ---- main loop.  The fragments of a k-step are read from LDS during the MFMAs of the k-step before it, and the copies
+  // of later k-tiles are spread over the MFMAs too: every memory instruction is pinned behind an MFMA of its own
+  // (sched_barrier fences).  Copies issued back to back hold the wave until the texture unit has accepted them (64 B per
+  // clk and compute unit), and with one wave per SIMD nothing else runs meanwhile.
+  // The barrier that publishes k-tile kt + 1 sits between the two k-steps of k-tile kt: by then every read of k-tile kt has
+  // been issued and has returned (lgkmcnt(0)), so its stage is free for the copies that follow the barrier.
+  constexpr int NMF = FR * FR;
   using Yes = std::true_type;
   using No = std::false_type;
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  using C1 = std::integral_constant<int, G1>;
-  using C2 = std::integral_constant<int, G2>;
-  using C3 = std::integral_constant<int, G3>;
-  using C4 = std::integral_constant<int, NGL>;
-  // k-steps 0..2 of k-tile kt (with the rest of the copies of kt+1), barrier, k-step 3 (with the first
-  // copies of kt+2).  COPY_REST / NEXT / COPY_FIRST: k-tiles kt+1 / kt+1 / kt+2 exist.  ACTIVE = false is the same
-  // sequence of copies, waits and barriers without the fragment reads and the MFMAs: what a wave runs whose sub-tile
-  // lies below the diagonal of a symmetric product (one code path, so the barriers of the two kinds of wave cannot
-  // drift apart).
-  auto ktile = [&](int kt, auto copy_rest, auto next, auto copy_first, auto active) {
-    constexpr bool COPY_REST = decltype(copy_rest)::value, NEXT = decltype(next)::value, COPY_FIRST = decltype(copy_first)::value;
-    using Act = std::integral_constant<bool, decltype(active)::value>;
-    const char* sP = smem + (kt & 1) * STAGE;
-    const char* sQ = sP + PBYTES;
-    const char* nP = smem + ((kt + 1) & 1) * STAGE;
-    const char* nQ = nP + PBYTES;
-    if constexpr (COPY_REST) {
-      phase(Act{}, Act{}, I0{}, I1{}, sP, sQ, I1{}, kt + 1, C1{}, C2{});
-      phase(Act{}, Act{}, I1{}, I0{}, sP, sQ, I2{}, kt + 1, C2{}, C3{});
-      phase(Act{}, Act{}, I0{}, I1{}, sP, sQ, I3{}, kt + 1, C3{}, C4{});
-    } else {
-      phase(Act{}, Act{}, I0{}, I1{}, sP, sQ, I1{}, 0, I0{}, I0{});
-      phase(Act{}, Act{}, I1{}, I0{}, sP, sQ, I2{}, 0, I0{}, I0{});
-      phase(Act{}, Act{}, I0{}, I1{}, sP, sQ, I3{}, 0, I0{}, I0{});
+  // one k-step: MFMAs on fragment set CBUF (when ACTIVE), reads of k-step RKK of the stages at (rsP, rsQ) into the other
+  // set, copies of P to stage dP (when CP) and of Q to stage dQ (when CQ) from src
+  auto kstep = [&](auto active, auto cbuf_, int rsP, int rsQ, auto rkk_, auto cp, auto cq, const Source& src, int dP, int dQ) __attribute__((always_inline)) {
+    constexpr bool ACTIVE = decltype(active)::value, CP = decltype(cp)::value, CQ = decltype(cq)::value;
+    constexpr int cbuf = decltype(cbuf_)::value;
+    constexpr int NCOPY = (CP ? NC : 0) + (CQ ? NC : 0);
+    // reads within the first three quarters of the k-step, copies over all of it
+    constexpr int RSPAN = NMF * 3 / 4;
+    static_for<NMF>([&](auto q_) __attribute__((always_inline)) {
+      constexpr int q = decltype(q_)::value;
+      if constexpr (ACTIVE) mfma16<IN16, AGPR>(acc[q / FR][q % FR], af[cbuf][q / FR], bq[cbuf][q % FR]);
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int c_lo = (q * NCOPY + NMF - 1) / NMF, c_hi = ((q + 1) * NCOPY + NMF - 1) / NMF;
+      static_for<c_hi - c_lo>([&](auto d_) __attribute__((always_inline)) {
+        constexpr int c = c_lo + decltype(d_)::value;
+        if constexpr (CP && c < NC) copyP(src, dP, c);
+        else copyQ(src, dQ, CP ? c - NC : c);
+      });
+      if constexpr (ACTIVE) {
+        constexpr int r_lo = q < RSPAN ? (q * NRD + RSPAN - 1) / RSPAN : NRD, r_hi = q + 1 < RSPAN ? ((q + 1) * NRD + RSPAN - 1) / RSPAN : NRD;
+        static_for<r_hi - r_lo>([&](auto d_) __attribute__((always_inline)) {
+          fread(std::integral_constant<int, cbuf ^ 1>{}, rsP, rsQ, rkk_, std::integral_constant<int, r_lo + decltype(d_)::value>{});
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (ACTIVE) land(std::integral_constant<int, cbuf ^ 1>{});
+  };
+  auto nextP = [](int s) { return s + OPBYTES == SP * OPBYTES ? 0 : s + OPBYTES; };
+  auto nextQ = [](int s) { return s + OPBYTES == QBASE + SQ * OPBYTES ? QBASE : s + OPBYTES; };
+  // In k-tile kt: Q of k-tile kt + SP in the first k-step when Q has the extra stage (the stage of kt - 1 is free), else
+  // after the barrier like P of kt + SP.  In flight at the barrier, younger than what it publishes:
+  constexpr int PAIR = 2 * NC;
+  constexpr int INFLIGHT = (SP - 2) * PAIR + (SQ > SP ? NC : 0);
+  using QX = std::integral_constant<bool, (SQ > SP)>;
+  using QN = std::integral_constant<bool, (SQ == SP)>;
+  auto k_range = [&](auto active) __attribute__((always_inline)) {
+    constexpr bool ACTIVE = decltype(active)::value;
+    int sP = 0, sQ = QBASE;               // stages of k-tile kt
+    if constexpr (ACTIVE) {
+      static_for<NRD>([&](auto r_) __attribute__((always_inline)) { fread(I0{}, 0, QBASE, I0{}, r_); });
+      land(I0{});
     }
-    if constexpr (NEXT) {
-      // this wave's copies of kt+1 have landed and its reads of kt are done; after the barrier that holds for all
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    for (int kt = 0; kt < KT_ALL; ++kt) {
+      const int nP = nextP(sP), nQ = nextQ(sQ);
+      // the Q stage before this one in the ring is the one that k-tile kt + SP goes to when Q has the extra stage
+      const int pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
+      const Source src = source(kt + SP);
+      kstep(active, I0{}, sP, sQ, I1{}, No{}, QX{}, src, 0, pQ);
+      wait_copies<INFLIGHT>();
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (COPY_FIRST) phase(Act{}, Act{}, I1{}, I0{}, nP, nQ, I0{}, kt + 2, I0{}, C1{});
-      else phase(Act{}, Act{}, I1{}, I0{}, nP, nQ, I0{}, 0, I0{}, I0{});
-    } else {
-      phase(Act{}, No{}, I1{}, I0{}, nP, nQ, I0{}, 0, I0{}, I0{});
+      kstep(active, I1{}, nP, nQ, I0{}, Yes{}, QN{}, src, sP, sQ);
+      sP = nP;
+      sQ = nQ;
     }
-  };
-  // the whole K range: ACTIVE waves multiply, the others only copy and meet the barriers
-  auto k_range = [&](auto active) {
-    using Act = std::integral_constant<bool, decltype(active)::value>;
-    if constexpr (Act::value) {
-#pragma unroll
-      for (int r = 0; r < NRD; ++r) fread(0, smem, smem + PBYTES, 0, r);
-    }
-    for (int kt = 0; kt + 2 < KT_ALL; ++kt) ktile(kt, Yes{}, Yes{}, Yes{}, Act{});
-    if (KT_ALL > 1) ktile(KT_ALL - 2, Yes{}, Yes{}, No{}, Act{});
-    ktile(KT_ALL - 1, No{}, No{}, No{}, Act{});
   };
 
+  // first SP k-tiles, oldest first; k-tile 0 has landed once only the younger ones are outstanding
 #pragma unroll
-  for (int g = 0; g < NGL; ++g) gload(0, g);
-  if (KT_ALL > 1) {
+  for (int s = 0; s < SP; ++s) {
+    const Source src = source(s);
 #pragma unroll
-    for (int g = 0; g < G1; ++g) gload(1, g);
-    // k-tile 0 has landed once at most the G1 younger copies are outstanding
-    if constexpr (G1 == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else if constexpr (G1 == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int j = 0; j < NC; ++j) copyQ(src, QBASE + s * OPBYTES, j);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copyP(src, s * OPBYTES, j);
   }
-  __syncthreads();
-  if (!idle) k_range(Yes{});
-  else k_range(No{});
+  wait_copies<(SP - 1) * PAIR>();
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (SYM) {
+    if (idle) {   // the same copies and barriers as its block, nothing else
+      k_range(No{});
+      wait_copies<0>();
+      if constexpr (SK) {
+        if (p.ksplit > 1) {
+          __syncthreads();
+          __syncthreads();
+          if (!*(volatile int*)smem) return;
+        }
+      }
+      __syncthreads();
+      return;
+    }
+  }
+  k_range(Yes{});
+  wait_copies<0>();   // (copies without records included: the epilogue reuses the stages)
+  acc_settle();
 
   // ---- epilogue.  acc[i][j][e] of lane l is element
-  //   rl = wr0 + i*32 + 8*(e/4) + 4*(l/32) + e%4  (row in the tile),   cl = wc0 + j*32 + l%32  (column)
+  //   r = wr0 + 16 i + 4 (l / 16) + e  (row in the tile),   c = wc0 + 16 j + l % 16  (column)
   // so a lane owns 4 consecutive rows of one column.  Every global access of the epilogue goes through
   // LDS (the operand stages are dead by now) so that it is a 16-byte, row-contiguous access:
-  //   * the addend tile is copied in as its transposed image  S[cl][rl]  (it is read as E[col][row..row+3]);
-  //   * the transposed output (mirror of a symmetric product, X'^T) is staged as S[cl][rl] with 8-byte
-  //     LDS writes and flushed row by row;
-  //   * the row-major output is staged as D[rl][cl] with 2-byte LDS writes and flushed row by row.
-  // Scattered 8-byte / 2-byte global accesses straight from the accumulator layout flood L2 with
+  // scattered 8-byte / 2-byte global accesses straight from the accumulator layout flood L2 with
   // partial-line requests and cost a quarter of the kernel.
-  static_assert(BM == BN, "square block tiles");
-  constexpr int NT = NW * 64;
   if constexpr (SK) {
     if (p.ksplit > 1) {
       // Every part leaves its accumulators in the workspace (accumulator layout: one word per lane and accumulator
@@ -475,125 +536,86 @@ ns_gemm_kernel(const GroupedGemmParams gp) {
       // waits for anybody.  The partial results travel as system-scope accesses (written through, read past the
       // caches): the eight L2 caches of the chip are not coherent with each other, and the alternative - a release /
       // acquire fence per block - writes back and invalidates a whole L2 each time (measured: the product twice as slow).
-      __shared__ int sk_last;
-      float* part = p.sk_partial + (size_t)sk_tile * p.ksplit * (BM * BN);
-      if (!idle) {
-        float* dst = part + (size_t)ks * (BM * BN);
+      int* sk_last = (int*)smem;   // the operand stages are dead after the barrier below
+      float* part = p.sk_partial + (size_t)sk_tile * p.ksplit * (BT * BT);
+      float* dst = part + (size_t)ks * (BT * BT);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FR; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FR; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-              __hip_atomic_store(dst + ((i * FN + j) * 16 + e) * NT + tid, acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      }
+          for (int e = 0; e < 4; ++e)
+            __hip_atomic_store(dst + ((i * FR + j) * 4 + e) * NT + tid, acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's stores have been acknowledged
       __syncthreads();
       if (tid == 0) {
         const int old = __hip_atomic_fetch_add(p.sk_counter + sk_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int last = old == p.ksplit - 1;
         if (last) __hip_atomic_store(p.sk_counter + sk_tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
-        sk_last = last;
+        *sk_last = last;
       }
       __syncthreads();
-      if (!sk_last) return;
-      if (!idle) {
+      if (!*sk_last) return;
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FR; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int sidx = 0; sidx < p.ksplit; ++sidx) {
+        const float* src = part + (size_t)sidx * (BT * BT);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-        for (int sidx = 0; sidx < p.ksplit; ++sidx) {
-          const float* src = part + (size_t)sidx * (BM * BN);
+        for (int i = 0; i < FR; ++i)
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
+          for (int j = 0; j < FR; ++j)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-              for (int e = 0; e < 16; ++e)
-                acc[i][j][e] += __hip_atomic_load(src + ((i * FN + j) * 16 + e) * NT + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+            for (int e = 0; e < 4; ++e)
+              acc[i][j][e] += __hip_atomic_load(src + ((i * FR + j) * 4 + e) * NT + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
   }
-  constexpr int TPITCH = BN * 2;            // bytes per staged row (both images)
-  constexpr int CPRT = BN / 8;              // 16-byte chunks per staged row
-  constexpr int PASSES = (BM * BN / 8) / NT;
-  static_assert(BM * BN * 2 <= 2 * STAGE, "staging tile must fit in the operand stages");
   // optional per-matrix scale of the operand that was left out of it (deferred normalisation): the product of two
   // such operands carries sc^2, a product with one of them (and its addend) carries sc
   const float sc = p.scale ? p.scale[b] : 1.f;
   const float bx_sc = sc * __builtin_ldexpf(1.f, p.out_shift);   // MODE_BX: scale of the result (a power of two from the host)
   const float alpha = SYRK_PLAIN ? p.alpha * sc * sc : p.alpha, beta = p.beta;
   // A diagonal tile of a product of a matrix with ITSELF is symmetric bit for bit as it comes out of the matrix cores
-  // (element (i,j) and element (j,i) are the same products summed in the same order over k), so it takes the wave-local
-  // epilogue below like any other tile and writes one image.  A diagonal tile of P Q^T with two different (commuting,
-  // symmetric) matrices is symmetric only up to rounding: it keeps its upper half and reflects it.
-  const bool self_product = p.P == p.Q && p.strideP == p.strideQ && p.ldp == p.ldq;
-  // (the instantiation that writes a hi+lo pair keeps the reflecting path for every diagonal tile: its epilogue has no
-  // registers to spare for the diagonal term in the wave-local one)
-  const bool reflect = diag && (!self_product || (SPLIT && MODE == MODE_SYRK2));
-  // S[cl][rl]: chunk index XOR cl, so the 32 lanes of an 8-byte access (32 different cl) spread over all banks
-  auto s_off = [](int cl, int rl) { return cl * TPITCH + ((((rl >> 3) ^ cl) & (CPRT - 1)) << 4) + ((rl & 7) << 1); };
-  auto s_chunk = [](int cl, int ch) { return cl * TPITCH + (((ch ^ cl) & (CPRT - 1)) << 4); };
-  // D[rl][cl]: 64-byte halves of a row swapped on rows with bit 2 set, so the two half-waves of a 2-byte
-  // access (rows r and r+4) hit different banks
-  auto d_off = [](int rl, int byte_in_row) { return rl * TPITCH + (byte_in_row ^ (((rl >> 2) & 1) << 6)); };
-
-  // row-contiguous copy of a staged image to global memory; `swz` maps (staged row, chunk) -> LDS offset
-  auto flush = [&](auto swz, __bf16* dst, long bstride, int ld, int row0, int col0, int rows_valid, int cols_valid) {
-    __bf16* base = dst + (size_t)b * bstride;
-    const bool vec_ok = !FINAL || ((ld & 7) == 0 && (bstride & 7) == 0 && (((uintptr_t)dst) & 15) == 0);
-#pragma unroll 4
-    for (int t = 0; t < PASSES; ++t) {
-      const int q = t * NT + tid;
-      const int sr = q / CPRT, ch = q - sr * CPRT;
-      const uint4 val = *(const uint4*)(smem + swz(sr, ch));
-      const int row = row0 + sr, col = col0 + ch * 8;
-      if (!FINAL) {
-        *(uint4*)(base + (size_t)row * ld + col) = val;
-      } else if (row < rows_valid) {  // caller's tensor: true extents, arbitrary leading dimension
-        if (vec_ok && col + 7 < cols_valid) {
-          *(uint4*)(base + (size_t)row * ld + col) = val;
-        } else {
-          const uint32_t w[4] = {val.x, val.y, val.z, val.w};
-#pragma unroll
-          for (int k = 0; k < 8; ++k)
-            if (col + k < cols_valid) ((uint16_t*)base)[(size_t)row * ld + col + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
-        }
-      }
-    }
-  };
-  auto s_swz = [&](int sr, int ch) { return s_chunk(sr, ch); };
-  auto d_swz = [&](int sr, int ch) { return d_off(sr, ch * 16); };
+  // (element (i,j) and element (j,i) are the same products summed in the same order over k), so it is stored like any
+  // other tile, as one image.  A diagonal tile of P Q^T with two different (commuting, symmetric) matrices is symmetric
+  // only up to rounding: it keeps its upper half and reflects it.
+  const bool reflect = MODE == MODE_SYRK && diag && !(p.P == p.Q && p.strideP == p.strideQ && p.ldp == p.ldq);
 
   __syncthreads();  // every wave is done reading the operand stages
+  // Wave-local: each wave stages its own WT x WT sub-tile in its own LDS region as the transposed image
+  // W[c][r] (c = column in the sub-tile, r = row), so nothing below needs a block barrier:
+  //   addend in:   16-byte direct copies of E[col][row..] rows into W, read back 8 bytes per lane
+  //   W <- values: 8-byte LDS writes (a lane owns 4 consecutive r of one c), in place of the addend it has read
+  //   transposed / mirrored image out: 16-byte reads of W rows -> 16-byte stores, up to 256 B contiguous per row
+  //   row-major image out: LDS transpose reads (ds_read_b64_tr_b16: a lane receives 4 consecutive c of one
+  //     r; two of them make 16 bytes) -> 16-byte stores, 64 B contiguous per row
+  // The values are formed where they are packed, fragment by fragment: 256 accumulators updated in place would not fit
+  // beside their copies in the register file.
+  constexpr int WROW = WT * 2;                  // bytes per W row
+  constexpr int RCH = WT / 8;                   // 16-byte chunks per W row
+  constexpr int WBYTES = WT * WROW;
+  constexpr int WSLABS = WBYTES / 1024;         // 64-chunk slabs of one region
+  static_assert(NW * WBYTES <= (SP + SQ) * OPBYTES, "wave regions must fit in the operand stages");
+  char* W = smem + wave * WBYTES;
+  // chunk swizzle: the 8-byte accesses of 16 columns, and the four W rows of a transpose read, fall on different banks
+  auto sw = [](int c) {
+    if constexpr (RCH == 16) return ((c & 7) << 1) | ((c >> 3) & 1);
+    else if constexpr (RCH == 8) return (((c >> 1) & 3) << 1) | ((c >> 3) & 1);
+    else return (((c >> 2) & 1) << 1) | ((c >> 3) & 1);
+  };
+  auto w_off = [&](int c, int r) { return c * WROW + (((r >> 3) ^ sw(c)) << 4) + ((r & 7) << 1); };
+  const int wrow0 = R0 + wr0, wcol0 = C0 + wc0;  // global origin of this wave's sub-tile
 
-  if (!reflect) {
-    if (idle) return;
-    // ---- wave-local epilogue (every tile except the diagonal tiles of a product of two different matrices).
-    // Each wave stages its own WM x WN sub-tile in its own LDS region as the transposed image
-    // W[c][r] (c = column in the sub-tile, r = row), so nothing below needs a block barrier:
-    //   addend in:   16-byte direct copies of E[col][row..] rows into W, read back 8 bytes per lane
-    //   W <- values: 8-byte LDS writes (a lane owns 4 consecutive r of one c)
-    //   transposed / mirrored image out: 16-byte reads of W rows -> 16-byte stores, 256 B contiguous per row
-    //   row-major image out: LDS transpose reads (ds_read_b64_tr_b16: a lane receives 4 consecutive c of one
-    //     r; two of them make 16 bytes) -> 16-byte stores, 64 B contiguous per row
-    constexpr int WROW = WM * 2;                  // bytes per W row
-    constexpr int RCH = WM / 8;                   // 16-byte chunks per W row
-    constexpr int WBYTES = WN * WROW;
-    constexpr int WSLABS = WBYTES / 1024;         // 64-chunk slabs of one region
-    static_assert(NW * WBYTES <= 2 * STAGE, "wave regions must fit in the operand stages");
-    char* W = smem + wave * WBYTES;
-    // chunk swizzle: 4 consecutive rows of W land in 4 different pairs of 16-byte bank groups
-    auto sw = [](int c) { return (((c & 7) << 1) | ((c >> 3) & 1)) & (RCH - 1); };
-    auto w_off = [&](int c, int r) { return c * WROW + ((((r >> 3) ^ sw(c)) & (RCH - 1)) << 4) + ((r & 7) << 1); };
-    const int wrow0 = R0 + wr0, wcol0 = C0 + wc0;  // global origin of this wave's sub-tile
-
-    // MODE_BX without an addend (ADDEND = false): a*I was folded into B's diagonal by the product that made B
-    constexpr bool has_e = !SYRK_PLAIN && (MODE != MODE_BX || ADDEND);
+  // MODE_BX without an addend (ADDEND = false): a*I was folded into B's diagonal by the product that made B
+  constexpr bool has_e = !SYRK_PLAIN && (MODE != MODE_BX || ADDEND);
+  const bool on_diag = diag && wr0 == wc0;       // the diagonal of the matrix runs through fragments (f, f) of this wave
+  // PART 0: the values (high halves of a split pair); PART 1: the low halves, value - bf16(value)
+  auto emit = [&](auto part_, __bf16* Cdst) __attribute__((always_inline)) {
+    constexpr int PART = decltype(part_)::value;
     if constexpr (has_e) {
+      if constexpr (PART == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of the high half's image
       const char* Eb = (const char*)(p.E + (size_t)b * p.strideE + (size_t)wcol0 * p.lde + wrow0);
 #pragma unroll
       for (int t = 0; t < WSLABS; ++t) {
@@ -603,281 +625,133 @@ ns_gemm_kernel(const GroupedGemmParams gp) {
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    if constexpr (MODE == MODE_BX && !has_e) {
-      if (bx_sc != 1.f) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FR; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < FR; ++j) {
+        const int c = j * 16 + l16, r = i * 16 + 4 * lg;
+        float v[4];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] *= bx_sc;
-      }
-    } else
+        for (int q = 0; q < 4; ++q) v[q] = acc[i][j][q];
+        if constexpr (SYRK_PLAIN) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+          for (int q = 0; q < 4; ++q) v[q] *= alpha;
+        } else if constexpr (has_e) {
+          const uint2 e = *(const uint2*)(W + w_off(c, r));
+          const float ev[4] = {dec(e.x & 0xffff), dec(e.x >> 16), dec(e.y & 0xffff), dec(e.y >> 16)};
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int c = j * 32 + l32;
+          for (int q = 0; q < 4; ++q) {
+            if constexpr (MODE == MODE_SYRK2) v[q] = fmaf(alpha, v[q], beta * ev[q]);
+            else v[q] = fmaf(alpha, ev[q], v[q]) * bx_sc;
+          }
+        } else {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int r = i * 32 + 8 * g + 4 * hi;
-          if (SYRK_PLAIN) {
+          for (int q = 0; q < 4; ++q) v[q] *= bx_sc;
+        }
+        if constexpr (MODE == MODE_SYRK2) {   // B + a I
+          if (i == j && on_diag) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[i][j][4 * g + q] *= alpha;
-          } else {
-            const uint2 e = *(const uint2*)(W + w_off(c, r));
-            const float e0 = dec(e.x & 0xffff), e1 = dec(e.x >> 16);
-            const float e2 = dec(e.y & 0xffff), e3 = dec(e.y >> 16);
-            if (MODE == MODE_SYRK2) {
-              acc[i][j][4 * g + 0] = fmaf(alpha, acc[i][j][4 * g + 0], beta * e0);
-              acc[i][j][4 * g + 1] = fmaf(alpha, acc[i][j][4 * g + 1], beta * e1);
-              acc[i][j][4 * g + 2] = fmaf(alpha, acc[i][j][4 * g + 2], beta * e2);
-              acc[i][j][4 * g + 3] = fmaf(alpha, acc[i][j][4 * g + 3], beta * e3);
-            } else {
-              acc[i][j][4 * g + 0] = fmaf(alpha, e0, acc[i][j][4 * g + 0]) * bx_sc;
-              acc[i][j][4 * g + 1] = fmaf(alpha, e1, acc[i][j][4 * g + 1]) * bx_sc;
-              acc[i][j][4 * g + 2] = fmaf(alpha, e2, acc[i][j][4 * g + 2]) * bx_sc;
-              acc[i][j][4 * g + 3] = fmaf(alpha, e3, acc[i][j][4 * g + 3]) * bx_sc;
+            for (int q = 0; q < 4; ++q) v[q] += (4 * lg + q == l16) ? p.diag_add : 0.f;
+          }
+        }
+        if constexpr (PART == 1) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] -= bf16_to_f32(bf16_bits(v[q]));
+        }
+        if (MODE == MODE_SYRK && reflect && on_diag) {
+          // upper half to both of its places
+          if (i <= j) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if (i < j || r + q <= c) {
+                const uint16_t bits = enc(v[q]);
+                *(uint16_t*)(W + w_off(c, r + q)) = bits;
+                *(uint16_t*)(W + w_off(r + q, c)) = bits;
+              }
             }
+          }
+        } else {
+          *(uint2*)(W + w_off(c, r)) = pk4(v[0], v[1], v[2], v[3]);
+        }
+        if ((j & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    // transposed / mirrored image: rows of W
+    __bf16* Tdst = SYM ? Cdst : p.Ct;
+    if (Tdst && (!diag || above)) {   // in a diagonal tile: only the image of the idle wave's part
+      const long tbs = SYM ? p.strideC : p.strideCt;
+      const int tld = SYM ? p.ldc : p.ldct;
+      __bf16* base = Tdst + (size_t)b * tbs;
+      const bool vec_ok = !FINAL || ((tld & 7) == 0 && (tbs & 7) == 0 && (((uintptr_t)Tdst) & 15) == 0);
+#pragma unroll 8
+      for (int t = 0; t < WSLABS; ++t) {
+        const int q = t * 64 + lane;
+        const int c = q / RCH, ch = q % RCH;
+        const uint4 val = *(const uint4*)(W + c * WROW + ((ch ^ sw(c)) << 4));
+        const int orow = wcol0 + c, ocol = wrow0 + ch * 8;   // row of the transposed image = column of the tile
+        if (!FINAL) {
+          *(uint4*)(base + (size_t)orow * tld + ocol) = val;
+        } else if (orow < p.n_valid) {
+          if (vec_ok && ocol + 7 < p.m_valid) {
+            *(uint4*)(base + (size_t)orow * tld + ocol) = val;
+          } else {
+            const uint32_t w[4] = {val.x, val.y, val.z, val.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (ocol + k < p.m_valid) ((uint16_t*)base)[(size_t)orow * tld + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
           }
         }
       }
-
-    if constexpr (MODE == MODE_SYRK2 && !SPLIT) {
-      // B + a I: in a diagonal tile (R0 == C0) the diagonal of the matrix runs through the 32x32 blocks (j + d32, j) of
-      // this wave's sub-tile with 32 d32 == wc0 - wr0, where it is the element with 8*g + q == l32 - 4*hi.  Only those
-      // blocks are touched, with a select per element.
-      const int d32 = (wc0 - wr0) / 32;   // wave-uniform
-      if (diag && d32 >= 0 && (wc0 - wr0) % 32 == 0) {
-        const int t = l32 - 4 * hi;
-        const float da = p.diag_add;
-#pragma unroll
-        for (int dd = 0; dd < FM; ++dd)
-          if (dd == d32) {
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-              if (j + dd < FM) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[j + dd][j][e] += (8 * (e >> 2) + (e & 3) == t) ? da : 0.f;
-              }
-          }
-      }
     }
-
-    auto store_wave = [&](__bf16* Cdst, int lane) {
-      const int l32 = lane & 31, hi = lane >> 5;
-      // W[c][r] <- bf16(acc)
+    // row-major image: transpose reads.  In a 16-lane group, source lane s points at W[c0 + s/4][r0 + 4*(s%4) ..+3];
+    // lane L of the group then holds W[c0 .. c0+3][r0 + L].
+    if (SYM || p.C) {
+      __bf16* base = Cdst + (size_t)b * p.strideC;
+      const bool vec_ok = !FINAL || ((p.ldc & 7) == 0 && (p.strideC & 7) == 0 && (((uintptr_t)Cdst) & 15) == 0);
+      const int s = l16;
+#pragma unroll 4
+      for (int rb = 0; rb < WT / 16; ++rb)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *(uint2*)(W + w_off(j * 32 + l32, i * 32 + 8 * g + 4 * hi)) =
-                pk4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-      // transposed / mirrored image: rows of W
-      __bf16* Tdst = SYM ? Cdst : p.Ct;
-      if (Tdst && (!diag || above)) {   // in a diagonal tile: only the image of the idle waves' part
-        const long tbs = SYM ? p.strideC : p.strideCt;
-        const int tld = SYM ? p.ldc : p.ldct;
-        __bf16* base = Tdst + (size_t)b * tbs;
-        const bool vec_ok = !FINAL || ((tld & 7) == 0 && (tbs & 7) == 0 && (((uintptr_t)Tdst) & 15) == 0);
-#pragma unroll
-        for (int t = 0; t < WSLABS; ++t) {
-          const int q = t * 64 + lane;
-          const int c = q / RCH, ch = q % RCH;
-          const uint4 val = *(const uint4*)(W + c * WROW + (((ch ^ sw(c)) & (RCH - 1)) << 4));
-          const int orow = wcol0 + c, ocol = wrow0 + ch * 8;   // row of the transposed image = column of the tile
+        for (int cb = 0; cb < WT / 32; ++cb) {
+          const int c0 = cb * 32 + lg * 8;
+          const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + (s >> 2), rb * 16 + 4 * (s & 3))));
+          const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + 4 + (s >> 2), rb * 16 + 4 * (s & 3))));
+          uint4 val;
+          val.x = (uint32_t)(uint16_t)lo4[0] | ((uint32_t)(uint16_t)lo4[1] << 16);
+          val.y = (uint32_t)(uint16_t)lo4[2] | ((uint32_t)(uint16_t)lo4[3] << 16);
+          val.z = (uint32_t)(uint16_t)hi4[0] | ((uint32_t)(uint16_t)hi4[1] << 16);
+          val.w = (uint32_t)(uint16_t)hi4[2] | ((uint32_t)(uint16_t)hi4[3] << 16);
+          const int orow = wrow0 + rb * 16 + s, ocol = wcol0 + c0;
           if (!FINAL) {
-            *(uint4*)(base + (size_t)orow * tld + ocol) = val;
-          } else if (orow < p.n_valid) {
-            if (vec_ok && ocol + 7 < p.m_valid) {
-              *(uint4*)(base + (size_t)orow * tld + ocol) = val;
+            *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
+          } else if (orow < p.m_valid) {
+            if (vec_ok && ocol + 7 < p.n_valid) {
+              *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
             } else {
               const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
               for (int k = 0; k < 8; ++k)
-                if (ocol + k < p.m_valid) ((uint16_t*)base)[(size_t)orow * tld + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+                if (ocol + k < p.n_valid) ((uint16_t*)base)[(size_t)orow * p.ldc + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
             }
           }
         }
-      }
-      // row-major image: transpose reads.  In a 16-lane group, source lane s points at W[c0 + s/4][r0 + 4*(s%4) ..+3];
-      // lane L of the group then holds W[c0 .. c0+3][r0 + L].
-      if (SYM || p.C) {
-        __bf16* base = Cdst + (size_t)b * p.strideC;
-        const bool vec_ok = !FINAL || ((p.ldc & 7) == 0 && (p.strideC & 7) == 0 && (((uintptr_t)Cdst) & 15) == 0);
-        const int grp = lane >> 4, s = lane & 15;
-#pragma unroll
-        for (int rb = 0; rb < WM / 16; ++rb)
-#pragma unroll
-          for (int cb = 0; cb < WN / 32; ++cb) {
-            const int c0 = cb * 32 + grp * 8;
-            const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + (s >> 2), rb * 16 + 4 * (s & 3))));
-            const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + 4 + (s >> 2), rb * 16 + 4 * (s & 3))));
-            uint4 val;
-            val.x = (uint32_t)(uint16_t)lo4[0] | ((uint32_t)(uint16_t)lo4[1] << 16);
-            val.y = (uint32_t)(uint16_t)lo4[2] | ((uint32_t)(uint16_t)lo4[3] << 16);
-            val.z = (uint32_t)(uint16_t)hi4[0] | ((uint32_t)(uint16_t)hi4[1] << 16);
-            val.w = (uint32_t)(uint16_t)hi4[2] | ((uint32_t)(uint16_t)hi4[3] << 16);
-            const int orow = wrow0 + rb * 16 + s, ocol = wcol0 + c0;
-            if (!FINAL) {
-              *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
-            } else if (orow < p.m_valid) {
-              if (vec_ok && ocol + 7 < p.n_valid) {
-                *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
-              } else {
-                const uint32_t w[4] = {val.x, val.y, val.z, val.w};
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                  if (ocol + k < p.n_valid) ((uint16_t*)base)[(size_t)orow * p.ldc + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
-              }
-            }
-          }
-      }
-    };
-
-    store_wave(p.C, lane);
-    if (SPLIT && MODE == MODE_SYRK2) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] -= bf16_to_f32(bf16_bits(acc[i][j][e]));
-      __builtin_amdgcn_sched_barrier(0);
-      // the second copy of the store code gets its lane id through an opaque move, so that its addresses are computed
-      // here and not hoisted above the first copy (where they cost hundreds of spilled registers)
-      int lane2 = lane;
-      asm volatile("" : "+v"(lane2));
-      store_wave(p.C2, lane2);
-    }
-    return;
-  }
-
-  // ---- block-cooperative epilogue for the diagonal tiles of a symmetric product (the upper half is
-  // reflected across waves so that the product is bit-symmetric)
-
-  // 1. fold the addend into the accumulators: acc <- alpha*acc + beta*E (SYRK2), acc + alpha*E (BX), alpha*acc (SYRK)
-  if (!SYRK_PLAIN) {
-    // E[C0 + cl][R0 + rl] -> S[cl][rl], two staged rows (1 KiB) per wave-wide copy
-    const char* Eb = (const char*)(p.E + (size_t)b * p.strideE + (size_t)C0 * p.lde + R0);
-#pragma unroll
-    for (int t = 0; t < PASSES; ++t) {
-      const int slab = wave * PASSES + t;                  // 64 chunks
-      const int q = slab * 64 + lane;
-      const int sr = q / CPRT, cpos = q - sr * CPRT;
-      const int src = (cpos ^ sr) & (CPRT - 1);
-      __builtin_amdgcn_global_load_lds((gptr_t)(Eb + ((size_t)sr * p.lde + src * 8) * 2), (lptr_t)(smem + slab * 1024), 16, 0, 0);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int cl = wc0 + j * 32 + l32;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int rl = wr0 + i * 32 + 8 * g + 4 * hi;
-        if (SYRK_PLAIN) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[i][j][4 * g + q] *= alpha;
-        } else {
-          const uint2 e = *(const uint2*)(smem + s_off(cl, rl));
-          const float e0 = dec(e.x & 0xffff), e1 = dec(e.x >> 16);
-          const float e2 = dec(e.y & 0xffff), e3 = dec(e.y >> 16);
-          if (MODE == MODE_SYRK2) {
-            acc[i][j][4 * g + 0] = fmaf(alpha, acc[i][j][4 * g + 0], beta * e0);
-            acc[i][j][4 * g + 1] = fmaf(alpha, acc[i][j][4 * g + 1], beta * e1);
-            acc[i][j][4 * g + 2] = fmaf(alpha, acc[i][j][4 * g + 2], beta * e2);
-            acc[i][j][4 * g + 3] = fmaf(alpha, acc[i][j][4 * g + 3], beta * e3);
-            // diagonal of the matrix (this path runs on diagonal tiles only: R0 == C0)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (rl + q == cl) acc[i][j][4 * g + q] += p.diag_add;
-          } else {
-            acc[i][j][4 * g + 0] = fmaf(alpha, e0, acc[i][j][4 * g + 0]) * bx_sc;
-            acc[i][j][4 * g + 1] = fmaf(alpha, e1, acc[i][j][4 * g + 1]) * bx_sc;
-            acc[i][j][4 * g + 2] = fmaf(alpha, e2, acc[i][j][4 * g + 2]) * bx_sc;
-            acc[i][j][4 * g + 3] = fmaf(alpha, e3, acc[i][j][4 * g + 3]) * bx_sc;
-          }
-        }
-      }
-    }
-  if (!SYRK_PLAIN) __syncthreads();  // the addend image is consumed; LDS is free again
-
-  // stores the accumulators as bf16 to Cdst (row-major image) and to its transposed / mirrored image
-  auto store_all = [&](__bf16* Cdst, int lane) {
-    const int l32 = lane & 31, hi = lane >> 5;
-    // 2. transposed image
-    const bool want_t = SYM ? !diag : (p.Ct != nullptr);
-    if (want_t) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int cl = wc0 + j * 32 + l32;
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int rl = wr0 + i * 32 + 8 * g + 4 * hi;
-            *(uint2*)(smem + s_off(cl, rl)) =
-                pk4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-          }
-        }
-      __syncthreads();
-      if (SYM) flush(s_swz, Cdst, p.strideC, p.ldc, C0, R0, 0, 0);
-      else flush(s_swz, p.Ct, p.strideCt, p.ldct, C0, R0, p.n_valid, p.m_valid);
-      __syncthreads();
-    }
-    // 3. row-major image
-    if (SYM || p.C) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int cl = wc0 + j * 32 + l32;
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int rl = wr0 + i * 32 + 8 * g + 4 * hi + q;
-              const uint16_t bits = enc(acc[i][j][4 * g + q]);
-              if (!diag) {
-                *(uint16_t*)(smem + d_off(rl, cl * 2)) = bits;
-              } else if (cl >= rl) {
-                // diagonal tile: keep the upper half and reflect it, so the product is bit-symmetric
-                *(uint16_t*)(smem + d_off(rl, cl * 2)) = bits;
-                *(uint16_t*)(smem + d_off(cl, rl * 2)) = bits;
-              }
-            }
-          }
-        }
-      __syncthreads();
-      flush(d_swz, Cdst, p.strideC, p.ldc, R0, C0, p.m_valid, p.n_valid);
     }
   };
+  emit(I0{}, p.C);
+  if constexpr (SPLIT && MODE == MODE_SYRK2) emit(I1{}, p.C2);
+#endif
+}
 
-  store_all(p.C, lane);
-  if (SPLIT && MODE == MODE_SYRK2) {
-    __builtin_amdgcn_sched_barrier(0);
-    // low half of the bf16 split: acc <- acc - bf16(acc), stored the same way to C2
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] -= bf16_to_f32(bf16_bits(acc[i][j][e]));
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    int lane2 = lane;
-    asm volatile("" : "+v"(lane2));   // as above: keep the second copy's addresses out of the first copy
-    store_all(p.C2, lane2);
-  }
+// LDS stages of P and Q: all 160 KiB of a compute unit for one block of the 256 configuration, half of it for each of the
+// two blocks that the 128 configuration keeps resident
+constexpr int STAGES_P = 2, STAGES_Q = 3;
+
+template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+__global__ void __launch_bounds__(256, BM == 256 ? 1 : 2)
+ns_gemm_kernel(const GroupedGemmParams gp) {
+  static_assert(BM == BN && WM == WN && BM == 2 * WM, "square block tiles, four waves in a 2 x 2 arrangement");
+  ns_gemm_tile<BM, STAGES_P, STAGES_Q, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
 }
 
 // ---------------------------------------------------------------------------
@@ -888,11 +762,11 @@ long ns_gemm_tiles(int mode, const GemmParams& p) {
   return (long)p.batch * (sym ? (long)p.tilesM * (p.tilesM + 1) / 2 : (long)p.tilesM * p.tilesN);
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, bool SK = false>
+template <int BT, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, bool SK = false>
 static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
-  constexpr int NT = (BM / WM) * (BN / WN) * 64;
-  constexpr int SMEM = 2 * (BM + BN) * ROW_BYTES;
-  auto kern = ns_gemm_kernel<BM, BN, WM, WN, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
+  constexpr int NT = 256;
+  constexpr int SMEM = (STAGES_P + STAGES_Q) * BT * ROW_BYTES;
+  auto kern = ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
   // the dynamic-LDS limit is an attribute of the function on ONE device: set it once per device and instantiation
   // (the call is idempotent, so two threads that race on the first launch only repeat it)
   static std::atomic<bool> attr_set[64];
@@ -912,39 +786,39 @@ static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int F16>
+template <int BT, int F16>
 static hipError_t launch_cfg(int mode, bool split, bool final_, const GroupedGemmParams& p, hipStream_t s) {
   if (F16 && split) return hipErrorInvalidValue;
   if constexpr (F16 == 2) {
     if (mode != MODE_BX || final_) return hipErrorInvalidValue;
-    return p.g[0].E ? launch_one<BM, BN, WM, WN, MODE_BX, false, false, true, 2>(p, s)
-                    : launch_one<BM, BN, WM, WN, MODE_BX, false, false, false, 2>(p, s);
+    return p.g[0].E ? launch_one<BT, MODE_BX, false, false, true, 2>(p, s)
+                    : launch_one<BT, MODE_BX, false, false, false, 2>(p, s);
   } else {
     switch (mode) {
       case MODE_SYRK:
-        return launch_one<BM, BN, WM, WN, MODE_SYRK, false, false, true, F16>(p, s);
+        return launch_one<BT, MODE_SYRK, false, false, true, F16>(p, s);
       case MODE_SYRKT:
-        return launch_one<BM, BN, WM, WN, MODE_SYRKT, false, false, true, F16>(p, s);
+        return launch_one<BT, MODE_SYRKT, false, false, true, F16>(p, s);
       case MODE_SYRK2:
         if constexpr (!F16) {
-          if (split) return launch_one<BM, BN, WM, WN, MODE_SYRK2, true, false>(p, s);
+          if (split) return launch_one<BT, MODE_SYRK2, true, false>(p, s);
         }
-        return launch_one<BM, BN, WM, WN, MODE_SYRK2, false, false, true, F16>(p, s);
+        return launch_one<BT, MODE_SYRK2, false, false, true, F16>(p, s);
       case MODE_BX:
         if constexpr (!F16) {
           if (split) {
             if (p.g[0].E)
-              return final_ ? launch_one<BM, BN, WM, WN, MODE_BX, true, true>(p, s)
-                            : launch_one<BM, BN, WM, WN, MODE_BX, true, false>(p, s);
-            return final_ ? launch_one<BM, BN, WM, WN, MODE_BX, true, true, false>(p, s)
-                          : launch_one<BM, BN, WM, WN, MODE_BX, true, false, false>(p, s);
+              return final_ ? launch_one<BT, MODE_BX, true, true>(p, s)
+                            : launch_one<BT, MODE_BX, true, false>(p, s);
+            return final_ ? launch_one<BT, MODE_BX, true, true, false>(p, s)
+                          : launch_one<BT, MODE_BX, true, false, false>(p, s);
           }
         }
         if (p.g[0].E)
-          return final_ ? launch_one<BM, BN, WM, WN, MODE_BX, false, true, true, F16>(p, s)
-                        : launch_one<BM, BN, WM, WN, MODE_BX, false, false, true, F16>(p, s);
-        return final_ ? launch_one<BM, BN, WM, WN, MODE_BX, false, true, false, F16>(p, s)
-                      : launch_one<BM, BN, WM, WN, MODE_BX, false, false, false, F16>(p, s);
+          return final_ ? launch_one<BT, MODE_BX, false, true, true, F16>(p, s)
+                        : launch_one<BT, MODE_BX, false, false, true, F16>(p, s);
+        return final_ ? launch_one<BT, MODE_BX, false, true, false, F16>(p, s)
+                      : launch_one<BT, MODE_BX, false, false, false, F16>(p, s);
     }
     return hipErrorInvalidValue;
   }
@@ -954,9 +828,9 @@ static hipError_t launch_cfg(int mode, bool split, bool final_, const GroupedGem
 template <int F16>
 static hipError_t launch_ksplit(int mode, const GroupedGemmParams& p, hipStream_t s) {
   switch (mode) {
-    case MODE_SYRK: return launch_one<128, 128, 64, 64, MODE_SYRK, false, false, true, F16, true>(p, s);
-    case MODE_SYRKT: return launch_one<128, 128, 64, 64, MODE_SYRKT, false, false, true, F16, true>(p, s);
-    case MODE_SYRK2: return launch_one<128, 128, 64, 64, MODE_SYRK2, false, false, true, F16, true>(p, s);
+    case MODE_SYRK: return launch_one<128, MODE_SYRK, false, false, true, F16, true>(p, s);
+    case MODE_SYRKT: return launch_one<128, MODE_SYRKT, false, false, true, F16, true>(p, s);
+    case MODE_SYRK2: return launch_one<128, MODE_SYRK2, false, false, true, F16, true>(p, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1000,14 +874,14 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
     return launch_ksplit<0>(mode, gp, stream);
   }
   if (f16 == 1) {
-    if (tile == 256) return launch_cfg<256, 256, 128, 64, 1>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 128, 64, 64, 1>(mode, split, final_, gp, stream);
+    if (tile == 256) return launch_cfg<256, 1>(mode, split, final_, gp, stream);
+    if (tile == 128) return launch_cfg<128, 1>(mode, split, final_, gp, stream);
   } else if (f16 == 2) {
-    if (tile == 256) return launch_cfg<256, 256, 128, 64, 2>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 128, 64, 64, 2>(mode, split, final_, gp, stream);
+    if (tile == 256) return launch_cfg<256, 2>(mode, split, final_, gp, stream);
+    if (tile == 128) return launch_cfg<128, 2>(mode, split, final_, gp, stream);
   } else if (f16 == 0) {
-    if (tile == 256) return launch_cfg<256, 256, 128, 64, 0>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 128, 64, 64, 0>(mode, split, final_, gp, stream);
+    if (tile == 256) return launch_cfg<256, 0>(mode, split, final_, gp, stream);
+    if (tile == 128) return launch_cfg<128, 0>(mode, split, final_, gp, stream);
   }
   return hipErrorInvalidValue;
 }
