@@ -193,22 +193,44 @@ hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const Grouped
                       [&] { return launch_ns_gemm_grouped(tile, mode, split, final_, g, stream, f16); });
 }
 
-// One product over all problems of a 256-tile launch.  When the last round of the grid would hold only a few tiles, the
-// full rounds run as they are and the tiles of the last round are handed, as four 128x128 quadrants each, to the small
-// configuration: a quarter of the time per block instead of a whole round for a few tiles.  The small configuration
-// runs at about half the rate of the large one, so this pays for at most QUARTER_MAX_TAIL tiles (measured: a tail of
-// 160 tiles on the depth-16 set costs 83 us quartered against 57 us as it is; tails of 16 and 128 tiles of single
-// 8192x8192 and 4096x14336 matrices: 10.33 -> 9.80 ms and 4.58 -> 4.44 ms per call); a launch smaller than one round
-// is quartered as a whole up to QUARTER_MAX_ALONE tiles.  ARCHSCALE_MUON_QUARTER=0 switches it off.
-constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_ALONE = 176;
+// One product over all problems of a launch, with tiles handed to the next smaller configuration (four quadrants each)
+// where the larger one would leave the chip idle.  The sums of an element are the same in every configuration.
+//
+// Tiles of 256, more than one round (256 compute units) of them: the full rounds run as they are, a last round of at most
+// QUARTER_MAX_TAIL tiles is quartered: a quarter of the time per block instead of a whole round for a few tiles (measured: a
+// tail of 160 tiles on the depth-16 set costs 83 us quartered against 57 us as it is; tails of 16 and 128 tiles of single
+// 8192x8192 and 4096x14336 matrices: 10.33 -> 9.80 ms and 4.58 -> 4.44 ms per call).
+// Less than one round: as tiles of 256 the launch takes as long as its longest tile; quartered, the tiles spread over the
+// chip, at about 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
+// (208 tiles of 2816 and 1024 k-values, five fp32 EMA-Muon products) the step takes 1250 us quartered, 1318 as it is; at 0.625
+// (160 equal tiles, power iteration over 16 x 1024 x 2816) 337 against 317 us.
+//
+// Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
+// a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
+// 1023 286 -> 198, 1500 x 2000 (78 tiles) 268 -> 241; 136 tiles: the fp32 decoder of width 384 284 -> 262, but 2048 x 8192
+// 709 -> 747; 192 tiles: 3001 x 1023 198 -> 208.
+// ARCHSCALE_MUON_QUARTER=0 switches all of it off.
+constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
+constexpr double QUARTER_LOAD = 0.6;
 hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream,
                          double fa, double fi, int f16) {
   const bool enabled = env_switches().quarter;
   const int total = gp.tile_start[gp.n_groups];
-  const int round = 256;
-  const int full = total / round * round, tail = total - full;
-  if (!enabled || tile != 256 || tail == 0 || tail > (full > 0 ? QUARTER_MAX_TAIL : QUARTER_MAX_ALONE))
-    return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+  double all = 0.0, longest = 0.0;   // k-values of all tiles, of the longest one
+  for (int i = 0; i < gp.n_groups; ++i) {
+    all += (double)(gp.tile_start[i + 1] - gp.tile_start[i]) * gp.g[i].K;
+    longest = std::max(longest, (double)gp.g[i].K);
+  }
+  int full = 0;
+  if (tile == 256) {
+    const int round = 256;
+    full = total / round * round;
+    const int tail = total - full;
+    if (!enabled || tail == 0 || (full > 0 ? tail > QUARTER_MAX_TAIL : all > QUARTER_LOAD * round * longest))
+      return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+  } else {
+    if (!enabled || tile != 128 || split || total > (longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT)) return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+  }
   const double share = (double)full / total;
   if (full > 0) {
     GroupedGemmParams m = gp;
@@ -230,7 +252,7 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     q.tile_start[q.n_groups + 1] = q.tile_start[q.n_groups] + 4 * (e - f);
     ++q.n_groups;
   }
-  return timed_gemm(128, mode, split, final_, q, stream, fa * (1.0 - share), fi * (1.0 - share), f16);
+  return timed_gemm(tile / 2, mode, split, final_, q, stream, fa * (1.0 - share), fi * (1.0 - share), f16);
 }
 
 }  // namespace
@@ -914,23 +936,58 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   __bf16* Ap = (__bf16*)ws;
   __bf16* Cp = (__bf16*)(ws + round_up((long)batch * Np * Kp * 2, 256));
   __bf16* Dp = (__bf16*)((char*)Cp + round_up((long)batch * Np * Np * 2, 256));
-  hipError_t e = launch_layout(a_dev, MUON_DTYPE_BF16, 0, a_batch_stride, lda, batch, n, k, nullptr, Ap,
-                               (long)Np * Kp, Kp, Np, Kp, nullptr, 0, 0, stream);
-  if (e != hipSuccess) return (int)e;
-  if (c_dev) {
+  // A tensor goes through the workspace only where the kernel cannot use it as it lies: extents that need padding, rows
+  // that are not 16-byte aligned (a copy of the loader is 16 bytes), row panels past the loader's 32-bit offsets, or a
+  // result that overlaps an operand (blocks would overwrite what others still read).  2048 x 5632: the copies were 17 of
+  // 132 us; with quartered tiles the call takes 39.
+  auto in_place = [&](const void* t, int64_t bstride, int ld) {
+    return ((uintptr_t)t & 15) == 0 && ld % 8 == 0 && (batch == 1 || (bstride >= 0 && bstride % 8 == 0)) && ld < (1 << 22);
+  };
+  auto overlaps = [&](const void* t, int64_t bstride, int rows, int cols, int ld) {
+    auto last = [&](int64_t bs, long r, long l, long c) { return 2 * ((size_t)(batch - 1) * bs + (size_t)(r - 1) * l + c); };
+    const uintptr_t t0 = (uintptr_t)t, t1 = t0 + last(bstride, rows, ld, cols);
+    const uintptr_t d0 = (uintptr_t)d_dev, d1 = d0 + last(d_batch_stride, n, ldd, n);
+    return t0 < d1 && d0 < t1;
+  };
+  const bool a_here = n == Np && k == Kp && in_place(a_dev, a_batch_stride, lda);
+  const bool c_here = c_dev && n == Np && in_place(c_dev, c_batch_stride, ldc);
+  const bool d_here = n == Np && in_place(d_dev, d_batch_stride, ldd) && (batch == 1 || d_batch_stride >= (int64_t)(n - 1) * ldd + n) &&
+                      !(a_here && overlaps(a_dev, a_batch_stride, n, k, lda)) &&
+                      !(c_here && overlaps(c_dev, c_batch_stride, n, n, ldc));
+  hipError_t e;
+  GemmParams g = {};
+  g.batch = batch;
+  if (a_here) {
+    g.P = (const __bf16*)a_dev; g.strideP = a_batch_stride; g.ldp = lda;
+  } else {
+    e = launch_layout(a_dev, MUON_DTYPE_BF16, 0, a_batch_stride, lda, batch, n, k, nullptr, Ap,
+                      (long)Np * Kp, Kp, Np, Kp, nullptr, 0, 0, stream);
+    if (e != hipSuccess) return (int)e;
+    g.P = Ap; g.strideP = (long)Np * Kp; g.ldp = Kp;
+  }
+  g.Q = g.P; g.strideQ = g.strideP; g.ldq = g.ldp; g.K = Kp;
+  if (c_here) {
+    g.E = (const __bf16*)c_dev; g.strideE = c_batch_stride; g.lde = ldc;
+  } else if (c_dev) {
     e = launch_layout(c_dev, MUON_DTYPE_BF16, 0, c_batch_stride, ldc, batch, n, n, nullptr, Cp, (long)Np * Np, Np, Np,
                       Np, nullptr, 0, 0, stream);
     if (e != hipSuccess) return (int)e;
+    g.E = Cp; g.strideE = (long)Np * Np; g.lde = Np;
   }
-  GemmParams g = {};
-  g.batch = batch;
-  g.P = Ap; g.Q = Ap; g.strideP = g.strideQ = (long)Np * Kp; g.ldp = g.ldq = Kp; g.K = Kp;
   g.tilesM = g.tilesN = Np / tile;
-  g.C = Dp; g.strideC = (long)Np * Np; g.ldc = Np;
+  if (d_here) { g.C = (__bf16*)d_dev; g.strideC = d_batch_stride; g.ldc = ldd; }
+  else { g.C = Dp; g.strideC = (long)Np * Np; g.ldc = Np; }
   g.alpha = alpha; g.beta = c_dev ? beta : 0.f;
-  g.E = Cp; g.strideE = (long)Np * Np; g.lde = Np;
-  e = launch_ns_gemm(tile, c_dev ? MODE_SYRK2 : MODE_SYRK, false, false, g, stream);
-  if (e != hipSuccess) return (int)e;
+  const int mode = c_dev ? MODE_SYRK2 : MODE_SYRK;
+  const long tiles = ns_gemm_tiles(mode, g);
+  if (tiles > 0x1ffffff0L) return MUON_E_UNSUPPORTED;
+  GroupedGemmParams gp = {};
+  gp.n_groups = 1;
+  gp.g[0] = g;
+  gp.tile_start[1] = (int)tiles;
+  e = launch_rounds(tile, mode, false, false, gp, stream, (double)batch * n * n * k,
+                    (double)batch * 2.0 * tile * tile * sym_tiles_issued(Np / tile) * Kp, 0);
+  if (e != hipSuccess || d_here) return (int)e;
   return (int)launch_unpad_copy(Dp, (long)Np * Np, Np, d_dev, d_batch_stride, ldd, batch, n, n, stream);
 }
 
@@ -1090,10 +1147,12 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
   auto gram = [&](auto&& src_of, auto&& k_of, auto&& dst_of, auto&& scale_of) -> int {
     for (int tile : {256, 128}) {
       GroupedGemmParams gp = {};
+      double fa = 0.0, fi = 0.0;
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
-        hipError_t err = launch_ns_gemm_grouped(tile, MODE_SYRK, false, false, gp, stream);
+        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, fa, fi, 0);
         gp = GroupedGemmParams{};
+        fa = fi = 0.0;
         return err;
       };
       for (const Prob& P : pr) {
@@ -1114,6 +1173,8 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
         gp.g[gp.n_groups] = g;
         gp.tile_start[gp.n_groups + 1] = gp.tile_start[gp.n_groups] + (int)tiles;
         ++gp.n_groups;
+        fa += (double)P.q.batch * pl.m * pl.m * K;
+        fi += (double)P.q.batch * 2.0 * tile * tile * sym_tiles_issued(pl.Mp / tile) * K;
       }
       if ((e = flush()) != hipSuccess) return (int)e;
     }

@@ -52,8 +52,8 @@ struct GemmParams {
 // argument (about 1.5 KiB).
 constexpr int MAX_GROUPS = 8;
 // Quarter mode: the blocks of the launch are the four half-size tiles of each tile of a 2x coarser enumeration
-// (tilesM, tilesN count the fine tiles; block 4q + s is quadrant s of coarse tile qt_first + q).  It lets the 128x128
-// configuration finish the last, partly filled round of a 256x256 launch.
+// (tilesM, tilesN count the fine tiles; block 4q + s is quadrant s of coarse tile qt_first + q).  It lets a smaller
+// configuration take over where the larger one would leave the chip idle.
 struct GroupedGemmParams {
   int n_groups;
   int quarter;
@@ -64,7 +64,7 @@ struct GroupedGemmParams {
 // number of block tiles of one problem
 long ns_gemm_tiles(int mode, const GemmParams& p);
 
-// tile: 256 (256x256 block tile, 8 waves) or 128 (128x128, 4 waves)
+// tile: side of the block tile, 256, 128 or 64 (four waves each; 64 without the hi+lo pair)
 // f16: 0 = the workspace matrices of the launch are bfloat16; 1 = IEEE half (see GemmParams::out_shift), not with split;
 // 2 = bfloat16 operands, IEEE-half result (MODE_BX, not the final launch)
 // ksplit: some problem of the launch has GemmParams::ksplit > 1 (symmetric modes, tile 128, no hi+lo pair)

@@ -85,6 +85,9 @@ __device__ __forceinline__ int kmaj_swz(int k) {
   return ROWS >= 128 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (((k >> 1) & 1) << 2) | (((k >> 3) & 1) << 1);
 }
 
+// consecutive tiles of a launch that go to one XCD (see the kernel); the grid is a multiple of eight runs
+__host__ __device__ constexpr int xcd_run(int tiles) { return tiles < 256 ? (tiles + 7) / 8 : 32; }
+
 // f(0), f(1), ... f(N - 1) with the index as a compile-time constant
 template <class F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
@@ -186,9 +189,11 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // ---- block -> (problem, matrix, tile).  Workgroups are dealt round-robin to the 8 XCDs; runs of 32
   // consecutive logical tiles (neighbouring tiles of one matrix: shared operand panels) are kept on ONE
   // XCD, i.e. in one L2, and successive runs go to successive XCDs so that long and short tiles of a
-  // grouped launch spread evenly over the chip.  The grid is a multiple of 8*32.
+  // grouped launch spread evenly over the chip.  A launch of fewer than 8 * 32 tiles is dealt out in eight shorter runs:
+  // runs of 32 would leave whole XCDs without work.
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int logical = (((slot >> 5) << 3) + xcd) * 32 + (slot & 31);
+  const int run = xcd_run(gp.tile_start[gp.n_groups]);
+  const int logical = ((slot / run) * 8 + xcd) * run + slot % run;
   if (logical >= gp.tile_start[gp.n_groups]) return;
   int grp = 0;
   while (grp + 1 < gp.n_groups && logical >= gp.tile_start[grp + 1]) ++grp;
@@ -743,15 +748,23 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 #endif
 }
 
-// LDS stages of P and Q: all 160 KiB of a compute unit for one block of the 256 configuration, half of it for each of the
-// two blocks that the 128 configuration keeps resident
-constexpr int STAGES_P = 2, STAGES_Q = 3;
+// Configurations: block tile, LDS stages of P and Q, blocks that a compute unit holds.
+//   256       all 160 KiB of LDS for one block
+//   128       half of it for each of two blocks
+//   128 deep  144 KiB for a block that has its compute unit to itself (a launch that gives no unit a second one): with two
+//             stages and nothing else resident, a k-tile waits for its copies
+//   64        launches that cannot occupy the chip with tiles of 128: latency bound, so as many stages as two blocks leave room for
+enum { CFG_256, CFG_128, CFG_128_DEEP, CFG_64 };
+template <int CFG> struct Config;
+template <> struct Config<CFG_256> { static constexpr int BT = 256, SP = 2, SQ = 3, BLOCKS = 1; };
+template <> struct Config<CFG_128> { static constexpr int BT = 128, SP = 2, SQ = 3, BLOCKS = 2; };
+template <> struct Config<CFG_128_DEEP> { static constexpr int BT = 128, SP = 4, SQ = 5, BLOCKS = 1; };
+template <> struct Config<CFG_64> { static constexpr int BT = 64, SP = 4, SQ = 5, BLOCKS = 2; };
 
-template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
-__global__ void __launch_bounds__(256, BM == 256 ? 1 : 2)
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+__global__ void __launch_bounds__(256, Config<CFG>::BLOCKS)
 ns_gemm_kernel(const GroupedGemmParams gp) {
-  static_assert(BM == BN && WM == WN && BM == 2 * WM, "square block tiles, four waves in a 2 x 2 arrangement");
-  ns_gemm_tile<BM, STAGES_P, STAGES_Q, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
+  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
 }
 
 // ---------------------------------------------------------------------------
@@ -762,11 +775,11 @@ long ns_gemm_tiles(int mode, const GemmParams& p) {
   return (long)p.batch * (sym ? (long)p.tilesM * (p.tilesM + 1) / 2 : (long)p.tilesM * p.tilesN);
 }
 
-template <int BT, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, bool SK = false>
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, bool SK = false>
 static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   constexpr int NT = 256;
-  constexpr int SMEM = (STAGES_P + STAGES_Q) * BT * ROW_BYTES;
-  auto kern = ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
+  constexpr int SMEM = (Config<CFG>::SP + Config<CFG>::SQ) * Config<CFG>::BT * ROW_BYTES;
+  auto kern = ns_gemm_kernel<CFG, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
   // the dynamic-LDS limit is an attribute of the function on ONE device: set it once per device and instantiation
   // (the call is idempotent, so two threads that race on the first launch only repeat it)
   static std::atomic<bool> attr_set[64];
@@ -781,44 +794,45 @@ static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   }
   const long tiles = gp.tile_start[gp.n_groups];
   if (tiles <= 0) return hipSuccess;
-  const long grid = (tiles + 255) / 256 * 256;
+  const long unit = 8L * xcd_run((int)tiles);
+  const long grid = (tiles + unit - 1) / unit * unit;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NT), SMEM, stream, gp);
   return hipGetLastError();
 }
 
-template <int BT, int F16>
+template <int CFG, int F16>
 static hipError_t launch_cfg(int mode, bool split, bool final_, const GroupedGemmParams& p, hipStream_t s) {
-  if (F16 && split) return hipErrorInvalidValue;
+  if ((F16 || CFG == CFG_64) && split) return hipErrorInvalidValue;
   if constexpr (F16 == 2) {
     if (mode != MODE_BX || final_) return hipErrorInvalidValue;
-    return p.g[0].E ? launch_one<BT, MODE_BX, false, false, true, 2>(p, s)
-                    : launch_one<BT, MODE_BX, false, false, false, 2>(p, s);
+    return p.g[0].E ? launch_one<CFG, MODE_BX, false, false, true, 2>(p, s)
+                    : launch_one<CFG, MODE_BX, false, false, false, 2>(p, s);
   } else {
     switch (mode) {
       case MODE_SYRK:
-        return launch_one<BT, MODE_SYRK, false, false, true, F16>(p, s);
+        return launch_one<CFG, MODE_SYRK, false, false, true, F16>(p, s);
       case MODE_SYRKT:
-        return launch_one<BT, MODE_SYRKT, false, false, true, F16>(p, s);
+        return launch_one<CFG, MODE_SYRKT, false, false, true, F16>(p, s);
       case MODE_SYRK2:
-        if constexpr (!F16) {
-          if (split) return launch_one<BT, MODE_SYRK2, true, false>(p, s);
+        if constexpr (!F16 && CFG != CFG_64) {
+          if (split) return launch_one<CFG, MODE_SYRK2, true, false>(p, s);
         }
-        return launch_one<BT, MODE_SYRK2, false, false, true, F16>(p, s);
+        return launch_one<CFG, MODE_SYRK2, false, false, true, F16>(p, s);
       case MODE_BX:
-        if constexpr (!F16) {
+        if constexpr (!F16 && CFG != CFG_64) {
           if (split) {
             if (p.g[0].E)
-              return final_ ? launch_one<BT, MODE_BX, true, true>(p, s)
-                            : launch_one<BT, MODE_BX, true, false>(p, s);
-            return final_ ? launch_one<BT, MODE_BX, true, true, false>(p, s)
-                          : launch_one<BT, MODE_BX, true, false, false>(p, s);
+              return final_ ? launch_one<CFG, MODE_BX, true, true>(p, s)
+                            : launch_one<CFG, MODE_BX, true, false>(p, s);
+            return final_ ? launch_one<CFG, MODE_BX, true, true, false>(p, s)
+                          : launch_one<CFG, MODE_BX, true, false, false>(p, s);
           }
         }
         if (p.g[0].E)
-          return final_ ? launch_one<BT, MODE_BX, false, true, true, F16>(p, s)
-                        : launch_one<BT, MODE_BX, false, false, true, F16>(p, s);
-        return final_ ? launch_one<BT, MODE_BX, false, true, false, F16>(p, s)
-                      : launch_one<BT, MODE_BX, false, false, false, F16>(p, s);
+          return final_ ? launch_one<CFG, MODE_BX, false, true, true, F16>(p, s)
+                        : launch_one<CFG, MODE_BX, false, false, true, F16>(p, s);
+        return final_ ? launch_one<CFG, MODE_BX, false, true, false, F16>(p, s)
+                      : launch_one<CFG, MODE_BX, false, false, false, F16>(p, s);
     }
     return hipErrorInvalidValue;
   }
@@ -828,9 +842,9 @@ static hipError_t launch_cfg(int mode, bool split, bool final_, const GroupedGem
 template <int F16>
 static hipError_t launch_ksplit(int mode, const GroupedGemmParams& p, hipStream_t s) {
   switch (mode) {
-    case MODE_SYRK: return launch_one<128, MODE_SYRK, false, false, true, F16, true>(p, s);
-    case MODE_SYRKT: return launch_one<128, MODE_SYRKT, false, false, true, F16, true>(p, s);
-    case MODE_SYRK2: return launch_one<128, MODE_SYRK2, false, false, true, F16, true>(p, s);
+    case MODE_SYRK: return launch_one<CFG_128, MODE_SYRK, false, false, true, F16, true>(p, s);
+    case MODE_SYRKT: return launch_one<CFG_128, MODE_SYRKT, false, false, true, F16, true>(p, s);
+    case MODE_SYRK2: return launch_one<CFG_128, MODE_SYRK2, false, false, true, F16, true>(p, s);
   }
   return hipErrorInvalidValue;
 }
@@ -873,16 +887,21 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
     if (f16 == 1) return launch_ksplit<1>(mode, gp, stream);
     return launch_ksplit<0>(mode, gp, stream);
   }
-  if (f16 == 1) {
-    if (tile == 256) return launch_cfg<256, 1>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 1>(mode, split, final_, gp, stream);
-  } else if (f16 == 2) {
-    if (tile == 256) return launch_cfg<256, 2>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 2>(mode, split, final_, gp, stream);
-  } else if (f16 == 0) {
-    if (tile == 256) return launch_cfg<256, 0>(mode, split, final_, gp, stream);
-    if (tile == 128) return launch_cfg<128, 0>(mode, split, final_, gp, stream);
-  }
+  // The deep form where every block finds a unit of its own and the reductions are long: 3001 x 1023 302 -> 286 us, 1500 x 2000
+  // 290 -> 270, a symmetric product of 2048 x 5632 47 -> 41; filling four stages costs reductions of 640 and less 1 to 4 %.
+  bool deep = tile == 128 && gp.tile_start[gp.n_groups] <= 256;
+  for (int i = 0; i < gp.n_groups; ++i) deep = deep && gp.g[i].K >= 1024;
+  auto by_storage = [&](auto cfg_) -> hipError_t {
+    constexpr int CFG = decltype(cfg_)::value;
+    if (f16 == 1) return launch_cfg<CFG, 1>(mode, split, final_, gp, stream);
+    if (f16 == 2) return launch_cfg<CFG, 2>(mode, split, final_, gp, stream);
+    if (f16 == 0) return launch_cfg<CFG, 0>(mode, split, final_, gp, stream);
+    return hipErrorInvalidValue;
+  };
+  if (tile == 256) return by_storage(std::integral_constant<int, CFG_256>{});
+  if (tile == 128 && deep) return by_storage(std::integral_constant<int, CFG_128_DEEP>{});
+  if (tile == 128) return by_storage(std::integral_constant<int, CFG_128>{});
+  if (tile == 64) return by_storage(std::integral_constant<int, CFG_64>{});
   return hipErrorInvalidValue;
 }
 

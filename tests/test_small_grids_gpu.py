@@ -1,0 +1,61 @@
+"""Launches too small for the large tiles: the smaller configurations give the bits of the larger ones, and symmetric products that
+read and write the caller's tensors directly."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (64, 64), (65, 130), (128, 384), (200, 900), (513, 520), (640, 1700), (1030, 1100), (1024, 3001)])
+@pytest.mark.parametrize("prec", ["bf16", "f16"])
+def test_matrix_alone_and_in_a_large_batch(gpu_device, m, n, prec):
+    """Alone: tiles of 64 or the deep pipeline; in the batch: the tiles of 128 and 256 that fill the chip."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    batch = 20 if m > 512 else 48
+    g = torch.Generator().manual_seed(m * 10000 + n)
+    x = (torch.randn(batch, m, n, generator=g) * 1e-3).to(torch.bfloat16).to(gpu_device)
+    for t in (x, x.mT.contiguous()):
+        all_ = ns.newton_schulz(t, prec=prec)
+        for i in (0, batch - 1):
+            assert torch.equal(ns.newton_schulz(t[i], prec=prec), all_[i])
+
+
+@pytest.mark.parametrize("n,k", [(128, 64), (256, 1024), (384, 320), (1280, 1024)])
+@pytest.mark.parametrize("addend", [False, True])
+def test_symmetric_product_in_place_and_through_the_workspace(gpu_device, n, k, addend):
+    """Aligned operands are used as they lie.  The same product from an unaligned view, into a strided result and over its own
+    operand goes through the workspace and gives the same bits."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator().manual_seed(n + k)
+    a = (torch.randn(2, n, k, generator=g)).to(torch.bfloat16).to(gpu_device)
+    c = (torch.randn(n, n, generator=g)).to(torch.bfloat16).to(gpu_device)
+    c = torch.triu(c) + torch.triu(c, 1).T
+
+    def product(t, cc=c, out=None):
+        return ns._syrk(t, cc if addend else None, 1.5, -0.75 if addend else 0.0, out)
+
+    got = product(a[0])
+    a64 = a[0].double()
+    want = 1.5 * (a64 @ a64.T) - (0.75 * c.double() if addend else 0)
+    mag = 1.5 * (a64.abs() @ a64.abs().T) + (0.75 * c.double().abs() if addend else 0)
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + mag * (k + 2) * 2.0 ** -24).all())
+    for pad, shift in ((8, 8), (8, 0), (3, 1)):      # rows and start aligned to 16 bytes, and not
+        wide = torch.zeros(n, k + pad, dtype=torch.bfloat16, device=gpu_device)
+        wide[:, shift:shift + k] = a[0]
+        cw = torch.zeros(n, n + pad, dtype=torch.bfloat16, device=gpu_device)
+        cw[:, shift:shift + n] = c
+        dw = torch.full((n, n + pad), 7.0, dtype=torch.bfloat16, device=gpu_device)
+        assert torch.equal(product(wide[:, shift:shift + k], cw[:, shift:shift + n], dw[:, shift:shift + n]), got)
+        rest = torch.cat([dw[:, :shift], dw[:, shift + n:]], 1)
+        assert bool((rest == 7.0).all())             # nothing beside the result is touched
+    if addend:
+        cc = c.clone()
+        assert torch.equal(product(a[0], cc, cc), got)          # over its own addend
+    else:
+        assert torch.equal(ns._syrk(a, None, 1.5, 0.0, None)[0], got)
+        if n == k:
+            t = a[0].clone()
+            assert torch.equal(product(t, out=t), got)
+    sq = torch.randn(n, n, generator=g).to(torch.bfloat16).to(gpu_device)
+    ref = ns._syrk(sq, None, 1.0, 0.0, None)
+    assert torch.equal(ns._syrk(sq, None, 1.0, 0.0, sq), ref)   # over its own operand
