@@ -466,24 +466,39 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   for (const NsProblem& P : pr)
     if (P.sk_counter && (e = launch_zero_i32(P.sk_counter, (long)P.q.batch * P.pl.sk_quadrants, stream)) != hipSuccess) return (int)e;
   // normalise into X^T (long side first): a wide input is transposed on the way, a tall one is copied as it is
-  for (int i = 0; i < n_problems && !fused; ++i) {
-    const NsProblem& P = pr[i];
-    const NsPlan& pl = P.pl;
-    const long xs = (long)pl.Mp * pl.Np;
-    const float* sc = !normalize ? nullptr : (P.defer ? P.pow2 : P.scale);   // null: copy unscaled
-    const int to_half = (f16 && !P.defer) ? 1 : 0;
-    if (normalize) {
-      e = launch_norm_scale(P.q.in, P.q.in_dtype, cast_first, P.q.in_batch_stride, P.q.in_ld, P.q.batch, P.q.rows,
-                            P.q.cols, eps, eps_mode, P.partial, P.scale, stream, P.defer ? P.pow2 : nullptr);
-      if (e != hipSuccess) return (int)e;
+  if (!fused) {
+    StageParams sp = {};
+    auto flush = [&]() -> hipError_t {
+      if (sp.n == 0) return hipSuccess;
+      const hipError_t err = launch_stage(sp, stream);
+      sp = StageParams{};
+      return err;
+    };
+    for (const NsProblem& P : pr) {
+      const NsPlan& pl = P.pl;
+      StageProblem q = {};
+      q.in = P.q.in; q.in_bstride = P.q.in_batch_stride; q.ld = P.q.in_ld;
+      q.rows = P.q.rows; q.cols = P.q.cols; q.batch = P.q.batch; q.cpm = pl.cpm;
+      q.partial = P.partial; q.scale = P.scale; q.pow2 = P.defer ? P.pow2 : nullptr;
+      q.dst = (uint16_t*)P.Xt[0]; q.d_bstride = (long)pl.Mp * pl.Np; q.ldd = pl.Mp;
+      q.transpose = P.tall ? 0 : 1;
+      q.d_rows = P.tall ? pl.Np : pl.Mp; q.d_cols = P.tall ? pl.Mp : pl.Np;
+      q.out_f16 = (f16 && !P.defer) ? 1 : 0;
+      q.out_shift = q.out_f16 ? P.sx : 0;
+      long sums, tiles;
+      if (!stage_blocks(q, &sums, &tiles)) return (int)hipErrorInvalidValue;
+      if (sp.n == STAGE_MAX || (sp.n > 0 && sp.in_dtype != P.q.in_dtype) || sp.sum_start[sp.n] + sums > 0x7ffffff0L ||
+          sp.tile_start[sp.n] + tiles > 0x7ffffff0L) {
+        if ((e = flush()) != hipSuccess) return (int)e;
+      }
+      sp.in_dtype = P.q.in_dtype; sp.cast_first = cast_first; sp.normalize = normalize ? 1 : 0;
+      sp.eps = eps; sp.eps_mode = eps_mode;
+      sp.p[sp.n] = q;
+      sp.sum_start[sp.n + 1] = sp.sum_start[sp.n] + (int)sums;
+      sp.tile_start[sp.n + 1] = sp.tile_start[sp.n] + (int)tiles;
+      ++sp.n;
     }
-    if (!P.tall)
-      e = launch_layout(P.q.in, P.q.in_dtype, cast_first, P.q.in_batch_stride, P.q.in_ld, P.q.batch, P.q.rows,
-                        P.q.cols, sc, nullptr, 0, 0, pl.Mp, pl.Np, P.Xt[0], xs, pl.Mp, stream, to_half, to_half ? P.sx : 0);
-    else
-      e = launch_layout(P.q.in, P.q.in_dtype, cast_first, P.q.in_batch_stride, P.q.in_ld, P.q.batch, P.q.rows,
-                        P.q.cols, sc, P.Xt[0], xs, pl.Mp, pl.Np, pl.Mp, nullptr, 0, 0, stream, to_half, to_half ? P.sx : 0);
-    if (e != hipSuccess) return (int)e;
+    if ((e = flush()) != hipSuccess) return (int)e;
   }
   // fused staging: momentum of every matrix, its bf16 update written unnormalised into X^T, norms from tile partials.
   // The matrices of ALL problems share launches (up to MOMG_MAX_MATS matrices of MOMG_MAX_CLS classes each): one

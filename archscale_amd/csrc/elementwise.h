@@ -27,11 +27,32 @@ struct MomentumCoef {
 hipError_t launch_momentum(const PreItem* items, const int32_t* prefix, int n_items, int total_chunks,
                            MomentumCoef c, hipStream_t stream);
 
-// per-matrix Frobenius norms of in[batch][rows][cols] -> scale[b] = 1/(|X|+eps) or 1/max(|X|,eps); with pow2 that
-// factor is split into pow2[b] (a power of two) times scale[b] (between 0.7 and 1.5)
-hipError_t launch_norm_scale(const void* in, int in_dtype, int cast_first, long in_bstride, int ld, int batch,
-                             int rows, int cols, float eps, int eps_mode, float* partial, float* scale,
-                             hipStream_t stream, float* pow2 = nullptr);
+// Staging of Newton-Schulz operands: per-matrix Frobenius norms and the scaled, padded, possibly transposed copy of every
+// matrix of up to STAGE_MAX batches, two launches in all (three where a matrix has more than STAGE_FOLD_MAX partial sums).
+//   dst = bf16(s * in), or half(2^out_shift * s * in), zero padded to d_rows x d_cols (multiples of 64), or its transpose
+//   normalize: f = 1 / (|in| + eps) or 1 / max(|in|, eps).  pow2 null: s = scale[b] = f.  Otherwise s = pow2[b], a power of
+//   two, and scale[b] = f / pow2[b] (between 0.7 and 1.5) is left to the reader of dst.  Not normalize: s = 1.
+constexpr int STAGE_MAX = 16;
+constexpr int STAGE_FOLD_MAX = 1024;
+struct StageProblem {
+  const void* in;
+  long in_bstride, d_bstride;
+  float *partial;        // [batch][cpm] sums of squares, one per MUON_CHUNK_ELEMS elements
+  float *scale, *pow2;   // [batch]
+  uint16_t* dst;
+  int ld, rows, cols, batch, cpm;
+  int ldd, d_rows, d_cols, transpose, out_f16, out_shift;
+};
+struct StageParams {
+  int n, in_dtype, cast_first, normalize, eps_mode;
+  float eps;
+  int32_t sum_start[STAGE_MAX + 1], tile_start[STAGE_MAX + 1];   // first block of problem i of the two launches
+  StageProblem p[STAGE_MAX];
+};
+static_assert(sizeof(StageParams) <= 4096, "kernel arguments are limited to 4 KiB");
+// blocks that a problem adds to the two launches; false: not a problem that the kernels take
+bool stage_blocks(const StageProblem& p, long* sum_blocks, long* tiles);
+hipError_t launch_stage(const StageParams& p, hipStream_t stream);
 
 // D = bf16(scale*in) in the input's orientation and T = its transpose (either may be null), both zero-padded to
 // d_rows x d_cols / d_cols x d_rows (multiples of 64); scale may be null (= 1).  tile_sumsq (optional): the sum of
@@ -84,13 +105,13 @@ struct MomGroupParams {
 static_assert(sizeof(MomGroupParams) <= 4096, "kernel arguments are limited to 4 KiB");
 int momentum_class_blocks(const MomClass& k, int linear);
 hipError_t launch_momentum_group(const MomGroupParams& p, hipStream_t stream);
-hipError_t launch_norm_scale_from_partials(const float* partial, int partials_per_mat, int batch, float eps, int eps_mode,
-                                           float* scale, hipStream_t stream);
-// the same for several batches in one launch: block b serves matrix b - mat_start[i] of batch i
+// scale[b] = 1 / (|X| + eps) or 1 / max(|X|, eps) of every matrix of several batches from partial sums of squares written by
+// another kernel: block b serves matrix b - mat_start[i] of batch i
 constexpr int NORMG_MAX = 16;
 struct NormGroup {
   const float* partial;   // [batch][per_mat]
   float* scale;           // [batch]
+  float* pow2;            // [batch], or null: the factor is split as for StageProblem
   int per_mat;
 };
 struct NormGroupParams {

@@ -203,11 +203,14 @@ hipError_t launch_momentum(const PreItem* items, const int32_t* prefix, int n_it
 // ---------------------------------------------------------------------------
 template <int DT, bool CAST_FIRST>
 __global__ void __launch_bounds__(EW_THREADS)
-sumsq_partial_kernel(const void* __restrict__ in, long batch_stride, int rows, int cols, int ld,
-                     int chunks_per_mat, float* __restrict__ partial) {
+stage_sumsq_kernel(const StageParams sp) {
   __shared__ float red[4];
-  const int b = blockIdx.y, chunk = blockIdx.x;
-  const char* base = (const char*)in + (size_t)b * batch_stride * sizeof(typename Elem<DT>::T);
+  const int pi = find_item(sp.sum_start, sp.n, blockIdx.x);
+  const StageProblem& q = sp.p[pi];
+  const int local = blockIdx.x - sp.sum_start[pi];
+  const int b = local / q.cpm, chunk = local - b * q.cpm;
+  const int rows = q.rows, cols = q.cols, ld = q.ld;
+  const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
   const long numel = (long)rows * cols;
   const long begin = (long)chunk * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < numel ? begin + MUON_CHUNK_ELEMS : numel;
@@ -233,30 +236,18 @@ sumsq_partial_kernel(const void* __restrict__ in, long batch_stride, int rows, i
     }
   }
   block_reduce<1>(s, red);
-  if (threadIdx.x == 0) partial[(size_t)b * chunks_per_mat + chunk] = s[0];
+  if (threadIdx.x == 0) q.partial[(size_t)b * q.cpm + chunk] = s[0];
 }
 
-__global__ void __launch_bounds__(EW_THREADS)
-norm_scale_kernel(const float* __restrict__ partial, int chunks_per_mat, float eps, int eps_mode,
-                  float* __restrict__ scale, float* __restrict__ pow2) {
-  __shared__ float red[4];
-  const int b = blockIdx.x;
-  float s[1] = {0.f};
-  for (int i = threadIdx.x; i < chunks_per_mat; i += EW_THREADS) s[0] += partial[(size_t)b * chunks_per_mat + i];
-  block_reduce<1>(s, red);
-  if (threadIdx.x == 0) {
-    const float n = sqrtf(s[0]);
-    const float sc = eps_mode == EPS_ADD ? 1.f / (n + eps) : 1.f / fmaxf(n, eps);
-    if (!pow2) {
-      scale[b] = sc;
-    } else {
-      // sc = pow2 * scale with pow2 a power of two (applied to the copy of the input, exactly) and scale in [0.7, 1.5]
-      const bool ok = sc > 0.f && sc < 3.0e38f;
-      const float p = ok ? exp2f(rintf(log2f(sc))) : sc;
-      pow2[b] = p;
-      scale[b] = ok ? sc / p : 1.f;
-    }
-  }
+// normalisation factor of a matrix from its sum of squares; with pow2 it is split into a power of two (applied to the copy
+// of the input, exactly) and a rest in [0.7, 1.5]
+__device__ __forceinline__ float2 norm_factor(float sumsq, float eps, int eps_mode, bool pow2) {
+  const float n = sqrtf(sumsq);
+  const float sc = eps_mode == EPS_ADD ? 1.f / (n + eps) : 1.f / fmaxf(n, eps);
+  if (!pow2) return make_float2(sc, 1.f);
+  const bool ok = sc > 0.f && sc < 3.0e38f;
+  const float p = ok ? exp2f(rintf(log2f(sc))) : sc;
+  return make_float2(ok ? sc / p : 1.f, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -264,26 +255,19 @@ norm_scale_kernel(const float* __restrict__ partial, int chunks_per_mat, float e
 //    both zero-padded to the tile multiples the GEMMs assume (replaces the
 //    X/(norm+eps), .mT and .contiguous() of newton_schulz_triton.py:358-366).
 // ---------------------------------------------------------------------------
+// one 64x64 tile (row tile ty, column tile tx) by one block; d_rows / d_cols are the padded extents (multiples of 64)
 template <int DT, bool CAST_FIRST>
-__global__ void __launch_bounds__(256)
-normalize_layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstride, int rows, int cols, int ld,
-                        const float* __restrict__ scale,
-                        uint16_t* __restrict__ D, long d_bstride, int ldd, int d_rows, int d_cols,
-                        uint16_t* __restrict__ T, long t_bstride, int ldt, int out_f16, int out_shift,
-                        float* __restrict__ tile_sumsq) {
-  // 64x64 tile; d_rows/d_cols are the padded extents (multiples of 64)
+__device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, int ty, int tx, int rows, int cols, int ld, float s,
+                                            uint16_t* D, int ldd, int d_rows, int d_cols, uint16_t* T, int ldt, int out_f16,
+                                            int out_shift, float* tile_sumsq) {
   __shared__ uint16_t tile[64][66];
   __shared__ float red[4];
   float ss[1] = {0.f};
-  const int b = blockIdx.z;
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  // the matrices of the batch: equally spaced from `in`, or (in == null) separate allocations listed in `ptrs`
-  const char* base = in ? (const char*)in + (size_t)b * in_bstride * sizeof(typename Elem<DT>::T) : (const char*)ptrs.p[b];
-  const float s = scale ? scale[b] : 1.f;
+  const int r0 = ty * 64, c0 = tx * 64;
   const float fs = __builtin_ldexpf(1.f, out_shift);
   const int tr = threadIdx.x >> 3;        // 0..31
   const int tc = (threadIdx.x & 7) * 8;   // 0..56
-  const bool vec = aligned16(base) && (ld % 8 == 0) && (!in || in_bstride % 8 == 0);
+  const bool vec = aligned16(base) && (ld % 8 == 0) && stride_ok;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int r = r0 + tr + h * 32, c = c0 + tc;
@@ -307,13 +291,12 @@ normalize_layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long
       u32x4 pk;
       pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
       pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      stream_store16(D + (size_t)b * d_bstride + (size_t)r * ldd + c, pk);
+      stream_store16(D + (size_t)r * ldd + c, pk);
     }
   }
   if (tile_sumsq) {   // sum of squares of what this block wrote (every block of the grid: one value per 64x64 tile)
     block_reduce<1>(ss, red);
-    if (threadIdx.x == 0)
-      tile_sumsq[((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = ss[0];
+    if (threadIdx.x == 0) *tile_sumsq = ss[0];
   }
   if (!T) return;
   __syncthreads();
@@ -328,28 +311,75 @@ normalize_layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long
       u32x4 pk;
       pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
       pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      stream_store16(T + (size_t)b * t_bstride + (size_t)c * ldt + r, pk);
+      stream_store16(T + (size_t)c * ldt + r, pk);
     }
   }
 }
 
-hipError_t launch_norm_scale(const void* in, int in_dtype, int cast_first, long in_bstride, int ld, int batch,
-                             int rows, int cols, float eps, int eps_mode, float* partial, float* scale,
-                             hipStream_t stream, float* pow2) {
-  const long numel = (long)rows * cols;
-  const int cpm = (int)((numel + MUON_CHUNK_ELEMS - 1) / MUON_CHUNK_ELEMS);
-  if (batch > 65535) return hipErrorInvalidValue;
-  dim3 g1(cpm, batch);
-#define ARCHSCALE_SS(DT, CF)                                                                                  \
-  hipLaunchKernelGGL((sumsq_partial_kernel<DT, CF>), g1, dim3(EW_THREADS), 0, stream, in, in_bstride, rows,   \
-                     cols, ld, cpm, partial)
-  if (in_dtype == DT_BF16) ARCHSCALE_SS(DT_BF16, false);
-  else if (cast_first) ARCHSCALE_SS(DT_F32, true);
-  else ARCHSCALE_SS(DT_F32, false);
-#undef ARCHSCALE_SS
-  hipLaunchKernelGGL(norm_scale_kernel, dim3(batch), dim3(EW_THREADS), 0, stream, partial, cpm, eps, eps_mode,
-                     scale, pow2);
-  return hipGetLastError();
+template <int DT, bool CAST_FIRST>
+__global__ void __launch_bounds__(256)
+normalize_layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstride, int rows, int cols, int ld,
+                        const float* __restrict__ scale,
+                        uint16_t* __restrict__ D, long d_bstride, int ldd, int d_rows, int d_cols,
+                        uint16_t* __restrict__ T, long t_bstride, int ldt, int out_f16, int out_shift,
+                        float* __restrict__ tile_sumsq) {
+  const int b = blockIdx.z;
+  // the matrices of the batch: equally spaced from `in`, or (in == null) separate allocations listed in `ptrs`
+  const char* base = in ? (const char*)in + (size_t)b * in_bstride * sizeof(typename Elem<DT>::T) : (const char*)ptrs.p[b];
+  layout_tile<DT, CAST_FIRST>(base, !in || in_bstride % 8 == 0, blockIdx.y, blockIdx.x, rows, cols, ld, scale ? scale[b] : 1.f,
+                              D ? D + (size_t)b * d_bstride : nullptr, ldd, d_rows, d_cols,
+                              T ? T + (size_t)b * t_bstride : nullptr, ldt, out_f16, out_shift,
+                              tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr);
+}
+
+// The copies of a staging launch.  Launch bound for all but the largest calls, hence one launch over all matrices and no
+// launch of its own for the norms: every block adds up its matrix's partial sums (at most STAGE_FOLD_MAX, from the cache;
+// in the order of norm_scale_groups_kernel) and the first block of a matrix stores the factor.  16 classes of a MuonBall
+// step with fused parameters: 48 launches of 250 us in all before.
+template <int DT, bool CAST_FIRST>
+__global__ void __launch_bounds__(256)
+stage_layout_kernel(const StageParams sp) {
+  __shared__ float red[4];
+  __shared__ float factor;
+  const int pi = find_item(sp.tile_start, sp.n, blockIdx.x);
+  const StageProblem& q = sp.p[pi];
+  const int tiles_x = q.d_cols / 64, tiles = tiles_x * (q.d_rows / 64);
+  const int local = blockIdx.x - sp.tile_start[pi];
+  const int b = local / tiles, t = local - b * tiles;
+  const int ty = t / tiles_x, tx = t - ty * tiles_x;
+  float s = 1.f;
+  if (sp.normalize) {
+    if (q.cpm <= STAGE_FOLD_MAX) {
+      float v[1] = {0.f};
+      for (int i = threadIdx.x; i < q.cpm; i += EW_THREADS) v[0] += q.partial[(size_t)b * q.cpm + i];
+      block_reduce<1>(v, red);
+      if (threadIdx.x == 0) {
+        const float2 f = norm_factor(v[0], sp.eps, sp.eps_mode, q.pow2 != nullptr);
+        factor = q.pow2 ? f.y : f.x;
+        if (t == 0) {
+          q.scale[b] = f.x;
+          if (q.pow2) q.pow2[b] = f.y;
+        }
+      }
+      __syncthreads();
+      s = factor;
+    } else {
+      s = q.pow2 ? q.pow2[b] : q.scale[b];
+    }
+  }
+  const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
+  uint16_t* dst = q.dst + (size_t)b * q.d_bstride;
+  layout_tile<DT, CAST_FIRST>(base, q.in_bstride % 8 == 0, ty, tx, q.rows, q.cols, q.ld, s, q.transpose ? nullptr : dst, q.ldd,
+                              q.d_rows, q.d_cols, q.transpose ? dst : nullptr, q.ldd, q.out_f16, q.out_shift, nullptr);
+}
+
+bool stage_blocks(const StageProblem& p, long* sum_blocks, long* tiles) {
+  if (!p.in || !p.dst || p.batch < 1 || p.batch > 65535 || p.rows < 1 || p.cols < 1) return false;
+  if (p.d_rows % 64 || p.d_cols % 64 || p.rows > p.d_rows || p.cols > p.d_cols || p.d_rows / 64 > 65535) return false;
+  if (p.cpm != ((long)p.rows * p.cols + MUON_CHUNK_ELEMS - 1) / MUON_CHUNK_ELEMS) return false;
+  *sum_blocks = (long)p.batch * p.cpm;
+  *tiles = (long)p.batch * (p.d_rows / 64) * (p.d_cols / 64);
+  return *sum_blocks < 0x7ffffff0L && *tiles < 0x7ffffff0L;
 }
 
 namespace {
@@ -603,15 +633,6 @@ hipError_t launch_momentum_group(const MomGroupParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// scale[b] from per-tile (or per-chunk) partial sums written by another kernel
-hipError_t launch_norm_scale_from_partials(const float* partial, int partials_per_mat, int batch, float eps, int eps_mode,
-                                           float* scale, hipStream_t stream) {
-  if (batch < 1 || partials_per_mat < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(norm_scale_kernel, dim3(batch), dim3(EW_THREADS), 0, stream, partial, partials_per_mat, eps, eps_mode,
-                     scale, (float*)nullptr);
-  return hipGetLastError();
-}
-
 __global__ void __launch_bounds__(EW_THREADS)
 norm_scale_groups_kernel(const NormGroupParams p, float eps, int eps_mode) {
   __shared__ float red[4];
@@ -622,8 +643,9 @@ norm_scale_groups_kernel(const NormGroupParams p, float eps, int eps_mode) {
   for (int t = threadIdx.x; t < g.per_mat; t += EW_THREADS) s[0] += g.partial[(size_t)b * g.per_mat + t];
   block_reduce<1>(s, red);
   if (threadIdx.x == 0) {
-    const float n = sqrtf(s[0]);
-    g.scale[b] = eps_mode == EPS_ADD ? 1.f / (n + eps) : 1.f / fmaxf(n, eps);
+    const float2 f = norm_factor(s[0], eps, eps_mode, g.pow2 != nullptr);
+    g.scale[b] = f.x;
+    if (g.pow2) g.pow2[b] = f.y;
   }
 }
 
@@ -632,6 +654,39 @@ hipError_t launch_norm_scale_groups(const NormGroupParams& p, float eps, int eps
   for (int i = 0; i < p.n; ++i)
     if (!p.g[i].partial || !p.g[i].scale || p.g[i].per_mat < 1 || p.mat_start[i + 1] <= p.mat_start[i]) return hipErrorInvalidValue;
   hipLaunchKernelGGL(norm_scale_groups_kernel, dim3(p.mat_start[p.n]), dim3(EW_THREADS), 0, stream, p, eps, eps_mode);
+  return hipGetLastError();
+}
+
+hipError_t launch_stage(const StageParams& p, hipStream_t stream) {
+  if (p.n < 1 || p.n > STAGE_MAX || p.sum_start[0] != 0 || p.tile_start[0] != 0) return hipErrorInvalidValue;
+  NormGroupParams ng = {};
+  for (int i = 0; i < p.n; ++i) {
+    const StageProblem& q = p.p[i];
+    long sums, tiles;
+    if (!stage_blocks(q, &sums, &tiles) || (p.normalize && (!q.partial || !q.scale))) return hipErrorInvalidValue;
+    if (p.sum_start[i + 1] - p.sum_start[i] != sums || p.tile_start[i + 1] - p.tile_start[i] != tiles) return hipErrorInvalidValue;
+    if (q.cpm > STAGE_FOLD_MAX) {
+      NormGroup& g = ng.g[ng.n];
+      g.partial = q.partial; g.scale = q.scale; g.pow2 = q.pow2; g.per_mat = q.cpm;
+      ng.mat_start[ng.n + 1] = ng.mat_start[ng.n] + q.batch;
+      ++ng.n;
+    }
+  }
+#define ARCHSCALE_STAGE(KERNEL, BLOCKS)                                                                                    \
+  do {                                                                                                                     \
+    if (p.in_dtype == DT_BF16) hipLaunchKernelGGL((KERNEL<DT_BF16, false>), dim3(BLOCKS), dim3(256), 0, stream, p);         \
+    else if (p.cast_first) hipLaunchKernelGGL((KERNEL<DT_F32, true>), dim3(BLOCKS), dim3(256), 0, stream, p);               \
+    else hipLaunchKernelGGL((KERNEL<DT_F32, false>), dim3(BLOCKS), dim3(256), 0, stream, p);                                \
+  } while (0)
+  if (p.normalize) {
+    ARCHSCALE_STAGE(stage_sumsq_kernel, p.sum_start[p.n]);
+    if (ng.n > 0) {
+      const hipError_t e = launch_norm_scale_groups(ng, p.eps, p.eps_mode, stream);
+      if (e != hipSuccess) return e;
+    }
+  }
+  ARCHSCALE_STAGE(stage_layout_kernel, p.tile_start[p.n]);
+#undef ARCHSCALE_STAGE
   return hipGetLastError();
 }
 

@@ -49,8 +49,8 @@ struct GemmParams {
 // Several independent problems of one kind (same tile configuration, mode, split and final flags) in ONE
 // launch: block b works on problem g with tile_start[g] <= b < tile_start[g+1] (a problem with a K-split owns
 // ksplit blocks per tile: block tile_start[g] + s * tiles + t is part s of tile t).  Passed by value as a kernel
-// argument (about 1.5 KiB).
-constexpr int MAX_GROUPS = 8;
+// argument (about 3 KiB).
+constexpr int MAX_GROUPS = 16;
 // Quarter mode: the blocks of the launch are the four half-size tiles of each tile of a 2x coarser enumeration
 // (tilesM, tilesN count the fine tiles; block 4q + s is quadrant s of coarse tile qt_first + q).  It lets a smaller
 // configuration take over where the larger one would leave the chip idle.
@@ -60,6 +60,7 @@ struct GroupedGemmParams {
   int tile_start[MAX_GROUPS + 1];
   GemmParams g[MAX_GROUPS];
 };
+static_assert(sizeof(GroupedGemmParams) <= 4096, "kernel arguments are limited to 4 KiB");
 
 // number of block tiles of one problem
 long ns_gemm_tiles(int mode, const GemmParams& p);

@@ -59,3 +59,23 @@ def test_symmetric_product_in_place_and_through_the_workspace(gpu_device, n, k, 
     sq = torch.randn(n, n, generator=g).to(torch.bfloat16).to(gpu_device)
     ref = ns._syrk(sq, None, 1.0, 0.0, None)
     assert torch.equal(ns._syrk(sq, None, 1.0, 0.0, sq), ref)   # over its own operand
+
+
+@pytest.mark.parametrize("normalize_by", ["add", "clamp"])
+def test_many_classes_in_one_call(gpu_device, normalize_by):
+    """More classes than one staging or product launch holds, both element types and orientations, padded extents, views, and a
+    matrix with more partial sums than a copy block adds up itself: every matrix as alone."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator().manual_seed(5)
+    shapes = [(64, 64), (65, 100), (100, 65), (1, 7), (7, 1), (3, 128, 200), (2, 200, 128), (300, 64), (64, 300), (129, 129),
+              (2, 640, 160), (160, 640), (512, 100), (33, 1000), (1000, 33), (2, 96, 96), (256, 512), (520, 513), (2900, 2900)]
+    xs = []
+    for i, s in enumerate(shapes):
+        t = torch.randn(*s[:-1], s[-1] + (8 if i % 4 == 1 else 0), generator=g) * 10.0 ** (i % 5 - 2)
+        t = t.to(torch.float32 if i % 3 == 0 else torch.bfloat16).to(gpu_device)
+        xs.append(t[..., 8:] if i % 4 == 1 else t)
+    for first in (True, False):
+        kw = dict(eps_mode=normalize_by, cast_input_first=first)
+        outs = ns.newton_schulz_grouped(xs, **kw)
+        for x, o in zip(xs, outs):
+            assert torch.equal(o, ns.newton_schulz(x, **kw)), tuple(x.shape)
