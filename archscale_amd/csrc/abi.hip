@@ -406,14 +406,32 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   size_t off = 0;
   // A call whose smallest launch (the symmetric products) would not even occupy half of the compute units with 256x256
   // tiles takes the 128x128 configuration for every problem: four times the blocks, a quarter of the time per block.
+  // A call whose problems would take both configurations one by one pays for a second launch of every product, about 10 us
+  // each: where that is more than the padding or the lower rate of ONE configuration costs, all problems take the cheaper one.
+  // (In the units of `work`, flops of an iteration at about 1250 TFLOP/s; the small configuration runs at 0.8 of that.)
   long sym_blocks = 0;
+  bool uses[2] = {false, false}, ksplit = false;   // 256, 128
+  double mixed = 0.0, all_256 = 0.0, all_128 = 0.0;
   for (int i = 0; i < n_problems; ++i) {
     const muon_ns_problem& q = problems_host[i];
     if (q.batch <= 0 || q.rows <= 0 || q.cols <= 0) return MUON_E_ARG;
     const NsPlan pl = make_plan(q.batch, q.rows, q.cols, prec_mode);
     sym_blocks += (long)q.batch * sym_tiles(pl.Mp / pl.tile);
+    auto work = [&](int t) {
+      const double Mp = (double)round_up(pl.m, t), Np = (double)round_up(pl.n, t);
+      return q.batch * Mp * Mp * (3.0 * Np + Mp) * (t == 128 ? 1.25 : 1.0);
+    };
+    mixed += work(pl.tile); all_256 += work(256); all_128 += work(128);
+    uses[pl.tile == 128] = true;
+    ksplit = ksplit || pl.sk_quadrants > 0;   // (the K-split is laid out in tiles of 256)
   }
-  const int force_tile = (!env_switches().tile && sym_blocks * 2 < compute_units()) ? 128 : 0;
+  int force_tile = 0;
+  if (!env_switches().tile) {
+    constexpr double SECOND_LAUNCHES = 3.1e10;   // 25 us of an iteration
+    if (sym_blocks * 2 < compute_units()) force_tile = 128;
+    else if (uses[0] && uses[1] && !ksplit && std::min(all_256, all_128) < mixed + SECOND_LAUNCHES)
+      force_tile = all_128 < all_256 ? 128 : 256;
+  }
   for (int i = 0; i < n_problems; ++i) {
     NsProblem& P = pr[i];
     P.q = problems_host[i];
