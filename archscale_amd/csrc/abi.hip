@@ -209,8 +209,13 @@ hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const Grouped
 // a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
 // 1023 286 -> 198, 1500 x 2000 (78 tiles) 268 -> 241; 136 tiles: the fp32 decoder of width 384 284 -> 262, but 2048 x 8192
 // 709 -> 747; 192 tiles: 3001 x 1023 198 -> 208.
+// The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
+// left beside whole rounds of either kind become sixteen tiles of 64 each, 256 blocks at most.  The 136 triangle tiles of a
+// short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
+// 14336 3353 -> 3255; more than 16 tiles so: no further gain.
 // ARCHSCALE_MUON_QUARTER=0 switches all of it off.
 constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
+constexpr int SIXTEENTH_MAX = 16;
 constexpr double QUARTER_LOAD = 0.6;
 hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream,
                          double fa, double fi, int f16) {
@@ -229,30 +234,38 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     if (!enabled || tail == 0 || (full > 0 ? tail > QUARTER_MAX_TAIL : all > QUARTER_LOAD * round * longest))
       return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
   } else {
-    if (!enabled || tile != 128 || split || total > (longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT)) return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+    if (!enabled || tile != 128 || split || total > (longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT))
+      return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
   }
-  const double share = (double)full / total;
-  if (full > 0) {
-    GroupedGemmParams m = gp;
-    for (int i = 0; i <= gp.n_groups; ++i) m.tile_start[i] = std::min(gp.tile_start[i], full);
-    hipError_t e = timed_gemm(tile, mode, split, final_, m, stream, fa * share, fi * share, f16);
-    if (e != hipSuccess) return e;
+  // tiles [begin, end) of the launch as (2^level)^2 tiles each of the configuration that is `level` smaller (level 0: as they are)
+  auto run = [&](int begin, int end, int level) -> hipError_t {
+    if (begin >= end) return hipSuccess;
+    const double share = (double)(end - begin) / total;
+    GroupedGemmParams q = {};
+    q.quarter = level;
+    for (int i = 0; i < gp.n_groups; ++i) {
+      const int s = gp.tile_start[i], f = std::max(s, begin), e = std::min(gp.tile_start[i + 1], end);
+      if (e <= f) continue;
+      GemmParams g = gp.g[i];
+      g.tilesM <<= level;
+      g.tilesN <<= level;
+      g.qt_first = level ? f - s : 0;
+      q.g[q.n_groups] = g;
+      q.tile_start[q.n_groups + 1] = q.tile_start[q.n_groups] + ((e - f) << 2 * level);
+      ++q.n_groups;
+    }
+    return timed_gemm(tile >> level, mode, split, final_, q, stream, fa * share, fi * share, f16);
+  };
+  hipError_t e = run(0, full, 0);
+  if (e != hipSuccess) return e;
+  if (tile == 256 && !split) {
+    if (full > 0 && total - full <= SIXTEENTH_MAX) return run(full, total, 2);
+    if (total - full > 128 && total - full - 128 <= SIXTEENTH_MAX) {
+      if ((e = run(full, full + 128, 1)) != hipSuccess) return e;
+      return run(full + 128, total, 2);
+    }
   }
-  GroupedGemmParams q = {};
-  q.quarter = 1;
-  for (int i = 0; i < gp.n_groups; ++i) {
-    const int s = gp.tile_start[i], e = gp.tile_start[i + 1];
-    const int f = std::max(s, full);
-    if (e <= f) continue;
-    GemmParams g = gp.g[i];
-    g.tilesM *= 2;
-    g.tilesN *= 2;
-    g.qt_first = f - s;
-    q.g[q.n_groups] = g;
-    q.tile_start[q.n_groups + 1] = q.tile_start[q.n_groups] + 4 * (e - f);
-    ++q.n_groups;
-  }
-  return timed_gemm(tile / 2, mode, split, final_, q, stream, fa * (1.0 - share), fi * (1.0 - share), f16);
+  return run(full, total, 1);
 }
 
 }  // namespace

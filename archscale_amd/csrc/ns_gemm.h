@@ -33,7 +33,7 @@ struct GemmParams {
   float diag_add;        // MODE_SYRK2: added to the diagonal of the result (B + a I, so that B X needs no addend)
   const float* scale;    // per batch element, or null: SYRK / SYRKT multiply the product by scale^2, BX the result by scale
   int m_valid, n_valid;  // true extents for the bounds-checked final store
-  int qt_first;          // quarter mode: first tile of this problem (in its own 2x coarser enumeration) that is covered
+  int qt_first;          // quarter mode: first tile of this problem (in its own coarser enumeration) that is covered
   // a launch may cover only tiles [t_first, t_first + t_count) of every matrix of the problem (in the matrix's own
   // enumeration; t_count = 0: all of them), the flat tile index of the launch then counts t_count tiles per matrix
   int t_first, t_count;
@@ -51,9 +51,9 @@ struct GemmParams {
 // ksplit blocks per tile: block tile_start[g] + s * tiles + t is part s of tile t).  Passed by value as a kernel
 // argument (about 3 KiB).
 constexpr int MAX_GROUPS = 16;
-// Quarter mode: the blocks of the launch are the four half-size tiles of each tile of a 2x coarser enumeration
-// (tilesM, tilesN count the fine tiles; block 4q + s is quadrant s of coarse tile qt_first + q).  It lets a smaller
-// configuration take over where the larger one would leave the chip idle.
+// Quarter mode (quarter = 1; 2: sixteenths): the blocks of the launch are the 4^quarter smaller tiles of each tile of a
+// 2^quarter times coarser enumeration (tilesM, tilesN count the fine tiles; block 4q + s is quadrant s of coarse tile
+// qt_first + q).  It lets a smaller configuration take over where the larger one would leave the chip idle.
 struct GroupedGemmParams {
   int n_groups;
   int quarter;

@@ -209,10 +209,10 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // grid the tile index is decoded in: the problem's own, or the 2x coarser one whose tiles this launch quarters
   int dM = p.tilesM, dN = p.tilesN, quadrant = 0;
   if (gp.quarter) {
-    quadrant = local & 3;
-    local = p.qt_first + (local >> 2);
-    dM >>= 1;
-    dN >>= 1;
+    quadrant = local & ((1 << 2 * gp.quarter) - 1);
+    local = p.qt_first + (local >> 2 * gp.quarter);
+    dM >>= gp.quarter;
+    dN >>= gp.quarter;
   }
   const int tiles_per_mat = SYM ? (dM * (dM + 1)) / 2 : dM * dN;
   // the launch may cover only tiles [t_first, t_first + t_count) of every matrix
@@ -267,9 +267,9 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     ti = t - tj * dM;
   }
   if (gp.quarter) {
-    ti = 2 * ti + (quadrant >> 1);
-    tj = 2 * tj + (quadrant & 1);
-    if (SYM && ti > tj) return;   // lower quadrant of a diagonal tile: its mirror image covers it
+    ti = (ti << gp.quarter) + (quadrant >> gp.quarter);
+    tj = (tj << gp.quarter) + (quadrant & ((1 << gp.quarter) - 1));
+    if (SYM && ti > tj) return;   // lower part of a diagonal tile: its mirror image covers it
   }
   const int R0 = ti * BT, C0 = tj * BT;
 
@@ -875,12 +875,14 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
       if (g.t_count ? (g.t_first + g.t_count > per || blocks > (long)g.batch * g.t_count) : blocks > ns_gemm_tiles(mode, g))
         return hipErrorInvalidValue;
     } else {
-      if ((g.tilesM & 1) || (!sym && (g.tilesN & 1)) || g.qt_first < 0 || (blocks & 3)) return hipErrorInvalidValue;
-      const long cm = g.tilesM / 2, cn = g.tilesN / 2;
+      const int side = 1 << gp.quarter;
+      if (gp.quarter > 2 || (ksplit && gp.quarter != 1)) return hipErrorInvalidValue;
+      if (g.tilesM % side || (!sym && g.tilesN % side) || g.qt_first < 0 || blocks % (side * side)) return hipErrorInvalidValue;
+      const long cm = g.tilesM / side, cn = g.tilesN / side;
       const long per = sym ? cm * (cm + 1) / 2 : cm * cn;
       if (g.t_count && g.t_first + g.t_count > per) return hipErrorInvalidValue;
       const long coarse = (long)g.batch * (g.t_count ? g.t_count : per);
-      if (g.qt_first + blocks / 4 > coarse) return hipErrorInvalidValue;
+      if (g.qt_first + blocks / (side * side) > coarse) return hipErrorInvalidValue;
     }
   }
   if (ksplit) {

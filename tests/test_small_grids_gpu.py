@@ -61,6 +61,19 @@ def test_symmetric_product_in_place_and_through_the_workspace(gpu_device, n, k, 
     assert torch.equal(ns._syrk(sq, None, 1.0, 0.0, sq), ref)   # over its own operand
 
 
+def test_leftover_tiles_in_sixteenths(gpu_device):
+    """136 triangle tiles of 256 (short side 4096): 128 in quadrants and 8 in sixteenths alone, whole rounds and a quartered or
+    sixteenth rest in batches of 2 and 3."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator(device=gpu_device).manual_seed(11)
+    x = (torch.randn(3, 4000, 4100, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
+    coeffs = ns.QUINTIC_SCHEDULE[:3]
+    three = ns.newton_schulz(x, coeffs)
+    assert torch.equal(ns.newton_schulz(x[:2], coeffs), three[:2])
+    for i in range(3):
+        assert torch.equal(ns.newton_schulz(x[i], coeffs), three[i])
+
+
 @pytest.mark.parametrize("normalize_by", ["add", "clamp"])
 def test_many_classes_in_one_call(gpu_device, normalize_by):
     """More classes than one staging or product launch holds, both element types and orientations, padded extents, views, and a
