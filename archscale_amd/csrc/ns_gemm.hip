@@ -761,10 +761,31 @@ template <> struct Config<CFG_128> { static constexpr int BT = 128, SP = 2, SQ =
 template <> struct Config<CFG_128_DEEP> { static constexpr int BT = 128, SP = 4, SQ = 5, BLOCKS = 1; };
 template <> struct Config<CFG_64> { static constexpr int BT = 64, SP = 4, SQ = 5, BLOCKS = 2; };
 
-template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
-__global__ void __launch_bounds__(256, Config<CFG>::BLOCKS)
+// The two configurations that fill the chip, by block tile and wave tile.
+template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+__global__ void __launch_bounds__(256, Config<BM == 256 ? CFG_256 : CFG_128>::BLOCKS)
 ns_gemm_kernel(const GroupedGemmParams gp) {
-  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
+  static_assert(BM == BN && WM == BM / 2 && WN == BN / 2 && (BM == 256 || BM == 128), "four waves of a quarter each");
+  using C = Config<BM == 256 ? CFG_256 : CFG_128>;
+  ns_gemm_tile<BM, C::SP, C::SQ, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
+}
+
+// The two configurations for launches that do not (deeper pipelines).
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16>
+__global__ void __launch_bounds__(256, Config<CFG>::BLOCKS)
+ns_gemm_deep_kernel(const GroupedGemmParams gp) {
+  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, false>(gp);
+}
+
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+static constexpr auto kernel_of() {
+  constexpr int BT = Config<CFG>::BT;
+  if constexpr (CFG == CFG_256 || CFG == CFG_128) {
+    return &ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
+  } else {
+    static_assert(!SK, "the K-split runs in the 128 configuration");
+    return &ns_gemm_deep_kernel<CFG, MODE, SPLIT, FINAL, ADDEND, F16>;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -779,7 +800,7 @@ template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16
 static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   constexpr int NT = 256;
   constexpr int SMEM = (Config<CFG>::SP + Config<CFG>::SQ) * Config<CFG>::BT * ROW_BYTES;
-  auto kern = ns_gemm_kernel<CFG, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
+  constexpr auto kern = kernel_of<CFG, MODE, SPLIT, FINAL, ADDEND, F16, SK>();
   // the dynamic-LDS limit is an attribute of the function on ONE device: set it once per device and instantiation
   // (the call is idempotent, so two threads that race on the first launch only repeat it)
   static std::atomic<bool> attr_set[64];
