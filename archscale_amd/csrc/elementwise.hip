@@ -993,7 +993,7 @@ __device__ __forceinline__ void scalar_range(const ScalarItem& it, long begin, l
     }
   }
 }
-// all arrays of one dtype (no branch per access), or each by its own
+// all arrays of one dtype (no branch per access), or each by its own dtype
 template <int DT> struct OneDtype {
   __device__ __forceinline__ void load(const void* p, int, long i, float (&v)[8]) const { Elem<DT>::load8(p, i, v); }
   __device__ __forceinline__ void store(void* p, int, long i, const float (&v)[8]) const { Elem<DT>::store8(p, i, v); }
@@ -1032,7 +1032,10 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
     const int dt = it.w_dtype;
     const bool one = it.m_dtype == dt && it.g_dtype == dt && (!has_v || it.v_dtype == dt);
     if (one && dt == DT_BF16) scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, OneDtype<DT_BF16>{});
-    else if (one) scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, OneDtype<DT_F32>{});
+    // (plain AdamW on fp32 arrays is bound by its seven streams and slower with all its loads issued at once: 18 million
+    // elements of 20000 x 900 twice, 238 us against 208 us with a branch at each access)
+    else if (one && !(ALGO == ALGO_ADAMW && PHASE == 0))
+      scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, OneDtype<DT_F32>{});
     else scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, MixedDtypes{});
   } else {
     for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
