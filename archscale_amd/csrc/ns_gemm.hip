@@ -105,8 +105,10 @@ __device__ __forceinline__ void wait_copies() {
 // acc += a * b on the matrix cores.  Inline assembly with the accumulator as a read-write operand: the builtin leaves the
 // destination free, and over a software-pipelined loop the register allocator then rotates the accumulators with
 // register moves between the MFMAs (measured: half the issue rate).  What the assembler statement hides from the compiler
-// is kept by hand: an empty statement after the zero-initialisation keeps it away from the first MFMA, and acc_settle()
-// stands between the last MFMA and the first read of a result.
+// is kept by hand: an empty statement after the zero-initialisation keeps it away from the first MFMA, acc_settle() stands
+// behind the last MFMA, and acc_touch() before every use of a result keeps that use behind acc_settle(), whose nops name no
+// register (without it the compiler moved accumulator reads above the nops).  One statement per use, not all of them right
+// after the nops: the registers then spill nowhere (64 of them in one instantiation otherwise).
 template <bool HALF, bool AGPR>
 __device__ __forceinline__ void mfma16(f32x4& acc, const u32x4& a, const u32x4& b) {
   if constexpr (AGPR) {
@@ -547,10 +549,12 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 #pragma unroll
       for (int i = 0; i < FR; ++i)
 #pragma unroll
-        for (int j = 0; j < FR; ++j)
+        for (int j = 0; j < FR; ++j) {
+          acc_touch<AGPR>(acc[i][j]);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             __hip_atomic_store(dst + ((i * FR + j) * 4 + e) * NT + tid, acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's stores have been acknowledged
       __syncthreads();
       if (tid == 0) {
@@ -636,6 +640,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       for (int j = 0; j < FR; ++j) {
         const int c = j * 16 + l16, r = i * 16 + 4 * lg;
         float v[4];
+        acc_touch<AGPR>(acc[i][j]);
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = acc[i][j][q];
         if constexpr (SYRK_PLAIN) {
