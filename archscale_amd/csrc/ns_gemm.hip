@@ -107,8 +107,9 @@ __device__ __forceinline__ void wait_copies() {
 // register moves between the MFMAs (measured: half the issue rate).  What the assembler statement hides from the compiler
 // is kept by hand: an empty statement after the zero-initialisation keeps it away from the first MFMA, acc_settle() stands
 // behind the last MFMA, and acc_touch() before every use of a result keeps that use behind acc_settle(), whose nops name no
-// register (without it the compiler moved accumulator reads above the nops).  One statement per use, not all of them right
-// after the nops: the registers then spill nowhere (64 of them in one instantiation otherwise).
+// register (without it the compiler moved accumulator reads above the nops).  The epilogue touches one row of fragments at a
+// time: all of them right after the nops cost one instantiation 64 spilled registers, one by one costs 2 to 5 % more
+// instructions (waits inside each fragment).
 template <bool HALF, bool AGPR>
 __device__ __forceinline__ void mfma16(f32x4& acc, const u32x4& a, const u32x4& b) {
   if constexpr (AGPR) {
@@ -635,12 +636,13 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
 #pragma unroll
-    for (int i = 0; i < FR; ++i)
+    for (int i = 0; i < FR; ++i) {
+#pragma unroll
+      for (int j = 0; j < FR; ++j) acc_touch<AGPR>(acc[i][j]);
 #pragma unroll
       for (int j = 0; j < FR; ++j) {
         const int c = j * 16 + l16, r = i * 16 + 4 * lg;
         float v[4];
-        acc_touch<AGPR>(acc[i][j]);
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = acc[i][j][q];
         if constexpr (SYRK_PLAIN) {
@@ -685,6 +687,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
         }
         if ((j & 1) == 1) __builtin_amdgcn_sched_barrier(0);
       }
+    }
     // transposed / mirrored image: rows of W
     __bf16* Tdst = SYM ? Cdst : p.Ct;
     if (Tdst && (!diag || above)) {   // in a diagonal tile: only the image of the idle wave's part
