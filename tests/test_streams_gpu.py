@@ -59,3 +59,52 @@ def test_singular_vectors_against_fp64(gpu_device, rows, cols):
             want = want * torch.sign((got * want).sum())
             assert ((got - want).norm() / want.norm()).item() < 2.0 ** -8
         assert abs(s[i].item() - S[i, 0].item()) < 3e-3 * S[i, 0].item()
+
+
+@pytest.mark.parametrize("numel", [8192 + 16, 8192 + 3])
+def test_adam_direction_with_an_epsilon_at_the_bottom_of_the_range(gpu_device, numel):
+    """eps sqrt(bias2) below the smallest normal number: a zero moment over a zero second moment stays a zero direction, a
+    tiny one gives the finite quotient.  Bound as above."""
+    from archscale_amd.optim import scalar_opts as H
+    lr, b1, b2, eps, step = 1e-2, 0.875, 1 - 2.0 ** -10, 1e-37, 1   # (betas that fp32 holds exactly)
+    x0 = torch.linspace(-1.0, 1.0, numel)
+    g0, m0, v0 = torch.zeros(numel), torch.zeros(numel), torch.zeros(numel)
+    m0[1::3] = 1e-37
+    v0[2::3], m0[2::3] = 1e-6, 1e-3
+    for hyper in (False, True):
+        x, g, m, v = (t.clone().to(gpu_device) for t in (x0, g0, m0, v0))
+        fn = H.hyperball_adamw_update_foreach if hyper else H.adamw_update_foreach
+        fn([x], [g], [m], [v], lr, b1, b2, 0.0, step, eps)
+        m64, v64 = m.cpu().double(), v.cpu().double()
+        u = m64 / (v64.sqrt() / math.sqrt(1 - b2 ** step) + eps) / (1 - b1 ** step)
+        x64 = x0.double()
+        if hyper:
+            t = lr * x64.norm() / u.norm()
+            want = x64 - t * u
+            want = want * (x64.norm() / want.norm())
+        else:
+            t, want = lr, x64 - lr * u
+        err = (x.cpu().double() - want).abs()
+        bound = 2.0 ** -21 * (x64.abs() + t * u.abs())
+        assert bool((err <= bound).all()), (hyper, err.max().item())
+
+
+@pytest.mark.parametrize("numel", [1 << 18, (1 << 18) + 1])
+def test_adam_direction_is_the_quotient_to_the_last_bit(gpu_device, numel):
+    """With beta1 = 1/2, beta2 = 3/4, step 1, lr = 1/2 and zero weights every other operation of the plain step is exact and
+    the new weight is minus the quotient.  The corrected quotient is off by at most 2^-23 + 2^-22 of an ulp (the error of the
+    uncorrected one, about two ulp, times the reciprocal's) before its one rounding: never by more than an ulp after it, and
+    another last bit in about one of 2^22 quotients."""
+    import numpy as np
+    from archscale_amd.optim import scalar_opts as H
+    gen = torch.Generator().manual_seed(numel)
+    eps = 2.0 ** -27
+    m0 = torch.randn(numel, generator=gen) * 10.0 ** (torch.rand(numel, generator=gen) * 8 - 6)
+    v0 = torch.rand(numel, generator=gen) * 10.0 ** (torch.rand(numel, generator=gen) * 16 - 14)
+    x, g, m, v = (t.clone().to(gpu_device) for t in (torch.zeros(numel), torch.zeros(numel), m0, v0))
+    H.adamw_update_foreach([x], [g], [m], [v], 0.5, 0.5, 0.75, 0.0, 1, eps)
+    mn, vn = m.cpu().numpy(), v.cpu().numpy()
+    want = (mn * np.float32(0.5)) / (np.sqrt(vn) + np.float32(eps * 0.5))
+    assert want.dtype == np.float32
+    off = np.abs((-x).cpu().numpy().view(np.int32).astype(np.int64) - want.view(np.int32).astype(np.int64))
+    assert off.max() <= 1 and (off > 0).mean() <= 1e-4, (off.max(), (off > 0).mean())
