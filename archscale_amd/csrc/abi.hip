@@ -217,8 +217,14 @@ hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const Grouped
 constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
 constexpr int SIXTEENTH_MAX = 16;
 constexpr double QUARTER_LOAD = 0.6;
+// (work: the FLOPs of a Newton-Schulz launch for its timing record; null: a product of another entry point, not recorded)
+struct LaunchWork { double algorithmic, issued; };
 hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream,
-                         double fa, double fi, int f16) {
+                         const LaunchWork* work, int f16) {
+  auto launch = [&](int t, const GroupedGemmParams& g, double share) -> hipError_t {
+    if (!work) return launch_ns_gemm_grouped(t, mode, split, final_, g, stream, f16);
+    return timed_gemm(t, mode, split, final_, g, stream, work->algorithmic * share, work->issued * share, f16);
+  };
   const bool enabled = env_switches().quarter;
   const int total = gp.tile_start[gp.n_groups];
   double all = 0.0, longest = 0.0;   // k-values of all tiles, of the longest one
@@ -232,15 +238,14 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     full = total / round * round;
     const int tail = total - full;
     if (!enabled || tail == 0 || (full > 0 ? tail > QUARTER_MAX_TAIL : all > QUARTER_LOAD * round * longest))
-      return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+      return launch(tile, gp, 1.0);
   } else {
     if (!enabled || tile != 128 || split || total > (longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT))
-      return timed_gemm(tile, mode, split, final_, gp, stream, fa, fi, f16);
+      return launch(tile, gp, 1.0);
   }
   // tiles [begin, end) of the launch as (2^level)^2 tiles each of the configuration that is `level` smaller (level 0: as they are)
   auto run = [&](int begin, int end, int level) -> hipError_t {
     if (begin >= end) return hipSuccess;
-    const double share = (double)(end - begin) / total;
     GroupedGemmParams q = {};
     q.quarter = level;
     for (int i = 0; i < gp.n_groups; ++i) {
@@ -254,7 +259,7 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
       q.tile_start[q.n_groups + 1] = q.tile_start[q.n_groups] + ((e - f) << 2 * level);
       ++q.n_groups;
     }
-    return timed_gemm(tile >> level, mode, split, final_, q, stream, fa * share, fi * share, f16);
+    return launch(tile >> level, q, (double)(end - begin) / total);
   };
   hipError_t e = run(0, full, 0);
   if (e != hipSuccess) return e;
@@ -635,7 +640,8 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       double fa = 0.0, fi = 0.0;
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
-        hipError_t err = launch_rounds(tile, mode, split_launch, final_, gp, stream, fa, fi, ws16);
+        const LaunchWork work = {fa, fi};
+        hipError_t err = launch_rounds(tile, mode, split_launch, final_, gp, stream, &work, ws16);
         gp = GroupedGemmParams{};
         fa = fi = 0.0;
         return err;
@@ -1031,8 +1037,7 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   gp.n_groups = 1;
   gp.g[0] = g;
   gp.tile_start[1] = (int)tiles;
-  e = launch_rounds(tile, mode, false, false, gp, stream, (double)batch * n * n * k,
-                    (double)batch * 2.0 * tile * tile * sym_tiles_issued(Np / tile) * Kp, 0);
+  e = launch_rounds(tile, mode, false, false, gp, stream, nullptr, 0);
   if (e != hipSuccess || d_here) return (int)e;
   return (int)launch_unpad_copy(Dp, (long)Np * Np, Np, d_dev, d_batch_stride, ldd, batch, n, n, stream);
 }
@@ -1193,12 +1198,10 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
   auto gram = [&](auto&& src_of, auto&& k_of, auto&& dst_of, auto&& scale_of) -> int {
     for (int tile : {256, 128}) {
       GroupedGemmParams gp = {};
-      double fa = 0.0, fi = 0.0;
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
-        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, fa, fi, 0);
+        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, nullptr, 0);
         gp = GroupedGemmParams{};
-        fa = fi = 0.0;
         return err;
       };
       for (const Prob& P : pr) {
@@ -1219,8 +1222,6 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
         gp.g[gp.n_groups] = g;
         gp.tile_start[gp.n_groups + 1] = gp.tile_start[gp.n_groups] + (int)tiles;
         ++gp.n_groups;
-        fa += (double)P.q.batch * pl.m * pl.m * K;
-        fi += (double)P.q.batch * 2.0 * tile * tile * sym_tiles_issued(pl.Mp / tile) * K;
       }
       if ((e = flush()) != hipSuccess) return (int)e;
     }

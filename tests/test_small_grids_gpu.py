@@ -92,3 +92,20 @@ def test_many_classes_in_one_call(gpu_device, normalize_by):
         outs = ns.newton_schulz_grouped(xs, **kw)
         for x, o in zip(xs, outs):
             assert torch.equal(o, ns.newton_schulz(x, **kw)), tuple(x.shape)
+
+
+def test_only_newton_schulz_launches_are_recorded(gpu_device):
+    """The launch records serve the accounting of a Newton-Schulz call: single products and the power iteration share its kernels
+    but not its records."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    from archscale_amd import _lib
+    from archscale_amd.emerging import spectral_norm
+    a = torch.randn(256, 512, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(gpu_device)
+    _lib.profile_begin()
+    ns.ns_line_1(a)
+    spectral_norm(a[None], 10)
+    assert _lib.profile_collect() == []
+    _lib.profile_begin()
+    ns.newton_schulz(a, gram_tail=False)
+    recs = _lib.profile_collect()
+    assert len(recs) == 15 and all(r["kind"] == "gemm" and r["flops_algorithmic"] > 0 for r in recs)
