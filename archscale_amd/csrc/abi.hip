@@ -12,6 +12,7 @@
 
 #include "../../include/archscale_muon.h"
 #include "elementwise.h"
+#include "launch_rules.h"
 #include "ns_gemm.h"
 #include "spectral.h"
 
@@ -187,62 +188,32 @@ hipError_t timed_launch(int key, double work_algorithmic, double work_issued, hi
 }
 
 hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const GroupedGemmParams& g, hipStream_t stream,
-                      double flops_algorithmic, double flops_issued, int f16 = 0) {
+                      int units, double flops_algorithmic, double flops_issued, int f16 = 0) {
   const int key = tile * 100 + mode * 10 + ((mode == MODE_BX && !g.g[0].E) ? 4 : 0) + (split ? 2 : 0) + (final_ ? 1 : 0);
   return timed_launch(key, flops_algorithmic, flops_issued, stream,
-                      [&] { return launch_ns_gemm_grouped(tile, mode, split, final_, g, stream, f16); });
+                      [&] { return launch_ns_gemm_grouped(tile, mode, split, final_, g, stream, units, f16); });
 }
 
-// One product over all problems of a launch, with tiles handed to the next smaller configuration (four quadrants each)
-// where the larger one would leave the chip idle.  The sums of an element are the same in every configuration.
-//
-// Tiles of 256, more than one round (256 compute units) of them: the full rounds run as they are, a last round of at most
-// QUARTER_MAX_TAIL tiles is quartered: a quarter of the time per block instead of a whole round for a few tiles (measured: a
-// tail of 160 tiles on the depth-16 set costs 83 us quartered against 57 us as it is; tails of 16 and 128 tiles of single
-// 8192x8192 and 4096x14336 matrices: 10.33 -> 9.80 ms and 4.58 -> 4.44 ms per call).
-// Less than one round: as tiles of 256 the launch takes as long as its longest tile; quartered, the tiles spread over the
-// chip, at about 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
-// (208 tiles of 2816 and 1024 k-values, five fp32 EMA-Muon products) the step takes 1250 us quartered, 1318 as it is; at 0.625
-// (160 equal tiles, power iteration over 16 x 1024 x 2816) 337 against 317 us.
-//
-// Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
-// a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
-// 1023 286 -> 198, 1500 x 2000 (78 tiles) 268 -> 241; 136 tiles: the fp32 decoder of width 384 284 -> 262, but 2048 x 8192
-// 709 -> 747; 192 tiles: 3001 x 1023 198 -> 208.
-// The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
-// left beside whole rounds of either kind become sixteen tiles of 64 each, 256 blocks at most.  The 136 triangle tiles of a
-// short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
-// 14336 3353 -> 3255; more than 16 tiles so: no further gain.
-// ARCHSCALE_MUON_QUARTER=0 switches all of it off.
-constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
-constexpr int SIXTEENTH_MAX = 16;
-constexpr double QUARTER_LOAD = 0.6;
+// One product over all problems of a launch, with tiles handed to the next smaller configurations where the larger one would
+// leave the chip idle (launch_rules.h).  ARCHSCALE_MUON_QUARTER=0 switches that off.
 // (work: the FLOPs of a Newton-Schulz launch for its timing record; null: a product of another entry point, not recorded)
 struct LaunchWork { double algorithmic, issued; };
 hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream,
                          const LaunchWork* work, int f16) {
+  const int units = compute_units();
   auto launch = [&](int t, const GroupedGemmParams& g, double share) -> hipError_t {
-    if (!work) return launch_ns_gemm_grouped(t, mode, split, final_, g, stream, f16);
-    return timed_gemm(t, mode, split, final_, g, stream, work->algorithmic * share, work->issued * share, f16);
+    if (!work) return launch_ns_gemm_grouped(t, mode, split, final_, g, stream, units, f16);
+    return timed_gemm(t, mode, split, final_, g, stream, units, work->algorithmic * share, work->issued * share, f16);
   };
-  const bool enabled = env_switches().quarter;
   const int total = gp.tile_start[gp.n_groups];
   double all = 0.0, longest = 0.0;   // k-values of all tiles, of the longest one
   for (int i = 0; i < gp.n_groups; ++i) {
     all += (double)(gp.tile_start[i + 1] - gp.tile_start[i]) * gp.g[i].K;
     longest = std::max(longest, (double)gp.g[i].K);
   }
-  int full = 0;
-  if (tile == 256) {
-    const int round = 256;
-    full = total / round * round;
-    const int tail = total - full;
-    if (!enabled || tail == 0 || (full > 0 ? tail > QUARTER_MAX_TAIL : all > QUARTER_LOAD * round * longest))
-      return launch(tile, gp, 1.0);
-  } else {
-    if (!enabled || tile != 128 || split || total > (longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT))
-      return launch(tile, gp, 1.0);
-  }
+  const LaunchSplit cut = env_switches().quarter ? launch_split(units, tile, split, total, all, longest)
+                                                 : LaunchSplit{total, 0, 0};
+  if (cut.whole == total) return launch(tile, gp, 1.0);
   // tiles [begin, end) of the launch as (2^level)^2 tiles each of the configuration that is `level` smaller (level 0: as they are)
   auto run = [&](int begin, int end, int level) -> hipError_t {
     if (begin >= end) return hipSuccess;
@@ -261,16 +232,10 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     }
     return launch(tile >> level, q, (double)(end - begin) / total);
   };
-  hipError_t e = run(0, full, 0);
-  if (e != hipSuccess) return e;
-  if (tile == 256 && !split) {
-    if (full > 0 && total - full <= SIXTEENTH_MAX) return run(full, total, 2);
-    if (total - full > 128 && total - full - 128 <= SIXTEENTH_MAX) {
-      if ((e = run(full, full + 128, 1)) != hipSuccess) return e;
-      return run(full + 128, total, 2);
-    }
-  }
-  return run(full, total, 1);
+  const int quartered = cut.whole + cut.quarters;
+  hipError_t e = run(0, cut.whole, 0);
+  if (e == hipSuccess) e = run(cut.whole, quartered, 1);
+  return e == hipSuccess ? run(quartered, total, 2) : e;
 }
 
 }  // namespace
@@ -628,7 +593,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       const int key = 128 * 100 + mode * 10;
       const GroupedGemmParams launch = sk;
       hipError_t err = timed_launch(key, sk_fa, sk_fi, stream, [&] {
-        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, ws16, true);
+        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, compute_units(), ws16, true);
       });
       sk = GroupedGemmParams{};
       sk.quarter = 1;

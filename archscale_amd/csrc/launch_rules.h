@@ -1,0 +1,59 @@
+// How the tiles of one product launch are cut for the chip: host arithmetic only (no HIP), so that it can be checked on any
+// number of compute units.  `units` is what the current device reports; the measured lines are those of 256 units (one MI355X)
+// and are scaled with it.  A choice made here never changes a result: the sums of an element are the same in every configuration.
+#pragma once
+
+namespace archscale {
+
+// Tiles with numbers [0, whole) of a launch run as they are, the next `quarters` as four tiles of half the side each, the next
+// `sixteenths` as sixteen of a quarter of it.
+struct LaunchSplit { int whole, quarters, sixteenths; };
+
+// Tiles of 256, more than one round (one tile per unit) of them: the full rounds run as they are, a last round of at most
+// QUARTER_MAX_TAIL tiles is quartered: a quarter of the time per block instead of a whole round for a few tiles (measured: a
+// tail of 160 tiles on the depth-16 set costs 83 us quartered against 57 us as it is; tails of 16 and 128 tiles of single
+// 8192x8192 and 4096x14336 matrices: 10.33 -> 9.80 ms and 4.58 -> 4.44 ms per call).
+// Less than one round: as tiles of 256 the launch takes as long as its longest tile; quartered, the tiles spread over the
+// chip, at about 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
+// (208 tiles of 2816 and 1024 k-values, five fp32 EMA-Muon products) the step takes 1250 us quartered, 1318 as it is; at 0.625
+// (160 equal tiles, power iteration over 16 x 1024 x 2816) 337 against 317 us.
+//
+// Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
+// a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
+// 1023 286 -> 198, 1500 x 2000 (78 tiles) 268 -> 241; 136 tiles: the fp32 decoder of width 384 284 -> 262, but 2048 x 8192
+// 709 -> 747; 192 tiles: 3001 x 1023 198 -> 208.
+// The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
+// left beside whole rounds of either kind become sixteen tiles of 64 each, one block per unit at most.  The 136 triangle tiles of
+// a short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
+// 14336 3353 -> 3255; more than 16 tiles so: no further gain.
+constexpr int RULE_UNITS = 256;   // the device of the figures
+constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
+constexpr int SIXTEENTH_MAX = 16;
+constexpr double QUARTER_LOAD = 0.6;
+
+// total: tiles of the launch; all, longest: k-values of all its tiles and of the longest one; pair: products of a hi+lo pair
+// (there is no configuration of 64 for them)
+inline LaunchSplit launch_split(int units, int tile, bool pair, int total, double all, double longest) {
+  auto scaled = [&](int tiles) { return (int)((long)tiles * units / RULE_UNITS); };
+  const LaunchSplit as_is = {total, 0, 0};
+  if (tile == 128) {
+    const int most = scaled(longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT);
+    return pair || total > most ? as_is : LaunchSplit{0, total, 0};
+  }
+  if (tile != 256) return as_is;
+  const int full = total / units * units, tail = total - full;
+  if (tail == 0 || (full > 0 ? tail > scaled(QUARTER_MAX_TAIL) : all > QUARTER_LOAD * units * longest)) return as_is;
+  const int half = units / 2, few = scaled(SIXTEENTH_MAX);   // half: one round of quadrants
+  if (!pair && full > 0 && tail <= few) return {full, 0, tail};
+  if (!pair && tail > half && tail - half <= few) return {full, half, tail - half};
+  return {full, tail, 0};
+}
+
+// Tiles of 128 in the deep form where every block finds a unit of its own and the reductions are long: 3001 x 1023 302 -> 286 us,
+// 1500 x 2000 290 -> 270, a symmetric product of 2048 x 5632 47 -> 41; filling four stages costs reductions of 640 and less
+// 1 to 4 %.
+inline bool deep_pipeline(int units, int tile, int blocks, int shortest_k) {
+  return tile == 128 && blocks <= units && shortest_k >= 1024;
+}
+
+}  // namespace archscale

@@ -68,11 +68,11 @@ long ns_gemm_tiles(int mode, const GemmParams& p);
 // tile: side of the block tile, 256, 128 or 64 (four waves each; 64 without the hi+lo pair)
 // f16: 0 = the workspace matrices of the launch are bfloat16; 1 = IEEE half (see GemmParams::out_shift), not with split;
 // 2 = bfloat16 operands, IEEE-half result (MODE_BX, not the final launch)
+// units: compute units of the device
 // ksplit: some problem of the launch has GemmParams::ksplit > 1 (symmetric modes, tile 128, no hi+lo pair)
 hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp,
-                                  hipStream_t stream, int f16 = 0, bool ksplit = false);
+                                  hipStream_t stream, int units, int f16 = 0, bool ksplit = false);
 // bytes of GemmParams::sk_partial per tile of a K-split launch
 constexpr long SK_TILE_BYTES = 128L * 128 * 4;
-hipError_t launch_ns_gemm(int tile, int mode, bool split, bool final_, const GemmParams& p, hipStream_t stream);
 
 }  // namespace archscale

@@ -25,6 +25,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "launch_rules.h"
 #include "ns_gemm.h"
 
 // The epilogue arithmetic is written out with explicit fmaf() and the compiler forms no fused operations of its own:
@@ -879,7 +880,7 @@ static hipError_t launch_ksplit(int mode, const GroupedGemmParams& p, hipStream_
 }
 
 hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp,
-                                  hipStream_t stream, int f16, bool ksplit) {
+                                  hipStream_t stream, int units, int f16, bool ksplit) {
   if (gp.n_groups < 1 || gp.n_groups > MAX_GROUPS) return hipErrorInvalidValue;
   const bool sym = (mode == MODE_SYRK || mode == MODE_SYRK2 || mode == MODE_SYRKT);
   if (ksplit && (!sym || tile != 128 || split || final_ || f16 == 2)) return hipErrorInvalidValue;
@@ -918,10 +919,9 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
     if (f16 == 1) return launch_ksplit<1>(mode, gp, stream);
     return launch_ksplit<0>(mode, gp, stream);
   }
-  // The deep form where every block finds a unit of its own and the reductions are long: 3001 x 1023 302 -> 286 us, 1500 x 2000
-  // 290 -> 270, a symmetric product of 2048 x 5632 47 -> 41; filling four stages costs reductions of 640 and less 1 to 4 %.
-  bool deep = tile == 128 && gp.tile_start[gp.n_groups] <= 256;
-  for (int i = 0; i < gp.n_groups; ++i) deep = deep && gp.g[i].K >= 1024;
+  int shortest = gp.g[0].K;
+  for (int i = 1; i < gp.n_groups; ++i) shortest = gp.g[i].K < shortest ? gp.g[i].K : shortest;
+  const bool deep = deep_pipeline(units, tile, gp.tile_start[gp.n_groups], shortest);
   auto by_storage = [&](auto cfg_) -> hipError_t {
     constexpr int CFG = decltype(cfg_)::value;
     if (f16 == 1) return launch_cfg<CFG, 1>(mode, split, final_, gp, stream);
@@ -934,16 +934,6 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
   if (tile == 128) return by_storage(std::integral_constant<int, CFG_128>{});
   if (tile == 64) return by_storage(std::integral_constant<int, CFG_64>{});
   return hipErrorInvalidValue;
-}
-
-hipError_t launch_ns_gemm(int tile, int mode, bool split, bool final_, const GemmParams& p, hipStream_t stream) {
-  GroupedGemmParams gp = {};
-  gp.n_groups = 1;
-  gp.g[0] = p;
-  const long tiles = ns_gemm_tiles(mode, p);
-  if (tiles > 0x7ffffff0L) return hipErrorInvalidValue;
-  gp.tile_start[1] = (int)tiles;
-  return launch_ns_gemm_grouped(tile, mode, split, final_, gp, stream);
 }
 
 }  // namespace archscale

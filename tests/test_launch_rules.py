@@ -1,0 +1,73 @@
+"""CPU-only: how the tiles of a launch are cut for devices of any number of compute units."""
+import os
+import subprocess
+
+import pytest
+
+PROGRAM = r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() {
+  int units, tile, pair, total, blocks, k;
+  double all, longest;
+  while (scanf("%d %d %d %d %lf %lf %d %d", &units, &tile, &pair, &total, &all, &longest, &blocks, &k) == 8) {
+    const archscale::LaunchSplit s = archscale::launch_split(units, tile, pair != 0, total, all, longest);
+    printf("%d %d %d %d\n", s.whole, s.quarters, s.sixteenths, (int)archscale::deep_pipeline(units, 128, blocks, k));
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    from archscale_amd.build import CSRC
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(d / "rules.cpp"), "-o", str(d / "rules")], check=True)
+
+    def ask(rows):
+        text = "".join("%d %d %d %d %.17g %.17g %d %d\n" % r for r in rows)
+        out = subprocess.run([str(d / "rules")], input=text, capture_output=True, text=True, check=True).stdout
+        return [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+
+    return ask
+
+
+def test_lines_on_256_units(rules):
+    # (tile, pair, total, all k-values, longest) -> (whole, quarters, sixteenths)
+    want = {
+        (256, 0, 256, 256e3, 1e3): (256, 0, 0),
+        (256, 0, 272, 272e3, 1e3): (256, 0, 16),
+        (256, 0, 273, 273e3, 1e3): (256, 17, 0),
+        (256, 1, 272, 272e3, 1e3): (256, 16, 0),
+        (256, 0, 384, 384e3, 1e3): (256, 128, 0),
+        (256, 0, 385, 385e3, 1e3): (385, 0, 0),
+        (256, 0, 128, 128e3, 1e3): (0, 128, 0),
+        (256, 0, 136, 136e3, 1e3): (0, 128, 8),
+        (256, 1, 136, 136e3, 1e3): (0, 136, 0),
+        (256, 0, 145, 145e3, 1e3): (0, 145, 0),
+        (256, 0, 160, 160e3, 1e3): (160, 0, 0),
+        (256, 0, 208, 208 * 590.0, 1e3): (0, 208, 0),
+        (128, 0, 100, 1.0, 1088.0): (0, 100, 0),
+        (128, 0, 101, 1.0, 1088.0): (101, 0, 0),
+        (128, 0, 140, 1.0, 1024.0): (0, 140, 0),
+        (128, 0, 141, 1.0, 1024.0): (141, 0, 0),
+        (128, 1, 10, 1.0, 1024.0): (10, 0, 0),
+    }
+    got = rules([(256, *k, 1, 64) for k in want])
+    for k, g in zip(want, got):
+        assert g[:3] == want[k], (k, g)
+
+
+@pytest.mark.parametrize("units", [32, 38, 64, 128, 256, 304])
+def test_every_tile_once_and_rounds_of_the_device(rules, units):
+    rows = [(units, tile, pair, total, total * load * 1e3, 1e3, blocks, k)
+            for tile in (256, 128, 64) for pair in (0, 1) for total in range(1, 3 * units + 2, max(1, units // 16))
+            for load in (0.5, 1.0) for blocks in (units - 1, units, units + 1) for k in (960, 1024)]
+    for (_, tile, pair, total, _, _, blocks, k), (whole, quarters, sixteenths, deep) in zip(rows, rules(rows)):
+        assert min(whole, quarters, sixteenths) >= 0 and whole + quarters + sixteenths == total
+        assert whole == total or whole % units == 0
+        assert not sixteenths or (tile == 256 and not pair and 16 * sixteenths <= units)
+        assert tile != 64 or whole == total
+        # a block of the deep form holds most of a unit's LDS: never more of them than the device has units
+        assert deep == (blocks <= units and k >= 1024)
