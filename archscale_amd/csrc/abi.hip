@@ -977,8 +977,7 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   if (a_here) {
     g.P = (const __bf16*)a_dev; g.strideP = a_batch_stride; g.ldp = lda;
   } else {
-    e = launch_layout(a_dev, MUON_DTYPE_BF16, 0, a_batch_stride, lda, batch, n, k, nullptr, Ap,
-                      (long)Np * Kp, Kp, Np, Kp, nullptr, 0, 0, stream);
+    e = launch_layout(a_dev, a_batch_stride, lda, batch, n, k, Ap, (long)Np * Kp, Kp, Np, Kp, stream);
     if (e != hipSuccess) return (int)e;
     g.P = Ap; g.strideP = (long)Np * Kp; g.ldp = Kp;
   }
@@ -986,8 +985,7 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   if (c_here) {
     g.E = (const __bf16*)c_dev; g.strideE = c_batch_stride; g.lde = ldc;
   } else if (c_dev) {
-    e = launch_layout(c_dev, MUON_DTYPE_BF16, 0, c_batch_stride, ldc, batch, n, n, nullptr, Cp, (long)Np * Np, Np, Np,
-                      Np, nullptr, 0, 0, stream);
+    e = launch_layout(c_dev, c_batch_stride, ldc, batch, n, n, Cp, (long)Np * Np, Np, Np, Np, stream);
     if (e != hipSuccess) return (int)e;
     g.E = Cp; g.strideE = (long)Np * Np; g.lde = Np;
   }
@@ -1149,12 +1147,8 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
       const int nb = std::min(LAYOUT_PTRS_MAX, P.q.batch - b0);
       for (int k = 0; k < nb; ++k) lp.p[k] = P.q.w_ptrs[b0 + k];
       __bf16* dst = P.X + (size_t)b0 * xs;
-      if (!P.use_t)
-        e = launch_layout_ptrs(lp, nb, P.q.dtype, P.q.ld, P.q.rows, P.q.cols, dst, xs, pl.Np, pl.Mp, pl.Np, nullptr, 0, 0,
-                               stream, P.xpart + (size_t)b0 * xt);
-      else
-        e = launch_layout_ptrs(lp, nb, P.q.dtype, P.q.ld, P.q.rows, P.q.cols, nullptr, 0, 0, pl.Np, pl.Mp, dst, xs, pl.Np,
-                               stream, P.xpart + (size_t)b0 * xt);
+      e = launch_layout_ptrs(lp, nb, P.q.dtype, P.q.ld, P.q.rows, P.q.cols, dst, P.use_t, xs, pl.Np, P.use_t ? pl.Np : pl.Mp,
+                             P.use_t ? pl.Mp : pl.Np, stream, P.xpart + (size_t)b0 * xt);
       if (e != hipSuccess) return (int)e;
     }
   }

@@ -54,24 +54,19 @@ static_assert(sizeof(StageParams) <= 4096, "kernel arguments are limited to 4 Ki
 bool stage_blocks(const StageProblem& p, long* sum_blocks, long* tiles);
 hipError_t launch_stage(const StageParams& p, hipStream_t stream);
 
-// D = bf16(scale*in) in the input's orientation and T = its transpose (either may be null), both zero-padded to
-// d_rows x d_cols / d_cols x d_rows (multiples of 64); scale may be null (= 1).  tile_sumsq (optional): the sum of
-// squares of the values written, one float per 64x64 tile: [batch][d_rows / 64][d_cols / 64].
-hipError_t launch_layout(const void* in, int in_dtype, int cast_first, long in_bstride, int ld, int batch, int rows,
-                         int cols, const float* scale, void* D, long d_bstride, int ldd, int d_rows, int d_cols,
-                         void* T, long t_bstride, int ldt, hipStream_t stream, int out_f16 = 0, int out_shift = 0,
-                         float* tile_sumsq = nullptr);
+// D = a batch of bf16 matrices as they are, zero padded to d_rows x d_cols (multiples of 64)
+hipError_t launch_layout(const void* in, long in_bstride, int ld, int batch, int rows, int cols, void* D, long d_bstride, int ldd,
+                         int d_rows, int d_cols, hipStream_t stream);
 
-// the same pass over up to LAYOUT_PTRS_MAX matrices of one shape that are separate allocations (pointers by value, as
-// they are: no scale, bf16 output), one launch: matrix i goes to D + i * d_bstride / T + i * t_bstride and its tile sums
-// to tile_sumsq + i * (d_rows / 64) * (d_cols / 64)
+// bf16(in) of up to LAYOUT_PTRS_MAX matrices of one shape that are separate allocations (pointers by value), one launch:
+// matrix i goes to dst + i * dst_bstride, zero padded to d_rows x d_cols, or transposed to d_cols x d_rows.  tile_sumsq: the
+// sum of squares of the values written, one float per 64x64 tile, matrix i at tile_sumsq + i * (d_rows / 64) * (d_cols / 64).
 constexpr int LAYOUT_PTRS_MAX = 64;
 struct LayoutPtrs {
   const void* p[LAYOUT_PTRS_MAX];
 };
-hipError_t launch_layout_ptrs(const LayoutPtrs& ptrs, int n_mats, int in_dtype, int ld, int rows, int cols, void* D,
-                              long d_bstride, int ldd, int d_rows, int d_cols, void* T, long t_bstride, int ldt,
-                              hipStream_t stream, float* tile_sumsq);
+hipError_t launch_layout_ptrs(const LayoutPtrs& ptrs, int n_mats, int in_dtype, int ld, int rows, int cols, void* dst, bool transpose,
+                              long dst_bstride, int ldd, int d_rows, int d_cols, hipStream_t stream, float* tile_sumsq);
 
 // momentum fused with the layout pass of the Newton-Schulz operand (see momentum_layout_kernel): one launch covers up
 // to MOMG_MAX_MATS matrices (separate allocations: pointers by value) of up to MOMG_MAX_CLS shape classes, either all by

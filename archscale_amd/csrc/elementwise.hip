@@ -316,20 +316,17 @@ __device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, in
   }
 }
 
-template <int DT, bool CAST_FIRST>
+template <int DT>
 __global__ void __launch_bounds__(256)
-normalize_layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstride, int rows, int cols, int ld,
-                        const float* __restrict__ scale,
-                        uint16_t* __restrict__ D, long d_bstride, int ldd, int d_rows, int d_cols,
-                        uint16_t* __restrict__ T, long t_bstride, int ldt, int out_f16, int out_shift,
-                        float* __restrict__ tile_sumsq) {
+layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstride, int rows, int cols, int ld,
+              uint16_t* __restrict__ D, uint16_t* __restrict__ T, long bstride, int ldd, int ldt, int d_rows, int d_cols,
+              float* __restrict__ tile_sumsq) {
   const int b = blockIdx.z;
   // the matrices of the batch: equally spaced from `in`, or (in == null) separate allocations listed in `ptrs`
   const char* base = in ? (const char*)in + (size_t)b * in_bstride * sizeof(typename Elem<DT>::T) : (const char*)ptrs.p[b];
-  layout_tile<DT, CAST_FIRST>(base, !in || in_bstride % 8 == 0, blockIdx.y, blockIdx.x, rows, cols, ld, scale ? scale[b] : 1.f,
-                              D ? D + (size_t)b * d_bstride : nullptr, ldd, d_rows, d_cols,
-                              T ? T + (size_t)b * t_bstride : nullptr, ldt, out_f16, out_shift,
-                              tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr);
+  layout_tile<DT, false>(base, !in || in_bstride % 8 == 0, blockIdx.y, blockIdx.x, rows, cols, ld, 1.f,
+                         D ? D + (size_t)b * bstride : nullptr, ldd, d_rows, d_cols, T ? T + (size_t)b * bstride : nullptr, ldt,
+                         0, 0, tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr);
 }
 
 // The copies of a staging launch.  Launch bound for all but the largest calls, hence one launch over all matrices and no
@@ -383,41 +380,33 @@ bool stage_blocks(const StageProblem& p, long* sum_blocks, long* tiles) {
 }
 
 namespace {
-hipError_t launch_layout_impl(const void* in, const LayoutPtrs& ptrs, int in_dtype, int cast_first, long in_bstride, int ld,
-                              int batch, int rows, int cols, const float* scale, void* D, long d_bstride, int ldd,
-                              int d_rows, int d_cols, void* T, long t_bstride, int ldt, hipStream_t stream, int out_f16,
-                              int out_shift, float* tile_sumsq) {
-  if (batch > 65535 || d_rows / 64 > 65535 || d_rows % 64 || d_cols % 64) return hipErrorInvalidValue;
-  dim3 g3(d_cols / 64, d_rows / 64, batch);
-#define ARCHSCALE_NL(DT, CF)                                                                                   \
-  hipLaunchKernelGGL((normalize_layout_kernel<DT, CF>), g3, dim3(256), 0, stream, in, ptrs, in_bstride, rows,  \
-                     cols, ld, scale, (uint16_t*)D, d_bstride, ldd, d_rows, d_cols, (uint16_t*)T, t_bstride,   \
-                     ldt, out_f16, out_shift, tile_sumsq)
-  if (in_dtype == DT_BF16) ARCHSCALE_NL(DT_BF16, false);
-  else if (cast_first) ARCHSCALE_NL(DT_F32, true);
-  else ARCHSCALE_NL(DT_F32, false);
-#undef ARCHSCALE_NL
-  return hipGetLastError();
+bool layout_grid(int batch, int d_rows, int d_cols, dim3* grid) {
+  *grid = dim3(d_cols / 64, d_rows / 64, batch);
+  return batch <= 65535 && d_rows / 64 <= 65535 && d_rows % 64 == 0 && d_cols % 64 == 0;
 }
 }  // namespace
 
-hipError_t launch_layout(const void* in, int in_dtype, int cast_first, long in_bstride, int ld, int batch, int rows,
-                         int cols, const float* scale, void* D, long d_bstride, int ldd, int d_rows, int d_cols,
-                         void* T, long t_bstride, int ldt, hipStream_t stream, int out_f16, int out_shift,
-                         float* tile_sumsq) {
-  if (!in) return hipErrorInvalidValue;
-  return launch_layout_impl(in, LayoutPtrs{}, in_dtype, cast_first, in_bstride, ld, batch, rows, cols, scale, D, d_bstride,
-                            ldd, d_rows, d_cols, T, t_bstride, ldt, stream, out_f16, out_shift, tile_sumsq);
+hipError_t launch_layout(const void* in, long in_bstride, int ld, int batch, int rows, int cols, void* D, long d_bstride, int ldd,
+                         int d_rows, int d_cols, hipStream_t stream) {
+  dim3 grid;
+  if (!in || !layout_grid(batch, d_rows, d_cols, &grid)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(layout_kernel<DT_BF16>, grid, dim3(256), 0, stream, in, LayoutPtrs{}, in_bstride, rows, cols, ld, (uint16_t*)D,
+                     (uint16_t*)nullptr, d_bstride, ldd, 0, d_rows, d_cols, (float*)nullptr);
+  return hipGetLastError();
 }
 
-hipError_t launch_layout_ptrs(const LayoutPtrs& ptrs, int n_mats, int in_dtype, int ld, int rows, int cols, void* D,
-                              long d_bstride, int ldd, int d_rows, int d_cols, void* T, long t_bstride, int ldt,
-                              hipStream_t stream, float* tile_sumsq) {
-  if (n_mats < 1 || n_mats > LAYOUT_PTRS_MAX) return hipErrorInvalidValue;
+hipError_t launch_layout_ptrs(const LayoutPtrs& ptrs, int n_mats, int in_dtype, int ld, int rows, int cols, void* dst, bool transpose,
+                              long dst_bstride, int ldd, int d_rows, int d_cols, hipStream_t stream, float* tile_sumsq) {
+  dim3 grid;
+  if (n_mats < 1 || n_mats > LAYOUT_PTRS_MAX || !layout_grid(n_mats, d_rows, d_cols, &grid)) return hipErrorInvalidValue;
   for (int i = 0; i < n_mats; ++i)
     if (!ptrs.p[i]) return hipErrorInvalidValue;
-  return launch_layout_impl(nullptr, ptrs, in_dtype, 0, 0, ld, n_mats, rows, cols, nullptr, D, d_bstride, ldd, d_rows,
-                            d_cols, T, t_bstride, ldt, stream, 0, 0, tile_sumsq);
+  uint16_t *D = transpose ? nullptr : (uint16_t*)dst, *T = transpose ? (uint16_t*)dst : nullptr;
+  const void* none = nullptr;
+  auto kernel = in_dtype == DT_BF16 ? layout_kernel<DT_BF16> : layout_kernel<DT_F32>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, none, ptrs, 0L, rows, cols, ld, D, T, dst_bstride, ldd, ldd, d_rows, d_cols,
+                     tile_sumsq);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------

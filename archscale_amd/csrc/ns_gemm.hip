@@ -29,16 +29,14 @@
 #include "ns_gemm.h"
 
 // The epilogue arithmetic is written out with explicit fmaf() and the compiler forms no fused operations of its own:
-// the same element is computed by different code depending on the grid (wave-local or block-cooperative epilogue,
-// 256x256 or 128x128 configuration), and all of them have to round in the same places for the result of a matrix not to
+// the same element is computed by different code depending on the grid (tiles of 256, 128 or 64, straight or mirrored
+// image), and all of them have to round in the same places for the result of a matrix not to
 // depend on how the launch was cut into blocks.  Left to itself the compiler fuses a multiply-add with the conversion
 // to half in one path and not in the other.
 #pragma clang fp contract(off)
 
 namespace archscale {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -64,14 +62,6 @@ __device__ __forceinline__ uint16_t f16_bits(float f) {
   return __builtin_bit_cast(uint16_t, (_Float16)f);
 }
 __device__ __forceinline__ float f16_to_f32(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
-  uint2 r;
-  r.x = (uint32_t)bf16_bits(a) | ((uint32_t)bf16_bits(b) << 16);
-  r.y = (uint32_t)bf16_bits(c) | ((uint32_t)bf16_bits(d) << 16);
-  return r;
-}
 
 // LDS placement of the 16-byte chunk (row r, k-chunk c) of a [rows][64] bf16 tile.
 // XOR with (r>>1)&7 makes any 16 consecutive rows at one k-chunk hit 16 distinct
@@ -148,7 +138,7 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 1
 // with four waves and 16x16x32 MFMAs, 1280 to 1300 with a third LDS stage for Q (zero operands, where power does not
 // limit: 1320 / 1330 / 1525).  A persistent form whose copies run on into the next tile measured the same (1300).
 //
-// LDS: SP stages of the P tile and SQ of the Q tile (SQ = SP or SP + 1).  The 256 configuration has room for 2 + 3: the
+// LDS: SP stages of the P tile and SQ = SP + 1 of the Q tile.  The 256 configuration has room for 2 + 3: the
 // operand that streams from memory (Q = X^T) gets two k-tiles of time to arrive, P, which the caches hold, gets one.
 template <int BT, int SP, int SQ, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
 __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
@@ -165,7 +155,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   constexpr int OPBYTES = BT * ROW_BYTES;   // one stage of one operand
   constexpr int NC = BT / 8 / NW;       // copies (1 KiB: 8 rows x 128 B) per wave, operand and k-tile
   static_assert(BT % (8 * NW) == 0, "tile rows must split over waves");
-  static_assert(SP >= 2 && (SQ == SP || SQ == SP + 1), "stages");
+  static_assert(SP >= 2 && SQ == SP + 1, "stages");
   // MODE_SYRKT is MODE_SYRK with the operand given K-major: P = Q = X^T stored [K][M] (leading dimension ldp), so the
   // iteration needs no row-major copy of X at all; the MFMA fragments then come from LDS transpose reads
   constexpr bool KMAJ = (MODE == MODE_SYRKT);
@@ -442,22 +432,21 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
   // one k-step: MFMAs on fragment set CBUF (when ACTIVE), reads of k-step RKK of the stages at (rsP, rsQ) into the other
-  // set, copies of P to stage dP (when CP) and of Q to stage dQ (when CQ) from src
-  auto kstep = [&](auto active, auto cbuf_, int rsP, int rsQ, auto rkk_, auto cp, auto cq, const Source& src, int dP, int dQ) __attribute__((always_inline)) {
-    constexpr bool ACTIVE = decltype(active)::value, CP = decltype(cp)::value, CQ = decltype(cq)::value;
+  // set, copies of P to stage dP (when CP) or of Q to stage dQ from src
+  auto kstep = [&](auto active, auto cbuf_, int rsP, int rsQ, auto rkk_, auto cp, const Source& src, int dP, int dQ) __attribute__((always_inline)) {
+    constexpr bool ACTIVE = decltype(active)::value, CP = decltype(cp)::value;
     constexpr int cbuf = decltype(cbuf_)::value;
-    constexpr int NCOPY = (CP ? NC : 0) + (CQ ? NC : 0);
     // reads within the first three quarters of the k-step, copies over all of it
     constexpr int RSPAN = NMF * 3 / 4;
     static_for<NMF>([&](auto q_) __attribute__((always_inline)) {
       constexpr int q = decltype(q_)::value;
       if constexpr (ACTIVE) mfma16<IN16, AGPR>(acc[q / FR][q % FR], af[cbuf][q / FR], bq[cbuf][q % FR]);
       __builtin_amdgcn_sched_barrier(0);
-      constexpr int c_lo = (q * NCOPY + NMF - 1) / NMF, c_hi = ((q + 1) * NCOPY + NMF - 1) / NMF;
+      constexpr int c_lo = (q * NC + NMF - 1) / NMF, c_hi = ((q + 1) * NC + NMF - 1) / NMF;
       static_for<c_hi - c_lo>([&](auto d_) __attribute__((always_inline)) {
         constexpr int c = c_lo + decltype(d_)::value;
-        if constexpr (CP && c < NC) copyP(src, dP, c);
-        else copyQ(src, dQ, CP ? c - NC : c);
+        if constexpr (CP) copyP(src, dP, c);
+        else copyQ(src, dQ, c);
       });
       if constexpr (ACTIVE) {
         constexpr int r_lo = q < RSPAN ? (q * NRD + RSPAN - 1) / RSPAN : NRD, r_hi = q + 1 < RSPAN ? ((q + 1) * NRD + RSPAN - 1) / RSPAN : NRD;
@@ -471,12 +460,10 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   };
   auto nextP = [](int s) { return s + OPBYTES == SP * OPBYTES ? 0 : s + OPBYTES; };
   auto nextQ = [](int s) { return s + OPBYTES == QBASE + SQ * OPBYTES ? QBASE : s + OPBYTES; };
-  // In k-tile kt: Q of k-tile kt + SP in the first k-step when Q has the extra stage (the stage of kt - 1 is free), else
-  // after the barrier like P of kt + SP.  In flight at the barrier, younger than what it publishes:
+  // In k-tile kt: Q of k-tile kt + SP in the first k-step (its extra stage is the one of kt - 1, which is free), P of it after
+  // the barrier.  In flight at the barrier, younger than what it publishes:
   constexpr int PAIR = 2 * NC;
-  constexpr int INFLIGHT = (SP - 2) * PAIR + (SQ > SP ? NC : 0);
-  using QX = std::integral_constant<bool, (SQ > SP)>;
-  using QN = std::integral_constant<bool, (SQ == SP)>;
+  constexpr int INFLIGHT = (SP - 2) * PAIR + NC;
   auto k_range = [&](auto active) __attribute__((always_inline)) {
     constexpr bool ACTIVE = decltype(active)::value;
     int sP = 0, sQ = QBASE;               // stages of k-tile kt
@@ -486,14 +473,14 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     }
     for (int kt = 0; kt < KT_ALL; ++kt) {
       const int nP = nextP(sP), nQ = nextQ(sQ);
-      // the Q stage before this one in the ring is the one that k-tile kt + SP goes to when Q has the extra stage
+      // the Q stage before this one in the ring is the one that k-tile kt + SP goes to
       const int pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
       const Source src = source(kt + SP);
-      kstep(active, I0{}, sP, sQ, I1{}, No{}, QX{}, src, 0, pQ);
+      kstep(active, I0{}, sP, sQ, I1{}, No{}, src, 0, pQ);
       wait_copies<INFLIGHT>();
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      kstep(active, I1{}, nP, nQ, I0{}, Yes{}, QN{}, src, sP, sQ);
+      kstep(active, I1{}, nP, nQ, I0{}, Yes{}, src, sP, 0);
       sP = nP;
       sQ = nQ;
     }
