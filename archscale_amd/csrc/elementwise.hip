@@ -909,16 +909,13 @@ __device__ __forceinline__ float fast_div(float m, float d) {
 
 // The direction M / (sqrt(V) / bias2_sqrt + eps) [/ bias1] as (M dm) / (sqrt(V) + de) with dm = bias2_sqrt [/ bias1] and
 // de = eps bias2_sqrt: one division per element instead of three, with as many roundings.  sqrt(V) is zero, infinite or
-// between 2^-75 and 2^64, so what fast_div needs is a matter of `de` alone (2^-100 and not 2^-126 below: an M dm that is no
-// normal number is then off by at most 2^-49 of a direction of one).  With an eps outside, 1e-37 say, the direction is formed
-// as written, with IEEE divisions, off the vector path.
-struct Direction {
-  float dm, de;
-  bool in_range;
-};
+// between 2^-75 and 2^64, so what fast_div needs is a matter of `de` alone: with an eps that takes de near an end of the range
+// (1e-37 say) the denominator carries a power of two `s`, which the quotient gets back; otherwise s = 1 and changes no bit.
+struct Direction { float dm, de, s; };
 __device__ __forceinline__ Direction direction_of(const ScalarHyper& h, bool with_bias1) {
-  const float de = h.eps * h.bias2_sqrt, a = fabsf(de);
-  return {with_bias1 ? h.bias2_sqrt / h.bias1 : h.bias2_sqrt, de, h.eps == 0.f || (a >= 0x1p-100f && a <= 0x1p125f)};
+  const float a = fabsf(h.eps * h.bias2_sqrt);
+  const float s = h.eps != 0.f && a < 0x1p-100f ? 0x1p40f : (a > 0x1p100f ? 0x1p-40f : 1.f);
+  return {with_bias1 ? h.bias2_sqrt / h.bias1 : h.bias2_sqrt, h.eps * (h.bias2_sqrt * s), s};
 }
 
 // one element; returns the new weight, updates m, v (as rounded to their dtypes), accumulates sums
@@ -941,8 +938,7 @@ __device__ __forceinline__ float scalar_elem(float x, float g, float& m, float& 
     const float g2 = round_v(gm * gm);
     v = round_v(v + h.w2 * (g2 - v));                          // V <- lerp(V, G*G, 1-beta2)
   }
-  if (dir.in_range) u = fast_div(m * dir.dm, sqrtf(v) + dir.de);
-  else u = m / (sqrtf(v) / h.bias2_sqrt + h.eps) / (PHASE == 0 ? 1.f : h.bias1);
+  u = fast_div(m * dir.dm, fmaf(sqrtf(v), dir.s, dir.de)) * dir.s;
   const float xd = decayed(x, u, h.lr_wd, h.cautious);
   if (PHASE == 0) return xd - lr1 * u;
   if (PHASE == 1) { s[0] += xd * xd; s[1] += u * u; s[2] += xd * u; return x; }
@@ -1025,7 +1021,7 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
   const Direction dir = direction_of(h, PHASE != 0);
   const float lr1 = h.lr / h.bias1;
   float s[3] = {0.f, 0.f, 0.f};
-  if (vec_ok && (ALGO == ALGO_LION || dir.in_range)) {
+  if (vec_ok) {
     // Bound by memory once the arithmetic is out of the way: the update of one element was about 100 vector instructions
     // (three IEEE divisions, a branch on the dtype per conversion), four clocks each.  206 million bf16 elements of two
     // vocabulary matrices: phase 1 678 -> 459 us (5.4 TB/s), phase 2 400 -> 280 us (5.9 TB/s).
