@@ -54,7 +54,9 @@ const EnvSwitches& env_switches() {
 
 int pick_tile(int m, int n) {
   if (env_switches().tile) return env_switches().tile;
-  // padded work, with the small tile charged for its lower arithmetic intensity
+  // padded work, with the small tile charged for its lower rate: full launches of it run at 0.71 to 0.93 of the large one's,
+  // by product and size (TFLOP/s, 128 / 256: X' = BX of 16 x 2048 x 5632 1064 / 1359, of 32 x 2048 x 2048 951 / 1342, of
+  // 64 x 1024 x 1024 835 / 1098; X X^T of 16 x 2048 x 5632 1030 / 1238, cAA+bA 834 / 999)
   auto cost = [&](int t, double penalty) {
     const double Mp = (double)round_up(m, t), Np = (double)round_up(n, t);
     return Mp * Mp * (3.0 * Np + Mp) * penalty;
@@ -71,9 +73,9 @@ inline long sym_tiles(int t) { return (long)t * (t + 1) / 2; }
 // k-tiles.  Only long reductions (KT >= 128, i.e. K >= 8192) of matrices with at least 16 tiles left over are split: the
 // partial results cost 64 KiB of traffic per block each way, which a block of 32 or more k-tiles hides, and a batch of
 // many small matrices (whose launches are full anyway) must not pay for it.  Measured on single matrices (us per
-// product, 2 / 4 / 8 parts against none): the 136 tiles of a 4096 x 14336 matrix 330 / 315 / 366 against 378, the 16 tiles
-// left over by an 8192 x 8192 matrix 55 / 40 / 43 against 83; a batch of eight 8192 x 8192 matrices, which needs no split,
-// pays 1.5 % of its time for the partial results.
+// product, 2 / 4 / 8 parts against none): X X^T of 4096 x 14336, 136 tiles, 252 / 254 / 301 against 258 (its first one, on the
+// input as it is, 277 / 261 / 307 against 314); the 16 tiles left over by an 8192 x 8192 matrix 42 / 32 / 38 against 36.  Whole
+// calls 3.12 -> 3.07 and 7.63 -> 7.61 ms; a batch of eight 8192 x 8192 matrices, which needs no split, pays 0.9 % of its time.
 struct SkRule { int full, rem, parts; };
 constexpr int SK_PARTS = 4, SK_MIN_KT = 128, SK_MIN_REM = 16;
 SkRule sk_rule(int tm, int KT) {
@@ -391,7 +393,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   // tiles takes the 128x128 configuration for every problem: four times the blocks, a quarter of the time per block.
   // A call whose problems would take both configurations one by one pays for a second launch of every product, about 10 us
   // each: where that is more than the padding or the lower rate of ONE configuration costs, all problems take the cheaper one.
-  // (In the units of `work`, flops of an iteration at about 1250 TFLOP/s; the small configuration runs at 0.8 of that.)
+  // (In the units of `work`, flops of an iteration at about 1250 TFLOP/s; the small configuration is charged as in pick_tile.)
   long sym_blocks = 0;
   bool uses[2] = {false, false}, ksplit = false;   // 256, 128
   double mixed = 0.0, all_256 = 0.0, all_128 = 0.0;

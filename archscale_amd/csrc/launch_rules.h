@@ -10,13 +10,15 @@ namespace archscale {
 struct LaunchSplit { int whole, quarters, sixteenths; };
 
 // Tiles of 256, more than one round (one tile per unit) of them: the full rounds run as they are, a last round of at most
-// QUARTER_MAX_TAIL tiles is quartered: a quarter of the time per block instead of a whole round for a few tiles (measured: a
-// tail of 160 tiles on the depth-16 set costs 83 us quartered against 57 us as it is; tails of 16 and 128 tiles of single
-// 8192x8192 and 4096x14336 matrices: 10.33 -> 9.80 ms and 4.58 -> 4.44 ms per call).
+// QUARTER_MAX_TAIL tiles is quartered.  A round of quadrants alone runs at about 0.6 of the rate of a full round of large tiles
+// (it neither overlaps the stores of the round before nor shares operand panels as well), but it takes time only for the tiles
+// that are there.  Per product: leftovers of 64 tiles (X X^T of 16 x 2048 x 5632) 379 -> 324 us, of 128 (X X^T of 32 x 2048 x
+// 2048; X' = BX of 4096 x 14336) 274 -> 264 and 355 -> 333; of 160 (X X^T of the depth-16 set) 1173 us as it is, 1218
+// quartered; of 176 (X' = BX of the EMA-Muon set of width 1024) 90 as it is, 93 quartered.
 // Less than one round: as tiles of 256 the launch takes as long as its longest tile; quartered, the tiles spread over the
-// chip, at about 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
-// (208 tiles of 2816 and 1024 k-values, five fp32 EMA-Muon products) the step takes 1250 us quartered, 1318 as it is; at 0.625
-// (160 equal tiles, power iteration over 16 x 1024 x 2816) 337 against 317 us.
+// chip, at the same 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
+// (208 tiles of 2816 and 1024 k-values, X X^T of that EMA-Muon set) a product takes 56 us quartered, 66 as it is; at 0.625
+// (160 equal tiles, power iteration over 16 x 1024 x 2816) the call takes 337 against 317 us.
 //
 // Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
 // a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x

@@ -30,7 +30,7 @@ def msign_schedule(steps: int) -> List[Tuple[float, float, float]]:
 @torch.no_grad()
 def msign(G: torch.Tensor, steps: int) -> torch.Tensor:
     """fp32 in, bf16 out: normalise in fp32 with ``max(|G|, 1e-7)``, round to bf16, iterate.
-    The steep first row of the table needs B = bA + cA^2 as a bf16 hi+lo pair to stay within 1e-2 of fp32."""
+    The steep first row of the table needs the half-precision workspace to stay within 1e-2 of fp32."""
     if G.ndim < 2:
         raise ValueError("Input tensor must have at least 2 dimensions.")
     if G.dtype != torch.float32:
