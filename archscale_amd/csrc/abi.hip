@@ -200,9 +200,8 @@ hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const Grouped
 // leave the chip idle (launch_rules.h).  ARCHSCALE_MUON_QUARTER=0 switches that off.
 // (work: the FLOPs of a Newton-Schulz launch for its timing record; null: a product of another entry point, not recorded)
 struct LaunchWork { double algorithmic, issued; };
-hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream,
+hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, hipStream_t stream, int units,
                          const LaunchWork* work, int f16) {
-  const int units = compute_units();
   auto launch = [&](int t, const GroupedGemmParams& g, double share) -> hipError_t {
     if (!work) return launch_ns_gemm_grouped(t, mode, split, final_, g, stream, units, f16);
     return timed_gemm(t, mode, split, final_, g, stream, units, work->algorithmic * share, work->issued * share, f16);
@@ -394,6 +393,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   // A call whose problems would take both configurations one by one pays for a second launch of every product, about 10 us
   // each: where that is more than the padding or the lower rate of ONE configuration costs, all problems take the cheaper one.
   // (In the units of `work`, flops of an iteration at about 1250 TFLOP/s; the small configuration is charged as in pick_tile.)
+  const int units = compute_units();
   long sym_blocks = 0;
   bool uses[2] = {false, false}, ksplit = false;   // 256, 128
   double mixed = 0.0, all_256 = 0.0, all_128 = 0.0;
@@ -413,7 +413,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   int force_tile = 0;
   if (!env_switches().tile) {
     constexpr double SECOND_LAUNCHES = 3.1e10;   // 25 us of an iteration
-    if (sym_blocks * 2 < compute_units()) force_tile = 128;
+    if (sym_blocks * 2 < units) force_tile = 128;
     else if (uses[0] && uses[1] && !ksplit && std::min(all_256, all_128) < mixed + SECOND_LAUNCHES)
       force_tile = all_128 < all_256 ? 128 : 256;
   }
@@ -595,7 +595,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       const int key = 128 * 100 + mode * 10;
       const GroupedGemmParams launch = sk;
       hipError_t err = timed_launch(key, sk_fa, sk_fi, stream, [&] {
-        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, compute_units(), ws16, true);
+        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, units, ws16, true);
       });
       sk = GroupedGemmParams{};
       sk.quarter = 1;
@@ -608,7 +608,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
         const LaunchWork work = {fa, fi};
-        hipError_t err = launch_rounds(tile, mode, split_launch, final_, gp, stream, &work, ws16);
+        hipError_t err = launch_rounds(tile, mode, split_launch, final_, gp, stream, units, &work, ws16);
         gp = GroupedGemmParams{};
         fa = fi = 0.0;
         return err;
@@ -1002,7 +1002,7 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   gp.n_groups = 1;
   gp.g[0] = g;
   gp.tile_start[1] = (int)tiles;
-  e = launch_rounds(tile, mode, false, false, gp, stream, nullptr, 0);
+  e = launch_rounds(tile, mode, false, false, gp, stream, compute_units(), nullptr, 0);
   if (e != hipSuccess || d_here) return (int)e;
   return (int)launch_unpad_copy(Dp, (long)Np * Np, Np, d_dev, d_batch_stride, ldd, batch, n, n, stream);
 }
@@ -1113,6 +1113,7 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
   // the transpose of the stored block
   struct Prob { muon_sn_problem q; SnPlan sp; __bf16 *X, *G, *G2, *G4; float *xscale, *xpart, *z, *part; bool tall, use_t; };
   const int levels = spectral_power_levels(steps);
+  const int units = compute_units();
   std::vector<Prob> pr(n_problems);
   size_t off = 0;
   for (int i = 0; i < n_problems; ++i) {
@@ -1161,7 +1162,7 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
       GroupedGemmParams gp = {};
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
-        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, nullptr, 0);
+        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, units, nullptr, 0);
         gp = GroupedGemmParams{};
         return err;
       };
