@@ -1,9 +1,25 @@
-// How the tiles of one product launch are cut for the chip: host arithmetic only (no HIP), so that it can be checked on any
+// How the tiles of one product launch are cut for the chip: plain arithmetic (no HIP), so that it can be checked on the host for any
 // number of compute units.  `units` is what the current device reports; the measured lines are those of 256 units (one MI355X)
 // and are scaled with it.  A choice made here never changes a result: the sums of an element are the same in every configuration.
 #pragma once
+#include <stdint.h>
 
 namespace archscale {
+
+// Division by multiplication, for the start of a tile (host and device): quotient and rest of x / d for 0 <= x < 2^31 and
+// 0 < d < 2^31 with inv = reciprocal(d).  The estimate is at most one too small.
+constexpr uint32_t reciprocal(int d) { return 0xffffffffu / (uint32_t)d; }
+constexpr int divide(int x, int d, uint32_t inv, int& rest) {
+  uint32_t q = (uint32_t)(((uint64_t)(uint32_t)x * inv) >> 32), r = (uint32_t)x - q * (uint32_t)d;
+  if (r >= (uint32_t)d) { ++q; r -= (uint32_t)d; }
+  rest = (int)r;
+  return (int)q;
+}
+// x / d for d = 1 .. 4 and 0 <= x < 2^31
+constexpr int divide_1_to_4(int x, int d) {
+  const int third = (int)(((uint64_t)(uint32_t)x * 0xaaaaaaabu) >> 33);
+  return d == 4 ? x >> 2 : (d == 3 ? third : (d == 2 ? x >> 1 : x));
+}
 
 // Tiles with numbers [0, whole) of a launch run as they are, the next `quarters` as four tiles of half the side each, the next
 // `sixteenths` as sixteen of a quarter of it.

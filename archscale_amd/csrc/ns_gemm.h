@@ -10,14 +10,25 @@ enum { MODE_SYRK = 0, MODE_SYRK2 = 1, MODE_BX = 2, MODE_SYRKT = 3 };
 
 // C[m][n] = sum_k P[m][k] * Q[n][k]; all leading dimensions / strides in elements.
 struct GemmParams {
+  // (what the start of a tile needs comes first and together)
   const __bf16* P;   // [batch][tilesM*BM][ldp]
-  const __bf16* P2;  // second pass over K for P (low half of a split B), or null
   const __bf16* Q;   // [batch][tilesN*BN][ldq]
   long strideP, strideQ;
   int ldp, ldq;
   int K;             // reduction length, multiple of 64
   int tilesM, tilesN;
+  int qt_first;          // quarter mode: first tile of this problem (in its own coarser enumeration) that is covered
+  // a launch may cover only tiles [t_first, t_first + t_count) of every matrix of the problem (in the matrix's own
+  // enumeration; t_count = 0: all of them), the flat tile index of the launch then counts t_count tiles per matrix
+  int t_first;
+  // filled in by the launch: tiles per matrix that it covers, reciprocals (floor((2^32 - 1) / d)) of that and of what a line
+  // of the tile order holds, blocks of one part of a K-split
+  int per_mat;
+  uint32_t inv_per_mat, inv_line;
+  int part_tiles;
+  int t_count;
   int batch;
+  const __bf16* P2;  // second pass over K for P (low half of a split B), or null
   const __bf16* E;   // epilogue addend, read as E[col][row..row+3]; MODE_BX: may be null (X' = B X, no addend)
   long strideE;
   int lde;
@@ -33,10 +44,6 @@ struct GemmParams {
   float diag_add;        // MODE_SYRK2: added to the diagonal of the result (B + a I, so that B X needs no addend)
   const float* scale;    // per batch element, or null: SYRK / SYRKT multiply the product by scale^2, BX the result by scale
   int m_valid, n_valid;  // true extents for the bounds-checked final store
-  int qt_first;          // quarter mode: first tile of this problem (in its own coarser enumeration) that is covered
-  // a launch may cover only tiles [t_first, t_first + t_count) of every matrix of the problem (in the matrix's own
-  // enumeration; t_count = 0: all of them), the flat tile index of the launch then counts t_count tiles per matrix
-  int t_first, t_count;
   // K-split (symmetric products of the 128x128 configuration only): `ksplit` > 1 blocks share every tile, block s of
   // them walks k-tiles [s KT / ksplit, (s + 1) KT / ksplit) and leaves its fp32 accumulators in sk_partial; the block
   // that finds itself last (sk_counter, one per tile, zero before the launch and zero again after it) adds the partial
@@ -57,7 +64,8 @@ constexpr int MAX_GROUPS = 16;
 struct GroupedGemmParams {
   int n_groups;
   int quarter;
-  int tile_start[MAX_GROUPS + 1];
+  int total;                        // filled in by the launch: tile_start[n_groups] ...
+  int tile_start[MAX_GROUPS + 1];   // ... and the places past n_groups, with the largest int
   GemmParams g[MAX_GROUPS];
 };
 static_assert(sizeof(GroupedGemmParams) <= 4096, "kernel arguments are limited to 4 KiB");

@@ -62,6 +62,18 @@ __device__ __forceinline__ uint16_t f16_bits(float f) {
   return __builtin_bit_cast(uint16_t, (_Float16)f);
 }
 __device__ __forceinline__ float f16_to_f32(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
+// two values at a time: one conversion instruction for both (converted one by one and put together afterwards they cost
+// four instructions more per pair, and the 256 values of a lane are what the epilogue spends its time on)
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+__device__ __forceinline__ uint32_t f16_pair(float a, float b) {
+  asm("" : "+v"(a), "+v"(b));   // (see f16_bits)
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
+}
 
 // LDS placement of the 16-byte chunk (row r, k-chunk c) of a [rows][64] bf16 tile.
 // XOR with (r>>1)&7 makes any 16 consecutive rows at one k-chunk hit 16 distinct
@@ -93,6 +105,44 @@ __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
+// What the start of a tile needs of its problem, and what its end needs.  The values are pinned to registers where they are
+// fetched: left alone the compiler fetches each where it is used, and every fetch is a wait of its own.
+struct TileArgs {
+  const __bf16 *P, *Q;
+  long strideP, strideQ;
+  int ldp, ldq, K, tilesM, tilesN, qt_first, t_first, per_mat;
+  uint32_t inv_per_mat, inv_line;
+  int part_tiles;
+};
+struct LaunchHead { int n_groups, quarter, total, first[3]; };   // first tiles of problems 1 to 3
+__device__ __forceinline__ TileArgs fetch_tile_args(const GemmParams& g) {
+  return TileArgs{g.P, g.Q, g.strideP, g.strideQ, g.ldp, g.ldq, g.K, g.tilesM, g.tilesN, g.qt_first, g.t_first,
+                  g.per_mat, g.inv_per_mat, g.inv_line, g.part_tiles};
+}
+#define ARCHSCALE_PIN_TILE_ARGS(a)                                                                                       \
+  "+s"(a.P), "+s"(a.Q), "+s"(a.strideP), "+s"(a.strideQ), "+s"(a.ldp), "+s"(a.ldq), "+s"(a.K), "+s"(a.tilesM), "+s"(a.tilesN), \
+      "+s"(a.qt_first), "+s"(a.t_first), "+s"(a.per_mat), "+s"(a.inv_per_mat), "+s"(a.inv_line), "+s"(a.part_tiles)
+__device__ __forceinline__ void pin(TileArgs& a) { asm volatile("" : ARCHSCALE_PIN_TILE_ARGS(a)); }
+__device__ __forceinline__ void pin(TileArgs& a, LaunchHead& h) {
+  asm volatile("" : ARCHSCALE_PIN_TILE_ARGS(a), "+s"(h.n_groups), "+s"(h.quarter), "+s"(h.total), "+s"(h.first[0]), "+s"(h.first[1]), "+s"(h.first[2]));
+}
+struct EndArgs {
+  // (a pointer that comes out of an assembler statement would count as a generic one)
+  const __attribute__((address_space(1))) __bf16* E;
+  __attribute__((address_space(1))) __bf16 *C, *Ct;
+  const __attribute__((address_space(1))) float* scale;
+  long strideE, strideC, strideCt;
+  int lde, ldc, ldct, out_shift, m_valid, n_valid;
+  float alpha, beta, diag_add;
+};
+__device__ __forceinline__ EndArgs end_args(const GemmParams& g) {
+  EndArgs a = {(const __attribute__((address_space(1))) __bf16*)g.E, (__attribute__((address_space(1))) __bf16*)g.C,
+               (__attribute__((address_space(1))) __bf16*)g.Ct, (const __attribute__((address_space(1))) float*)g.scale,
+               g.strideE, g.strideC, g.strideCt, g.lde, g.ldc, g.ldct, g.out_shift, g.m_valid, g.n_valid, g.alpha, g.beta, g.diag_add};
+  asm volatile("" : "+s"(a.E), "+s"(a.C), "+s"(a.Ct), "+s"(a.scale), "+s"(a.strideE), "+s"(a.strideC), "+s"(a.strideCt), "+s"(a.lde),
+                    "+s"(a.ldc), "+s"(a.ldct), "+s"(a.out_shift), "+s"(a.m_valid), "+s"(a.n_valid), "+s"(a.alpha), "+s"(a.beta), "+s"(a.diag_add));
+  return a;
+}
 // acc += a * b on the matrix cores.  Inline assembly with the accumulator as a read-write operand: the builtin leaves the
 // destination free, and over a software-pipelined loop the register allocator then rotates the accumulators with
 // register moves between the MFMAs (measured: half the issue rate).  What the assembler statement hides from the compiler
@@ -168,8 +218,8 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   auto enc = [](float f) { return (OUT16 && !FINAL) ? f16_bits(f) : bf16_bits(f); };
   auto pk4 = [&](float a, float b, float c, float d) {
     uint2 r;
-    r.x = (uint32_t)enc(a) | ((uint32_t)enc(b) << 16);
-    r.y = (uint32_t)enc(c) | ((uint32_t)enc(d) << 16);
+    if constexpr (OUT16 && !FINAL) { r.x = f16_pair(a, b); r.y = f16_pair(c, d); }
+    else { r.x = bf16_pair(a, b); r.y = bf16_pair(c, d); }
     return r;
   };
 
@@ -185,34 +235,51 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // XCD, i.e. in one L2, and successive runs go to successive XCDs so that long and short tiles of a
   // grouped launch spread evenly over the chip.  A launch of fewer than 8 * 32 tiles is dealt out in eight shorter runs:
   // runs of 32 would leave whole XCDs without work.
+  // All of this is paid at the start of every tile, before its first copy: there is no division in it (the host sends
+  // reciprocals), and it waits for the kernel arguments once - the first problem's come with the header, another
+  // problem's take a second wait.  From the start of a tile to its first copy, with the accumulators cleared behind the copies
+  // instead of before them: 1.1 to 2.2 -> 0.55 to 1.0 us (divisions and fields fetched where they are used before); the 64
+  // expert matrices of 512 x 2048 and 2048 x 256 1375 -> 1320 us per step, one 512 x 2048 matrix 130 -> 123 us per call, both
+  // together with the epilogue's paired conversions and running store addresses.
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int run = xcd_run(gp.tile_start[gp.n_groups]);
-  const int logical = ((slot / run) * 8 + xcd) * run + slot % run;
-  if (logical >= gp.tile_start[gp.n_groups]) return;
-  int grp = 0;
-  while (grp + 1 < gp.n_groups && logical >= gp.tile_start[grp + 1]) ++grp;
-  const GemmParams p = gp.g[grp];
-  int local = logical - gp.tile_start[grp];
+  TileArgs p = fetch_tile_args(gp.g[0]);
+  LaunchHead head = {gp.n_groups, gp.quarter, gp.total, {gp.tile_start[1], gp.tile_start[2], gp.tile_start[3]}};
+  pin(p, head);
+  const int total = head.total, quarter = head.quarter;
+  const int run = xcd_run(total);
+  const int lap = total < 256 ? 0 : slot >> 5;   // (a launch of fewer than 256 tiles has `run` slots per XCD)
+  const int logical = (lap * 8 + xcd) * run + slot - lap * run;
+  if (logical >= total) return;
+  int grp = 0, start = 0;
+  auto from = [&](int i, int first) { if (logical >= first) { grp = i; start = first; } };   // (past every tile for i >= n_groups)
+#pragma unroll
+  for (int i = 1; i <= 3; ++i) from(i, head.first[i - 1]);
+  if (head.n_groups > 4) {
+#pragma unroll
+    for (int i = 4; i < MAX_GROUPS; ++i) from(i, gp.tile_start[i]);
+  }
+  if (grp) {
+    p = fetch_tile_args(gp.g[grp]);
+    pin(p);
+  }
+  const GemmParams& g = gp.g[grp];
+  int local = logical - start;
   int ks = 0;   // part of the K range this block walks
   if constexpr (SK) {
-    const int launch_tiles = (gp.tile_start[grp + 1] - gp.tile_start[grp]) / p.ksplit;
-    ks = local / launch_tiles;
-    local -= ks * launch_tiles;
+    while (local >= p.part_tiles) { local -= p.part_tiles; ++ks; }   // (up to `ksplit` parts)
   }
   const int sk_tile = local;   // this tile among the problem's tiles in the launch
-  // grid the tile index is decoded in: the problem's own, or the 2x coarser one whose tiles this launch quarters
-  int dM = p.tilesM, dN = p.tilesN, quadrant = 0;
-  if (gp.quarter) {
-    quadrant = local & ((1 << 2 * gp.quarter) - 1);
-    local = p.qt_first + (local >> 2 * gp.quarter);
-    dM >>= gp.quarter;
-    dN >>= gp.quarter;
+  // grid the tile index is decoded in: the problem's own, or the coarser one whose tiles this launch quarters
+  int quadrant = 0;
+  const int dM = p.tilesM >> quarter, dN = p.tilesN >> quarter;
+  if (quarter) {
+    quadrant = local & ((1 << 2 * quarter) - 1);
+    local = p.qt_first + (local >> 2 * quarter);
   }
-  const int tiles_per_mat = SYM ? (dM * (dM + 1)) / 2 : dM * dN;
-  // the launch may cover only tiles [t_first, t_first + t_count) of every matrix
-  const int per_mat = p.t_count > 0 ? p.t_count : tiles_per_mat;
-  const int b = local / per_mat;
-  int t = p.t_first + (local - b * per_mat);
+  // the launch may cover only tiles [t_first, t_first + per_mat) of every matrix
+  int t;
+  const int b = divide(local, p.per_mat, p.inv_per_mat, t);
+  t += p.t_first;
   int ti, tj;
   if (SYM && dM > 8) {
     // A large upper triangle in blocks of 4 x 4 tiles, block row by block row (a diagonal block holds the 10 tiles of
@@ -246,23 +313,21 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     // per k-step.  Whole columns of dM tiles at a time would stream dM + 32 / dM panels (33 for dM = 32, 24 for 22).
     // The last block row and the last block of a row are as narrow as the grid leaves them (1 to 4 tiles).
     const int nbi = (dM + 3) >> 2, nbj = (dN + 3) >> 2;
-    int bi = t / (4 * dN);
-    if (bi >= nbi) bi = nbi - 1;
-    const int r = t - bi * 4 * dN;
+    int r, bi = divide(t, 4 * dN, p.inv_line, r);
+    if (bi >= nbi) { r += (bi - (nbi - 1)) * 4 * dN; bi = nbi - 1; }
     const int h = dM - 4 * bi < 4 ? dM - 4 * bi : 4;
-    int bj = r / (4 * h);
+    int bj = divide_1_to_4(r, h) >> 2;
     if (bj >= nbj) bj = nbj - 1;
     const int q = r - bj * 4 * h;
-    const int qc = q / h;
+    const int qc = divide_1_to_4(q, h);
     ti = 4 * bi + (q - qc * h);
     tj = 4 * bj + qc;
   } else {
-    tj = t / dM;   // up to 8 row panels: whole columns, 8 x 4 tiles per XCD for dM = 8
-    ti = t - tj * dM;
+    tj = divide(t, dM, p.inv_line, ti);   // up to 8 row panels: whole columns, 8 x 4 tiles per XCD for dM = 8
   }
-  if (gp.quarter) {
-    ti = (ti << gp.quarter) + (quadrant >> gp.quarter);
-    tj = (tj << gp.quarter) + (quadrant & ((1 << gp.quarter) - 1));
+  if (quarter) {
+    ti = (ti << quarter) + (quadrant >> quarter);
+    tj = (tj << quarter) + (quadrant & ((1 << quarter) - 1));
     if (SYM && ti > tj) return;   // lower part of a diagonal tile: its mirror image covers it
   }
   const int R0 = ti * BT, C0 = tj * BT;
@@ -274,7 +339,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   int KT = p.K / BK;
   if constexpr (SK) {
     // part ks of ksplit: k-tiles [ks KT / ksplit, (ks + 1) KT / ksplit), at least one (the host checks KT >= ksplit)
-    const int kt0 = (int)((long)ks * KT / p.ksplit), kt1 = (int)((long)(ks + 1) * KT / p.ksplit);
+    const int kt0 = (int)((long)ks * KT / g.ksplit), kt1 = (int)((long)(ks + 1) * KT / g.ksplit);
     Pb += KMAJ ? (size_t)kt0 * BK * p.ldp * 2 : (size_t)kt0 * ROW_BYTES;
     Qb += KMAJ ? (size_t)kt0 * BK * p.ldq * 2 : (size_t)kt0 * ROW_BYTES;
     KT = kt1 - kt0;
@@ -302,7 +367,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   }
   const uint32_t kstepP = KMAJ ? (uint32_t)BK * (uint32_t)p.ldp * 2u : (uint32_t)ROW_BYTES;
   const uint32_t kstepQ = KMAJ ? (uint32_t)BK * (uint32_t)p.ldq * 2u : (uint32_t)ROW_BYTES;
-  const char* P2b = KSPLIT ? (const char*)(p.P2 + (size_t)b * p.strideP + (size_t)R0 * p.ldp) : Pb;
+  const char* P2b = KSPLIT ? (const char*)(g.P2 + (size_t)b * p.strideP + (size_t)R0 * p.ldp) : Pb;
   // (the descriptors have to be seen to be uniform: each is a loop over the lanes otherwise)
   auto uniform = [](const char* q) {
     const uint64_t v = (uint64_t)q;
@@ -331,14 +396,16 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   };
   constexpr int QBASE = SP * OPBYTES;   // the Q stages follow the P stages
 
-  const int wr0 = (wave >> 1) * WT;     // wave origin inside the block tile
-  const int wc0 = (wave & 1) * WT;
-  // Diagonal tile of a symmetric product: wave (1, 0), whose sub-tile lies wholly BELOW the diagonal, computes nothing (it
-  // only takes part in the copies and the barriers); its part of the tile is the mirror image of the sub-tile of wave
-  // (0, 1), which writes it (a quarter of the tile's matrix-core work is saved).
-  const bool diag = SYM && (ti == tj);
-  const bool idle = diag && wave == 2;
-  const bool above = diag && wave == 1;
+  // first SP k-tiles, oldest first, on their way before anything else is set up (clearing 256 accumulators alone takes 1024 clk)
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    const Source src = source(s);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copyQ(src, QBASE + s * OPBYTES, j);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copyP(src, s * OPBYTES, j);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 
   f32x4 acc[FR][FR];
 #pragma unroll
@@ -349,6 +416,16 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   for (int i = 0; i < FR; ++i)
 #pragma unroll
     for (int j = 0; j < FR; ++j) acc_touch<AGPR>(acc[i][j]);
+  const EndArgs out = end_args(g);   // (the wait for them falls into the one for the first copies)
+
+  const int wr0 = (wave >> 1) * WT;     // wave origin inside the block tile
+  const int wc0 = (wave & 1) * WT;
+  // Diagonal tile of a symmetric product: wave (1, 0), whose sub-tile lies wholly BELOW the diagonal, computes nothing (it
+  // only takes part in the copies and the barriers); its part of the tile is the mirror image of the sub-tile of wave
+  // (0, 1), which writes it (a quarter of the tile's matrix-core work is saved).
+  const bool diag = SYM && (ti == tj);
+  const bool idle = diag && wave == 2;
+  const bool above = diag && wave == 1;
 
   // ---- operand fragments.  A k-tile is two k-steps of 32.  Fragment f of a wave in k-step kk holds, in lane l16 + 16 lg, the
   // eight k-values 32 kk + 8 lg .. + 7 of row (column) 16 f + l16 of the wave's sub-tile: one 16-byte read.
@@ -486,15 +563,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     }
   };
 
-  // first SP k-tiles, oldest first; k-tile 0 has landed once only the younger ones are outstanding
-#pragma unroll
-  for (int s = 0; s < SP; ++s) {
-    const Source src = source(s);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) copyQ(src, QBASE + s * OPBYTES, j);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) copyP(src, s * OPBYTES, j);
-  }
+  // (k-tile 0 has landed once only the copies of the younger ones are outstanding)
   wait_copies<(SP - 1) * PAIR>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
@@ -503,7 +572,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       k_range(No{});
       wait_copies<0>();
       if constexpr (SK) {
-        if (p.ksplit > 1) {
+        if (g.ksplit > 1) {
           __syncthreads();
           __syncthreads();
           if (!*(volatile int*)smem) return;
@@ -524,7 +593,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // scattered 8-byte / 2-byte global accesses straight from the accumulator layout flood L2 with
   // partial-line requests and cost a quarter of the kernel.
   if constexpr (SK) {
-    if (p.ksplit > 1) {
+    if (g.ksplit > 1) {
       // Every part leaves its accumulators in the workspace (accumulator layout: one word per lane and accumulator
       // register, so every access of a wave is a run of 256 bytes), waits until they have arrived, and counts itself in.
       // The block that finds itself last adds ALL parts in the order 0, 1, ... (its own from memory like the others: the
@@ -533,7 +602,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       // caches): the eight L2 caches of the chip are not coherent with each other, and the alternative - a release /
       // acquire fence per block - writes back and invalidates a whole L2 each time (measured: the product twice as slow).
       int* sk_last = (int*)smem;   // the operand stages are dead after the barrier below
-      float* part = p.sk_partial + (size_t)sk_tile * p.ksplit * (BT * BT);
+      float* part = g.sk_partial + (size_t)sk_tile * g.ksplit * (BT * BT);
       float* dst = part + (size_t)ks * (BT * BT);
 #pragma unroll
       for (int i = 0; i < FR; ++i)
@@ -547,9 +616,9 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this lane's stores have been acknowledged
       __syncthreads();
       if (tid == 0) {
-        const int old = __hip_atomic_fetch_add(p.sk_counter + sk_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int last = old == p.ksplit - 1;
-        if (last) __hip_atomic_store(p.sk_counter + sk_tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+        const int old = __hip_atomic_fetch_add(g.sk_counter + sk_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int last = old == g.ksplit - 1;
+        if (last) __hip_atomic_store(g.sk_counter + sk_tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
         *sk_last = last;
       }
       __syncthreads();
@@ -558,7 +627,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       for (int i = 0; i < FR; ++i)
 #pragma unroll
         for (int j = 0; j < FR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int sidx = 0; sidx < p.ksplit; ++sidx) {
+      for (int sidx = 0; sidx < g.ksplit; ++sidx) {
         const float* src = part + (size_t)sidx * (BT * BT);
 #pragma unroll
         for (int i = 0; i < FR; ++i)
@@ -572,9 +641,9 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   }
   // optional per-matrix scale of the operand that was left out of it (deferred normalisation): the product of two
   // such operands carries sc^2, a product with one of them (and its addend) carries sc
-  const float sc = p.scale ? p.scale[b] : 1.f;
-  const float bx_sc = sc * __builtin_ldexpf(1.f, p.out_shift);   // MODE_BX: scale of the result (a power of two from the host)
-  const float alpha = SYRK_PLAIN ? p.alpha * sc * sc : p.alpha, beta = p.beta;
+  const float sc = out.scale ? out.scale[b] : 1.f;
+  const float bx_sc = sc * __builtin_ldexpf(1.f, out.out_shift);   // MODE_BX: scale of the result (a power of two from the host)
+  const float alpha = SYRK_PLAIN ? out.alpha * sc * sc : out.alpha, beta = out.beta;
   // A diagonal tile of a product of a matrix with ITSELF is symmetric bit for bit as it comes out of the matrix cores
   // (element (i,j) and element (j,i) are the same products summed in the same order over k), so it is stored like any
   // other tile, as one image.  A diagonal tile of P Q^T with two different (commuting, symmetric) matrices is symmetric
@@ -603,6 +672,8 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     else if constexpr (RCH == 8) return (((c >> 1) & 3) << 1) | ((c >> 3) & 1);
     else return (((c >> 2) & 1) << 1) | ((c >> 3) & 1);
   };
+  constexpr int SLAB_ROWS = 64 / RCH;           // W rows of a slab; sw() repeats after SW_PERIOD slabs
+  constexpr int SW_PERIOD = RCH == 16 ? 4 : (RCH == 8 ? 2 : 1);
   auto w_off = [&](int c, int r) { return c * WROW + (((r >> 3) ^ sw(c)) << 4) + ((r & 7) << 1); };
   const int wrow0 = R0 + wr0, wcol0 = C0 + wc0;  // global origin of this wave's sub-tile
 
@@ -614,13 +685,16 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     constexpr int PART = decltype(part_)::value;
     if constexpr (has_e) {
       if constexpr (PART == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of the high half's image
-      const char* Eb = (const char*)(p.E + (size_t)b * p.strideE + (size_t)wcol0 * p.lde + wrow0);
+      // as in the main loop: a descriptor, a constant offset per lane and a scalar one per slab
+      void* const Eb = uniform((const char*)(out.E + (size_t)b * out.strideE + (size_t)wcol0 * out.lde + wrow0));
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(Eb, 0, -1, 0x00027000);
+      uint32_t off[SW_PERIOD];
 #pragma unroll
-      for (int t = 0; t < WSLABS; ++t) {
-        const int q = t * 64 + lane;
-        const int c = q / RCH, ch = (q % RCH) ^ sw(c);
-        __builtin_amdgcn_global_load_lds((gptr_t)(Eb + ((size_t)c * p.lde + ch * 8) * 2), (lptr_t)(W + t * 1024), 16, 0, 0);
-      }
+      for (int t = 0; t < SW_PERIOD; ++t)
+        off[t] = (uint32_t)(lane / RCH) * (uint32_t)out.lde * 2u + (uint32_t)(((lane % RCH) ^ sw(t * SLAB_ROWS + lane / RCH)) * 16);
+#pragma unroll
+      for (int t = 0; t < WSLABS; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lptr_t)(W + t * 1024), 16, (int)off[t % SW_PERIOD], (int)(t * SLAB_ROWS * (uint32_t)out.lde * 2u), 0, 0);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
 #pragma unroll
@@ -651,7 +725,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
         if constexpr (MODE == MODE_SYRK2) {   // B + a I
           if (i == j && on_diag) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] += (4 * lg + q == l16) ? p.diag_add : 0.f;
+            for (int q = 0; q < 4; ++q) v[q] += (4 * lg + q == l16) ? out.diag_add : 0.f;
           }
         }
         if constexpr (PART == 1) {
@@ -677,70 +751,88 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       }
     }
     // transposed / mirrored image: rows of W
-    __bf16* Tdst = SYM ? Cdst : p.Ct;
+    __bf16* Tdst = SYM ? Cdst : (__bf16*)out.Ct;
     if (Tdst && (!diag || above)) {   // in a diagonal tile: only the image of the idle wave's part
-      const long tbs = SYM ? p.strideC : p.strideCt;
-      const int tld = SYM ? p.ldc : p.ldct;
+      const long tbs = SYM ? out.strideC : out.strideCt;
+      const int tld = SYM ? out.ldc : out.ldct;
       __bf16* base = Tdst + (size_t)b * tbs;
       const bool vec_ok = !FINAL || ((tld & 7) == 0 && (tbs & 7) == 0 && (((uintptr_t)Tdst) & 15) == 0);
-#pragma unroll 8
-      for (int t = 0; t < WSLABS; ++t) {
-        const int q = t * 64 + lane;
-        const int c = q / RCH, ch = q % RCH;
-        const uint4 val = *(const uint4*)(W + c * WROW + ((ch ^ sw(c)) << 4));
-        const int orow = wcol0 + c, ocol = wrow0 + ch * 8;   // row of the transposed image = column of the tile
-        if (!FINAL) {
-          *(uint4*)(base + (size_t)orow * tld + ocol) = val;
-        } else if (orow < p.n_valid) {
-          if (vec_ok && ocol + 7 < p.m_valid) {
-            *(uint4*)(base + (size_t)orow * tld + ocol) = val;
-          } else {
-            const uint32_t w[4] = {val.x, val.y, val.z, val.w};
+      const int row = lane / RCH, ch = lane % RCH;   // of a slab of SLAB_ROWS rows of W; W's rows are the tile's columns
+      auto slab = [&](int t) { return *(const uint4*)(W + t * 1024 + row * WROW + ((ch ^ sw(t * SLAB_ROWS + row)) << 4)); };
+      if (!FINAL || (vec_ok && wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
+        char* to = (char*)(base + (size_t)(wcol0 + row) * tld + wrow0 + ch * 8);
+        static_for<WSLABS>([&](auto t_) __attribute__((always_inline)) {
+          constexpr int t = decltype(t_)::value;
+          *(uint4*)(to + (long)(t * SLAB_ROWS * 2) * tld) = slab(t);
+          if constexpr (t % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+#pragma unroll 4
+        for (int t = 0; t < WSLABS; ++t) {
+          const uint4 val = slab(t);
+          const int orow = wcol0 + t * SLAB_ROWS + row, ocol = wrow0 + ch * 8;
+          if (orow < out.n_valid) {
+            if (vec_ok && ocol + 7 < out.m_valid) {
+              *(uint4*)(base + (size_t)orow * tld + ocol) = val;
+            } else {
+              const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-              if (ocol + k < p.m_valid) ((uint16_t*)base)[(size_t)orow * tld + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+              for (int k = 0; k < 8; ++k)
+                if (ocol + k < out.m_valid) ((uint16_t*)base)[(size_t)orow * tld + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+            }
           }
         }
       }
     }
     // row-major image: transpose reads.  In a 16-lane group, source lane s points at W[c0 + s/4][r0 + 4*(s%4) ..+3];
     // lane L of the group then holds W[c0 .. c0+3][r0 + L].
-    if (SYM || p.C) {
-      __bf16* base = Cdst + (size_t)b * p.strideC;
-      const bool vec_ok = !FINAL || ((p.ldc & 7) == 0 && (p.strideC & 7) == 0 && (((uintptr_t)Cdst) & 15) == 0);
+    if (SYM || out.C) {
+      __bf16* base = Cdst + (size_t)b * out.strideC;
+      const bool vec_ok = !FINAL || ((out.ldc & 7) == 0 && (out.strideC & 7) == 0 && (((uintptr_t)Cdst) & 15) == 0);
       const int s = l16;
-#pragma unroll 4
-      for (int rb = 0; rb < WT / 16; ++rb)
+      // 16 rows, from row rb * 16 on, of the eight columns from cb * 32 + lg * 8 on
+      auto rows16 = [&](int rb, int cb) {
+        const int c0 = cb * 32 + lg * 8;
+        const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + (s >> 2), rb * 16 + 4 * (s & 3))));
+        const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + 4 + (s >> 2), rb * 16 + 4 * (s & 3))));
+        const uint2 lo = __builtin_bit_cast(uint2, lo4), hi = __builtin_bit_cast(uint2, hi4);
+        return make_uint4(lo.x, lo.y, hi.x, hi.y);
+      };
+      if (!FINAL || (vec_ok && wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
+        char* to = (char*)(base + (size_t)(wrow0 + s) * out.ldc + wcol0 + lg * 8);
+        static_for<WT / 16>([&](auto rb_) __attribute__((always_inline)) {
+          constexpr int rb = decltype(rb_)::value;
+          static_for<WT / 32>([&](auto cb_) __attribute__((always_inline)) {
+            constexpr int cb = decltype(cb_)::value;
+            *(uint4*)(to + (long)(rb * 32) * out.ldc + cb * 64) = rows16(rb, cb);
+          });
+          if constexpr (rb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+#pragma unroll 2
+        for (int rb = 0; rb < WT / 16; ++rb)
 #pragma unroll
-        for (int cb = 0; cb < WT / 32; ++cb) {
-          const int c0 = cb * 32 + lg * 8;
-          const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + (s >> 2), rb * 16 + 4 * (s & 3))));
-          const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + 4 + (s >> 2), rb * 16 + 4 * (s & 3))));
-          uint4 val;
-          val.x = (uint32_t)(uint16_t)lo4[0] | ((uint32_t)(uint16_t)lo4[1] << 16);
-          val.y = (uint32_t)(uint16_t)lo4[2] | ((uint32_t)(uint16_t)lo4[3] << 16);
-          val.z = (uint32_t)(uint16_t)hi4[0] | ((uint32_t)(uint16_t)hi4[1] << 16);
-          val.w = (uint32_t)(uint16_t)hi4[2] | ((uint32_t)(uint16_t)hi4[3] << 16);
-          const int orow = wrow0 + rb * 16 + s, ocol = wcol0 + c0;
-          if (!FINAL) {
-            *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
-          } else if (orow < p.m_valid) {
-            if (vec_ok && ocol + 7 < p.n_valid) {
-              *(uint4*)(base + (size_t)orow * p.ldc + ocol) = val;
-            } else {
-              const uint32_t w[4] = {val.x, val.y, val.z, val.w};
+          for (int cb = 0; cb < WT / 32; ++cb) {
+            const uint4 val = rows16(rb, cb);
+            const int orow = wrow0 + rb * 16 + s, ocol = wcol0 + cb * 32 + lg * 8;
+            if (orow < out.m_valid) {
+              if (vec_ok && ocol + 7 < out.n_valid) {
+                *(uint4*)(base + (size_t)orow * out.ldc + ocol) = val;
+              } else {
+                const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
-              for (int k = 0; k < 8; ++k)
-                if (ocol + k < p.n_valid) ((uint16_t*)base)[(size_t)orow * p.ldc + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+                for (int k = 0; k < 8; ++k)
+                  if (ocol + k < out.n_valid) ((uint16_t*)base)[(size_t)orow * out.ldc + ocol + k] = (uint16_t)(w[k >> 1] >> ((k & 1) * 16));
+              }
             }
           }
-        }
+      }
     }
   };
-  emit(I0{}, p.C);
-  if constexpr (SPLIT && MODE == MODE_SYRK2) emit(I1{}, p.C2);
+  emit(I0{}, (__bf16*)out.C);
+  if constexpr (SPLIT && MODE == MODE_SYRK2) emit(I1{}, g.C2);
 #endif
 }
 
@@ -809,7 +901,7 @@ static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
     if (e != hipSuccess) return e;
     if (slot) attr_set[dev].store(true, std::memory_order_release);
   }
-  const long tiles = gp.tile_start[gp.n_groups];
+  const long tiles = gp.total;
   if (tiles <= 0) return hipSuccess;
   const long unit = 8L * xcd_run((int)tiles);
   const long grid = (tiles + unit - 1) / unit * unit;
@@ -866,13 +958,14 @@ static hipError_t launch_ksplit(int mode, const GroupedGemmParams& p, hipStream_
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp,
+hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& asked,
                                   hipStream_t stream, int units, int f16, bool ksplit) {
+  GroupedGemmParams gp = asked;
   if (gp.n_groups < 1 || gp.n_groups > MAX_GROUPS) return hipErrorInvalidValue;
   const bool sym = (mode == MODE_SYRK || mode == MODE_SYRK2 || mode == MODE_SYRKT);
   if (ksplit && (!sym || tile != 128 || split || final_ || f16 == 2)) return hipErrorInvalidValue;
   for (int i = 0; i < gp.n_groups; ++i) {
-    const GemmParams& g = gp.g[i];
+    GemmParams& g = gp.g[i];
     if (g.K % BK != 0 || g.K <= 0 || gp.tile_start[i + 1] < gp.tile_start[i]) return hipErrorInvalidValue;
     if (mode == MODE_SYRK2 && !g.E) return hipErrorInvalidValue;
     if (mode == MODE_BX && (g.E == nullptr) != (gp.g[0].E == nullptr)) return hipErrorInvalidValue;  // one kernel per launch
@@ -902,13 +995,25 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
       if (g.qt_first + blocks / (side * side) > coarse) return hipErrorInvalidValue;
     }
   }
+  // what the kernel would otherwise divide for at the start of every tile
+  for (int i = 0; i < gp.n_groups; ++i) {
+    GemmParams& g = gp.g[i];
+    const int dM = g.tilesM >> gp.quarter, dN = g.tilesN >> gp.quarter;
+    g.per_mat = g.t_count > 0 ? g.t_count : (sym ? dM * (dM + 1) / 2 : dM * dN);
+    g.part_tiles = (gp.tile_start[i + 1] - gp.tile_start[i]) / (ksplit ? g.ksplit : 1);
+    if (g.per_mat < 1 || (ksplit && g.part_tiles < 1)) return hipErrorInvalidValue;
+    g.inv_per_mat = reciprocal(g.per_mat);
+    g.inv_line = sym ? 0u : reciprocal(dM > 8 ? 4 * dN : dM);
+  }
+  gp.total = gp.tile_start[gp.n_groups];
+  for (int i = gp.n_groups + 1; i <= MAX_GROUPS; ++i) gp.tile_start[i] = 0x7fffffff;
   if (ksplit) {
     if (f16 == 1) return launch_ksplit<1>(mode, gp, stream);
     return launch_ksplit<0>(mode, gp, stream);
   }
   int shortest = gp.g[0].K;
   for (int i = 1; i < gp.n_groups; ++i) shortest = gp.g[i].K < shortest ? gp.g[i].K : shortest;
-  const bool deep = deep_pipeline(units, tile, gp.tile_start[gp.n_groups], shortest);
+  const bool deep = deep_pipeline(units, tile, gp.total, shortest);
   auto by_storage = [&](auto cfg_) -> hipError_t {
     constexpr int CFG = decltype(cfg_)::value;
     if (f16 == 1) return launch_cfg<CFG, 1>(mode, split, final_, gp, stream);

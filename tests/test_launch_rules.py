@@ -71,3 +71,35 @@ def test_every_tile_once_and_rounds_of_the_device(rules, units):
         assert tile != 64 or whole == total
         # a block of the deep form holds most of a unit's LDS: never more of them than the device has units
         assert deep == (blocks <= units and k >= 1024)
+
+
+def test_division_by_reciprocals(tmp_path):
+    """What the start of a tile computes instead of dividing: exact over the whole range, the ends of it included."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "divide.cpp").write_text(r"""
+#include <cstdio>
+#include <initializer_list>
+#include "launch_rules.h"
+int main() {
+  const int top = 0x7fffffff;
+  long wrong = 0;
+  auto check = [&](int x, int d) {
+    if (x < 0 || d < 1) return;
+    int rest = -1;
+    const int q = archscale::divide(x, d, archscale::reciprocal(d), rest);
+    wrong += q != x / d || rest != x % d;
+    if (d <= 4) wrong += archscale::divide_1_to_4(x, d) != x / d;
+  };
+  for (int d = 1; d <= 300; ++d)
+    for (int x = 0; x <= 3000; ++x) check(x, d);
+  for (long d = 1; d <= top; d = d * 5 / 3 + 1)
+    for (long near : {0L, d, 7 * d, (top / d) * d, (long)top})
+      for (long e = -2; e <= 2; ++e)
+        if (near + e <= top) check((int)(near + e), (int)d);
+  printf("%ld\n", wrong);
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "divide.cpp"), "-o", str(tmp_path / "divide")],
+                   check=True)
+    out = subprocess.run([str(tmp_path / "divide")], capture_output=True, text=True, check=True).stdout
+    assert out.strip() == "0", out
