@@ -14,6 +14,7 @@
 #include "elementwise.h"
 #include "launch_rules.h"
 #include "ns_gemm.h"
+#include "ns_small.h"
 #include "spectral.h"
 
 using namespace archscale;
@@ -464,12 +465,22 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
     return (long)pr[a].pl.Mp * pr[a].pl.Np > (long)pr[b].pl.Mp * pr[b].pl.Np;
   });
 
+  // A call of nothing but small matrices: the whole chain in one launch, a block per matrix, with the same bits as the launches
+  // below (ns_small.hip).  Where a call holds larger matrices too, the small ones stay in its chain: their tiles cost the
+  // shared launches next to nothing, a launch of their own would add its time.  (A tile configuration forced through the
+  // environment forces the chain as well.)  One 128 x 384 matrix, staging included: 83 us as 18 launches, 46 as one; where the line lies
+  // is what the LDS of a compute unit holds, and every matrix that fits is faster so (64 x 1024 88 -> 45, 64 x 128 85 -> 19;
+  // 1000 of 128 x 384 522 -> 219).
+  bool small = !split_any && iters <= SMALL_NS_MAX_ITERS && !env_switches().tile;
+  for (const NsProblem& P : pr)
+    small = small && small_ns_extents(P.pl.m, P.pl.n, nullptr, nullptr) && P.defer == pr[0].defer;
+
   hipError_t e;
   // K-split counters start at zero (every launch leaves them at zero again); the workspace is the caller's and holds anything
   for (const NsProblem& P : pr)
     if (P.sk_counter && (e = launch_zero_i32(P.sk_counter, (long)P.q.batch * P.pl.sk_quadrants, stream)) != hipSuccess) return (int)e;
   // normalise into X^T (long side first): a wide input is transposed on the way, a tall one is copied as it is
-  if (!fused) {
+  if (!fused && !small) {
     StageParams sp = {};
     auto flush = [&]() -> hipError_t {
       if (sp.n == 0) return hipSuccess;
@@ -819,6 +830,40 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       return true;
     });
   };
+  if (small) {
+    for (const int side : {64, 128}) {   // one kernel each
+      SmallNsParams sp = {};
+      auto flush = [&]() -> hipError_t {
+        if (sp.n == 0) return hipSuccess;
+        sp.iters = iters; sp.sa = SH_A; sp.sb = SH_B;
+        sp.eps = eps; sp.eps_mode = eps_mode;
+        sp.normalize = normalize; sp.cast_first = cast_first; sp.defer = pr[0].defer; sp.half = f16 && !pr[0].defer;
+        for (int it = 0; it < iters; ++it) {
+          const ItCfg k = it_cfg(it);
+          sp.it[it] = SmallNsIteration{k.a, k.b, k.c, (uint8_t)k.half_ops, (uint8_t)k.half_out, (uint8_t)k.fold};
+        }
+        const hipError_t err = launch_small_ns(sp, stream);
+        sp = SmallNsParams{};
+        return err;
+      };
+      for (const NsProblem& P : pr) {
+        int mp = 0;
+        small_ns_extents(P.pl.m, P.pl.n, &mp, nullptr);
+        if (mp != side) continue;
+        if ((sp.n == SMALL_NS_MAX_PROBLEMS || (long)sp.block_start[sp.n] + P.q.batch > 0x7fffffffL) && (e = flush()) != hipSuccess) return (int)e;
+        SmallNsProblem& q = sp.p[sp.n];
+        if (fused) { q.in = P.Xt[0]; q.in_stride = (long)P.pl.Mp * P.pl.Np; q.in_ld = P.pl.Mp; q.in_dtype = -1; q.scale = P.scale; }
+        else { q.in = P.q.in; q.in_stride = P.q.in_batch_stride; q.in_ld = P.q.in_ld; q.in_dtype = (int8_t)P.q.in_dtype; }
+        q.out = (uint16_t*)P.q.out; q.out_stride = P.q.out_batch_stride; q.out_ld = P.q.out_ld;
+        q.rows = P.q.rows; q.cols = P.q.cols; q.sx = P.sx; q.gram_tail = P.gram_tail;
+        sp.block_start[sp.n + 1] = sp.block_start[sp.n] + P.q.batch;
+        ++sp.n;
+      }
+      if ((e = flush()) != hipSuccess) return (int)e;
+    }
+    return 0;
+  }
+
   auto every = [](const NsProblem&) { return true; };
   auto on_gram = [](const NsProblem& P) { return P.gram_tail; };
   auto plain = [](const NsProblem& P) { return !P.gram_tail; };

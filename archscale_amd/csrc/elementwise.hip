@@ -12,67 +12,9 @@
 #include <stdint.h>
 
 #include "elementwise.h"
+#include "streaming.h"
 
 namespace archscale {
-
-static constexpr int EW_THREADS = 256;
-static constexpr int EW_VEC = 8;                                   // elements per thread per trip
-static constexpr int EW_TRIPS = MUON_CHUNK_ELEMS / (EW_THREADS * EW_VEC);
-static_assert(EW_TRIPS * EW_THREADS * EW_VEC == MUON_CHUNK_ELEMS, "chunk must be a whole number of trips");
-
-// ---------------------------------------------------------------------------
-// small helpers
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
-__device__ __forceinline__ float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
-
-// Every kernel of this file streams: an element is touched once per launch and the tensors of a step are far larger
-// than the caches, so all 16-byte accesses carry the non-temporal hint (measured on a 2-read / 2-write stream of
-// 1 GiB arrays: 5.87 TB/s with it, 5.57 TB/s without; a plain copy 6.29 against 5.72 TB/s).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x4 stream_load16(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
-__device__ __forceinline__ void stream_store16(void* p, u32x4 v) { __builtin_nontemporal_store(v, (u32x4*)p); }
-
-template <int DT> struct Elem;  // DT_BF16 / DT_F32 access of 8 consecutive elements
-template <> struct Elem<DT_BF16> {
-  typedef uint16_t T;
-  static __device__ __forceinline__ void load8(const void* p, long i, float (&v)[8]) {
-    const u32x4 r = stream_load16((const uint16_t*)p + i);
-    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(w[k] & 0xffff); v[2 * k + 1] = bf2f(w[k] >> 16); }
-  }
-  static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) {
-    u32x4 r;
-    r.x = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-    r.y = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-    r.z = f2bf(v[4]) | ((uint32_t)f2bf(v[5]) << 16);
-    r.w = f2bf(v[6]) | ((uint32_t)f2bf(v[7]) << 16);
-    stream_store16((uint16_t*)p + i, r);
-  }
-  static __device__ __forceinline__ float load1(const void* p, long i) { return bf2f(((const uint16_t*)p)[i]); }
-  static __device__ __forceinline__ void store1(void* p, long i, float v) { ((uint16_t*)p)[i] = f2bf(v); }
-  static __device__ __forceinline__ float round(float v) { return bf2f(f2bf(v)); }
-};
-template <> struct Elem<DT_F32> {
-  typedef float T;
-  static __device__ __forceinline__ void load8(const void* p, long i, float (&v)[8]) {
-    const f32x4 a = __builtin_nontemporal_load((const f32x4*)((const float*)p + i));
-    const f32x4 b = __builtin_nontemporal_load((const f32x4*)((const float*)p + i + 4));
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  }
-  static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) {
-    const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
-    __builtin_nontemporal_store(a, (f32x4*)((float*)p + i));
-    __builtin_nontemporal_store(b, (f32x4*)((float*)p + i + 4));
-  }
-  static __device__ __forceinline__ float load1(const void* p, long i) { return ((const float*)p)[i]; }
-  static __device__ __forceinline__ void store1(void* p, long i, float v) { ((float*)p)[i] = v; }
-  static __device__ __forceinline__ float round(float v) { return v; }
-};
-
-__device__ __forceinline__ bool aligned16(const void* p) { return (((uintptr_t)p) & 15) == 0; }
 
 // item that owns global chunk c: largest i with prefix[i] <= c
 __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int n_items, int c) {
@@ -82,26 +24,6 @@ __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int
     if (prefix[mid] <= c) lo = mid; else hi = mid;
   }
   return lo;
-}
-
-// ordered block reduction of up to 3 values; result valid in thread 0
-template <int N>
-__device__ __forceinline__ void block_reduce(float (&v)[N], float* smem /* N * 4 floats */) {
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
-  }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < N; ++k) smem[k * 4 + w] = v[k];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = (smem[k * 4 + 0] + smem[k * 4 + 1]) + (smem[k * 4 + 2] + smem[k * 4 + 3]);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -211,43 +133,10 @@ stage_sumsq_kernel(const StageParams sp) {
   const int b = local / q.cpm, chunk = local - b * q.cpm;
   const int rows = q.rows, cols = q.cols, ld = q.ld;
   const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
-  const long numel = (long)rows * cols;
-  const long begin = (long)chunk * MUON_CHUNK_ELEMS;
-  const long end = begin + MUON_CHUNK_ELEMS < numel ? begin + MUON_CHUNK_ELEMS : numel;
-  float s[1] = {0.f};
-  const bool dense = (ld == cols);
-  if (dense && aligned16(base) && numel % EW_VEC == 0) {
-#pragma unroll
-    for (int t = 0; t < EW_TRIPS; ++t) {
-      const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
-        float v[8];
-        Elem<DT>::load8(base, i, v);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) { const float x = CAST_FIRST ? bf2f(f2bf(v[k])) : v[k]; s[0] += x * x; }
-      }
-    }
-  } else {
-    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
-      const long r = i / cols, cc = i - r * cols;
-      float x = Elem<DT>::load1(base, r * ld + cc);
-      if (CAST_FIRST) x = bf2f(f2bf(x));
-      s[0] += x * x;
-    }
-  }
+  float s[1] = {dense_sumsq_ok(base, rows, cols, ld) ? thread_sumsq_dense<DT>(base, (long)rows * cols, chunk, threadIdx.x, CAST_FIRST)
+                                                     : thread_sumsq_strided<DT>(base, rows, cols, ld, chunk, threadIdx.x, CAST_FIRST)};
   block_reduce<1>(s, red);
   if (threadIdx.x == 0) q.partial[(size_t)b * q.cpm + chunk] = s[0];
-}
-
-// normalisation factor of a matrix from its sum of squares; with pow2 it is split into a power of two (applied to the copy
-// of the input, exactly) and a rest in [0.7, 1.5]
-__device__ __forceinline__ float2 norm_factor(float sumsq, float eps, int eps_mode, bool pow2) {
-  const float n = sqrtf(sumsq);
-  const float sc = eps_mode == EPS_ADD ? 1.f / (n + eps) : 1.f / fmaxf(n, eps);
-  if (!pow2) return make_float2(sc, 1.f);
-  const bool ok = sc > 0.f && sc < 3.0e38f;
-  const float p = ok ? exp2f(rintf(log2f(sc))) : sc;
-  return make_float2(ok ? sc / p : 1.f, p);
 }
 
 // ---------------------------------------------------------------------------

@@ -164,7 +164,8 @@ void muon_ns_ksplit_info(int rows, int cols, int* info);
 
 /* Per-launch timing of the Newton-Schulz GEMM kernels, for roofline accounting (no counterpart in the
  * reference).  Between muon_profile_begin() and muon_profile_collect() every GEMM launch of muon_ns_batched is
- * bracketed by a pair of HIP events on its stream.  muon_profile_collect waits for them, writes up to `capacity`
+ * bracketed by a pair of HIP events on its stream (a call of matrices so small that one launch does everything records
+ * nothing).  muon_profile_collect waits for them, writes up to `capacity`
  * records to the HOST arrays (any may be NULL) and returns the number of launches recorded (< 0 on error):
  *   ms                elapsed milliseconds of the launch
  *   key               tile*100 + mode*10 + 4*noaddend + split*2 + final  (mode 0 = X X^T, 1 = cAA+bA, 2 = aX + BX,

@@ -1,0 +1,69 @@
+"""GPU: matrices whose whole iteration runs in one block, against the same matrices in the chain of product launches.
+
+A call that holds a larger matrix as well takes the chain for all of its matrices, so a grouped call with a filler matrix is the
+general path.  Both do the same products in the same order with the same rounding: the bits have to agree.
+"""
+import pytest
+import torch
+
+from archscale_amd.optim import newton_schulz_hip as H
+
+pytestmark = pytest.mark.gpu
+
+POLAR = [(8.2051, -22.9019, 16.4607), (4.0664, -2.8612, 0.5184), (3.9096, -2.8234, 0.5250), (3.2856, -2.4153, 0.4853),
+         (2.2779, -1.6198, 0.3985)]
+KINDS = {
+    "quintic": dict(coeffs=H.QUINTIC_SCHEDULE),
+    "no tail": dict(coeffs=H.QUINTIC_SCHEDULE, gram_tail=False),
+    "constant, half": dict(coeffs=[H.SIMPLE_ROW] * 5, prec="f16"),
+    "polar, half, fp32 norm": dict(coeffs=POLAR, prec="f16", cast_input_first=False),
+    "half with tail": dict(coeffs=H.QUINTIC_SCHEDULE, prec="f16", gram_tail=True),
+    "one row": dict(coeffs=[H.SIMPLE_ROW]),
+}
+# (batch, rows, cols): edges of the fragments, of the two kernels (short side 64 / 128) and of what fits one compute unit
+SHAPES = [(1, 1, 1), (2, 1, 9), (1, 15, 17), (3, 64, 64), (2, 65, 64), (1, 128, 128), (2, 127, 129), (1, 128, 384), (1, 384, 127),
+          (2, 97, 383), (1, 64, 1152), (1, 1151, 33), (1, 63, 770), (1, 128, 385), (1, 64, 1153)]
+
+
+def _input(batch, rows, cols, dtype, ld=None):
+    g = torch.Generator().manual_seed(1000 * rows + cols)
+    x = torch.randn(batch, rows, ld or cols, generator=g) * 1e-3
+    return x.to(dtype).cuda()[..., :cols]
+
+
+def _chain(x, **kw):
+    filler = torch.randn(160, 160, generator=torch.Generator().manual_seed(0)).to(x.dtype).cuda()
+    return H.newton_schulz_grouped([x, filler], **kw)[0]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_block_gives_the_bits_of_the_chain(kind, dtype):
+    kw = KINDS[kind]
+    for batch, rows, cols in SHAPES:
+        x = _input(batch, rows, cols, dtype)
+        got, want = H.newton_schulz(x, **kw), _chain(x, **kw)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (batch, rows, cols)
+
+
+@pytest.mark.parametrize("rows,cols,ld", [(100, 200, 203), (96, 384, 400), (200, 48, 56), (7, 5, 8)])
+def test_strided_rows_and_the_input_as_result(rows, cols, ld):
+    x = _input(2, rows, cols, torch.bfloat16, ld)
+    want = _chain(x)
+    assert torch.equal(H.newton_schulz(x).view(torch.int16), want.view(torch.int16))
+    y = x.contiguous()
+    H.newton_schulz(y, out=y)
+    assert torch.equal(y.view(torch.int16), H.newton_schulz(x.contiguous()).view(torch.int16))
+
+
+def test_many_classes_zeros_and_tiny_norms_in_one_call():
+    shapes = [(33 + 3 * i, 40 + 7 * i) for i in range(28)] + [(128, 384), (5, 1000)]
+    xs = [_input(1, r, c, torch.bfloat16)[0] for r, c in shapes]
+    xs[3].zero_()
+    xs[4].mul_(1e-9)
+    small = H.newton_schulz_grouped(xs)
+    filler = torch.randn(160, 160, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).cuda()
+    chain = H.newton_schulz_grouped(xs + [filler])
+    for x, a, b in zip(xs, small, chain):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), x.shape
+    assert not small[3].any()
