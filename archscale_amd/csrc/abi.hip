@@ -1084,7 +1084,7 @@ int muon_scalar_update_dev(const muon_scalar_item* items_dev, const int32_t* pre
 namespace {
 struct SnPlan {
   NsPlan pl;
-  size_t off_x, off_g, off_g2, off_g4, off_xscale, off_xpart, off_z, off_part, total;
+  size_t off_x, off_g, off_g2, off_g4, off_xscale, off_xpart, off_z, off_part, off_long, total;
 };
 SnPlan make_sn_plan(int batch, int rows, int cols) {
   SnPlan s;
@@ -1096,9 +1096,11 @@ SnPlan make_sn_plan(int batch, int rows, int cols) {
   s.off_g2 = take((size_t)batch * s.pl.Mp * s.pl.Mp * 2);   // G^2 and G^4 of the grouped rounds (used from 6 / 16 rounds on)
   s.off_g4 = take((size_t)batch * s.pl.Mp * s.pl.Mp * 2);
   s.off_xscale = take((size_t)batch * sizeof(float));
-  s.off_xpart = take((size_t)batch * (s.pl.Mp / 64) * (s.pl.Np / 64) * sizeof(float));
+  // sums of squares: per 64x64 tile of a copy, or per strip of the short side
+  s.off_xpart = take((size_t)batch * std::max((s.pl.Mp / 64) * (s.pl.Np / 64), s.pl.Mp / SN_ROWS) * sizeof(float));
   s.off_z = take((size_t)2 * batch * s.pl.Mp * sizeof(float));
   s.off_part = take((size_t)2 * batch * (s.pl.Mp / SN_ROWS) * 2 * sizeof(float));
+  s.off_long = take((size_t)batch * s.pl.n * sizeof(float));   // the long-side vectors before they are made unit vectors
   s.total = off;
   return s;
 }
@@ -1125,38 +1127,66 @@ size_t muon_spectral_norm_workspace_bytes(const muon_sn_problem* problems_host, 
 }
 
 namespace {
+// singular vectors of a call with one problem: unnormalised in fp32, or unit vectors in bfloat16
+struct SnOutputs { float *short_out, *long_out; uint16_t *short_unit, *long_unit; };
 int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int steps, void* ws_dev, size_t ws_bytes,
-                       void* stream_, float* short_out, float* long_out);
+                       void* stream_, const SnOutputs& out);
+muon_sn_problem one_sn_problem(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, float* sigma_out_dev) {
+  muon_sn_problem q = {};
+  q.w_ptrs = w_ptrs_host; q.sigma_out = sigma_out_dev;
+  q.dtype = dtype; q.ld = ld; q.batch = batch; q.rows = rows; q.cols = cols; q.flags = 0;
+  return q;
 }
+}  // namespace
 
 int muon_spectral_norm(const muon_sn_problem* problems_host, int n_problems, int steps, void* ws_dev, size_t ws_bytes,
                        void* stream) {
-  return spectral_norm_impl(problems_host, n_problems, steps, ws_dev, ws_bytes, stream, nullptr, nullptr);
+  return spectral_norm_impl(problems_host, n_problems, steps, ws_dev, ws_bytes, stream, SnOutputs{});
 }
 
+// (the short-side vector is u for a wide matrix and v for a tall one)
 int muon_power_iteration(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, int steps,
                          float* sigma_out_dev, float* u_out_dev, float* v_out_dev, void* ws_dev, size_t ws_bytes,
                          void* stream) {
   if (!u_out_dev || !v_out_dev) return MUON_E_ARG;
-  muon_sn_problem q = {};
-  q.w_ptrs = w_ptrs_host; q.sigma_out = sigma_out_dev;
-  q.dtype = dtype; q.ld = ld; q.batch = batch; q.rows = rows; q.cols = cols; q.flags = 0;
-  // the short-side vector is u for a wide matrix and v for a tall one
+  const muon_sn_problem q = one_sn_problem(w_ptrs_host, dtype, ld, batch, rows, cols, sigma_out_dev);
   const bool tall = rows > cols;
-  return spectral_norm_impl(&q, 1, steps, ws_dev, ws_bytes, stream, tall ? v_out_dev : u_out_dev,
-                            tall ? u_out_dev : v_out_dev);
+  return spectral_norm_impl(&q, 1, steps, ws_dev, ws_bytes, stream,
+                            SnOutputs{tall ? v_out_dev : u_out_dev, tall ? u_out_dev : v_out_dev, nullptr, nullptr});
+}
+
+int muon_power_iteration_units(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, int steps,
+                               float* sigma_out_dev, void* u_out_dev, void* v_out_dev, void* ws_dev, size_t ws_bytes,
+                               void* stream) {
+  if (!u_out_dev || !v_out_dev) return MUON_E_ARG;
+  const muon_sn_problem q = one_sn_problem(w_ptrs_host, dtype, ld, batch, rows, cols, sigma_out_dev);
+  const bool tall = rows > cols;
+  return spectral_norm_impl(&q, 1, steps, ws_dev, ws_bytes, stream,
+                            SnOutputs{nullptr, nullptr, (uint16_t*)(tall ? v_out_dev : u_out_dev), (uint16_t*)(tall ? u_out_dev : v_out_dev)});
 }
 
 namespace {
 int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int steps, void* ws_dev, size_t ws_bytes,
-                       void* stream_, float* short_out, float* long_out) {
+                       void* stream_, const SnOutputs& out) {
   hipStream_t stream = (hipStream_t)stream_;
   if (!problems_host || n_problems <= 0 || steps < 1 || !ws_dev) return MUON_E_ARG;
-  if ((short_out || long_out) && (n_problems != 1 || !short_out || !long_out)) return MUON_E_ARG;
+  const bool vectors = out.short_out || out.short_unit;
+  if (vectors && n_problems != 1) return MUON_E_ARG;
   if ((uintptr_t)ws_dev & 255) return MUON_E_WORKSPACE;
   // tall: the matrix meant (after MUON_SN_TRANSPOSED) has more rows than columns; use_t: its short-side-first copy is
   // the transpose of the stored block
-  struct Prob { muon_sn_problem q; SnPlan sp; __bf16 *X, *G, *G2, *G4; float *xscale, *xpart, *z, *part; bool tall, use_t; };
+  // own: the products and passes read the caller's matrices where they lie (src, stride, ld); all of a call's problems by rows
+  // (short side first), or all by columns (long_first: the operand of the Gram product is K-major)
+  struct Prob {
+    muon_sn_problem q;
+    SnPlan sp;
+    __bf16 *X, *G, *G2, *G4;
+    float *xscale, *xpart, *z, *part;
+    bool tall, use_t, own;
+    const __bf16* src;
+    long stride;
+    int ld, L;   // leading dimension of src; its extent along the long side, padding included
+  };
   const int levels = spectral_power_levels(steps);
   const int units = compute_units();
   std::vector<Prob> pr(n_problems);
@@ -1182,10 +1212,34 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
     const bool transposed = (P.q.flags & MUON_SN_TRANSPOSED) != 0;
     P.tall = transposed ? P.q.cols > P.q.rows : P.q.rows > P.q.cols;
     P.use_t = transposed != P.tall;
+    P.src = P.X; P.stride = (long)P.sp.pl.Mp * P.sp.pl.Np; P.ld = P.L = P.sp.pl.Np;
+  }
+  // A matrix goes through the workspace only where the kernels cannot use it as it lies: other types, extents that need
+  // padding (the short side to tiles, the long one to k-tiles), rows that are not 16-byte aligned, separate allocations that
+  // are not equally spaced.  Long side first only where the whole call is: a product of either operand order is a launch of
+  // its own.  16 x 1024 x 2816: the copy was 35 us of 312.
+  auto usable = [](const muon_sn_problem& q, int short_side, int long_side, int Mp) {
+    const int64_t step = q.batch > 1 ? ((const char*)q.w_ptrs[1] - (const char*)q.w_ptrs[0]) : 0;
+    if (q.dtype != MUON_DTYPE_BF16 || short_side != Mp || long_side % 64 || q.ld % 8 || q.ld >= (1 << 22) || step < 0 || step % 16) return false;
+    if ((double)q.rows * q.ld * 2.0 >= 4294967296.0) return false;
+    for (int b = 0; b < q.batch; ++b)
+      if (((uintptr_t)q.w_ptrs[b] & 15) || (const char*)q.w_ptrs[b] != (const char*)q.w_ptrs[0] + b * step) return false;
+    return true;
+  };
+  bool long_first = true;
+  for (Prob& P : pr) long_first = long_first && P.use_t && P.tall && usable(P.q, P.q.cols, P.q.rows, P.sp.pl.Mp);
+  for (Prob& P : pr) {
+    P.own = long_first || (!P.use_t && usable(P.q, P.q.rows, P.q.cols, P.sp.pl.Mp));
+    if (!P.own) continue;
+    P.src = (const __bf16*)P.q.w_ptrs[0];
+    P.stride = P.q.batch > 1 ? ((const char*)P.q.w_ptrs[1] - (const char*)P.q.w_ptrs[0]) / 2 : 0;
+    P.ld = P.q.ld;
+    P.L = P.sp.pl.n;
   }
   hipError_t e;
   // bf16 copy of every matrix with its short side first, zero padded to the GEMM tile, and its sums of squares per tile
   for (const Prob& P : pr) {
+    if (P.own) continue;
     const NsPlan& pl = P.sp.pl;
     const long xs = (long)pl.Mp * pl.Np;
     const size_t xt = (size_t)(pl.Mp / 64) * (pl.Np / 64);
@@ -1200,14 +1254,16 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
       if (e != hipSuccess) return (int)e;
     }
   }
-  // a symmetric product for every problem, problems of one tile size sharing launches: dst = scale^2 * src src^T
-  // (src: [d_p][K] row-major per matrix)
-  auto gram = [&](auto&& src_of, auto&& k_of, auto&& dst_of, auto&& scale_of) -> int {
+  // a symmetric product for every problem, problems of one tile size sharing launches: dst = scale^2 * src src^T, or
+  // scale^2 * src^T src of a K-major operand
+  struct Operand { const __bf16* src; long stride; int ld, K; };
+  auto gram = [&](bool kmajor, auto&& operand_of, auto&& dst_of, auto&& scale_of) -> int {
+    const int mode = kmajor ? MODE_SYRKT : MODE_SYRK;
     for (int tile : {256, 128}) {
       GroupedGemmParams gp = {};
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
-        hipError_t err = launch_rounds(tile, MODE_SYRK, false, false, gp, stream, units, nullptr, 0);
+        hipError_t err = launch_rounds(tile, mode, false, false, gp, stream, units, nullptr, 0);
         gp = GroupedGemmParams{};
         return err;
       };
@@ -1215,13 +1271,13 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
         const NsPlan& pl = P.sp.pl;
         if (pl.tile != tile) continue;
         GemmParams g = {};
-        const int K = k_of(P);
+        const Operand o = operand_of(P);
         g.batch = P.q.batch;
-        g.P = src_of(P); g.Q = g.P; g.strideP = g.strideQ = (long)pl.Mp * K; g.ldp = g.ldq = K; g.K = K;
+        g.P = o.src; g.Q = o.src; g.strideP = g.strideQ = o.stride; g.ldp = g.ldq = o.ld; g.K = o.K;
         g.tilesM = g.tilesN = pl.Mp / pl.tile;
         g.C = dst_of(P); g.strideC = (long)pl.Mp * pl.Mp; g.ldc = pl.Mp; g.alpha = 1.f; g.beta = 0.f;
         g.scale = scale_of(P);
-        const long tiles = ns_gemm_tiles(MODE_SYRK, g);
+        const long tiles = ns_gemm_tiles(mode, g);
         if (tiles > 0x7ffffff0L) return MUON_E_UNSUPPORTED;
         if (gp.n_groups == MAX_GROUPS || tiles + gp.tile_start[gp.n_groups] > 0x7ffffff0L) {
           if ((e = flush()) != hipSuccess) return (int)e;
@@ -1249,30 +1305,35 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
       const long blocks = (long)P.q.batch * (pl.Mp / SN_ROWS);
       if (blocks > 0x3ffffff0L) return MUON_E_UNSUPPORTED;
       SnClass& c = sp.c[sp.n];
-      c.X = P.X; c.G = P.G; c.G2 = P.G2; c.G4 = P.G4;
-      c.xscale = P.xscale; c.xpart = P.xpart; c.xtiles = (pl.Mp / 64) * (pl.Np / 64);
+      c.X = P.src; c.strideX = P.stride; c.ldx = P.ld;
+      c.G = P.G; c.G2 = P.G2; c.G4 = P.G4;
+      c.xscale = P.xscale; c.xpart = P.xpart; c.xparts = P.own ? pl.Mp / SN_ROWS : (pl.Mp / 64) * (pl.Np / 64);
       c.z = P.z; c.part = P.part; c.sigma = P.q.sigma_out;
-      c.batch = P.q.batch; c.d = pl.m; c.d_p = pl.Mp; c.L_p = pl.Np; c.nblk = pl.Mp / SN_ROWS; c.tall = P.tall ? 1 : 0;
+      c.batch = P.q.batch; c.d = pl.m; c.d_p = pl.Mp; c.L_p = P.L; c.nblk = pl.Mp / SN_ROWS;
+      c.tall = P.tall; c.own = P.own; c.long_first = long_first;
       sp.blk_start[sp.n + 1] = sp.blk_start[sp.n] + (int)blocks;
       ++sp.n;
     }
     return 0;
   };
   int st;
+  // start vectors (and what the next launch needs of the caller's own matrices)
+  if ((st = for_class_chunks([&](const SnParams& sp) { return launch_spectral_init(sp, stream); })) != 0) return st;
   // G = s^2 X X^T with s a power of two near sqrt(d) / |X|_F (mean eigenvalue about 1: no power of G leaves the bf16 range)
   if ((st = for_class_chunks([&](const SnParams& sp) { return launch_spectral_xscale(sp, stream); })) != 0) return st;
-  if ((st = gram([](const Prob& P) { return P.X; }, [](const Prob& P) { return P.sp.pl.Np; },
+  if ((st = gram(long_first, [](const Prob& P) { return Operand{P.src, P.stride, P.ld, P.L}; },
                  [](const Prob& P) { return P.G; }, [](const Prob& P) { return (const float*)P.xscale; })) != 0)
     return st;
   // G2 = G^2, G4 = G2^2
+  auto square_of = [](const Prob& P, const __bf16* src) { return Operand{src, (long)P.sp.pl.Mp * P.sp.pl.Mp, P.sp.pl.Mp, P.sp.pl.Mp}; };
   if (levels >= 1) {
-    if ((st = gram([](const Prob& P) { return P.G; }, [](const Prob& P) { return P.sp.pl.Mp; },
-                   [](const Prob& P) { return P.G2; }, [](const Prob&) { return (const float*)nullptr; })) != 0)
+    if ((st = gram(false, [&](const Prob& P) { return square_of(P, P.G); }, [](const Prob& P) { return P.G2; },
+                   [](const Prob&) { return (const float*)nullptr; })) != 0)
       return st;
   }
   if (levels >= 2) {
-    if ((st = gram([](const Prob& P) { return P.G2; }, [](const Prob& P) { return P.sp.pl.Mp; },
-                   [](const Prob& P) { return P.G4; }, [](const Prob&) { return (const float*)nullptr; })) != 0)
+    if ((st = gram(false, [&](const Prob& P) { return square_of(P, P.G2); }, [](const Prob& P) { return P.G4; },
+                   [](const Prob&) { return (const float*)nullptr; })) != 0)
       return st;
   }
   // the rounds: every application of G (or of a power of it) is one launch over all classes
@@ -1283,10 +1344,15 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
          return launch_spectral_iterate(sp, steps, stream, final_src);
        })) != 0)
     return st;
-  if (short_out) {   // one problem, one class: its singular vectors from the iterates that are still in the workspace
+  if (vectors) {   // one problem, one class: its singular vectors from the iterates that are still in the workspace
     const SnClass& c = last.c[0];
-    const int L = pr[0].sp.pl.n;
-    if ((e = launch_spectral_vectors(c, L, final_src[c.tall ? 1 : 0], short_out, long_out, stream)) != hipSuccess) return (int)e;
+    const int L = pr[0].sp.pl.n, src = final_src[c.tall ? 1 : 0];
+    float* const long_out = out.long_unit ? (float*)((char*)ws_dev + pr[0].sp.off_long) : out.long_out;
+    if ((e = launch_spectral_vectors(c, L, src, out.short_out, long_out, stream)) != hipSuccess) return (int)e;
+    if (out.short_unit &&
+        (e = launch_spectral_units(SnVectors{spectral_short_vectors(c, src), c.d_p, out.short_unit, c.d},
+                                   SnVectors{long_out, L, out.long_unit, L}, c.batch, stream)) != hipSuccess)
+      return (int)e;
   }
   return 0;
 }

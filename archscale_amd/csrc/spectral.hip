@@ -24,6 +24,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "spectral.h"
 
@@ -34,51 +35,115 @@ namespace {
 __device__ __forceinline__ float bf2f_(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 __device__ __forceinline__ uint16_t f2bf_(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
+// sum over the wave, lanes i and i + 32, then 16, 8, 4, 2, 1 apart; in registers (by LDS permutes the six steps of a sum are six
+// LDS latencies, a fifth of a round)
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return __shfl(v, 0, 64);
+  // (the two operands of a swap are two registers: one value in both, which the compiler must not know to be one)
+  auto halves = [](auto swap, float x) {
+    unsigned a = __builtin_bit_cast(unsigned, x), b = a;
+    asm("" : "+v"(b));
+    const auto r = swap(a, b);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  };
+  v = halves([](unsigned a, unsigned b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); }, v);
+  v = halves([](unsigned a, unsigned b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); }, v);
+  auto from = [&](auto n_) {   // lane + n of the same 16 lanes
+    constexpr int n = decltype(n_)::value;
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 | n, 0xf, 0xf, true));
+  };
+  v += from(std::integral_constant<int, 8>{});
+  v += from(std::integral_constant<int, 4>{});
+  v += from(std::integral_constant<int, 2>{});
+  v += from(std::integral_constant<int, 1>{});
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
 // block -> (class, matrix, 16-row strip)
-__device__ __forceinline__ bool locate(const SnParams& sp, int& g, int& b, int& s) {
+__device__ __forceinline__ void locate(const SnParams& sp, int& g, int& b, int& s) {
+  // (all first blocks in one fetch instead of one after the other)
   const int blk = blockIdx.x;
-  if (blk >= sp.blk_start[sp.n]) return false;
+  int first = 0;
   g = 0;
-  while (g + 1 < sp.n && blk >= sp.blk_start[g + 1]) ++g;
-  const int local = blk - sp.blk_start[g];
+#pragma unroll
+  for (int i = 1; i < SN_MAX_CLASSES; ++i) {
+    const int at = sp.blk_start[i];
+    if (i < sp.n && blk >= at) { g = i; first = at; }
+  }
+  const int local = blk - first;
   b = local / sp.c[g].nblk;
   s = local - b * sp.c[g].nblk;
-  return true;
 }
 
-// dot products of 4 consecutive rows of a row-major bf16 matrix (leading dimension ld, a multiple of 8)
-// with an fp32 vector, over n_cols columns (a multiple of 8); result broadcast to all lanes
-__device__ __forceinline__ void rows4_dot(const uint16_t* __restrict__ row0, long ld, const float* __restrict__ x,
-                                          int n_cols, int lane, float (&acc)[4]) {
-  acc[0] = acc[1] = acc[2] = acc[3] = 0.f;
-  for (int j = lane * 8; j < n_cols; j += 512) {
-    float xv[8];
-    if (x) {
-      const float4 a = *(const float4*)(x + j), c = *(const float4*)(x + j + 4);
-      xv[0] = a.x; xv[1] = a.y; xv[2] = a.z; xv[3] = a.w; xv[4] = c.x; xv[5] = c.y; xv[6] = c.z; xv[7] = c.w;
-    } else {
+// Dot products of four rows of a row-major bf16 matrix (leading dimension ld, a multiple of 8) with an fp32 vector, over n_cols
+// columns (a multiple of 8).  The first AHEAD runs of a lane can be fetched before anything else is known.
+constexpr int AHEAD = 2;   // 1024 columns
+struct Rows4 {
+  uint4 r[AHEAD][4];
+  float4 x[AHEAD][2];
+};
+__device__ __forceinline__ void rows4_fetch(Rows4& f, const uint16_t* __restrict__ row0, long ld, const float* __restrict__ x,
+                                            int n_cols, int lane) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) xv[k] = 1.f;
+  for (int t = 0; t < AHEAD; ++t) {
+    const int j = t * 512 + lane * 8 < n_cols ? t * 512 + lane * 8 : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.r[t][i] = *(const uint4*)(row0 + (size_t)i * ld + j);
+    f.x[t][0] = *(const float4*)(x + j);
+    f.x[t][1] = *(const float4*)(x + j + 4);
+  }
+}
+__device__ __forceinline__ void rows4_add(const uint4 (&r)[4], const float4& a, const float4& c, float (&acc)[4]) {
+  const float xv[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      acc[i] += bf2f_(w[k] & 0xffff) * xv[2 * k];
+      acc[i] += bf2f_(w[k] >> 16) * xv[2 * k + 1];
     }
+  }
+}
+__device__ __forceinline__ void rows4_finish(const Rows4& f, const uint16_t* __restrict__ row0, long ld, const float* __restrict__ x,
+                                             int n_cols, int lane, float (&acc)[4]) {
+  acc[0] = acc[1] = acc[2] = acc[3] = 0.f;
+#pragma unroll
+  for (int t = 0; t < AHEAD; ++t)
+    if (t * 512 + lane * 8 < n_cols) rows4_add(f.r[t], f.x[t][0], f.x[t][1], acc);
+  for (int j = AHEAD * 512 + lane * 8; j < n_cols; j += 512) {
+    uint4 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = *(const uint4*)(row0 + (size_t)i * ld + j);
+    rows4_add(r, *(const float4*)(x + j), *(const float4*)(x + j + 4), acc);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = wave_sum(acc[i]);
+}
+// row sums of four rows and the sum of their squares (this lane's share)
+__device__ __forceinline__ float rows4_sums(const uint16_t* __restrict__ row0, long ld, int n_cols, int lane, float (&acc)[4]) {
+  acc[0] = acc[1] = acc[2] = acc[3] = 0.f;
+  float sq = 0.f;
+#pragma unroll 2
+  for (int j = lane * 8; j < n_cols; j += 512) {
+    uint4 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = *(const uint4*)(row0 + (size_t)i * ld + j);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint4 r = *(const uint4*)(row0 + (size_t)i * ld + j);
-      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+      const uint32_t w[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        acc[i] += bf2f_(w[k] & 0xffff) * xv[2 * k];
-        acc[i] += bf2f_(w[k] >> 16) * xv[2 * k + 1];
+        const float lo = bf2f_(w[k] & 0xffff), hi = bf2f_(w[k] >> 16);
+        acc[i] += lo;
+        acc[i] += hi;
+        sq = fmaf(lo, lo, sq);
+        sq = fmaf(hi, hi, sq);
       }
     }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i] = wave_sum(acc[i]);
+  return sq;
 }
 
 // sums `n` (S, D) pairs in a fixed lane-strided order; result in all lanes
@@ -91,22 +156,41 @@ __device__ __forceinline__ void sum_pairs(const float* __restrict__ part, int n,
 
 }  // namespace
 
-// x0 = X 1 (row sums of the short-side-first operand) or 1;  z[0] <- x0, z[1] <- 0, part[0] <- (|x0|^2 per strip, 0)
+// x0 = X 1 (row sums of the short-side-first operand) or 1;  z[0] <- x0, z[1] <- 0, part[0] <- (|x0|^2 per strip, 0); where X is
+// the caller's, its sums of squares: one read of X, which the Gram product then finds in the caches.
+// 16 matrices of 1024 x 2816: 16 us, where a copy of them with its sums took 35 and this pass came on top.
 __global__ void __launch_bounds__(256)
 sn_init_kernel(const SnParams sp) {
   __shared__ float red[8];
   int g, b, s;
-  if (!locate(sp, g, b, s)) return;
+  locate(sp, g, b, s);
   const SnClass c = sp.c[g];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r0 = s * SN_ROWS + wave * 4;
-  float v[4];
-  if (c.tall) {
+  const uint16_t* X = (const uint16_t*)c.X + (size_t)b * c.strideX;
+  float v[4] = {1.f, 1.f, 1.f, 1.f}, sq = 0.f;
+  if (c.long_first) {
+    // (tall matrices only: nothing but the squares) rows of d elements, a strip of the short side taking every nblk-th four
+    for (int r = s * 4 + wave; r < c.L_p; r += c.nblk * 4)
+      for (int j = lane * 8; j < c.d; j += 512) {
+        const uint4 q = *(const uint4*)(X + (size_t)r * c.ldx + j);
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = 1.f;
-  } else {
-    rows4_dot((const uint16_t*)c.X + (size_t)b * c.d_p * c.L_p + (size_t)r0 * c.L_p, c.L_p, nullptr, c.L_p, lane, v);
+        for (int k = 0; k < 4; ++k) {
+          const float lo = bf2f_(w[k] & 0xffff), hi = bf2f_(w[k] >> 16);
+          sq = fmaf(lo, lo, sq);
+          sq = fmaf(hi, hi, sq);
+        }
+      }
+  } else if (!c.tall || c.own) {
+    float sums[4];
+    sq = rows4_sums(X + (size_t)r0 * c.ldx, c.ldx, c.L_p, lane, sums);
+    if (!c.tall) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = sums[i];
+    }
   }
+  if (c.own) sq = wave_sum(sq);
   float S = 0.f;
   float* z0 = c.z + (size_t)b * c.d_p;
   float* z1 = c.z + ((size_t)c.batch + b) * c.d_p;
@@ -116,50 +200,60 @@ sn_init_kernel(const SnParams sp) {
     if (lane == 0) { z0[r0 + i] = val; z1[r0 + i] = 0.f; }
     S += val * val;
   }
-  if (lane == 0) red[wave] = S;
+  if (lane == 0) { red[wave] = S; red[4 + wave] = sq; }
   __syncthreads();
   if (threadIdx.x == 0) {
     float* p = c.part + ((size_t)b * c.nblk + s) * 2;
     p[0] = (red[0] + red[1]) + (red[2] + red[3]);
     p[1] = 0.f;
+    if (c.own) c.xpart[(size_t)b * c.xparts + s] = (red[4] + red[5]) + (red[6] + red[7]);
   }
 }
 
 // z[dst] <- M z[src] / max(|z[src]|, 1e-12);  part[dst] <- per strip (|z[dst]|^2,  z[src]^T z[dst] / |z[src]|)
 // M = G, G2 or G4 (which = 0, 1, 2) and the source buffer are given per kind of class (wide, tall), whose sequences
 // differ; which < 0: the classes of that kind sit this launch out.
+// Latency bound (16 matrices of 1024: 32 MB that the caches hold): every load of the first 1024 columns is on its way before the
+// norm of z[src] is added up, and no sum goes through LDS: 5.3 us a launch, 6.2 before.
 __global__ void __launch_bounds__(256)
 sn_step_kernel(const SnParams sp, int src_wide, int which_wide, int src_tall, int which_tall) {
   __shared__ float red[8];
   int g, b, s;
-  if (!locate(sp, g, b, s)) return;
-  const SnClass c = sp.c[g];
+  locate(sp, g, b, s);
+  const SnClass& c = sp.c[g];
   const int src = c.tall ? src_tall : src_wide, which = c.tall ? which_tall : which_wide;
   if (which < 0) return;
   const __bf16* M = which == 0 ? c.G : (which == 1 ? c.G2 : c.G4);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int dst = src ^ 1;
-  const float* zin = c.z + ((size_t)src * c.batch + b) * c.d_p;
-  float* zout = c.z + ((size_t)dst * c.batch + b) * c.d_p;
-  const float* pin = c.part + (((size_t)src * c.batch + b) * c.nblk) * 2;
-  float Sin, Din;
-  sum_pairs(pin, c.nblk, lane, Sin, Din);
-  const float inv = 1.f / fmaxf(sqrtf(Sin), 1e-12f);
+  const int dst = src ^ 1, d = c.d, d_p = c.d_p, nblk = c.nblk, batch = c.batch;
+  const float* zin = c.z + ((size_t)src * batch + b) * d_p;
+  float* zout = c.z + ((size_t)dst * batch + b) * d_p;
+  float* const part = c.part;
+  const float* pin = part + (((size_t)src * batch + b) * nblk) * 2;
   const int r0 = s * SN_ROWS + wave * 4;
+  const uint16_t* row0 = (const uint16_t*)M + (size_t)b * d_p * d_p + (size_t)r0 * d_p;
+  Rows4 ahead;
+  rows4_fetch(ahead, row0, d_p, zin, d_p, lane);
+  float own[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) own[i] = zin[r0 + i];
+  float Sin, Din;
+  sum_pairs(pin, nblk, lane, Sin, Din);
+  const float inv = 1.f / fmaxf(sqrtf(Sin), 1e-12f);
   float acc[4];
-  rows4_dot((const uint16_t*)M + (size_t)b * c.d_p * c.d_p + (size_t)r0 * c.d_p, c.d_p, zin, c.d_p, lane, acc);
+  rows4_finish(ahead, row0, d_p, zin, d_p, lane, acc);
   float S = 0.f, D = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float out = (r0 + i < c.d) ? acc[i] * inv : 0.f;
+    const float out = (r0 + i < d) ? acc[i] * inv : 0.f;
     if (lane == 0) zout[r0 + i] = out;
     S += out * out;
-    D += zin[r0 + i] * inv * out;
+    D += own[i] * inv * out;
   }
   if (lane == 0) { red[wave] = S; red[4 + wave] = D; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    float* p = c.part + (((size_t)dst * c.batch + b) * c.nblk + s) * 2;
+    float* p = part + (((size_t)dst * batch + b) * nblk + s) * 2;
     p[0] = (red[0] + red[1]) + (red[2] + red[3]);
     p[1] = (red[4] + red[5]) + (red[6] + red[7]);
   }
@@ -189,9 +283,9 @@ sn_xscale_kernel(const SnParams sp) {
   while (g < sp.n && blk >= sp.c[g].batch) { blk -= sp.c[g].batch; ++g; }
   if (g >= sp.n) return;
   const SnClass c = sp.c[g];
-  const float* part = c.xpart + (size_t)blk * c.xtiles;
+  const float* part = c.xpart + (size_t)blk * c.xparts;
   float t = 0.f;
-  for (int i = threadIdx.x; i < c.xtiles; i += 64) t += part[i];
+  for (int i = threadIdx.x; i < c.xparts; i += 64) t += part[i];
   t = wave_sum(t);
   // a power of two: X and G are scaled exactly
   // (exponent clamped: xscale^2 multiplies an fp32 accumulator)
@@ -208,7 +302,7 @@ hipError_t launch_spectral_xscale(const SnParams& sp, hipStream_t stream) {
   if (sp.n < 1 || sp.n > SN_MAX_CLASSES) return hipErrorInvalidValue;
   int matrices = 0;
   for (int g = 0; g < sp.n; ++g) {
-    if (sp.c[g].batch <= 0 || !sp.c[g].xscale || !sp.c[g].xpart || sp.c[g].xtiles < 1) return hipErrorInvalidValue;
+    if (sp.c[g].batch <= 0 || !sp.c[g].xscale || !sp.c[g].xpart || sp.c[g].xparts < 1) return hipErrorInvalidValue;
     matrices += sp.c[g].batch;
   }
   hipLaunchKernelGGL(sn_xscale_kernel, dim3(matrices), dim3(64), 0, stream, sp);
@@ -224,21 +318,21 @@ hipError_t launch_spectral_xscale(const SnParams& sp, hipStream_t stream) {
 // now (6.1 TB/s).
 constexpr int SNV_COLS = 64, SNV_GROUPS = 256 / (SNV_COLS / 8);
 __global__ void __launch_bounds__(256)
-sn_vectors_kernel(const uint16_t* __restrict__ X, const float* __restrict__ z_prev, const float* __restrict__ z_short,
+sn_vectors_kernel(const uint16_t* __restrict__ X, long strideX, int ldx, const float* __restrict__ z_prev, const float* __restrict__ z_short,
                   float* __restrict__ short_out, float* __restrict__ long_out, int d, int d_p, int L, int L_p) {
   __shared__ float red[SNV_GROUPS][SNV_COLS + 4];   // (rows of 272 bytes: the row groups of a wave start on different banks)
   const int b = blockIdx.y;
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t < d) short_out[(size_t)b * d + t] = z_short[(size_t)b * d_p + t];
+  if (short_out && t < d) short_out[(size_t)b * d + t] = z_short[(size_t)b * d_p + t];
   const int cg = threadIdx.x & (SNV_COLS / 8 - 1), rg = threadIdx.x / (SNV_COLS / 8);
   const long c0 = (long)blockIdx.x * SNV_COLS, j0 = c0 + cg * 8;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (j0 < L_p) {
-    const uint16_t* col = X + (size_t)b * d_p * L_p + j0;
+    const uint16_t* col = X + (size_t)b * strideX + j0;
     const float* zp = z_prev + (size_t)b * d_p;
 #pragma unroll 8
     for (int i = rg; i < d; i += SNV_GROUPS) {
-      const uint4 r = *(const uint4*)(col + (size_t)i * L_p);
+      const uint4 r = *(const uint4*)(col + (size_t)i * ldx);
       const float zi = zp[i];
       const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
@@ -259,38 +353,108 @@ sn_vectors_kernel(const uint16_t* __restrict__ X, const float* __restrict__ z_pr
   }
 }
 
+// the same of matrices stored long side first, [L][d]: four rows per wave against the vector
+__global__ void __launch_bounds__(256)
+sn_vectors_rows_kernel(const uint16_t* __restrict__ X, long strideX, int ldx, const float* __restrict__ z_prev, const float* __restrict__ z_short,
+                       float* __restrict__ short_out, float* __restrict__ long_out, int d, int d_p, int L) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (short_out && t < d) short_out[(size_t)b * d + t] = z_short[(size_t)b * d_p + t];
+  const int r0 = (blockIdx.x * 4 + wave) * 4;
+  if (r0 >= L) return;   // (L is a multiple of 4)
+  const uint16_t* row0 = X + (size_t)b * strideX + (size_t)r0 * ldx;
+  const float* zp = z_prev + (size_t)b * d_p;
+  Rows4 ahead;
+  rows4_fetch(ahead, row0, ldx, zp, d, lane);
+  float acc[4];
+  rows4_finish(ahead, row0, ldx, zp, d, lane, acc);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) long_out[(size_t)b * L + r0 + i] = acc[i];
+  }
+}
+
+const float* spectral_short_vectors(const SnClass& c, int src_final) {
+  // wide matrices (G = W W^T): the short vector is the LAST iterate, G^steps W 1 (the reference's u); tall ones
+  // (G = W^T W): the one before it, G^steps 1 (the reference's v)
+  return c.z + (size_t)(c.tall ? src_final ^ 1 : src_final) * c.batch * c.d_p;
+}
+
 hipError_t launch_spectral_vectors(const SnClass& c, int L, int src_final, float* short_out, float* long_out,
                                    hipStream_t stream) {
-  if (!short_out || !long_out || c.batch <= 0 || c.batch > 65535 || c.d <= 0 || c.d > c.d_p || L <= 0 || L > c.L_p ||
+  if (!long_out || c.batch <= 0 || c.batch > 65535 || c.d <= 0 || c.d > c.d_p || L <= 0 || L > c.L_p ||
       c.L_p % 8 || (src_final != 0 && src_final != 1))
     return hipErrorInvalidValue;
-  const float* z_final = c.z + (size_t)src_final * c.batch * c.d_p;
-  const float* z_prev = c.z + (size_t)(src_final ^ 1) * c.batch * c.d_p;
-  // wide matrices (G = W W^T): the short vector is the LAST iterate, G^steps W 1 (the reference's u); tall ones
-  // (G = W^T W): the one before it, G^steps 1 (the reference's v); the long vector is X^T times the one before the last
-  const float* z_short = c.tall ? z_prev : z_final;
+  const float* z_prev = c.z + (size_t)(src_final ^ 1) * c.batch * c.d_p;   // the long vector is X^T times the one before the last
+  const float* z_short = spectral_short_vectors(c, src_final);
+  if (c.long_first) {
+    if (L % 4 || c.d % 8) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)std::max((L / 4 + 3) / 4, (c.d + 255) / 256);
+    hipLaunchKernelGGL(sn_vectors_rows_kernel, dim3(blocks, c.batch), dim3(256), 0, stream, (const uint16_t*)c.X, c.strideX, c.ldx, z_prev,
+                       z_short, short_out, long_out, c.d, c.d_p, L);
+    return hipGetLastError();
+  }
   const unsigned blocks = (unsigned)std::max(((long)c.L_p + SNV_COLS - 1) / SNV_COLS, ((long)c.d + 255) / 256);
-  hipLaunchKernelGGL(sn_vectors_kernel, dim3(blocks, c.batch), dim3(256), 0, stream, (const uint16_t*)c.X, z_prev, z_short,
+  hipLaunchKernelGGL(sn_vectors_kernel, dim3(blocks, c.batch), dim3(256), 0, stream, (const uint16_t*)c.X, c.strideX, c.ldx, z_prev, z_short,
                      short_out, long_out, c.d, c.d_p, L, c.L_p);
   return hipGetLastError();
 }
 
-hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src) {
-  if (sp.n < 1 || sp.n > SN_MAX_CLASSES || steps < 1) return hipErrorInvalidValue;
-  const int blocks = sp.blk_start[sp.n];
-  int matrices = 0;
-  bool have2 = true, have4 = true, any[2] = {false, false};
+// one block per vector; the vectors are short (one read from the caches), the launch is what it costs: 16 pairs of 1024 and 2816
+// in 6 us, eight launches of the tensor library 25
+__global__ void __launch_bounds__(256)
+sn_units_kernel(const SnVectors a, const SnVectors c) {
+  __shared__ float red[4];
+  const SnVectors v = blockIdx.y ? c : a;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float* x = v.x + (size_t)blockIdx.x * v.stride;
+  float s = 0.f;
+  for (int i = threadIdx.x; i < v.len; i += 256) s = fmaf(x[i], x[i], s);
+  s = wave_sum(s);
+  if (lane == 0) red[wave] = s;
+  __syncthreads();
+  const float norm = fmaxf(sqrtf((red[0] + red[1]) + (red[2] + red[3])), 1e-12f);
+  for (int i = threadIdx.x; i < v.len; i += 256) v.unit[(size_t)blockIdx.x * v.len + i] = f2bf_(x[i] / norm);
+}
+
+hipError_t launch_spectral_units(const SnVectors& a, const SnVectors& b, int batch, hipStream_t stream) {
+  if (batch < 1 || !a.x || !b.x || !a.unit || !b.unit || a.len < 1 || b.len < 1 || a.stride < a.len || b.stride < b.len) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(sn_units_kernel, dim3(batch, 2), dim3(256), 0, stream, a, b);
+  return hipGetLastError();
+}
+
+namespace {
+bool classes_ok(const SnParams& sp, int* matrices) {
+  if (sp.n < 1 || sp.n > SN_MAX_CLASSES || sp.blk_start[sp.n] <= 0) return false;
+  *matrices = 0;
   for (int g = 0; g < sp.n; ++g) {
     const SnClass& c = sp.c[g];
-    if (c.batch <= 0 || c.d <= 0 || c.d_p % 128 || c.L_p % 8 || c.d > c.d_p || c.nblk * SN_ROWS != c.d_p || !c.xscale)
-      return hipErrorInvalidValue;
-    matrices += c.batch;
-    have2 = have2 && c.G2 != nullptr;
-    have4 = have4 && c.G4 != nullptr;
-    any[c.tall ? 1 : 0] = true;
+    if (c.batch <= 0 || c.d <= 0 || c.d_p % 128 || c.L_p % 8 || c.d > c.d_p || c.nblk * SN_ROWS != c.d_p || !c.xscale || c.ldx % 8) return false;
+    // the caller's own matrices fill the extents that the kernels walk
+    if (c.own && (c.d != c.d_p || c.xparts != c.nblk || (c.long_first && !c.tall))) return false;
+    *matrices += c.batch;
   }
-  if (blocks <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(sn_init_kernel, dim3(blocks), dim3(256), 0, stream, sp);
+  return true;
+}
+}  // namespace
+
+hipError_t launch_spectral_init(const SnParams& sp, hipStream_t stream) {
+  int matrices;
+  if (!classes_ok(sp, &matrices)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(sn_init_kernel, dim3(sp.blk_start[sp.n]), dim3(256), 0, stream, sp);
+  return hipGetLastError();
+}
+
+hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src) {
+  int matrices;
+  if (steps < 1 || !classes_ok(sp, &matrices)) return hipErrorInvalidValue;
+  const int blocks = sp.blk_start[sp.n];
+  bool have2 = true, have4 = true, any[2] = {false, false};
+  for (int g = 0; g < sp.n; ++g) {
+    have2 = have2 && sp.c[g].G2 != nullptr;
+    have4 = have4 && sp.c[g].G4 != nullptr;
+    any[sp.c[g].tall ? 1 : 0] = true;
+  }
   // applications before the final one: `steps` for tall matrices (one more than for wide ones, see the file comment),
   // as many as possible with the highest power
   int seq[2][3];   // per kind: how many applications of G4, G2, G, in this order

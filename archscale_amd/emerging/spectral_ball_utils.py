@@ -80,7 +80,7 @@ def spectral_norm(w: torch.Tensor, steps: int = 50) -> torch.Tensor:
 def power_iteration(w: torch.Tensor, steps: int = 50, eps: float = 1e-20):
     """(sigma, u, v) like spectral_ball_utils.py:151-166 of the reference: ``sigma`` fp32 of shape ``w.shape[:-2]``,
     ``u`` ``[..., rows, 1]`` and ``v`` ``[..., cols, 1]`` unit vectors in bf16, all from the HIP path
-    (``muon_power_iteration``: the vector sequence runs on the Gram matrix of the short side; the short-side vector is
+    (``muon_power_iteration_units``: the vector sequence runs on the Gram matrix of the short side; the short-side vector is
     its last iterate, the long-side one a single pass over the matrix). ``eps`` is unused, as in the reference."""
     import ctypes
 
@@ -98,8 +98,8 @@ def power_iteration(w: torch.Tensor, steps: int = 50, eps: float = 1e-20):
         mats = mats.contiguous()
     batch = mats.shape[0]
     sigma = torch.empty(batch, dtype=torch.float32, device=w.device)
-    u = torch.empty(batch, rows, dtype=torch.float32, device=w.device)
-    v = torch.empty(batch, cols, dtype=torch.float32, device=w.device)
+    u = torch.empty(batch, rows, dtype=torch.bfloat16, device=w.device)
+    v = torch.empty(batch, cols, dtype=torch.bfloat16, device=w.device)
     ptrs = (ctypes.c_void_p * batch)(*[mats[b].data_ptr() for b in range(batch)])
     prob = (_lib.SnProblem * 1)()
     q = prob[0]
@@ -108,14 +108,12 @@ def power_iteration(w: torch.Tensor, steps: int = 50, eps: float = 1e-20):
     L = _lib.lib()
     ws = _lib.workspace(w.device, L.muon_spectral_norm_workspace_bytes(prob, 1), tag="sn")
     with torch.cuda.device(w.device):
-        st = L.muon_power_iteration(ctypes.cast(ptrs, ctypes.POINTER(ctypes.c_void_p)), q.dtype, q.ld, batch, rows, cols,
-                                    steps, sigma.data_ptr(), u.data_ptr(), v.data_ptr(), ws.data_ptr(), ws.numel(),
-                                    _lib.current_stream_ptr(w.device))
-    _lib.check(st, "muon_power_iteration")
+        st = L.muon_power_iteration_units(ctypes.cast(ptrs, ctypes.POINTER(ctypes.c_void_p)), q.dtype, q.ld, batch, rows, cols,
+                                          steps, sigma.data_ptr(), u.data_ptr(), v.data_ptr(), ws.data_ptr(), ws.numel(),
+                                          _lib.current_stream_ptr(w.device))
+    _lib.check(st, "muon_power_iteration_units")
     lead = w.shape[:-2]
-    u = torch.nn.functional.normalize(u, dim=-1).to(torch.bfloat16).reshape(*lead, rows, 1)
-    v = torch.nn.functional.normalize(v, dim=-1).to(torch.bfloat16).reshape(*lead, cols, 1)
-    return sigma.reshape(lead), u, v
+    return sigma.reshape(lead), u.reshape(*lead, rows, 1), v.reshape(*lead, cols, 1)
 
 
 @torch.no_grad()

@@ -356,6 +356,10 @@ int muon_spectral_norm(const muon_sn_problem* problems_host, int n_problems, int
 int muon_power_iteration(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, int steps,
                          float* sigma_out_dev, float* u_out_dev, float* v_out_dev, void* workspace_dev,
                          size_t workspace_bytes, void* stream);
+/* The same with unit vectors: u and v bfloat16, each divided by max(its norm, 1e-12). */
+int muon_power_iteration_units(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, int steps,
+                               float* sigma_out_dev, void* u_out_dev, void* v_out_dev, void* workspace_dev,
+                               size_t workspace_bytes, void* stream);
 
 /* muon_ball_apply: for every item (a strided rows x cols block of a weight tensor)
  *   W <- f * decay * W - lr * lr_ratio * Phi

@@ -109,3 +109,23 @@ def test_only_newton_schulz_launches_are_recorded(gpu_device):
     ns.newton_schulz(a, gram_tail=False)
     recs = _lib.profile_collect()
     assert len(recs) == 15 and all(r["kind"] == "gemm" and r["flops_algorithmic"] > 0 for r in recs)
+
+
+@pytest.mark.parametrize("shape", [(1, 128, 128), (3, 128, 192), (2, 192, 128), (2, 256, 320), (1, 1024, 1088), (2, 640, 256), (1, 1152, 1024),
+                                   (2, 128, 200), (2, 130, 256), (1, 256, 1028)])
+def test_spectral_norms_of_matrices_where_they_lie(gpu_device, shape):
+    """bfloat16 matrices whose extents need no padding are read in place, fp32 copies of the same values through the workspace:
+    the same norms bit for bit, rows apart and matrices apart included."""
+    from archscale_amd.emerging.spectral_ball_utils import power_iteration, spectral_norm
+    g = torch.Generator().manual_seed(shape[1] + shape[2])
+    b, r, c = shape
+    wide = (torch.randn(2 * b, r, c + 24, generator=g) * 0.02).to(torch.bfloat16).to(gpu_device)
+    for W in (wide[:b, :, :c].contiguous(), wide[::2, :, 8:8 + c], wide[b:, :, 4:4 + c]):   # dense; strided; not 16-byte aligned
+        for steps in (1, 7, 50):
+            assert torch.equal(spectral_norm(W, steps), spectral_norm(W.float(), steps)), steps
+        for got, want in zip(power_iteration(W, 7), power_iteration(W.float(), 7)):
+            # (the long-side vector of a tall matrix in place is summed in another order: an fp32 sum of unit size moves by about
+            # 1e-6, a value that is then rounded to bfloat16 by one place, 2^-7 at most)
+            assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2e-6)
+        u = power_iteration(W, 7)[1].float().squeeze(-1)
+        assert torch.allclose(u.norm(dim=-1), torch.ones(b, device=gpu_device), atol=4e-3)
