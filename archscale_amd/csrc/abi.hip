@@ -221,6 +221,7 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     if (begin >= end) return hipSuccess;
     GroupedGemmParams q = {};
     q.quarter = level;
+    q.backwards = gp.backwards;
     for (int i = 0; i < gp.n_groups; ++i) {
       const int s = gp.tile_start[i], f = std::max(s, begin), e = std::min(gp.tile_start[i + 1], end);
       if (e <= f) continue;
@@ -593,6 +594,9 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
     }
   }
 
+  long iterate_bytes = 0;
+  for (const NsProblem& P : pr) iterate_bytes += 2L * P.q.batch * P.pl.Mp * P.pl.Np;
+  const int backwards = iterate_bytes <= BACKWARDS_BYTES ? 1 : 0;
   // one product of the iteration for every problem that `fill` accepts: problems that share a tile configuration go
   // into one launch (at most MAX_GROUPS per launch)
   auto run_mode = [&](int mode, bool split_launch, bool final_, int ws16, auto&& fill) -> hipError_t {
@@ -619,6 +623,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       auto flush = [&]() -> hipError_t {
         if (gp.n_groups == 0) return hipSuccess;
         const LaunchWork work = {fa, fi};
+        gp.backwards = backwards;
         hipError_t err = launch_rounds(tile, mode, split_launch, final_, gp, stream, units, &work, ws16);
         gp = GroupedGemmParams{};
         fa = fi = 0.0;

@@ -69,7 +69,7 @@ __device__ __forceinline__ void momentum_range(const PreItem& it, long begin, lo
           if (SS) { const float x = Elem<UD>::round(uv[k]); *ss += x * x; }
         }
         Elem<MD>::store8(m, i, mv[t]);
-        Elem<UD>::store8(u, i, uv);
+        Elem<UD>::keep8(u, i, uv);
       }
     }
   } else {
@@ -180,7 +180,7 @@ __device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, in
       u32x4 pk;
       pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
       pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      stream_store16(D + (size_t)r * ldd + c, pk);
+      *(u32x4*)(D + (size_t)r * ldd + c) = pk;
     }
   }
   if (tile_sumsq) {   // sum of squares of what this block wrote (every block of the grid: one value per 64x64 tile)
@@ -200,7 +200,7 @@ __device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, in
       u32x4 pk;
       pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
       pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      stream_store16(T + (size_t)c * ldt + r, pk);
+      *(u32x4*)(T + (size_t)c * ldt + r) = pk;
     }
   }
 }
@@ -399,7 +399,7 @@ __device__ __forceinline__ void momlay_tile(const MomMat& p, int r0, int c0,
         u32x4 pk;
         pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
         pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-        stream_store16(p.dst + (size_t)r * p.ldd + c, pk);
+        *(u32x4*)(p.dst + (size_t)r * p.ldd + c) = pk;
       }
     }
   }
@@ -444,7 +444,7 @@ momentum_layout_kernel(const MomGroupParams p) {
       u32x4 pk;
       pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
       pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      stream_store16(mt.dst + (size_t)c * mt.ldd + r, pk);
+      *(u32x4*)(mt.dst + (size_t)c * mt.ldd + r) = pk;
     }
   }
   block_reduce<1>(s, red);
@@ -670,6 +670,8 @@ muonh_coef_kernel(const int32_t* __restrict__ prefix, const float* __restrict__ 
   if (hdev) { lr = hdev->lr; eps = hdev->eps; }
   const int ii = blockIdx.x;
   double s[3] = {0.0, 0.0, 0.0};
+  // (8 trips of loads in flight: a vocabulary matrix of 50304 x 2048 has 49 trips, 18 us one after the other, 9 so)
+#pragma unroll 8
   for (int c = prefix[ii] + threadIdx.x; c < prefix[ii + 1]; c += EW_THREADS) {
     s[0] += partial[(size_t)c * 3 + 0];
     s[1] += partial[(size_t)c * 3 + 1];

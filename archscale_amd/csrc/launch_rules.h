@@ -67,6 +67,12 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   return {full, tail, 0};
 }
 
+// X' = B X walks its problems and matrices backwards where the iterates of a call (bf16 bytes) are at most this: it then meets the
+// matrices that X X^T has read last first, and the next X X^T the ones that it has written last, while the memory-side cache
+// (256 MB for X, X' and the square matrices) still holds them.  Iterates of 90 MB: MuonBall step 1519 -> 1494 us, EMA Muon 1216 ->
+// 1209; of 200 MB (64 experts), where neither order finds them, 1329 -> 1343; of 1.4 GB no difference.
+constexpr long BACKWARDS_BYTES = 128L << 20;
+
 // Tiles of 128 in the deep form where every block finds a unit of its own and the reductions are long: 3001 x 1023 302 -> 286 us,
 // 1500 x 2000 290 -> 270, a symmetric product of 2048 x 5632 47 -> 41; filling four stages costs reductions of 640 and less
 // 1 to 4 %.

@@ -64,6 +64,7 @@ constexpr int MAX_GROUPS = 16;
 struct GroupedGemmParams {
   int n_groups;
   int quarter;
+  int backwards;                    // MODE_BX: the last tile of the last problem first (see BACKWARDS_BYTES)
   int total;                        // filled in by the launch: tile_start[n_groups] ...
   int tile_start[MAX_GROUPS + 1];   // ... and the places past n_groups, with the largest int
   GemmParams g[MAX_GROUPS];

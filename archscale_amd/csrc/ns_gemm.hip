@@ -114,7 +114,7 @@ struct TileArgs {
   uint32_t inv_per_mat, inv_line;
   int part_tiles;
 };
-struct LaunchHead { int n_groups, quarter, total, first[3]; };   // first tiles of problems 1 to 3
+struct LaunchHead { int n_groups, quarter, backwards, total, first[3]; };   // first tiles of problems 1 to 3
 __device__ __forceinline__ TileArgs fetch_tile_args(const GemmParams& g) {
   return TileArgs{g.P, g.Q, g.strideP, g.strideQ, g.ldp, g.ldq, g.K, g.tilesM, g.tilesN, g.qt_first, g.t_first,
                   g.per_mat, g.inv_per_mat, g.inv_line, g.part_tiles};
@@ -124,7 +124,7 @@ __device__ __forceinline__ TileArgs fetch_tile_args(const GemmParams& g) {
       "+s"(a.qt_first), "+s"(a.t_first), "+s"(a.per_mat), "+s"(a.inv_per_mat), "+s"(a.inv_line), "+s"(a.part_tiles)
 __device__ __forceinline__ void pin(TileArgs& a) { asm volatile("" : ARCHSCALE_PIN_TILE_ARGS(a)); }
 __device__ __forceinline__ void pin(TileArgs& a, LaunchHead& h) {
-  asm volatile("" : ARCHSCALE_PIN_TILE_ARGS(a), "+s"(h.n_groups), "+s"(h.quarter), "+s"(h.total), "+s"(h.first[0]), "+s"(h.first[1]), "+s"(h.first[2]));
+  asm volatile("" : ARCHSCALE_PIN_TILE_ARGS(a), "+s"(h.n_groups), "+s"(h.quarter), "+s"(h.backwards), "+s"(h.total), "+s"(h.first[0]), "+s"(h.first[1]), "+s"(h.first[2]));
 }
 struct EndArgs {
   // (a pointer that comes out of an assembler statement would count as a generic one)
@@ -243,13 +243,14 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // together with the epilogue's paired conversions and running store addresses.
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   TileArgs p = fetch_tile_args(gp.g[0]);
-  LaunchHead head = {gp.n_groups, gp.quarter, gp.total, {gp.tile_start[1], gp.tile_start[2], gp.tile_start[3]}};
+  LaunchHead head = {gp.n_groups, gp.quarter, gp.backwards, gp.total, {gp.tile_start[1], gp.tile_start[2], gp.tile_start[3]}};
   pin(p, head);
   const int total = head.total, quarter = head.quarter;
   const int run = xcd_run(total);
   const int lap = total < 256 ? 0 : slot >> 5;   // (a launch of fewer than 256 tiles has `run` slots per XCD)
-  const int logical = (lap * 8 + xcd) * run + slot - lap * run;
+  int logical = (lap * 8 + xcd) * run + slot - lap * run;
   if (logical >= total) return;
+  if (MODE == MODE_BX && head.backwards) logical = total - 1 - logical;
   int grp = 0, start = 0;
   auto from = [&](int i, int first) { if (logical >= first) { grp = i; start = first; } };   // (past every tile for i >= n_groups)
 #pragma unroll

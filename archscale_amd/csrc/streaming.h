@@ -18,9 +18,11 @@ static_assert(EW_TRIPS * EW_THREADS * EW_VEC == MUON_CHUNK_ELEMS, "chunk must be
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 
-// Every kernel of this file streams: an element is touched once per launch and the tensors of a step are far larger
-// than the caches, so all 16-byte accesses carry the non-temporal hint (measured on a 2-read / 2-write stream of
-// 1 GiB arrays: 5.87 TB/s with it, 5.57 TB/s without; a plain copy 6.29 against 5.72 TB/s).
+// Most accesses stream: an element is touched once per launch and the tensors of a step are far larger than the caches, so
+// 16-byte accesses carry the non-temporal hint (measured on a 2-read / 2-write stream of 1 GiB arrays: 5.87 TB/s with it,
+// 5.57 TB/s without; a plain copy 6.29 against 5.72 TB/s).  Not the stores of what the next launch reads, the operand images and
+// the update: where they fit the memory-side cache it serves them (steps of width 1024: EMA Muon 1210 -> 1192 us, MuonBall
+// 1494 -> 1463; 3001 x 1023 188.5 -> 186), and where they do not nothing is lost (depth-16 set 22.15 ms either way).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x4 stream_load16(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
@@ -35,14 +37,16 @@ template <> struct Elem<DT_BF16> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(w[k] & 0xffff); v[2 * k + 1] = bf2f(w[k] >> 16); }
   }
-  static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) {
+  static __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
     u32x4 r;
     r.x = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
     r.y = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
     r.z = f2bf(v[4]) | ((uint32_t)f2bf(v[5]) << 16);
     r.w = f2bf(v[6]) | ((uint32_t)f2bf(v[7]) << 16);
-    stream_store16((uint16_t*)p + i, r);
+    return r;
   }
+  static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) { stream_store16((uint16_t*)p + i, pack8(v)); }
+  static __device__ __forceinline__ void keep8(void* p, long i, const float (&v)[8]) { *(u32x4*)((uint16_t*)p + i) = pack8(v); }
   static __device__ __forceinline__ float load1(const void* p, long i) { return bf2f(((const uint16_t*)p)[i]); }
   static __device__ __forceinline__ void store1(void* p, long i, float v) { ((uint16_t*)p)[i] = f2bf(v); }
   static __device__ __forceinline__ float round(float v) { return bf2f(f2bf(v)); }
@@ -58,6 +62,10 @@ template <> struct Elem<DT_F32> {
     const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
     __builtin_nontemporal_store(a, (f32x4*)((float*)p + i));
     __builtin_nontemporal_store(b, (f32x4*)((float*)p + i + 4));
+  }
+  static __device__ __forceinline__ void keep8(void* p, long i, const float (&v)[8]) {
+    *(f32x4*)((float*)p + i) = f32x4{v[0], v[1], v[2], v[3]};
+    *(f32x4*)((float*)p + i + 4) = f32x4{v[4], v[5], v[6], v[7]};
   }
   static __device__ __forceinline__ float load1(const void* p, long i) { return ((const float*)p)[i]; }
   static __device__ __forceinline__ void store1(void* p, long i, float v) { ((float*)p)[i] = v; }
