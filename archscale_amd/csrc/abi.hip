@@ -984,11 +984,24 @@ int muon_ns_batched_static(const void* in_dev, int in_dtype, int64_t in_batch_st
   return rc;
 }
 
+namespace {
+// K-split of a symmetric product: parts per tile of 128, tiles, and what it adds to the workspace (partial results, counters)
+struct SyrkSplit { int parts; long tiles; size_t bytes; };
+SyrkSplit syrk_split(int batch, int Np, int Kp) {
+  SyrkSplit s = {1, (long)batch * sym_tiles(Np / 128), 0};
+  if (env_switches().ksplit == 0 || env_switches().tile != 0) return s;
+  s.parts = product_parts(compute_units(), s.tiles, Kp / 64);
+  if (s.parts > 1) s.bytes = (size_t)s.tiles * s.parts * SK_TILE_BYTES + (size_t)round_up(s.tiles * (long)sizeof(int), 256);
+  return s;
+}
+}  // namespace
+
 size_t muon_syrk_workspace_bytes(int batch, int n, int k) {
   if (batch <= 0 || n <= 0 || k <= 0) return 0;
   const int tile = pick_tile(n, k);
   const size_t Np = (size_t)round_up(n, tile), Kp = (size_t)round_up(k, 64);
-  return (size_t)round_up((long)(batch * Np * Kp * 2), 256) + 2 * (size_t)round_up((long)(batch * Np * Np * 2), 256);
+  return (size_t)round_up((long)(batch * Np * Kp * 2), 256) + 2 * (size_t)round_up((long)(batch * Np * Np * 2), 256) +
+         syrk_split(batch, (int)Np, (int)Kp).bytes;
 }
 
 int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_dev, int64_t c_batch_stride, int ldc,
@@ -1052,7 +1065,19 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   gp.n_groups = 1;
   gp.g[0] = g;
   gp.tile_start[1] = (int)tiles;
-  e = launch_rounds(tile, mode, false, false, gp, stream, compute_units(), nullptr, 0);
+  const SyrkSplit split = syrk_split(batch, Np, Kp);
+  if (split.parts > 1) {
+    GemmParams& q = gp.g[0];
+    q.tilesM = q.tilesN = Np / 128;
+    q.ksplit = split.parts;
+    q.sk_partial = (float*)((char*)Dp + round_up((long)batch * Np * Np * 2, 256));
+    q.sk_counter = (int*)((char*)q.sk_partial + split.tiles * split.parts * SK_TILE_BYTES);
+    gp.tile_start[1] = (int)(split.tiles * split.parts);
+    e = launch_zero_i32(q.sk_counter, split.tiles, stream);
+    if (e == hipSuccess) e = launch_ns_gemm_grouped(128, mode, false, false, gp, stream, compute_units(), 0, true);
+  } else {
+    e = launch_rounds(tile, mode, false, false, gp, stream, compute_units(), nullptr, 0);
+  }
   if (e != hipSuccess || d_here) return (int)e;
   return (int)launch_unpad_copy(Dp, (long)Np * Np, Np, d_dev, d_batch_stride, ldd, batch, n, n, stream);
 }

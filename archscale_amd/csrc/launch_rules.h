@@ -67,6 +67,21 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   return {full, tail, 0};
 }
 
+// Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 with at most
+// one block to a unit.  Few tiles walk a long reduction on few units; a part costs 64 KiB of traffic each way and the call a
+// launch that clears the counters, so a part has at least SPLIT_PART_KT k-tiles and there are three of them or none (five where there
+// are only one or two tiles, which tiles of 64 walk faster: 100 x 4000 23.5 whole, 27.7 in three; 128 x 8192 25.6 / 23.2).
+// us, whole / as split here: 512 x 4096 27.0 / 21.9, 512 x 16384 89 / 31, 1024 x 4096 27.9 / 22.4, 1024 x 8192 48.7 / 26.8, 1536 x
+// 8192 50.1 / 34.6, 256 x 4096 26.2 / 24.2.  Not split: 512 x 2048 (16.5 whole, 18.8 in two), 2048 x 5632 (136 tiles: 37.7 whole, 41.3 in
+// three with two blocks to a unit, which share the LDS port that bounds a lone one).
+constexpr int SPLIT_PART_KT = 20, SPLIT_MIN_PARTS = 3, SPLIT_MAX_PARTS = 8;
+inline int product_parts(int units, long tiles, int kt) {
+  long parts = units / tiles;
+  if (parts > kt / SPLIT_PART_KT) parts = kt / SPLIT_PART_KT;
+  if (parts > SPLIT_MAX_PARTS) parts = SPLIT_MAX_PARTS;
+  return parts < (tiles < 3 ? SPLIT_MIN_PARTS + 2 : SPLIT_MIN_PARTS) ? 1 : (int)parts;
+}
+
 // X' = B X walks its problems and matrices backwards where the iterates of a call (bf16 bytes) are at most this: it then meets the
 // matrices that X X^T has read last first, and the next X X^T the ones that it has written last, while the memory-side cache
 // (256 MB for X, X' and the square matrices) still holds them.  Iterates of 90 MB: MuonBall step 1519 -> 1494 us, EMA Muon 1216 ->

@@ -103,3 +103,19 @@ int main() {
                    check=True)
     out = subprocess.run([str(tmp_path / "divide")], capture_output=True, text=True, check=True).stdout
     assert out.strip() == "0", out
+
+
+def test_parts_of_a_single_product(tmp_path):
+    """Parts of the K-split on 256 units: (tiles, k-tiles) -> parts; every part walks at least 20 k-tiles, one block to a unit."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "parts.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int u, t, k; while (scanf("%d %d %d", &u, &t, &k) == 3) printf("%d\n", archscale::product_parts(u, t, k)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "parts.cpp"), "-o", str(tmp_path / "parts")], check=True)
+    want = {(3, 59): 1, (3, 60): 3, (2, 99): 1, (1, 100): 5, (3, 64): 3, (10, 128): 6, (10, 256): 8, (36, 64): 3, (36, 256): 7, (78, 128): 3, (85, 256): 3,
+            (86, 256): 1, (136, 88): 1, (1, 4096): 8}
+    text = "".join(f"256 {t} {k}\n" for t, k in want)
+    out = subprocess.run([str(tmp_path / "parts")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())

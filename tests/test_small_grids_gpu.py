@@ -129,3 +129,33 @@ def test_spectral_norms_of_matrices_where_they_lie(gpu_device, shape):
             assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2e-6)
         u = power_iteration(W, 7)[1].float().squeeze(-1)
         assert torch.allclose(u.norm(dim=-1), torch.ones(b, device=gpu_device), atol=4e-3)
+
+
+@pytest.mark.parametrize("batch,n,k", [(1, 128, 3840), (1, 256, 4096), (2, 300, 4000), (1, 1000, 8200), (1, 640, 16384), (3, 512, 4096)])
+@pytest.mark.parametrize("addend", [False, True])
+def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
+    """Products whose reduction is cut into parts: bf16 rounding of the fp32 result, the same bits every time, symmetric."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    from archscale_amd import _lib
+    if addend and batch > 1:
+        pytest.skip("the entry point with an addend takes one matrix")
+    g = torch.Generator().manual_seed(n + k)
+    a = (torch.randn(batch, n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(gpu_device)
+    a = a[0] if batch == 1 else a
+    c = None
+    if addend:
+        c = torch.randn(n, n, generator=g) * 0.1
+        c = (c + c.t()).to(torch.bfloat16).to(gpu_device)
+    want = a.float() @ a.float().mT.contiguous()
+    if addend:
+        want = 1.2 * want - 0.7 * c.float()
+    first = None
+    for fill in (0, 0x7f, 0xff):   # whatever the workspace holds
+        for ws in list(_lib._workspaces.values()):
+            ws.fill_(fill)
+        got = ns.ns_line_1(a) if c is None else ns.tsyrk_ex(a, c, alpha=1.2, beta=-0.7)
+        assert torch.equal(got, got.mT)
+        first = got if first is None else first
+        assert torch.equal(got, first)
+    # one bf16 rounding (2^-9 of the value) beside sums of k products in fp32 (k 2^-24 of the root mean square at most)
+    assert ((first.float() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-3 * want.pow(2).mean().sqrt()).all()
