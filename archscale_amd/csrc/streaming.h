@@ -17,6 +17,13 @@ static_assert(EW_TRIPS * EW_THREADS * EW_VEC == MUON_CHUNK_ELEMS, "chunk must be
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
+// two at a time: one conversion for both instead of two and their merging (vocabulary matrices on the sphere 725 -> 717 us per
+// step, 64 experts 1317 -> 1313)
+__device__ __forceinline__ uint32_t f2bf_pair(float a, float b) {
+  typedef float f32x2_ __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_ __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_){a, b}, bf16x2_));
+}
 
 // Most accesses stream: an element is touched once per launch and the tensors of a step are far larger than the caches, so
 // 16-byte accesses carry the non-temporal hint (measured on a 2-read / 2-write stream of 1 GiB arrays: 5.87 TB/s with it,
@@ -38,12 +45,7 @@ template <> struct Elem<DT_BF16> {
     for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(w[k] & 0xffff); v[2 * k + 1] = bf2f(w[k] >> 16); }
   }
   static __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
-    u32x4 r;
-    r.x = f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-    r.y = f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-    r.z = f2bf(v[4]) | ((uint32_t)f2bf(v[5]) << 16);
-    r.w = f2bf(v[6]) | ((uint32_t)f2bf(v[7]) << 16);
-    return r;
+    return u32x4{f2bf_pair(v[0], v[1]), f2bf_pair(v[2], v[3]), f2bf_pair(v[4], v[5]), f2bf_pair(v[6], v[7])};
   }
   static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) { stream_store16((uint16_t*)p + i, pack8(v)); }
   static __device__ __forceinline__ void keep8(void* p, long i, const float (&v)[8]) { *(u32x4*)((uint16_t*)p + i) = pack8(v); }
