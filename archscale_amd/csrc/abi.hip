@@ -213,8 +213,10 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
     all += (double)(gp.tile_start[i + 1] - gp.tile_start[i]) * gp.g[i].K;
     longest = std::max(longest, (double)gp.g[i].K);
   }
-  const LaunchSplit cut = env_switches().quarter ? launch_split(units, tile, split, total, all, longest)
-                                                 : LaunchSplit{total, 0, 0};
+  LaunchSplit cut = {total, 0, 0};
+  if (env_switches().quarter)
+    cut = mode == MODE_SYRKT && !split && fine_tiles(units, tile, total, longest) ? LaunchSplit{0, 0, total}
+                                                                                   : launch_split(units, tile, split, total, all, longest);
   if (cut.whole == total) return launch(tile, gp, 1.0);
   // tiles [begin, end) of the launch as (2^level)^2 tiles each of the configuration that is `level` smaller (level 0: as they are)
   auto run = [&](int begin, int end, int level) -> hipError_t {

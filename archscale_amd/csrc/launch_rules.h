@@ -88,6 +88,15 @@ inline int product_parts(int units, long tiles, int kt) {
 // 1209; of 200 MB (64 experts), where neither order finds them, 1329 -> 1343; of 1.4 GB no difference.
 constexpr long BACKWARDS_BYTES = 128L << 20;
 
+// X X^T of so few tiles of 128 over a long reduction that even as tiles of 64 it leaves most of the chip idle: as tiles of 32, one
+// block to a unit.  us per call, as tiles of 64 / of 32: 512 x 2048 119.5 / 108.3, 512 x 8192 215 / 183, 256 x 2048 104 / 90, 640 x
+// 4096 (15 tiles) 167 / 147, 256 x 1024 88.6 / 82.5; beyond one block to a unit they lose: 700 x 3000 (21 tiles) 160 / 171, 1023 x 3001
+// (36) 193 / 227.
+constexpr int FINE_MAX_128 = 16, FINE_MIN_K = 1024;
+inline bool fine_tiles(int units, int tile, int total, double longest) {
+  return tile == 128 && (long)total * RULE_UNITS <= (long)FINE_MAX_128 * units && longest >= FINE_MIN_K;
+}
+
 // Tiles of 128 in the deep form where every block finds a unit of its own and the reductions are long: 3001 x 1023 302 -> 286 us,
 // 1500 x 2000 290 -> 270, a symmetric product of 2048 x 5632 47 -> 41; filling four stages costs reductions of 640 and less
 // 1 to 4 %.

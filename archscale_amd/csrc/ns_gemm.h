@@ -74,7 +74,7 @@ static_assert(sizeof(GroupedGemmParams) <= 4096, "kernel arguments are limited t
 // number of block tiles of one problem
 long ns_gemm_tiles(int mode, const GemmParams& p);
 
-// tile: side of the block tile, 256, 128 or 64 (four waves each; 64 without the hi+lo pair)
+// tile: side of the block tile, 256, 128, 64 or 32 (four waves each; 64 without the hi+lo pair, 32 for MODE_SYRKT alone)
 // f16: 0 = the workspace matrices of the launch are bfloat16; 1 = IEEE half (see GemmParams::out_shift), not with split;
 // 2 = bfloat16 operands, IEEE-half result (MODE_BX, not the final launch)
 // units: compute units of the device

@@ -85,7 +85,9 @@ __device__ __forceinline__ int lds_chunk_off(int r, int c) { return r * ROW_BYTE
 // each) covers all 64 banks.
 template <int ROWS>
 __device__ __forceinline__ int kmaj_swz(int k) {
-  return ROWS >= 128 ? ((k & 3) << 2) | (((k >> 3) & 1) << 1) : (((k >> 1) & 1) << 2) | (((k >> 3) & 1) << 1);
+  if constexpr (ROWS >= 128) return ((k & 3) << 2) | (((k >> 3) & 1) << 1);
+  else if constexpr (ROWS == 64) return (((k >> 1) & 1) << 2) | (((k >> 3) & 1) << 1);
+  else return ((k >> 3) & 1) << 1;
 }
 
 // consecutive tiles of a launch that go to one XCD (see the kernel); the grid is a multiple of eight runs
@@ -193,7 +195,7 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 1
 template <int BT, int SP, int SQ, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
 __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know the buffer descriptor type)
-  static_assert(BT == 256 || BT == 128 || BT == 64, "block tiles");
+  static_assert(BT == 256 || BT == 128 || BT == 64 || (BT == 32 && MODE == MODE_SYRKT && !SPLIT && !SK), "block tiles");
   static_assert(!(F16 && SPLIT), "the hi+lo pair is a bfloat16 device");
   static_assert(!SK || (BT == 128 && !SPLIT && !FINAL && MODE != MODE_BX), "the K-split serves symmetric products in the 128 configuration");
   static_assert(F16 != 2 || (MODE == MODE_BX && !FINAL), "only X' changes its storage type");
@@ -515,7 +517,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     constexpr bool ACTIVE = decltype(active)::value, CP = decltype(cp)::value;
     constexpr int cbuf = decltype(cbuf_)::value;
     // reads within the first three quarters of the k-step, copies over all of it
-    constexpr int RSPAN = NMF * 3 / 4;
+    constexpr int RSPAN = NMF > 1 ? NMF * 3 / 4 : 1;
     static_for<NMF>([&](auto q_) __attribute__((always_inline)) {
       constexpr int q = decltype(q_)::value;
       if constexpr (ACTIVE) mfma16<IN16, AGPR>(acc[q / FR][q % FR], af[cbuf][q / FR], bq[cbuf][q % FR]);
@@ -545,6 +547,43 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   auto k_range = [&](auto active) __attribute__((always_inline)) {
     constexpr bool ACTIVE = decltype(active)::value;
     int sP = 0, sQ = QBASE;               // stages of k-tile kt
+    if constexpr (BT == 32) {
+      // A wave has one MFMA per k-step here, and what a k-step takes is the wait for its LDS reads: a whole k-tile at a time, the
+      // reads of the next one behind the MFMAs of this one that used their registers (X X^T of 512 x 8192 188.6 -> 183.5 us a call;
+      // tiles of 64, which the LDS port bounds, are 1 to 2 % slower so).
+      auto reads = [&](auto kk_, int stP, int stQ) __attribute__((always_inline)) {
+        if constexpr (ACTIVE) static_for<NRD>([&](auto r_) __attribute__((always_inline)) { fread(kk_, stP, stQ, kk_, r_); });
+      };
+      auto multiply = [&](auto kk_) __attribute__((always_inline)) {
+        constexpr int kk = decltype(kk_)::value;
+        if constexpr (ACTIVE) mfma16<IN16, AGPR>(acc[0][0], af[kk][0], bq[kk][0]);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto arrive = [&]() __attribute__((always_inline)) {
+        if constexpr (ACTIVE) { land(I0{}); land(I1{}); }
+      };
+      reads(I0{}, 0, QBASE);
+      reads(I1{}, 0, QBASE);
+      arrive();
+      for (int kt = 0; kt < KT_ALL; ++kt) {
+        const int nP = nextP(sP), nQ = nextQ(sQ), pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
+        const Source src = source(kt + SP);
+        wait_copies<(SP - 2) * PAIR>();   // k-tile kt + 1 has landed, and every wave has its fragments of kt
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(I0{});
+        reads(I0{}, nP, nQ);
+        multiply(I1{});
+        reads(I1{}, nP, nQ);
+        copyQ(src, pQ, 0);
+        copyP(src, sP, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        arrive();
+        sP = nP;
+        sQ = nQ;
+      }
+      return;
+    }
     if constexpr (ACTIVE) {
       static_for<NRD>([&](auto r_) __attribute__((always_inline)) { fread(I0{}, 0, QBASE, I0{}, r_); });
       land(I0{});
@@ -579,7 +618,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
           if (!*(volatile int*)smem) return;
         }
       }
-      __syncthreads();
+      if constexpr (BT > 32) __syncthreads();   // (the one before the epilogue)
       return;
     }
   }
@@ -645,6 +684,21 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   const float sc = out.scale ? out.scale[b] : 1.f;
   const float bx_sc = sc * __builtin_ldexpf(1.f, out.out_shift);   // MODE_BX: scale of the result (a power of two from the host)
   const float alpha = SYRK_PLAIN ? out.alpha * sc * sc : out.alpha, beta = out.beta;
+  if constexpr (BT == 32) {
+    // One fragment per wave, stored straight from the registers (a lane has four consecutive rows of one column).  On the
+    // diagonal the fragment is its own mirror image.
+    acc_touch<AGPR>(acc[0][0]);
+    const uint2 bits = pk4(acc[0][0][0] * alpha, acc[0][0][1] * alpha, acc[0][0][2] * alpha, acc[0][0][3] * alpha);
+    const int r = R0 + wr0 + 4 * lg, c = C0 + wc0 + l16;
+    __bf16* const base = (__bf16*)out.C + (size_t)b * out.strideC;
+    *(uint2*)(base + (size_t)c * out.ldc + r) = bits;
+    if (!diag || above) {
+      const uint16_t e[4] = {(uint16_t)bits.x, (uint16_t)(bits.x >> 16), (uint16_t)bits.y, (uint16_t)(bits.y >> 16)};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ((uint16_t*)base)[(size_t)(r + q) * out.ldc + c] = e[q];
+    }
+    return;
+  }
   // A diagonal tile of a product of a matrix with ITSELF is symmetric bit for bit as it comes out of the matrix cores
   // (element (i,j) and element (j,i) are the same products summed in the same order over k), so it is stored like any
   // other tile, as one image.  A diagonal tile of P Q^T with two different (commuting, symmetric) matrices is symmetric
@@ -843,12 +897,14 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 //   128 deep  144 KiB for a block that has its compute unit to itself (a launch that gives no unit a second one): with two
 //             stages and nothing else resident, a k-tile waits for its copies
 //   64        launches that cannot occupy the chip with tiles of 128: latency bound, so as many stages as two blocks leave room for
-enum { CFG_256, CFG_128, CFG_128_DEEP, CFG_64 };
+//   32        X X^T of few tiles over a long reduction, which tiles of 64 walk at the rate of the LDS port of a few units
+enum { CFG_256, CFG_128, CFG_128_DEEP, CFG_64, CFG_32 };
 template <int CFG> struct Config;
 template <> struct Config<CFG_256> { static constexpr int BT = 256, SP = 2, SQ = 3, BLOCKS = 1; };
 template <> struct Config<CFG_128> { static constexpr int BT = 128, SP = 2, SQ = 3, BLOCKS = 2; };
 template <> struct Config<CFG_128_DEEP> { static constexpr int BT = 128, SP = 4, SQ = 5, BLOCKS = 1; };
 template <> struct Config<CFG_64> { static constexpr int BT = 64, SP = 4, SQ = 5, BLOCKS = 2; };
+template <> struct Config<CFG_32> { static constexpr int BT = 32, SP = 4, SQ = 5, BLOCKS = 2; };
 
 // The two configurations that fill the chip, by block tile and wave tile.
 template <int BM, int BN, int WM, int WN, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
@@ -866,9 +922,19 @@ ns_gemm_deep_kernel(const GroupedGemmParams gp) {
   ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, false>(gp);
 }
 
+// Tiles of 32 (X X^T only).
+template <int MODE, int F16>
+__global__ void __launch_bounds__(256, Config<CFG_32>::BLOCKS)
+ns_gemm_fine_kernel(const GroupedGemmParams gp) {
+  ns_gemm_tile<Config<CFG_32>::BT, Config<CFG_32>::SP, Config<CFG_32>::SQ, MODE, false, false, true, F16, false>(gp);
+}
+
 template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
 static constexpr auto kernel_of() {
   constexpr int BT = Config<CFG>::BT;
+  if constexpr (CFG == CFG_32) {
+    return &ns_gemm_fine_kernel<MODE, F16>;
+  } else
   if constexpr (CFG == CFG_256 || CFG == CFG_128) {
     return &ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
   } else {
@@ -1026,6 +1092,8 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
   if (tile == 128 && deep) return by_storage(std::integral_constant<int, CFG_128_DEEP>{});
   if (tile == 128) return by_storage(std::integral_constant<int, CFG_128>{});
   if (tile == 64) return by_storage(std::integral_constant<int, CFG_64>{});
+  if (tile == 32 && mode == MODE_SYRKT && !split && !final_ && f16 != 2)
+    return f16 ? launch_one<CFG_32, MODE_SYRKT, false, false, true, 1>(gp, stream) : launch_one<CFG_32, MODE_SYRKT, false, false, true, 0>(gp, stream);
   return hipErrorInvalidValue;
 }
 

@@ -159,3 +159,15 @@ def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
         assert torch.equal(got, first)
     # one bf16 rounding (2^-9 of the value) beside sums of k products in fp32 (k 2^-24 of the root mean square at most)
     assert ((first.float() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-3 * want.pow(2).mean().sqrt()).all()
+
+
+@pytest.mark.parametrize("m,n", [(130, 1024), (256, 1090), (511, 1500), (512, 2048), (640, 1025), (2100, 300)])
+@pytest.mark.parametrize("prec", ["bf16", "f16"])
+def test_tiles_of_32_give_the_bits_of_larger_ones(gpu_device, m, n, prec):
+    """Alone, X X^T of these matrices runs in tiles of 32 (short side up to 640, long side from 1024 on); sixteen of them, in larger ones."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator().manual_seed(m + n)
+    x = (torch.randn(16, m, n, generator=g) * 1e-3).to(torch.bfloat16).to(gpu_device)
+    batch = ns.newton_schulz(x, prec=prec)
+    for i in (0, 15):
+        assert torch.equal(ns.newton_schulz(x[i], prec=prec), batch[i])
