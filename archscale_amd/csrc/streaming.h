@@ -131,6 +131,15 @@ __device__ __forceinline__ float thread_sumsq_strided(const char* base, int rows
   const long numel = (long)rows * cols, begin = (long)chunk * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < numel ? begin + MUON_CHUNK_ELEMS : numel;
   float s = 0.f;
+  if (ld == cols) {   // rows one after the other, but in odd numbers or not aligned: nothing to divide, eight loads in flight
+#pragma unroll 8
+    for (long i = begin + tid; i < end; i += EW_THREADS) {
+      float x = Elem<DT>::load1(base, i);
+      if (cast_first) x = bf2f(f2bf(x));
+      s = fmaf(x, x, s);
+    }
+    return s;
+  }
   for (long i = begin + tid; i < end; i += EW_THREADS) {
     const long r = i / cols, cc = i - r * cols;
     float x = Elem<DT>::load1(base, r * ld + cc);
