@@ -1373,7 +1373,7 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
   SnParams last = {};
   if ((st = for_class_chunks([&](const SnParams& sp) {
          last = sp;
-         return launch_spectral_iterate(sp, steps, stream, final_src);
+         return launch_spectral_iterate(sp, steps, stream, final_src, !out.short_unit);
        })) != 0)
     return st;
   if (vectors) {   // one problem, one class: its singular vectors from the iterates that are still in the workspace
@@ -1383,7 +1383,7 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
     if ((e = launch_spectral_vectors(c, L, src, out.short_out, long_out, stream)) != hipSuccess) return (int)e;
     if (out.short_unit &&
         (e = launch_spectral_units(SnVectors{spectral_short_vectors(c, src), c.d_p, out.short_unit, c.d},
-                                   SnVectors{long_out, L, out.long_unit, L}, c.batch, stream)) != hipSuccess)
+                                   SnVectors{long_out, L, out.long_unit, L}, c, src, stream)) != hipSuccess)
       return (int)e;
   }
   return 0;

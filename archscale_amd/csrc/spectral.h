@@ -49,18 +49,18 @@ hipError_t launch_spectral_xscale(const SnParams& sp, hipStream_t stream);
 hipError_t launch_spectral_init(const SnParams& sp, hipStream_t stream);
 
 // the applications of G that `steps` rounds stand for (`steps` for wide matrices, `steps + 1` for tall ones, the
-// last one always G itself; the others G^4, G^2 or G as far as the class has them) + final
+// last one always G itself; the others G^4, G^2 or G as far as the class has them) + sigma, unless launch_spectral_units follows
 // final_src (optional, two ints): which of the two z buffers holds the last iterate of the wide / of the tall classes
-hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src = nullptr);
+hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src = nullptr, bool sigma = true);
 
 // after launch_spectral_iterate, for one class: short_out[b][d] = the short-side singular vector (unnormalised: u of a
 // wide matrix, v of a tall one), long_out[b][L] = X^T times the iterate before the last (v of a wide matrix, u of a
 // tall one, unnormalised); L = the true long extent
 hipError_t launch_spectral_vectors(const SnClass& c, int L, int src_final, float* short_out, float* long_out,
                                    hipStream_t stream);
-// unit[b] = bf16(x[b] / max(|x[b]|, 1e-12)) of two stacks of vectors, x[b] at x + b * stride
+// unit[b] = bf16(x[b] / max(|x[b]|, 1e-12)) of two stacks of vectors, x[b] at x + b * stride; and sigma
 struct SnVectors { const float* x; long stride; uint16_t* unit; int len; };
-hipError_t launch_spectral_units(const SnVectors& a, const SnVectors& b, int batch, hipStream_t stream);
+hipError_t launch_spectral_units(const SnVectors& a, const SnVectors& b, const SnClass& c, int src_final, hipStream_t stream);
 // the short-side vectors where launch_spectral_vectors takes them from
 const float* spectral_short_vectors(const SnClass& c, int src_final);
 

@@ -259,21 +259,21 @@ sn_step_kernel(const SnParams sp, int src_wide, int which_wide, int src_tall, in
   }
 }
 
-// sigma[b] from the partials of the last round
+// sigma[blk] of a class from the partials of the last round, by one wave
+__device__ __forceinline__ void sigma_of(const SnClass& c, int blk, int src, int lane) {
+  float S, D;
+  sum_pairs(c.part + (((size_t)src * c.batch + blk) * c.nblk) * 2, c.nblk, lane, S, D);
+  const float s2 = c.tall ? D : (D > 0.f ? S / D : 0.f);
+  const float xs = c.xscale[blk];   // G = xs^2 X X^T
+  if (lane == 0) c.sigma[blk] = xs > 0.f ? sqrtf(fmaxf(s2, 0.f)) / xs : 0.f;
+}
 __global__ void __launch_bounds__(64)
 sn_final_kernel(const SnParams sp, int src_wide, int src_tall) {
   // one wave per matrix: blocks are numbered class by class
   int blk = blockIdx.x, g = 0;
   while (g < sp.n && blk >= sp.c[g].batch) { blk -= sp.c[g].batch; ++g; }
   if (g >= sp.n) return;
-  const SnClass c = sp.c[g];
-  const int src = c.tall ? src_tall : src_wide;
-  const int lane = threadIdx.x;
-  float S, D;
-  sum_pairs(c.part + (((size_t)src * c.batch + blk) * c.nblk) * 2, c.nblk, lane, S, D);
-  const float s2 = c.tall ? D : (D > 0.f ? S / D : 0.f);
-  const float xs = c.xscale[blk];   // G = xs^2 X X^T
-  if (lane == 0) c.sigma[blk] = xs > 0.f ? sqrtf(fmaxf(s2, 0.f)) / xs : 0.f;
+  sigma_of(sp.c[g], blk, sp.c[g].tall ? src_tall : src_wide, threadIdx.x);
 }
 
 // xscale[b]: one wave per matrix, blocks numbered class by class; the tile sums are added in a fixed order
@@ -400,26 +400,48 @@ hipError_t launch_spectral_vectors(const SnClass& c, int L, int src_final, float
   return hipGetLastError();
 }
 
-// one block per vector; the vectors are short (one read from the caches), the launch is what it costs: 16 pairs of 1024 and 2816
-// in 6 us, eight launches of the tensor library 25
+// one block per vector and one for sigma; the vectors are short, so the launch and its chain of loads are what it costs: 16 loads
+// in flight per thread instead of one, and no launch of its own for sigma.  16 matrices of 1024 x 2816 with their vectors, 50
+// rounds: 249.8 -> 243.4 us the whole call (as launches of the tensor library the unit vectors alone were 25)
 __global__ void __launch_bounds__(256)
-sn_units_kernel(const SnVectors a, const SnVectors c) {
+sn_units_kernel(const SnVectors a, const SnVectors o, const SnClass c, int src_final) {
   __shared__ float red[4];
-  const SnVectors v = blockIdx.y ? c : a;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.y == 2) {
+    if (wave == 0) sigma_of(c, blockIdx.x, src_final, lane);
+    return;
+  }
+  const SnVectors v = blockIdx.y ? o : a;
   const float* x = v.x + (size_t)blockIdx.x * v.stride;
-  float s = 0.f;
-  for (int i = threadIdx.x; i < v.len; i += 256) s = fmaf(x[i], x[i], s);
+  uint16_t* unit = v.unit + (size_t)blockIdx.x * v.len;
+  constexpr int RUN = 16;
+  float f[RUN], s = 0.f;
+  auto fetch = [&](int i0) {
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) f[k] = x[min(i0 + k * 256, v.len - 1)];
+  };
+  for (int i0 = threadIdx.x; i0 < v.len; i0 += RUN * 256) {
+    fetch(i0);
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) s = i0 + k * 256 < v.len ? fmaf(f[k], f[k], s) : s;
+  }
   s = wave_sum(s);
   if (lane == 0) red[wave] = s;
   __syncthreads();
   const float norm = fmaxf(sqrtf((red[0] + red[1]) + (red[2] + red[3])), 1e-12f);
-  for (int i = threadIdx.x; i < v.len; i += 256) v.unit[(size_t)blockIdx.x * v.len + i] = f2bf_(x[i] / norm);
+  for (int i0 = threadIdx.x; i0 < v.len; i0 += RUN * 256) {
+    if (v.len > RUN * 256) fetch(i0);   // (else the run of the first loop)
+#pragma unroll
+    for (int k = 0; k < RUN; ++k)
+      if (i0 + k * 256 < v.len) unit[i0 + k * 256] = f2bf_(f[k] / norm);
+  }
 }
 
-hipError_t launch_spectral_units(const SnVectors& a, const SnVectors& b, int batch, hipStream_t stream) {
-  if (batch < 1 || !a.x || !b.x || !a.unit || !b.unit || a.len < 1 || b.len < 1 || a.stride < a.len || b.stride < b.len) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(sn_units_kernel, dim3(batch, 2), dim3(256), 0, stream, a, b);
+hipError_t launch_spectral_units(const SnVectors& a, const SnVectors& b, const SnClass& c, int src_final, hipStream_t stream) {
+  if (c.batch < 1 || !a.x || !b.x || !a.unit || !b.unit || a.len < 1 || b.len < 1 || a.stride < a.len || b.stride < b.len ||
+      !c.part || !c.sigma || !c.xscale || (src_final != 0 && src_final != 1))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(sn_units_kernel, dim3(c.batch, 3), dim3(256), 0, stream, a, b, c, src_final);
   return hipGetLastError();
 }
 
@@ -445,7 +467,7 @@ hipError_t launch_spectral_init(const SnParams& sp, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src) {
+hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t stream, int* final_src, bool sigma) {
   int matrices;
   if (steps < 1 || !classes_ok(sp, &matrices)) return hipErrorInvalidValue;
   const int blocks = sp.blk_start[sp.n];
@@ -481,7 +503,7 @@ hipError_t launch_spectral_iterate(const SnParams& sp, int steps, hipStream_t st
     if (w0 >= 0) src[0] ^= 1;
     if (w1 >= 0) src[1] ^= 1;
   }
-  hipLaunchKernelGGL(sn_final_kernel, dim3(matrices), dim3(64), 0, stream, sp, src[0], src[1]);
+  if (sigma) hipLaunchKernelGGL(sn_final_kernel, dim3(matrices), dim3(64), 0, stream, sp, src[0], src[1]);
   if (final_src) { final_src[0] = src[0]; final_src[1] = src[1]; }
   return hipGetLastError();
 }

@@ -131,6 +131,34 @@ def test_spectral_norms_of_matrices_where_they_lie(gpu_device, shape):
         assert torch.allclose(u.norm(dim=-1), torch.ones(b, device=gpu_device), atol=4e-3)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 1, 257), (2, 255, 256), (2, 130, 4096), (1, 4097, 64), (1, 33, 8200)])
+def test_unit_vectors_and_norm_from_one_launch(gpu_device, shape):
+    """Around the ends of a thread's run of 16 elements: sigma has the bits of the call for norms alone, the unit vectors are those of
+    the call that leaves them unnormalised (an fp32 norm of n elements is off by less than n 2^-24, then one rounding to bfloat16)."""
+    import ctypes
+    from archscale_amd import _lib
+    from archscale_amd.emerging.spectral_ball_utils import power_iteration, spectral_norm
+    b, r, c = shape
+    g = torch.Generator().manual_seed(r + c)
+    W = (torch.randn(b, r, c, generator=g) * 0.02).to(torch.bfloat16).to(gpu_device)
+    sigma, u, v = power_iteration(W, 6)
+    assert torch.equal(sigma, spectral_norm(W, 6))
+    raw = [torch.empty(b, n, device=gpu_device) for n in (r, c)]
+    s = torch.empty(b, device=gpu_device)
+    ptrs = (ctypes.c_void_p * b)(*[W[i].data_ptr() for i in range(b)])
+    pp = ctypes.cast(ptrs, ctypes.POINTER(ctypes.c_void_p))
+    prob = (_lib.SnProblem * 1)()
+    prob[0].w_ptrs, prob[0].sigma_out, prob[0].dtype, prob[0].ld, prob[0].batch, prob[0].rows, prob[0].cols, prob[0].flags = pp, s.data_ptr(), 0, c, b, r, c, 0
+    L = _lib.lib()
+    ws = _lib.workspace(W.device, L.muon_spectral_norm_workspace_bytes(prob, 1), tag="sn")
+    _lib.check(L.muon_power_iteration(pp, 0, c, b, r, c, 6, s.data_ptr(), raw[0].data_ptr(), raw[1].data_ptr(), ws.data_ptr(),
+                                      ws.numel(), _lib.current_stream_ptr(W.device)), "muon_power_iteration")
+    assert torch.equal(s, sigma)
+    for got, x in zip((u, v), raw):
+        want = x.double() / x.double().norm(dim=-1, keepdim=True)
+        assert bool(((got.squeeze(-1).double() - want).abs() <= want.abs() * (2.0 ** -8 + x.shape[-1] * 2.0 ** -24)).all())
+
+
 @pytest.mark.parametrize("batch,n,k", [(1, 128, 3840), (1, 256, 4096), (2, 300, 4000), (1, 1000, 8200), (1, 640, 16384), (3, 512, 4096)])
 @pytest.mark.parametrize("addend", [False, True])
 def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
