@@ -34,7 +34,7 @@ struct LaunchSplit { int whole, quarters, sixteenths; };
 // Less than one round: as tiles of 256 the launch takes as long as its longest tile; quartered, the tiles spread over the
 // chip, at the same 0.6 of the rate.  Quartered when the mean load of a unit is below QUARTER_LOAD of the longest tile.  At 0.59
 // (208 tiles of 2816 and 1024 k-values, X X^T of that EMA-Muon set) a product takes 56 us quartered, 66 as it is; at 0.625
-// (160 equal tiles, power iteration over 16 x 1024 x 2816) the call takes 337 against 317 us.
+// (160 equal tiles, power iteration over 16 x 1024 x 2816) the call takes 259 against 250 us.
 //
 // Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
 // a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
