@@ -991,7 +991,8 @@ namespace {
 struct SyrkSplit { int parts; long tiles; size_t bytes; };
 SyrkSplit syrk_split(int batch, int Np, int Kp) {
   SyrkSplit s = {1, (long)batch * sym_tiles(Np / 128), 0};
-  if (env_switches().ksplit == 0 || env_switches().tile != 0) return s;
+  // (short reductions, the most frequent calls, do without asking the device)
+  if (Kp / 64 < SPLIT_MIN_PARTS * SPLIT_PART_KT || env_switches().ksplit == 0 || env_switches().tile != 0) return s;
   s.parts = product_parts(compute_units(), s.tiles, Kp / 64);
   if (s.parts > 1) s.bytes = (size_t)s.tiles * s.parts * SK_TILE_BYTES + (size_t)round_up(s.tiles * (long)sizeof(int), 256);
   return s;
