@@ -612,7 +612,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
       const int key = 128 * 100 + mode * 10;
       const GroupedGemmParams launch = sk;
       hipError_t err = timed_launch(key, sk_fa, sk_fi, stream, [&] {
-        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, units, ws16, true);
+        return launch_ns_gemm_grouped(128, mode, false, false, launch, stream, units, ws16, CUT_BLOCKS);
       });
       sk = GroupedGemmParams{};
       sk.quarter = 1;
@@ -987,14 +987,16 @@ int muon_ns_batched_static(const void* in_dev, int in_dtype, int64_t in_batch_st
 }
 
 namespace {
-// K-split of a symmetric product: parts per tile of 128, tiles, and what it adds to the workspace (partial results, counters)
-struct SyrkSplit { int parts; long tiles; size_t bytes; };
+// K-split of a symmetric product: parts per tile of 128, tiles of all matrices, whether a block takes one part of a tile or all, and
+// what it adds to the workspace (partial results, counters)
+struct SyrkSplit { int parts; long tiles; KCut cut; size_t bytes; };
 SyrkSplit syrk_split(int batch, int Np, int Kp) {
-  SyrkSplit s = {1, (long)batch * sym_tiles(Np / 128), 0};
-  // (short reductions, the most frequent calls, do without asking the device)
-  if (Kp / 64 < SPLIT_MIN_PARTS * SPLIT_PART_KT || env_switches().ksplit == 0 || env_switches().tile != 0) return s;
-  s.parts = product_parts(compute_units(), s.tiles, Kp / 64);
-  if (s.parts > 1) s.bytes = (size_t)s.tiles * s.parts * SK_TILE_BYTES + (size_t)round_up(s.tiles * (long)sizeof(int), 256);
+  SyrkSplit s = {1, (long)batch * sym_tiles(Np / 128), CUT_NONE, 0};
+  if (env_switches().ksplit == 0 || env_switches().tile != 0) return s;
+  s.parts = product_parts(RULE_UNITS, sym_tiles(Np / 128), Kp / 64);
+  if (s.parts == 1) return s;
+  s.cut = parts_by_blocks(s.tiles) ? CUT_BLOCKS : CUT_SEQUENCE;
+  if (s.cut == CUT_BLOCKS) s.bytes = (size_t)s.tiles * s.parts * SK_TILE_BYTES + (size_t)round_up(s.tiles * (long)sizeof(int), 256);
   return s;
 }
 }  // namespace
@@ -1069,15 +1071,20 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   gp.g[0] = g;
   gp.tile_start[1] = (int)tiles;
   const SyrkSplit split = syrk_split(batch, Np, Kp);
-  if (split.parts > 1) {
+  if (split.cut != CUT_NONE) {
     GemmParams& q = gp.g[0];
     q.tilesM = q.tilesN = Np / 128;
     q.ksplit = split.parts;
-    q.sk_partial = (float*)((char*)Dp + round_up((long)batch * Np * Np * 2, 256));
-    q.sk_counter = (int*)((char*)q.sk_partial + split.tiles * split.parts * SK_TILE_BYTES);
-    gp.tile_start[1] = (int)(split.tiles * split.parts);
-    e = launch_zero_i32(q.sk_counter, split.tiles, stream);
-    if (e == hipSuccess) e = launch_ns_gemm_grouped(128, mode, false, false, gp, stream, compute_units(), 0, true);
+    long blocks = split.tiles;
+    e = hipSuccess;
+    if (split.cut == CUT_BLOCKS) {
+      blocks *= split.parts;
+      q.sk_partial = (float*)((char*)Dp + round_up((long)batch * Np * Np * 2, 256));
+      q.sk_counter = (int*)((char*)q.sk_partial + blocks * SK_TILE_BYTES);
+      e = launch_zero_i32(q.sk_counter, split.tiles, stream);
+    }
+    gp.tile_start[1] = (int)blocks;   // (four tiles of 128 to one of 256 at most)
+    if (e == hipSuccess) e = launch_ns_gemm_grouped(128, mode, false, false, gp, stream, compute_units(), 0, split.cut);
   } else {
     e = launch_rounds(tile, mode, false, false, gp, stream, compute_units(), nullptr, 0);
   }

@@ -1,6 +1,7 @@
 // How the tiles of one product launch are cut for the chip: plain arithmetic (no HIP), so that it can be checked on the host for any
 // number of compute units.  `units` is what the current device reports; the measured lines are those of 256 units (one MI355X)
-// and are scaled with it.  A choice made here never changes a result: the sums of an element are the same in every configuration.
+// and are scaled with it.  What is chosen for a launch never changes a result: the sums of an element are the same in every
+// configuration.  The one rule that cuts sums (product_parts) is asked about one matrix at RULE_UNITS, whatever the stack and the device.
 #pragma once
 #include <stdint.h>
 
@@ -67,8 +68,9 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   return {full, tail, 0};
 }
 
-// Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 with at most
-// one block to a unit.  Few tiles walk a long reduction on few units; a part costs 64 KiB of traffic each way and the call a
+// Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 (`tiles` of one
+// matrix) with at most one block to a unit.  The cut fixes the order of the sums, so callers ask for RULE_UNITS units and one
+// matrix: a matrix has the same bits alone, in a stack and on any device.  Few tiles walk a long reduction on few units; a part costs 64 KiB of traffic each way and the call a
 // launch that clears the counters, so a part has at least SPLIT_PART_KT k-tiles and there are three of them or none (five where there
 // are only one or two tiles, which tiles of 64 walk faster: 100 x 4000 23.5 whole, 27.7 in three; 128 x 8192 25.6 / 23.2).
 // us, whole / as split here: 512 x 4096 27.0 / 21.9, 512 x 16384 89 / 31, 1024 x 4096 27.9 / 22.4, 1024 x 8192 48.7 / 26.8, 1536 x
@@ -81,6 +83,14 @@ inline int product_parts(int units, long tiles, int kt) {
   if (parts > SPLIT_MAX_PARTS) parts = SPLIT_MAX_PARTS;
   return parts < (tiles < 3 ? SPLIT_MIN_PARTS + 2 : SPLIT_MIN_PARTS) ? 1 : (int)parts;
 }
+
+// Who walks the parts of a stack's tiles (`tiles` of all its matrices): a block each while the tiles alone would leave two thirds of
+// the chip idle, one block all of them otherwise.  us, in sequence / by blocks: 60 tiles of 640 x 16384 (8 parts) 94 / 48, 72 of 1024 x
+// 8192 (6) 51 / 38, 84 of 700 x 5800 (4) 61 / 60; 90 of 640 x 4096 (3) 29 / 31, 108 of 1000 x 4000 (3) 50 / 58, 120 of 256 x 8192
+// (6) 54 / 61.  Large stacks pay for bits that do not depend on them: whole, in tiles of 256, 64 of 512 x 4096 take 97 us,
+// in sequence 124; 256 of them 326 / 379, 64 of 1024 x 4096 275 / 325, 16 of them 89 / 88; extents that tiles of 128 serve
+// anyway lose nothing (64 of 640 x 8192 267 / 268, 1000 of 128 x 8192 403 / 403).
+inline bool parts_by_blocks(long tiles) { return tiles <= RULE_UNITS / SPLIT_MIN_PARTS; }
 
 // X' = B X walks its problems and matrices backwards where the iterates of a call (bf16 bytes) are at most this: it then meets the
 // matrices that X X^T has read last first, and the next X X^T the ones that it has written last, while the memory-side cache

@@ -8,6 +8,9 @@ namespace archscale {
 // MODE_SYRKT: as MODE_SYRK, but P = Q is given K-major ([K][M] row-major, ldp = leading dimension; P == Q required)
 enum { MODE_SYRK = 0, MODE_SYRK2 = 1, MODE_BX = 2, MODE_SYRKT = 3 };
 
+// who walks the parts of a reduction that is cut (GemmParams::ksplit): nobody has any, a block each, one block all of them
+enum KCut { CUT_NONE = 0, CUT_BLOCKS, CUT_SEQUENCE };
+
 // C[m][n] = sum_k P[m][k] * Q[n][k]; all leading dimensions / strides in elements.
 struct GemmParams {
   // (what the start of a tile needs comes first and together)
@@ -47,7 +50,8 @@ struct GemmParams {
   // K-split (symmetric products of the 128x128 configuration only): `ksplit` > 1 blocks share every tile, block s of
   // them walks k-tiles [s KT / ksplit, (s + 1) KT / ksplit) and leaves its fp32 accumulators in sk_partial; the block
   // that finds itself last (sk_counter, one per tile, zero before the launch and zero again after it) adds the partial
-  // results in the order s = 0, 1, ... and runs the epilogue.  The sums do not depend on which block came last.
+  // results in the order s = 0, 1, ... and runs the epilogue.  The sums do not depend on which block came last.  With
+  // CUT_SEQUENCE one block walks the parts one after the other and adds in that order: the same bits, no partial results in memory.
   int ksplit;
   float* sk_partial;     // [tiles of this problem in the launch][ksplit][128 * 128] fp32, accumulator layout
   int* sk_counter;       // [tiles of this problem in the launch]
@@ -78,9 +82,9 @@ long ns_gemm_tiles(int mode, const GemmParams& p);
 // f16: 0 = the workspace matrices of the launch are bfloat16; 1 = IEEE half (see GemmParams::out_shift), not with split;
 // 2 = bfloat16 operands, IEEE-half result (MODE_BX, not the final launch)
 // units: compute units of the device
-// ksplit: some problem of the launch has GemmParams::ksplit > 1 (symmetric modes, tile 128, no hi+lo pair)
+// cut: some problem of the launch has GemmParams::ksplit > 1 (symmetric modes, tile 128, no hi+lo pair)
 hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp,
-                                  hipStream_t stream, int units, int f16 = 0, bool ksplit = false);
+                                  hipStream_t stream, int units, int f16 = 0, KCut cut = CUT_NONE);
 // bytes of GemmParams::sk_partial per tile of a K-split launch
 constexpr long SK_TILE_BYTES = 128L * 128 * 4;
 

@@ -178,9 +178,10 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 1
 // F16 = 1: the workspace matrices (operands, addend, non-final outputs) are IEEE half instead of bfloat16 (the caller's
 // tensors stay bfloat16); the host keeps them in range with power-of-two factors folded into alpha / beta / out_shift.
 // F16 = 2: bfloat16 operands and addend, IEEE-half output (the step from a bfloat16 iteration to a half one).
-// SK: problems of the launch may carry a K-split (GemmParams::ksplit; symmetric products, 128x128 configuration): the
-// blocks that share a tile leave their fp32 accumulators in the workspace and the last one to arrive adds them up in
-// the order of the parts and runs the epilogue.
+// CUT: problems of the launch may carry a K-split (GemmParams::ksplit; symmetric products, 128x128 configuration).
+// CUT_BLOCKS: the blocks that share a tile leave their fp32 accumulators in the workspace and the last one to arrive adds
+// them up in the order of the parts and runs the epilogue.  CUT_SEQUENCE: one block walks all parts of its tile and adds up in the
+// same order, in registers: the same bits for launches that fill the chip without the cut.
 //
 // One block is four waves (one per SIMD of a compute unit), wave (r, c) of the 2 x 2 arrangement computes rows
 // r BT/2 .., columns c BT/2 .. of the BT x BT tile.  What bounds the 256 configuration is the LDS port and, at the power
@@ -192,12 +193,13 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 1
 //
 // LDS: SP stages of the P tile and SQ = SP + 1 of the Q tile.  The 256 configuration has room for 2 + 3: the
 // operand that streams from memory (Q = X^T) gets two k-tiles of time to arrive, P, which the caches hold, gets one.
-template <int BT, int SP, int SQ, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+template <int BT, int SP, int SQ, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, int CUT>
 __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass does not know the buffer descriptor type)
-  static_assert(BT == 256 || BT == 128 || BT == 64 || (BT == 32 && MODE == MODE_SYRKT && !SPLIT && !SK), "block tiles");
+  static_assert(BT == 256 || BT == 128 || BT == 64 || (BT == 32 && MODE == MODE_SYRKT && !SPLIT && CUT == CUT_NONE), "block tiles");
+  constexpr bool SK = CUT == CUT_BLOCKS, SEQUENCE = CUT == CUT_SEQUENCE;
   static_assert(!(F16 && SPLIT), "the hi+lo pair is a bfloat16 device");
-  static_assert(!SK || (BT == 128 && !SPLIT && !FINAL && MODE != MODE_BX), "the K-split serves symmetric products in the 128 configuration");
+  static_assert(CUT == CUT_NONE || (BT == 128 && !SPLIT && !FINAL && MODE != MODE_BX), "the K-split serves symmetric products in the 128 configuration");
   static_assert(F16 != 2 || (MODE == MODE_BX && !FINAL), "only X' changes its storage type");
   constexpr bool IN16 = F16 == 1, OUT16 = F16 != 0;
   constexpr int NW = 4, NT = 256;
@@ -544,6 +546,7 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   // the barrier.  In flight at the barrier, younger than what it publishes:
   constexpr int PAIR = 2 * NC;
   constexpr int INFLIGHT = (SP - 2) * PAIR + NC;
+  f32x4 sum[SEQUENCE ? FR : 1][SEQUENCE ? FR : 1] = {};   // CUT_SEQUENCE: the parts that are done
   auto k_range = [&](auto active) __attribute__((always_inline)) {
     constexpr bool ACTIVE = decltype(active)::value;
     int sP = 0, sQ = QBASE;               // stages of k-tile kt
@@ -588,7 +591,8 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       static_for<NRD>([&](auto r_) __attribute__((always_inline)) { fread(I0{}, 0, QBASE, I0{}, r_); });
       land(I0{});
     }
-    for (int kt = 0; kt < KT_ALL; ++kt) {
+    int kt = 0;
+    auto walk = [&](int end) __attribute__((always_inline)) { for (; kt < end; ++kt) {
       const int nP = nextP(sP), nQ = nextQ(sQ);
       // the Q stage before this one in the ring is the one that k-tile kt + SP goes to
       const int pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
@@ -600,6 +604,27 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       kstep(active, I1{}, nP, nQ, I0{}, Yes{}, src, sP, 0);
       sP = nP;
       sQ = nQ;
+    } };
+    if constexpr (!SEQUENCE) {
+      walk(KT_ALL);
+    } else {
+      // part by part; a part's sum joins those before it, and the next part starts from zero
+      for (int part = 1; part <= g.ksplit; ++part) {
+        walk((int)((long)part * KT / g.ksplit));
+        if constexpr (ACTIVE) {
+          acc_settle();
+#pragma unroll
+          for (int i = 0; i < FR; ++i)
+#pragma unroll
+            for (int j = 0; j < FR; ++j) {
+              acc_touch<AGPR>(acc[i][j]);
+              sum[i][j] += acc[i][j];
+              acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+              acc_touch<AGPR>(acc[i][j]);
+            }
+          acc_settle();   // (and these writes are away from the next MFMA)
+        }
+      }
     }
   };
 
@@ -625,6 +650,12 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
   k_range(Yes{});
   wait_copies<0>();   // (copies without records included: the epilogue reuses the stages)
   acc_settle();
+  if constexpr (SEQUENCE) {
+#pragma unroll
+    for (int i = 0; i < FR; ++i)
+#pragma unroll
+      for (int j = 0; j < FR; ++j) acc[i][j] = sum[i][j];
+  }
 
   // ---- epilogue.  acc[i][j][e] of lane l is element
   //   r = wr0 + 16 i + 4 (l / 16) + e  (row in the tile),   c = wc0 + 16 j + l % 16  (column)
@@ -912,33 +943,42 @@ __global__ void __launch_bounds__(256, Config<BM == 256 ? CFG_256 : CFG_128>::BL
 ns_gemm_kernel(const GroupedGemmParams gp) {
   static_assert(BM == BN && WM == BM / 2 && WN == BN / 2 && (BM == 256 || BM == 128), "four waves of a quarter each");
   using C = Config<BM == 256 ? CFG_256 : CFG_128>;
-  ns_gemm_tile<BM, C::SP, C::SQ, MODE, SPLIT, FINAL, ADDEND, F16, SK>(gp);
+  ns_gemm_tile<BM, C::SP, C::SQ, MODE, SPLIT, FINAL, ADDEND, F16, SK ? CUT_BLOCKS : CUT_NONE>(gp);
 }
 
 // The two configurations for launches that do not (deeper pipelines).
 template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16>
 __global__ void __launch_bounds__(256, Config<CFG>::BLOCKS)
 ns_gemm_deep_kernel(const GroupedGemmParams gp) {
-  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, false>(gp);
+  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, SPLIT, FINAL, ADDEND, F16, CUT_NONE>(gp);
 }
 
 // Tiles of 32 (X X^T only).
 template <int MODE, int F16>
 __global__ void __launch_bounds__(256, Config<CFG_32>::BLOCKS)
 ns_gemm_fine_kernel(const GroupedGemmParams gp) {
-  ns_gemm_tile<Config<CFG_32>::BT, Config<CFG_32>::SP, Config<CFG_32>::SQ, MODE, false, false, true, F16, false>(gp);
+  ns_gemm_tile<Config<CFG_32>::BT, Config<CFG_32>::SP, Config<CFG_32>::SQ, MODE, false, false, true, F16, CUT_NONE>(gp);
 }
 
-template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, bool SK>
+// Symmetric products whose reduction is cut, one block for all parts of a tile.
+template <int CFG, int MODE>
+__global__ void __launch_bounds__(256, Config<CFG>::BLOCKS)
+ns_gemm_sequence_kernel(const GroupedGemmParams gp) {
+  ns_gemm_tile<Config<CFG>::BT, Config<CFG>::SP, Config<CFG>::SQ, MODE, false, false, true, 0, CUT_SEQUENCE>(gp);
+}
+
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND, int F16, int CUT>
 static constexpr auto kernel_of() {
   constexpr int BT = Config<CFG>::BT;
-  if constexpr (CFG == CFG_32) {
+  if constexpr (CUT == CUT_SEQUENCE) {
+    return &ns_gemm_sequence_kernel<CFG, MODE>;
+  } else if constexpr (CFG == CFG_32) {
     return &ns_gemm_fine_kernel<MODE, F16>;
   } else
   if constexpr (CFG == CFG_256 || CFG == CFG_128) {
-    return &ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, SK>;
+    return &ns_gemm_kernel<BT, BT, BT / 2, BT / 2, MODE, SPLIT, FINAL, ADDEND, F16, CUT == CUT_BLOCKS>;
   } else {
-    static_assert(!SK, "the K-split runs in the 128 configuration");
+    static_assert(CUT == CUT_NONE, "the K-split runs in the 128 configuration");
     return &ns_gemm_deep_kernel<CFG, MODE, SPLIT, FINAL, ADDEND, F16>;
   }
 }
@@ -951,11 +991,11 @@ long ns_gemm_tiles(int mode, const GemmParams& p) {
   return (long)p.batch * (sym ? (long)p.tilesM * (p.tilesM + 1) / 2 : (long)p.tilesM * p.tilesN);
 }
 
-template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, bool SK = false>
+template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, int CUT = CUT_NONE>
 static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   constexpr int NT = 256;
   constexpr int SMEM = (Config<CFG>::SP + Config<CFG>::SQ) * Config<CFG>::BT * ROW_BYTES;
-  constexpr auto kern = kernel_of<CFG, MODE, SPLIT, FINAL, ADDEND, F16, SK>();
+  constexpr auto kern = kernel_of<CFG, MODE, SPLIT, FINAL, ADDEND, F16, CUT>();
   // the dynamic-LDS limit is an attribute of the function on ONE device: set it once per device and instantiation
   // (the call is idempotent, so two threads that race on the first launch only repeat it)
   static std::atomic<bool> attr_set[64];
@@ -1018,27 +1058,41 @@ static hipError_t launch_cfg(int mode, bool split, bool final_, const GroupedGem
 template <int F16>
 static hipError_t launch_ksplit(int mode, const GroupedGemmParams& p, hipStream_t s) {
   switch (mode) {
-    case MODE_SYRK: return launch_one<CFG_128, MODE_SYRK, false, false, true, F16, true>(p, s);
-    case MODE_SYRKT: return launch_one<CFG_128, MODE_SYRKT, false, false, true, F16, true>(p, s);
-    case MODE_SYRK2: return launch_one<CFG_128, MODE_SYRK2, false, false, true, F16, true>(p, s);
+    case MODE_SYRK: return launch_one<CFG_128, MODE_SYRK, false, false, true, F16, CUT_BLOCKS>(p, s);
+    case MODE_SYRKT: return launch_one<CFG_128, MODE_SYRKT, false, false, true, F16, CUT_BLOCKS>(p, s);
+    case MODE_SYRK2: return launch_one<CFG_128, MODE_SYRK2, false, false, true, F16, CUT_BLOCKS>(p, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+// the same with all parts of a tile in one block (bfloat16 operands in the caller's orientation: the products of muon_syrk)
+template <int CFG>
+static hipError_t launch_sequence(int mode, const GroupedGemmParams& p, hipStream_t s) {
+  switch (mode) {
+    case MODE_SYRK: return launch_one<CFG, MODE_SYRK, false, false, true, 0, CUT_SEQUENCE>(p, s);
+    case MODE_SYRK2: return launch_one<CFG, MODE_SYRK2, false, false, true, 0, CUT_SEQUENCE>(p, s);
   }
   return hipErrorInvalidValue;
 }
 
 hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, const GroupedGemmParams& asked,
-                                  hipStream_t stream, int units, int f16, bool ksplit) {
+                                  hipStream_t stream, int units, int f16, KCut cut) {
+  const bool ksplit = cut == CUT_BLOCKS;
   GroupedGemmParams gp = asked;
   if (gp.n_groups < 1 || gp.n_groups > MAX_GROUPS) return hipErrorInvalidValue;
   const bool sym = (mode == MODE_SYRK || mode == MODE_SYRK2 || mode == MODE_SYRKT);
-  if (ksplit && (!sym || tile != 128 || split || final_ || f16 == 2)) return hipErrorInvalidValue;
+  if (cut != CUT_NONE && (!sym || tile != 128 || split || final_ || f16 == 2)) return hipErrorInvalidValue;
+  if (cut == CUT_SEQUENCE && (asked.quarter || f16)) return hipErrorInvalidValue;
   for (int i = 0; i < gp.n_groups; ++i) {
     GemmParams& g = gp.g[i];
     if (g.K % BK != 0 || g.K <= 0 || gp.tile_start[i + 1] < gp.tile_start[i]) return hipErrorInvalidValue;
     if (mode == MODE_SYRK2 && !g.E) return hipErrorInvalidValue;
     if (mode == MODE_BX && (g.E == nullptr) != (gp.g[0].E == nullptr)) return hipErrorInvalidValue;  // one kernel per launch
     long blocks = (long)gp.tile_start[i + 1] - gp.tile_start[i];
-    if (!ksplit) {
+    if (cut == CUT_NONE) {
       if (g.ksplit > 1) return hipErrorInvalidValue;
+    } else if (cut == CUT_SEQUENCE) {
+      if (g.ksplit < 1 || g.ksplit > g.K / BK) return hipErrorInvalidValue;
     } else {
       // every part walks at least one k-tile; the parts of a tile find their partial results and their counter
       if (g.ksplit < 1 || g.ksplit > g.K / BK || blocks % g.ksplit) return hipErrorInvalidValue;
@@ -1081,6 +1135,7 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
   int shortest = gp.g[0].K;
   for (int i = 1; i < gp.n_groups; ++i) shortest = gp.g[i].K < shortest ? gp.g[i].K : shortest;
   const bool deep = deep_pipeline(units, tile, gp.total, shortest);
+  if (cut == CUT_SEQUENCE) return deep ? launch_sequence<CFG_128_DEEP>(mode, gp, stream) : launch_sequence<CFG_128>(mode, gp, stream);
   auto by_storage = [&](auto cfg_) -> hipError_t {
     constexpr int CFG = decltype(cfg_)::value;
     if (f16 == 1) return launch_cfg<CFG, 1>(mode, split, final_, gp, stream);

@@ -196,6 +196,9 @@ int muon_calibration_stream(int mode, const void* a_dev, void* b_dev, void* c_de
  * D = alpha * A A^T + beta * C, A [batch] n x k (bf16, row-major, ld lda), C symmetric n x n or NULL, D n x n,
  * both triangles written.  Replaces ns_line_1 / ns_line_2 (newton_schulz_triton.py:142-178, 269-310) and
  * tsyrk_ex (emerging_optimizers/triton_kernels/syrk.py:188-261).
+ * The reduction of a matrix with few tiles and a long k is summed in several parts; how many depends on (n, k) alone, so a
+ * matrix has the same bits alone and in any batch.  The workspace holds their partial results where the batch is small; its size
+ * depends on the arguments alone, not on the device.
  */
 size_t muon_syrk_workspace_bytes(int batch, int n, int k);
 int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda,

@@ -189,6 +189,24 @@ def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
     assert ((first.float() - want).abs() <= want.abs() * 2.0 ** -8 + 2e-3 * want.pow(2).mean().sqrt()).all()
 
 
+@pytest.mark.parametrize("batch,n,k", [(4, 640, 16384), (2, 1000, 4000), (4, 1000, 4000), (8, 512, 4096), (17, 512, 4090), (16, 1024, 4096),
+                                       (90, 100, 6400)])
+@pytest.mark.parametrize("addend", [False, True])
+def test_parts_of_a_reduction_do_not_depend_on_the_stack(gpu_device, batch, n, k, addend):
+    """Products whose reduction is cut, alone (a block to a part) and in stacks (the same up to 85 tiles of 128, then one block to all
+    parts, with both pipelines): equal bits, matrix by matrix."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator(device=gpu_device).manual_seed(n + k)
+    a = (torch.randn(batch, n, k, generator=g, device=gpu_device) / k ** 0.5).to(torch.bfloat16)
+    c = None
+    if addend:
+        c = torch.randn(batch, n, n, generator=g, device=gpu_device) * 0.1
+        c = (c + c.mT).to(torch.bfloat16)
+    stack = ns._syrk(a, c, 1.2, -0.7 if addend else 0.0, None)
+    for i in (0, 1, batch - 1):
+        assert torch.equal(ns._syrk(a[i], c[i] if addend else None, 1.2, -0.7 if addend else 0.0, None), stack[i])
+
+
 @pytest.mark.parametrize("m,n", [(130, 1024), (256, 1090), (511, 1500), (512, 2048), (640, 1025), (2100, 300)])
 @pytest.mark.parametrize("prec", ["bf16", "f16"])
 def test_tiles_of_32_give_the_bits_of_larger_ones(gpu_device, m, n, prec):
