@@ -1136,8 +1136,9 @@ SnPlan make_sn_plan(int batch, int rows, int cols) {
   s.off_g2 = take((size_t)batch * s.pl.Mp * s.pl.Mp * 2);   // G^2 and G^4 of the grouped rounds (used from 6 / 16 rounds on)
   s.off_g4 = take((size_t)batch * s.pl.Mp * s.pl.Mp * 2);
   s.off_xscale = take((size_t)batch * sizeof(float));
-  // sums of squares: per 64x64 tile of a copy, or per strip of the short side
-  s.off_xpart = take((size_t)batch * std::max((s.pl.Mp / 64) * (s.pl.Np / 64), s.pl.Mp / SN_ROWS) * sizeof(float));
+  // sums of squares: per 64x64 tile of a copy, or per block that sums a matrix where it lies
+  const int blocks = sum_blocks((long)s.pl.m * s.pl.n / 8, s.pl.Mp / SN_ROWS);
+  s.off_xpart = take((size_t)batch * std::max((s.pl.Mp / 64) * (s.pl.Np / 64), blocks) * sizeof(float));
   s.off_z = take((size_t)2 * batch * s.pl.Mp * sizeof(float));
   s.off_part = take((size_t)2 * batch * (s.pl.Mp / SN_ROWS) * 2 * sizeof(float));
   s.off_long = take((size_t)batch * s.pl.n * sizeof(float));   // the long-side vectors before they are made unit vectors
@@ -1347,7 +1348,7 @@ int spectral_norm_impl(const muon_sn_problem* problems_host, int n_problems, int
       SnClass& c = sp.c[sp.n];
       c.X = P.src; c.strideX = P.stride; c.ldx = P.ld;
       c.G = P.G; c.G2 = P.G2; c.G4 = P.G4;
-      c.xscale = P.xscale; c.xpart = P.xpart; c.xparts = P.own ? pl.Mp / SN_ROWS : (pl.Mp / 64) * (pl.Np / 64);
+      c.xscale = P.xscale; c.xpart = P.xpart; c.xparts = P.own ? (P.tall ? sum_blocks((long)pl.m * pl.n / 8, pl.Mp / SN_ROWS) : pl.Mp / SN_ROWS) : (pl.Mp / 64) * (pl.Np / 64);
       c.z = P.z; c.part = P.part; c.sigma = P.q.sigma_out;
       c.batch = P.q.batch; c.d = pl.m; c.d_p = pl.Mp; c.L_p = P.L; c.nblk = pl.Mp / SN_ROWS;
       c.tall = P.tall; c.own = P.own; c.long_first = long_first;

@@ -114,4 +114,14 @@ inline bool deep_pipeline(int units, int tile, int blocks, int shortest_k) {
   return tile == 128 && blocks <= units && shortest_k >= 1024;
 }
 
+// Blocks that sum the squares of one matrix of the power iteration that is read in place and needs no row sums (a tall one), each
+// eight 16-byte runs per thread at a time: as many as the matrix has loads for, whatever its short side (`strips`, which the start
+// vector is written by), up to two rounds of the chip, which keep the memory busy.
+constexpr int SUM_RUNS = 2048, SUM_MAX_BLOCKS = 512;
+inline int sum_blocks(long runs, int strips) {
+  const long blocks = (runs + SUM_RUNS - 1) / SUM_RUNS;
+  const int most = strips > SUM_MAX_BLOCKS ? strips : SUM_MAX_BLOCKS;
+  return blocks < strips ? strips : (blocks > most ? most : (int)blocks);
+}
+
 }  // namespace archscale

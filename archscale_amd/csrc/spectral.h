@@ -24,13 +24,15 @@ struct SnClass {
   const __bf16* G2;
   const __bf16* G4;
   float* xscale;       // [batch], written by launch_spectral_xscale; the result is divided by it
-  float* xpart;        // [batch][xparts] sums of squares of X (from the layout kernel, or from launch_spectral_init)
+  // [batch][xparts] sums of squares of X (from the layout kernel, or from launch_spectral_init: one per strip of the short side where
+  // the row sums are needed as well, else sum_blocks of them)
+  float* xpart;
   int xparts;
   float* z;      // [2][batch][d_p]
   float* part;   // [2][batch][nblk][2]
   float* sigma;  // [batch], result
   int batch, d, d_p, L_p, ldx, nblk;
-  uint8_t tall, own, long_first;   // own: X is the caller's, launch_spectral_init sums its squares (xparts = nblk)
+  uint8_t tall, own, long_first;   // own: X is the caller's, launch_spectral_init sums its squares
 };
 
 struct SnParams {

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "launch_rules.h"
 #include "spectral.h"
 
 namespace archscale {
@@ -58,8 +59,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
-// block -> (class, matrix, 16-row strip)
-__device__ __forceinline__ void locate(const SnParams& sp, int& g, int& b, int& s) {
+// block -> (class, matrix, 16-row strip); per(class): blocks per matrix
+template <class F>
+__device__ __forceinline__ void locate(const SnParams& sp, int& g, int& b, int& s, F&& per) {
   // (all first blocks in one fetch instead of one after the other)
   const int blk = blockIdx.x;
   int first = 0;
@@ -70,9 +72,13 @@ __device__ __forceinline__ void locate(const SnParams& sp, int& g, int& b, int& 
     if (i < sp.n && blk >= at) { g = i; first = at; }
   }
   const int local = blk - first;
-  b = local / sp.c[g].nblk;
-  s = local - b * sp.c[g].nblk;
+  const int n = per(sp.c[g]);
+  b = local / n;
+  s = local - b * n;
 }
+// blocks per matrix of a launch over the strips, and of the first one
+__host__ __device__ __forceinline__ int strips_of(const SnClass& c) { return c.nblk; }
+__host__ __device__ __forceinline__ int init_blocks_of(const SnClass& c) { return c.own ? c.xparts : c.nblk; }
 
 // Dot products of four rows of a row-major bf16 matrix (leading dimension ld, a multiple of 8) with an fp32 vector, over n_cols
 // columns (a multiple of 8).  The first AHEAD runs of a lane can be fetched before anything else is known.
@@ -146,6 +152,36 @@ __device__ __forceinline__ float rows4_sums(const uint16_t* __restrict__ row0, l
   return sq;
 }
 
+// This lane's share of the sum of squares of `rows` x `cols` elements (cols a multiple of 8), by block `part` of `parts`.  The runs of
+// all rows are dealt out as one sequence: every lane has work whatever the rows are, and eight loads in flight.
+__device__ __forceinline__ float runs_sumsq(const uint16_t* __restrict__ X, int ld, int rows, int cols, int part, int parts) {
+  constexpr int U = SUM_RUNS / 256;
+  const int per_row = cols / 8, total = rows * per_row;
+  const uint32_t inv = reciprocal(per_row);
+  float sq = 0.f;
+  for (int q0 = part * SUM_RUNS + threadIdx.x; q0 < total; q0 += parts * SUM_RUNS) {
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int at;
+      const int row = divide(min(q0 + u * 256, total - 1), per_row, inv, at);
+      v[u] = *(const uint4*)(X + (size_t)row * ld + at * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = q0 + u * 256 < total;
+      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float lo = in ? bf2f_(w[k] & 0xffff) : 0.f, hi = in ? bf2f_(w[k] >> 16) : 0.f;
+        sq = fmaf(lo, lo, sq);
+        sq = fmaf(hi, hi, sq);
+      }
+    }
+  }
+  return sq;
+}
+
 // sums `n` (S, D) pairs in a fixed lane-strided order; result in all lanes
 __device__ __forceinline__ void sum_pairs(const float* __restrict__ part, int n, int lane, float& S, float& D) {
   float s = 0.f, d = 0.f;
@@ -158,54 +194,45 @@ __device__ __forceinline__ void sum_pairs(const float* __restrict__ part, int n,
 
 // x0 = X 1 (row sums of the short-side-first operand) or 1;  z[0] <- x0, z[1] <- 0, part[0] <- (|x0|^2 per strip, 0); where X is
 // the caller's, its sums of squares: one read of X, which the Gram product then finds in the caches.
-// 16 matrices of 1024 x 2816: 16 us, where a copy of them with its sums took 35 and this pass came on top.
+// 16 matrices of 1024 x 2816: 16 us, where a copy of them with its sums took 35 and this pass came on top.  Tall matrices (x0 = 1)
+// have as many blocks as they have data, not one per strip: us per spectral_norm call of 5 rounds, copied / one block per strip and one
+// load per lane in flight / as here: 6144 x 128 67 / 91 / 55, 16384 x 128 96 / 181 / 72, 16 of 6144 x 128 84 / 111 / 62, 4096 x 1024
+// 83 / 80 / 69, 2816 x 1024 76 / 67 / 63, 16 of them 155 / 124 / 125, 50304 x 512 474 / 482 / 363.
 __global__ void __launch_bounds__(256)
 sn_init_kernel(const SnParams sp) {
   __shared__ float red[8];
   int g, b, s;
-  locate(sp, g, b, s);
+  locate(sp, g, b, s, init_blocks_of);
   const SnClass c = sp.c[g];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r0 = s * SN_ROWS + wave * 4;
   const uint16_t* X = (const uint16_t*)c.X + (size_t)b * c.strideX;
   float v[4] = {1.f, 1.f, 1.f, 1.f}, sq = 0.f;
-  if (c.long_first) {
-    // (tall matrices only: nothing but the squares) rows of d elements, a strip of the short side taking every nblk-th four
-    for (int r = s * 4 + wave; r < c.L_p; r += c.nblk * 4)
-      for (int j = lane * 8; j < c.d; j += 512) {
-        const uint4 q = *(const uint4*)(X + (size_t)r * c.ldx + j);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float lo = bf2f_(w[k] & 0xffff), hi = bf2f_(w[k] >> 16);
-          sq = fmaf(lo, lo, sq);
-          sq = fmaf(hi, hi, sq);
-        }
-      }
-  } else if (!c.tall || c.own) {
-    float sums[4];
-    sq = rows4_sums(X + (size_t)r0 * c.ldx, c.ldx, c.L_p, lane, sums);
-    if (!c.tall) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = sums[i];
-    }
+  if (!c.tall) {
+    sq = rows4_sums(X + (size_t)r0 * c.ldx, c.ldx, c.L_p, lane, v);
+  } else if (c.own) {
+    sq = c.long_first ? runs_sumsq(X, c.ldx, c.L_p, c.d, s, c.xparts) : runs_sumsq(X, c.ldx, c.d, c.L_p, s, c.xparts);
   }
   if (c.own) sq = wave_sum(sq);
   float S = 0.f;
-  float* z0 = c.z + (size_t)b * c.d_p;
-  float* z1 = c.z + ((size_t)c.batch + b) * c.d_p;
+  if (s < c.nblk) {
+    float* z0 = c.z + (size_t)b * c.d_p;
+    float* z1 = c.z + ((size_t)c.batch + b) * c.d_p;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float val = (r0 + i < c.d) ? v[i] : 0.f;
-    if (lane == 0) { z0[r0 + i] = val; z1[r0 + i] = 0.f; }
-    S += val * val;
+    for (int i = 0; i < 4; ++i) {
+      const float val = (r0 + i < c.d) ? v[i] : 0.f;
+      if (lane == 0) { z0[r0 + i] = val; z1[r0 + i] = 0.f; }
+      S += val * val;
+    }
   }
   if (lane == 0) { red[wave] = S; red[4 + wave] = sq; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    float* p = c.part + ((size_t)b * c.nblk + s) * 2;
-    p[0] = (red[0] + red[1]) + (red[2] + red[3]);
-    p[1] = 0.f;
+    if (s < c.nblk) {
+      float* p = c.part + ((size_t)b * c.nblk + s) * 2;
+      p[0] = (red[0] + red[1]) + (red[2] + red[3]);
+      p[1] = 0.f;
+    }
     if (c.own) c.xpart[(size_t)b * c.xparts + s] = (red[4] + red[5]) + (red[6] + red[7]);
   }
 }
@@ -219,7 +246,7 @@ __global__ void __launch_bounds__(256)
 sn_step_kernel(const SnParams sp, int src_wide, int which_wide, int src_tall, int which_tall) {
   __shared__ float red[8];
   int g, b, s;
-  locate(sp, g, b, s);
+  locate(sp, g, b, s, strips_of);
   const SnClass& c = sp.c[g];
   const int src = c.tall ? src_tall : src_wide, which = c.tall ? which_tall : which_wide;
   if (which < 0) return;
@@ -453,7 +480,9 @@ bool classes_ok(const SnParams& sp, int* matrices) {
     const SnClass& c = sp.c[g];
     if (c.batch <= 0 || c.d <= 0 || c.d_p % 128 || c.L_p % 8 || c.d > c.d_p || c.nblk * SN_ROWS != c.d_p || !c.xscale || c.ldx % 8) return false;
     // the caller's own matrices fill the extents that the kernels walk
-    if (c.own && (c.d != c.d_p || c.xparts != c.nblk || (c.long_first && !c.tall))) return false;
+    if (c.own && (c.d != c.d_p || (c.long_first && !c.tall))) return false;
+    // (blocks of the first launch: one sum each, a wide matrix's over the rows of a strip)
+    if (c.own && (c.xparts < c.nblk || (!c.tall && c.xparts != c.nblk))) return false;
     *matrices += c.batch;
   }
   return true;
@@ -463,7 +492,13 @@ bool classes_ok(const SnParams& sp, int* matrices) {
 hipError_t launch_spectral_init(const SnParams& sp, hipStream_t stream) {
   int matrices;
   if (!classes_ok(sp, &matrices)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(sn_init_kernel, dim3(sp.blk_start[sp.n]), dim3(256), 0, stream, sp);
+  SnParams ip = sp;
+  for (int g = 0; g < ip.n; ++g) {
+    const long end = ip.blk_start[g] + (long)ip.c[g].batch * init_blocks_of(ip.c[g]);
+    if (end > 0x7ffffff0L) return hipErrorInvalidValue;
+    ip.blk_start[g + 1] = (int)end;
+  }
+  hipLaunchKernelGGL(sn_init_kernel, dim3(ip.blk_start[ip.n]), dim3(256), 0, stream, ip);
   return hipGetLastError();
 }
 

@@ -119,3 +119,18 @@ int main() { int u, t, k; while (scanf("%d %d %d", &u, &t, &k) == 3) printf("%d\
     text = "".join(f"256 {t} {k}\n" for t, k in want)
     out = subprocess.run([str(tmp_path / "parts")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in out] == list(want.values())
+
+
+def test_blocks_that_sum_squares_follow_the_data(tmp_path):
+    """(16-byte runs, strips of the short side) -> blocks: eight runs per thread at a time up to 512 blocks, never fewer than strips."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "sums.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { long r; int s; while (scanf("%ld %d", &r, &s) == 2) printf("%d\n", archscale::sum_blocks(r, s)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "sums.cpp"), "-o", str(tmp_path / "sums")], check=True)
+    want = {(6144 * 16, 8): 48, (4096 * 128, 64): 256, (2816 * 128, 64): 176, (1, 8): 8, (2048 * 512, 8): 512, (2048 * 512 + 1, 8): 512,
+            (1 << 28, 600): 600, (2048 * 9, 8): 9, (2048 * 9 + 1, 8): 10}
+    out = subprocess.run([str(tmp_path / "sums")], input="".join(f"{r} {s}\n" for r, s in want), capture_output=True, text=True, check=True)
+    assert [int(v) for v in out.stdout.split()] == list(want.values())

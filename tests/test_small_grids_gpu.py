@@ -131,6 +131,36 @@ def test_spectral_norms_of_matrices_where_they_lie(gpu_device, shape):
         assert torch.allclose(u.norm(dim=-1), torch.ones(b, device=gpu_device), atol=4e-3)
 
 
+@pytest.mark.parametrize("shape", [(1, 6144, 128), (3, 192, 128), (2, 1088, 1024), (1, 8256, 128), (2, 3008, 384), (1, 9024, 1152)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_squares_of_tall_matrices_where_they_lie(gpu_device, shape, transposed):
+    """Fewer and more elements than the blocks of the first launch take at once, rows that a wave fills several times and only in part;
+    stored long side first, or short side first and meant transposed: the norms of fp32 copies, bit for bit."""
+    import ctypes
+    from archscale_amd import _lib
+    b, rows, cols = shape if not transposed else (shape[0], shape[2], shape[1])
+    g = torch.Generator(device=gpu_device).manual_seed(rows)
+    wide = (torch.randn(2 * b, rows, cols + 24, generator=g, device=gpu_device) * 0.02).to(torch.bfloat16)
+    L = _lib.lib()
+
+    def norms(w, steps):
+        n, out = w.shape[0], torch.empty(w.shape[0], device=gpu_device)
+        ptrs = (ctypes.c_void_p * n)(*[w[i].data_ptr() for i in range(n)])
+        q = (_lib.SnProblem * 1)()
+        q[0].w_ptrs, q[0].sigma_out = ctypes.cast(ptrs, ctypes.POINTER(ctypes.c_void_p)), out.data_ptr()
+        q[0].dtype, q[0].ld, q[0].batch, q[0].rows, q[0].cols = _lib.dtype_code(w.dtype), w.stride(-2), n, rows, cols
+        q[0].flags = _lib.SN_TRANSPOSED if transposed else 0
+        ws = _lib.workspace(gpu_device, L.muon_spectral_norm_workspace_bytes(q, 1), tag="sn")
+        _lib.check(L.muon_spectral_norm(q, 1, steps, ws.data_ptr(), ws.numel(), _lib.current_stream_ptr(gpu_device)), "muon_spectral_norm")
+        return out
+
+    for w in (wide[:b, :, :cols].contiguous(), wide[::2, :, 8:8 + cols]):
+        for steps in (1, 7):
+            assert torch.equal(norms(w, steps), norms(w.float(), steps))
+    w.fill_(0)
+    assert not norms(w, 2).any()
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 1, 257), (2, 255, 256), (2, 130, 4096), (1, 4097, 64), (1, 33, 8200)])
 def test_unit_vectors_and_norm_from_one_launch(gpu_device, shape):
     """Around the ends of a thread's run of 16 elements: sigma has the bits of the call for norms alone, the unit vectors are those of
