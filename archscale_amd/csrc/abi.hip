@@ -351,6 +351,33 @@ int check_problem(const muon_ns_problem& q, bool no_input = false) {
   if (q.in_dtype != MUON_DTYPE_BF16 && q.in_dtype != MUON_DTYPE_F32) return MUON_E_ARG;
   return 0;
 }
+
+// Whether no result of a call shares memory with an input, except a matrix's result with its own input (same place, type and
+// strides).  The chain of product launches reads every input before it writes the first result; blocks that take a
+// matrix each do not wait for one another, so they need this.
+bool results_clear_of_other_inputs(const std::vector<NsProblem>& pr) {
+  struct Span { uintptr_t lo, hi; size_t i; };
+  auto span = [](const muon_ns_problem& q, const void* at, int64_t stride, int ld, int size, size_t i) {
+    const int64_t last = (q.batch - 1) * stride;
+    return Span{(uintptr_t)at + (uintptr_t)(std::min<int64_t>(last, 0) * size),
+                (uintptr_t)at + (uintptr_t)((std::max<int64_t>(last, 0) + (int64_t)(q.rows - 1) * ld + q.cols) * size), i};
+  };
+  std::vector<Span> in;
+  for (size_t i = 0; i < pr.size(); ++i)
+    in.push_back(span(pr[i].q, pr[i].q.in, pr[i].q.in_batch_stride, pr[i].q.in_ld, pr[i].q.in_dtype == MUON_DTYPE_BF16 ? 2 : 4, i));
+  std::sort(in.begin(), in.end(), [](const Span& a, const Span& b) { return a.lo < b.lo; });
+  std::vector<uintptr_t> reach;   // the highest end of the inputs up to this one
+  for (const Span& s : in) reach.push_back(reach.empty() ? s.hi : std::max(reach.back(), s.hi));
+  for (size_t j = 0; j < pr.size(); ++j) {
+    const muon_ns_problem& q = pr[j].q;
+    const Span out = span(q, q.out, q.out_batch_stride, q.out_ld, 2, j);
+    const bool same = q.in == q.out && q.in_dtype == MUON_DTYPE_BF16 && q.in_ld == q.out_ld && (q.batch == 1 || q.in_batch_stride == q.out_batch_stride);
+    size_t k = std::lower_bound(in.begin(), in.end(), out.hi, [](const Span& s, uintptr_t end) { return s.lo < end; }) - in.begin();
+    for (; k > 0 && reach[k - 1] > out.lo; --k)
+      if (in[k - 1].hi > out.lo && !(same && in[k - 1].i == j)) return false;
+  }
+  return true;
+}
 }  // namespace
 
 size_t muon_ns_grouped_workspace_bytes(const muon_ns_problem* problems_host, int n_problems, int prec_mode) {
@@ -477,6 +504,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   bool small = !split_any && iters <= SMALL_NS_MAX_ITERS && !env_switches().tile;
   for (const NsProblem& P : pr)
     small = small && small_ns_extents(P.pl.m, P.pl.n, nullptr, nullptr) && P.defer == pr[0].defer;
+  small = small && (fused || results_clear_of_other_inputs(pr));   // (fused: the inputs are in the workspace)
 
   hipError_t e;
   // K-split counters start at zero (every launch leaves them at zero again); the workspace is the caller's and holds anything

@@ -87,7 +87,8 @@ const char* muon_status_string(int status);
  * in  : [batch] matrices of rows x cols, leading dimension in_ld, batch stride in_batch_stride (elements),
  *       dtype in_dtype.  Not modified.
  * out : bf16, same logical shape, leading dimension out_ld, batch stride out_batch_stride.  May alias `in`
- *       only if in_dtype is bf16 and the strides are equal.
+ *       only if in_dtype is bf16 and the strides are equal.  (Every input is read before the first result is written, in a
+ *       grouped call too: a result may lie over the input of another matrix.)
  * abc : HOST array of 3*iters floats, one (a, b, c) row per iteration (the reference has three different
  *       tables; none is compiled in).
  * Each matrix is normalised by its own Frobenius norm, tall matrices (rows > cols) are iterated transposed

@@ -56,6 +56,28 @@ def test_strided_rows_and_the_input_as_result(rows, cols, ld):
     assert torch.equal(y.view(torch.int16), H.newton_schulz(x.contiguous()).view(torch.int16))
 
 
+def test_results_in_the_place_of_other_inputs():
+    """Every input is read before any result is written, also where a result lies over the input of another matrix."""
+    # the same stack one matrix further on: more matrices than a round of blocks
+    stack = _input(600, 64, 200, torch.bfloat16).contiguous()
+    want = H.newton_schulz(stack[:-1].clone())
+    H.newton_schulz(stack[:-1], out=stack[1:])
+    assert torch.equal(stack[1:].view(torch.int16), want.view(torch.int16))
+    # results of one kernel (short side up to 64) over inputs of the other, and each over the other's
+    a, b, c = (_input(1, r, k, torch.bfloat16)[0].contiguous() for r, k in ((64, 128), (128, 300), (64, 128)))
+    wants = [H.newton_schulz(x.clone()) for x in (a, b, c)]
+    over = [b.view(-1)[:64 * 128].view(64, 128), torch.empty_like(b), a]
+    outs = H.newton_schulz_grouped([a, b, c], outs=over)
+    for got, want in zip(outs, wants):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    # a result within its own fp32 input
+    x = _input(3, 50, 70, torch.float32).contiguous()
+    want = H.newton_schulz(x.clone())
+    out = x.view(torch.bfloat16).view(-1)[:x.numel()].view(x.shape)
+    H.newton_schulz(x, out=out)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
 def test_many_classes_zeros_and_tiny_norms_in_one_call():
     shapes = [(33 + 3 * i, 40 + 7 * i) for i in range(28)] + [(128, 384), (5, 1000)]
     xs = [_input(1, r, c, torch.bfloat16)[0] for r, c in shapes]
