@@ -32,6 +32,7 @@ NS_STATIC_SCRATCH_BYTES = 64 << 20
 STREAM_COPY, STREAM_READ, STREAM_MIX = 0, 1, 2
 E_STATIC_LIMIT = -4
 PROF_KEY_MOMENTUM_LAYOUT = 90000
+PROF_KEY_SMALL_NS = 91000
 ABI_VERSION = 3
 
 #: numpy layouts of muon_pre_item / muon_post_item (natural C alignment)
@@ -304,8 +305,9 @@ def profile_begin() -> None:
 def profile_collect(capacity: int = 4096):
     """Per-launch records of the Newton-Schulz GEMMs since profile_begin():
     list of dicts {kind="gemm", ms, tile, mode, split, final, folded, flops_algorithmic, flops_issued} (``folded`` marks
-    the X' = (B + aI) X launches that read no addend) and {kind="momentum_layout", ms, bytes} for the fused momentum
-    launches (``bytes`` = algorithmic HBM bytes of the launch)."""
+    the X' = (B + aI) X launches that read no addend), {kind="momentum_layout", ms, bytes} for the fused momentum
+    launches (``bytes`` = algorithmic HBM bytes of the launch) and {kind="small", ms, side, flops_algorithmic, flops_issued}
+    for launches that run the whole iteration of small matrices (short side up to ``side``), a block each."""
     ms = (ctypes.c_float * capacity)()
     key = (ctypes.c_int32 * capacity)()
     fa = (ctypes.c_double * capacity)()
@@ -318,6 +320,9 @@ def profile_collect(capacity: int = 4096):
         k = key[i]
         if k == PROF_KEY_MOMENTUM_LAYOUT:   # the fused momentum launch: the work fields carry bytes
             out.append(dict(kind="momentum_layout", ms=ms[i], bytes=fa[i]))
+            continue
+        if k > PROF_KEY_SMALL_NS:
+            out.append(dict(kind="small", ms=ms[i], side=k - PROF_KEY_SMALL_NS, flops_algorithmic=fa[i], flops_issued=fi[i]))
             continue
         out.append(dict(kind="gemm", ms=ms[i], tile=k // 100, mode=(k // 10) % 10, split=bool((k % 10) & 2),
                         final=bool((k % 10) & 1), folded=bool((k % 10) & 4), flops_algorithmic=fa[i], flops_issued=fi[i]))

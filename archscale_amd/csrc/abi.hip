@@ -165,11 +165,13 @@ int compute_units() {
 // pool that muon_profile_begin creates, so a timed call creates nothing; launches beyond the pool run untimed.
 // Profiling is a single-threaded debugging mode: every timed launch takes one process-wide lock.
 struct ProfRec {
-  int key;  // tile*100 + mode*10 + 4*(BX without addend) + split*2 + final; PROF_KEY_MOMENTUM_LAYOUT for the fused momentum
+  // tile*100 + mode*10 + 4*(BX without addend) + split*2 + final; PROF_KEY_MOMENTUM_LAYOUT for the fused momentum; PROF_KEY_SMALL_NS + 64
+  // or 128 for the whole iteration of small matrices
+  int key;
   double work_algorithmic, work_issued;   // FLOPs of a GEMM launch; bytes of a momentum launch
 };
 constexpr int PROF_POOL = 1024;
-constexpr int PROF_KEY_MOMENTUM_LAYOUT = 90000;
+constexpr int PROF_KEY_MOMENTUM_LAYOUT = 90000, PROF_KEY_SMALL_NS = 91000;
 std::mutex g_prof_mutex;
 std::vector<hipEvent_t> g_prof_start, g_prof_stop;   // the pool
 std::vector<ProfRec> g_prof;                         // g_prof[i] used events i
@@ -868,6 +870,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   if (small) {
     for (const int side : {64, 128}) {   // one kernel each
       SmallNsParams sp = {};
+      double fa = 0.0, fi = 0.0;
       auto flush = [&]() -> hipError_t {
         if (sp.n == 0) return hipSuccess;
         sp.iters = iters; sp.sa = SH_A; sp.sb = SH_B;
@@ -877,13 +880,14 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
           const ItCfg k = it_cfg(it);
           sp.it[it] = SmallNsIteration{k.a, k.b, k.c, (uint8_t)k.half_ops, (uint8_t)k.half_out, (uint8_t)k.fold};
         }
-        const hipError_t err = launch_small_ns(sp, stream);
+        const hipError_t err = timed_launch(PROF_KEY_SMALL_NS + side, fa, fi, stream, [&] { return launch_small_ns(sp, stream); });
         sp = SmallNsParams{};
+        fa = fi = 0.0;
         return err;
       };
       for (const NsProblem& P : pr) {
-        int mp = 0;
-        small_ns_extents(P.pl.m, P.pl.n, &mp, nullptr);
+        int mp = 0, np = 0;
+        small_ns_extents(P.pl.m, P.pl.n, &mp, &np);
         if (mp != side) continue;
         if ((sp.n == SMALL_NS_MAX_PROBLEMS || (long)sp.block_start[sp.n] + P.q.batch > 0x7fffffffL) && (e = flush()) != hipSuccess) return (int)e;
         SmallNsProblem& q = sp.p[sp.n];
@@ -893,6 +897,11 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
         q.rows = P.q.rows; q.cols = P.q.cols; q.sx = P.sx; q.gram_tail = P.gram_tail;
         sp.block_start[sp.n + 1] = sp.block_start[sp.n] + P.q.batch;
         ++sp.n;
+        // products over the long side (an X X^T and an X' each) and symmetric m x m ones (the tail: two iterations in one and five)
+        const double longs = iters - (P.gram_tail ? 1 : 0), squares = iters + (P.gram_tail ? 3 : 0);
+        const double bm = P.q.batch, dm = P.pl.m, dn = P.pl.n, upper = 0.5 * (mp / 16) * (mp / 16 + 1);
+        fa += bm * (longs * 3.0 * dm * dm * dn + squares * dm * dm * dm);
+        fi += bm * (longs * (512.0 * upper * np + 2.0 * mp * mp * np) + squares * 512.0 * upper * mp);
       }
       if ((e = flush()) != hipSuccess) return (int)e;
     }

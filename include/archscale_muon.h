@@ -165,12 +165,14 @@ void muon_ns_ksplit_info(int rows, int cols, int* info);
 
 /* Per-launch timing of the Newton-Schulz GEMM kernels, for roofline accounting (no counterpart in the
  * reference).  Between muon_profile_begin() and muon_profile_collect() every GEMM launch of muon_ns_batched is
- * bracketed by a pair of HIP events on its stream (a call of matrices so small that one launch does everything records
- * nothing).  muon_profile_collect waits for them, writes up to `capacity`
+ * bracketed by a pair of HIP events on its stream (a call of matrices so small that a block does everything for one of
+ * them: the launches of that kernel).  muon_profile_collect waits for them, writes up to `capacity`
  * records to the HOST arrays (any may be NULL) and returns the number of launches recorded (< 0 on error):
  *   ms                elapsed milliseconds of the launch
  *   key               tile*100 + mode*10 + 4*noaddend + split*2 + final  (mode 0 = X X^T, 1 = cAA+bA, 2 = aX + BX,
- *                     3 = X X^T from the transposed iterate; noaddend: an X' = (B + aI) X launch)
+ *                     3 = X X^T from the transposed iterate; noaddend: an X' = (B + aI) X launch); 91000 + side (64 or
+ *                     128) for a launch that runs the whole iteration of matrices with at most that short side, staging
+ *                     included; 90000 for a fused momentum launch, whose work fields carry bytes
  *   flops_algorithmic minimum FLOPs of the product (symmetric products counted once)
  *   flops_issued      FLOPs of the matrix-core instructions actually issued (whole tiles; three quarters of a diagonal
  *                     tile of a symmetric product)

@@ -89,3 +89,21 @@ def test_many_classes_zeros_and_tiny_norms_in_one_call():
     for x, a, b in zip(xs, small, chain):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), x.shape
     assert not small[3].any()
+
+
+def test_calls_of_small_matrices_leave_records():
+    """One record per kernel of a call, with the work of the chain's products."""
+    from archscale_amd import _lib
+    a, b = _input(3, 64, 200, torch.bfloat16), _input(2, 100, 120, torch.bfloat16)
+    _lib.profile_begin()
+    H.newton_schulz_grouped([a, b])
+    recs = _lib.profile_collect()
+    assert [(r["kind"], r["side"]) for r in recs] == [("small", 64), ("small", 128)] and all(r["ms"] > 0 for r in recs)
+    filler = torch.randn(160, 160, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).cuda()
+    for x, r in zip((a, b), recs):
+        work = []
+        for xs in ([x, filler], [filler]):
+            _lib.profile_begin()
+            H.newton_schulz_grouped(xs)
+            work.append(sum(q["flops_algorithmic"] for q in _lib.profile_collect()))
+        assert r["flops_algorithmic"] == pytest.approx(work[0] - work[1], rel=1e-9) and r["flops_issued"] >= r["flops_algorithmic"]
