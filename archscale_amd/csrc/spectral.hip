@@ -455,7 +455,8 @@ sn_units_kernel(const SnVectors a, const SnVectors o, const SnClass c, int src_f
   s = wave_sum(s);
   if (lane == 0) red[wave] = s;
   __syncthreads();
-  const float norm = fmaxf(sqrtf((red[0] + red[1]) + (red[2] + red[3])), 1e-12f);
+  const float length = sqrtf((red[0] + red[1]) + (red[2] + red[3]));
+  const float norm = length < 1e-12f ? 1e-12f : length;   // (a length that is not a number makes the whole vector so; fmaxf would hide it)
   for (int i0 = threadIdx.x; i0 < v.len; i0 += RUN * 256) {
     if (v.len > RUN * 256) fetch(i0);   // (else the run of the first loop)
 #pragma unroll

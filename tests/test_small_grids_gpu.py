@@ -189,6 +189,34 @@ def test_unit_vectors_and_norm_from_one_launch(gpu_device, shape):
         assert bool(((got.squeeze(-1).double() - want).abs() <= want.abs() * (2.0 ** -8 + x.shape[-1] * 2.0 ** -24)).all())
 
 
+@pytest.mark.parametrize("shape", [(192, 128), (100, 130), (128, 128), (33, 8200)])
+@pytest.mark.parametrize("value", [float("inf"), 3e38, float("nan")])
+def test_unit_vectors_of_lengths_that_are_not_numbers(gpu_device, shape, value):
+    """A vector with a NaN or an infinity after the last round is what dividing it by its norm makes of it: NaN in every place the
+    norm is one, not only where the vector was."""
+    import ctypes
+    from archscale_amd import _lib
+    from archscale_amd.emerging.spectral_ball_utils import power_iteration
+    W = (torch.randn(1, *shape, generator=torch.Generator().manual_seed(8)) * 0.02)
+    W.view(-1)[W.numel() // 3] = value
+    W = W.to(torch.bfloat16).to(gpu_device)
+    r, c = shape
+    L = _lib.lib()
+    for steps in (1, 2, 7):
+        _, u, v = power_iteration(W, steps)
+        raw = [torch.empty(1, n, device=gpu_device) for n in (r, c)]
+        s = torch.empty(1, device=gpu_device)
+        pp = ctypes.cast((ctypes.c_void_p * 1)(W.data_ptr()), ctypes.POINTER(ctypes.c_void_p))
+        prob = (_lib.SnProblem * 1)()
+        prob[0].w_ptrs, prob[0].sigma_out, prob[0].ld, prob[0].batch, prob[0].rows, prob[0].cols = pp, s.data_ptr(), c, 1, r, c
+        ws = _lib.workspace(W.device, L.muon_spectral_norm_workspace_bytes(prob, 1), tag="sn")
+        _lib.check(L.muon_power_iteration(pp, 0, c, 1, r, c, steps, s.data_ptr(), raw[0].data_ptr(), raw[1].data_ptr(), ws.data_ptr(),
+                                          ws.numel(), _lib.current_stream_ptr(W.device)), "muon_power_iteration")
+        for got, x in zip((u, v), raw):
+            want = x / x.norm(dim=-1, keepdim=True).clamp_min(1e-12)
+            assert torch.equal(got.squeeze(-1).isnan(), want.isnan()), steps
+
+
 @pytest.mark.parametrize("batch,n,k", [(1, 128, 3840), (1, 256, 4096), (2, 300, 4000), (1, 1000, 8200), (1, 640, 16384), (3, 512, 4096)])
 @pytest.mark.parametrize("addend", [False, True])
 def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
