@@ -1027,10 +1027,10 @@ namespace {
 // K-split of a symmetric product: parts per tile of 128, tiles of all matrices, whether a block takes one part of a tile or all, and
 // what it adds to the workspace (partial results, counters)
 struct SyrkSplit { int parts; long tiles; KCut cut; size_t bytes; };
-SyrkSplit syrk_split(int batch, int Np, int Kp) {
+SyrkSplit syrk_split(int batch, int tile, int Np, int Kp) {
   SyrkSplit s = {1, (long)batch * sym_tiles(Np / 128), CUT_NONE, 0};
   if (env_switches().ksplit == 0 || env_switches().tile != 0) return s;
-  s.parts = product_parts(RULE_UNITS, sym_tiles(Np / 128), Kp / 64);
+  s.parts = matrix_parts(tile, sym_tiles(Np / 128), Kp / 64);
   if (s.parts == 1) return s;
   s.cut = parts_by_blocks(s.tiles) ? CUT_BLOCKS : CUT_SEQUENCE;
   if (s.cut == CUT_BLOCKS) s.bytes = (size_t)s.tiles * s.parts * SK_TILE_BYTES + (size_t)round_up(s.tiles * (long)sizeof(int), 256);
@@ -1043,7 +1043,7 @@ size_t muon_syrk_workspace_bytes(int batch, int n, int k) {
   const int tile = pick_tile(n, k);
   const size_t Np = (size_t)round_up(n, tile), Kp = (size_t)round_up(k, 64);
   return (size_t)round_up((long)(batch * Np * Kp * 2), 256) + 2 * (size_t)round_up((long)(batch * Np * Np * 2), 256) +
-         syrk_split(batch, (int)Np, (int)Kp).bytes;
+         syrk_split(batch, tile, (int)Np, (int)Kp).bytes;
 }
 
 int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_dev, int64_t c_batch_stride, int ldc,
@@ -1107,7 +1107,7 @@ int muon_syrk(const void* a_dev, int64_t a_batch_stride, int lda, const void* c_
   gp.n_groups = 1;
   gp.g[0] = g;
   gp.tile_start[1] = (int)tiles;
-  const SyrkSplit split = syrk_split(batch, Np, Kp);
+  const SyrkSplit split = syrk_split(batch, tile, Np, Kp);
   if (split.cut != CUT_NONE) {
     GemmParams& q = gp.g[0];
     q.tilesM = q.tilesN = Np / 128;

@@ -84,6 +84,15 @@ inline int product_parts(int units, long tiles, int kt) {
   return parts < (tiles < 3 ? SPLIT_MIN_PARTS + 2 : SPLIT_MIN_PARTS) ? 1 : (int)parts;
 }
 
+// The same for a matrix whose extents call for tiles of `tile`.  Where that is 128, three tiles and more run whole as tiles of 64, which keep
+// up with the parts until the reduction is SPLIT_MIN_KT_128 k-tiles long.  us, whole / cut: 384 x 4480 16.9 / 20.6, 640 x 3840 16.3 /
+// 20.7, 896 x 4480 16.9 / 23.1, 1152 x 4480 17.5 / 24.2, 896 x 6400 22.0 / 23.8, 640 x 7680 25.2 / 25.7, 640 x 8192 26.6 / 25.2, 896 x
+// 8192 26.6 / 25.2, 384 x 10240 31.9 / 25.9.
+constexpr int SPLIT_MIN_KT_128 = 128;
+inline int matrix_parts(int tile, long tiles, int kt) {
+  return tile == 128 && tiles >= 3 && kt < SPLIT_MIN_KT_128 ? 1 : product_parts(RULE_UNITS, tiles, kt);
+}
+
 // Who walks the parts of a stack's tiles (`tiles` of all its matrices): a block each while the tiles alone would leave two thirds of
 // the chip idle, one block all of them otherwise.  us, in sequence / by blocks: 60 tiles of 640 x 16384 (8 parts) 94 / 48, 72 of 1024 x
 // 8192 (6) 51 / 38, 84 of 700 x 5800 (4) 61 / 60; 90 of 640 x 4096 (3) 29 / 31, 108 of 1000 x 4000 (3) 50 / 58, 120 of 256 x 8192

@@ -134,3 +134,18 @@ int main() { long r; int s; while (scanf("%ld %d", &r, &s) == 2) printf("%d\n", 
             (1 << 28, 600): 600, (2048 * 9, 8): 9, (2048 * 9 + 1, 8): 10}
     out = subprocess.run([str(tmp_path / "sums")], input="".join(f"{r} {s}\n" for r, s in want), capture_output=True, text=True, check=True)
     assert [int(v) for v in out.stdout.split()] == list(want.values())
+
+
+def test_products_that_tiles_of_64_serve_are_cut_later(tmp_path):
+    """(tile that the extents call for, tiles of 128, k-tiles) -> parts."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "cut.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int c, t, k; while (scanf("%d %d %d", &c, &t, &k) == 3) printf("%d\n", archscale::matrix_parts(c, t, k)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "cut.cpp"), "-o", str(tmp_path / "cut")], check=True)
+    want = {(256, 10, 60): 3, (256, 10, 127): 6, (128, 6, 70): 1, (128, 15, 60): 1, (128, 28, 127): 1, (128, 28, 128): 6, (128, 45, 70): 1,
+            (128, 1, 100): 5, (128, 1, 99): 1, (256, 36, 64): 3, (256, 3, 59): 1}
+    out = subprocess.run([str(tmp_path / "cut")], input="".join(f"{c} {t} {k}\n" for c, t, k in want), capture_output=True, text=True, check=True)
+    assert [int(v) for v in out.stdout.split()] == list(want.values())
