@@ -82,7 +82,9 @@ __host__ __device__ __forceinline__ int init_blocks_of(const SnClass& c) { retur
 
 // Dot products of four rows of a row-major bf16 matrix (leading dimension ld, a multiple of 8) with an fp32 vector, over n_cols
 // columns (a multiple of 8).  The first AHEAD runs of a lane can be fetched before anything else is known.
-constexpr int AHEAD = 2;   // 1024 columns
+// (More of them make the waves of a launch ask for the same part of their rows at the same time: two against one, us per step, 15
+// matrices of 1920 26.1 / 22.9, 16 of 2048 31.1 / 26.7, 8 of 2048 17.7 / 15.5; none ahead 24.2, 28.3, 15.8.  16 of 1024 5.5 / 5.3.)
+constexpr int AHEAD = 1;   // 512 columns
 struct Rows4 {
   uint4 r[AHEAD][4];
   float4 x[AHEAD][2];
@@ -240,7 +242,7 @@ sn_init_kernel(const SnParams sp) {
 // z[dst] <- M z[src] / max(|z[src]|, 1e-12);  part[dst] <- per strip (|z[dst]|^2,  z[src]^T z[dst] / |z[src]|)
 // M = G, G2 or G4 (which = 0, 1, 2) and the source buffer are given per kind of class (wide, tall), whose sequences
 // differ; which < 0: the classes of that kind sit this launch out.
-// Latency bound (16 matrices of 1024: 32 MB that the caches hold): every load of the first 1024 columns is on its way before the
+// Latency bound (16 matrices of 1024: 32 MB that the caches hold): every load of the first 512 columns is on its way before the
 // norm of z[src] is added up, and no sum goes through LDS: 5.3 us a launch, 6.2 before.
 __global__ void __launch_bounds__(256)
 sn_step_kernel(const SnParams sp, int src_wide, int which_wide, int src_tall, int which_tall) {
