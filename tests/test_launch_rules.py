@@ -149,3 +149,19 @@ int main() { int c, t, k; while (scanf("%d %d %d", &c, &t, &k) == 3) printf("%d\
             (128, 1, 100): 5, (128, 1, 99): 1, (256, 36, 64): 3, (256, 3, 59): 1}
     out = subprocess.run([str(tmp_path / "cut")], input="".join(f"{c} {t} {k}\n" for c, t, k in want), capture_output=True, text=True, check=True)
     assert [int(v) for v in out.stdout.split()] == list(want.values())
+
+
+def test_lines_of_the_tiles_of_32(tmp_path):
+    """(units, tile, tiles, longest reduction) -> tiles of 32 or not: sixteen tiles of 128 on 256 units and as many per unit elsewhere."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "fine.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int u, t, n, k; while (scanf("%d %d %d %d", &u, &t, &n, &k) == 4) printf("%d\n", (int)archscale::fine_tiles(u, t, n, k)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "fine.cpp"), "-o", str(tmp_path / "fine")], check=True)
+    want = {(256, 128, 1, 1024): 1, (256, 128, 16, 1024): 1, (256, 128, 17, 1024): 0, (256, 128, 16, 960): 0, (256, 256, 1, 4096): 0,
+            (128, 128, 8, 2048): 1, (128, 128, 9, 2048): 0, (38, 128, 2, 2048): 1, (38, 128, 3, 2048): 0, (304, 128, 19, 2048): 1, (304, 128, 20, 2048): 0}
+    text = "".join("%d %d %d %d\n" % w for w in want)
+    out = subprocess.run([str(tmp_path / "fine")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())

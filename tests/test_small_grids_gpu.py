@@ -223,15 +223,13 @@ def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
     """Products whose reduction is cut into parts: bf16 rounding of the fp32 result, the same bits every time, symmetric."""
     import archscale_amd.optim.newton_schulz_hip as ns
     from archscale_amd import _lib
-    if addend and batch > 1:
-        pytest.skip("the entry point with an addend takes one matrix")
     g = torch.Generator().manual_seed(n + k)
     a = (torch.randn(batch, n, k, generator=g) / k ** 0.5).to(torch.bfloat16).to(gpu_device)
     a = a[0] if batch == 1 else a
     c = None
     if addend:
-        c = torch.randn(n, n, generator=g) * 0.1
-        c = (c + c.t()).to(torch.bfloat16).to(gpu_device)
+        c = torch.randn(*a.shape[:-2], n, n, generator=g) * 0.1
+        c = (c + c.mT).to(torch.bfloat16).to(gpu_device)
     want = a.float() @ a.float().mT.contiguous()
     if addend:
         want = 1.2 * want - 0.7 * c.float()
@@ -239,7 +237,7 @@ def test_few_tiles_with_a_long_reduction(gpu_device, batch, n, k, addend):
     for fill in (0, 0x7f, 0xff):   # whatever the workspace holds
         for ws in list(_lib._workspaces.values()):
             ws.fill_(fill)
-        got = ns.ns_line_1(a) if c is None else ns.tsyrk_ex(a, c, alpha=1.2, beta=-0.7)
+        got = ns.ns_line_1(a) if c is None else (ns.tsyrk_ex(a, c, alpha=1.2, beta=-0.7) if batch == 1 else ns._syrk(a, c, 1.2, -0.7, None))
         assert torch.equal(got, got.mT)
         first = got if first is None else first
         assert torch.equal(got, first)
@@ -275,3 +273,34 @@ def test_tiles_of_32_give_the_bits_of_larger_ones(gpu_device, m, n, prec):
     batch = ns.newton_schulz(x, prec=prec)
     for i in (0, 15):
         assert torch.equal(ns.newton_schulz(x[i], prec=prec), batch[i])
+
+
+@pytest.mark.parametrize("m,n,fine", [(130, 1024, True), (512, 2048, True), (640, 1025, True), (512, 890, False), (512, 1000, True), (700, 1500, False), (2100, 300, True)])
+def test_which_products_take_tiles_of_32(gpu_device, m, n, fine):
+    """X X^T of up to 16 tiles of 128 over at least 1024 k-values (padded to tiles: 890 has 896 of them, 1000 has 1024), alone; none of sixteen such matrices together, and no other product."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    from archscale_amd import _lib
+    x = (torch.randn(16, m, n, generator=torch.Generator().manual_seed(m + n)) * 1e-3).to(torch.bfloat16).to(gpu_device)
+    for t, want in ((x[0], fine), (x, False)):
+        _lib.profile_begin()
+        ns.newton_schulz(t, gram_tail=False)
+        recs = _lib.profile_collect()
+        grams = [r for r in recs if r["mode"] == 3]
+        assert len(grams) == 5 and all((r["tile"] == 32) == want for r in grams)
+        assert all(r["tile"] != 32 for r in recs if r["mode"] != 3)
+
+
+@pytest.mark.parametrize("shape", [(2, 192, 128), (2, 128, 192), (1, 6144, 128)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 3e38])
+def test_values_out_of_range_in_matrices_where_they_lie(gpu_device, shape, value):
+    """One such value: the norms and vectors of its matrix are those of the fp32 copy, NaN in the same places, and the other matrix of the
+    stack does not see it."""
+    from archscale_amd.emerging.spectral_ball_utils import power_iteration, spectral_norm
+    W = torch.randn(*shape, generator=torch.Generator().manual_seed(4)) * 0.02
+    clean = spectral_norm(W.to(torch.bfloat16).to(gpu_device), 5)
+    W[0].view(-1)[W[0].numel() // 3] = value
+    W = W.to(torch.bfloat16).to(gpu_device)
+    for steps in (1, 5):
+        for got, want in zip((spectral_norm(W, steps), *power_iteration(W, steps)), (spectral_norm(W.float(), steps), *power_iteration(W.float(), steps))):
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(spectral_norm(W, 5)[1:], clean[1:])

@@ -107,3 +107,30 @@ def test_calls_of_small_matrices_leave_records():
             H.newton_schulz_grouped(xs)
             work.append(sum(q["flops_algorithmic"] for q in _lib.profile_collect()))
         assert r["flops_algorithmic"] == pytest.approx(work[0] - work[1], rel=1e-9) and r["flops_issued"] >= r["flops_algorithmic"]
+
+
+def test_more_classes_than_one_launch_takes():
+    """30 classes with a short side up to 64 and 27 above it: two launches of either kernel."""
+    from archscale_amd import _lib
+    shapes = [(2 + 2 * i, 64 + 5 * i) for i in range(30)] + [(66 + 2 * i, 129 + 9 * i) for i in range(27)]
+    xs = [_input(1 + i % 3, r, c, torch.bfloat16 if i % 2 else torch.float32) for i, (r, c) in enumerate(shapes)]
+    _lib.profile_begin()
+    small = H.newton_schulz_grouped(xs)
+    assert [r["side"] for r in _lib.profile_collect()] == [64, 64, 128, 128]
+    filler = torch.randn(160, 160, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).cuda()
+    for x, a, b in zip(xs, small, H.newton_schulz_grouped(xs + [filler])):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), x.shape
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -3e38, 1e-38])
+def test_values_out_of_range(dtype, value):
+    """One such value in the first matrix of a stack: what the chain makes of it, and nothing in the other matrices."""
+    for rows, cols in ((64, 64), (40, 300), (128, 384), (97, 30)):
+        for kind in ("quintic", "polar, half, fp32 norm"):
+            x = _input(3, rows, cols, dtype).contiguous()
+            clean = H.newton_schulz(x, **KINDS[kind])
+            x[0].view(-1)[rows * cols // 3] = value
+            got, want = H.newton_schulz(x, **KINDS[kind]), _chain(x, **KINDS[kind])
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0)), (rows, cols, kind)
+            assert torch.equal(got[1:], clean[1:])
