@@ -500,7 +500,7 @@ int ns_grouped_impl(const muon_ns_problem* problems_host, const muon_mns_problem
   // A call of nothing but small matrices: the whole chain in one launch, a block per matrix, with the same bits as the launches
   // below (ns_small.hip).  Where a call holds larger matrices too, the small ones stay in its chain: their tiles cost the
   // shared launches next to nothing, a launch of their own would add its time.  (A tile configuration forced through the
-  // environment forces the chain as well.)  One 128 x 384 matrix, staging included: 83 us as 18 launches, 46 as one; where the line lies
+  // environment forces the chain as well.)  One 128 x 384 matrix, staging included: 83 us as 18 launches (two of staging, 16 products), 46 as one; where the line lies
   // is what the LDS of a compute unit holds, and every matrix that fits is faster so (64 x 1024 88 -> 45, 64 x 128 85 -> 19;
   // 1000 of 128 x 384 522 -> 219).
   bool small = !split_any && iters <= SMALL_NS_MAX_ITERS && !env_switches().tile;

@@ -1,6 +1,6 @@
 // The whole Newton-Schulz iteration of a small matrix in ONE block for gfx950: iterate, A and B stay in the LDS of one compute unit.
 //
-// As launches over tiles (ns_gemm.hip) a 128 x 384 matrix is a chain of 16 launches of 3 us and 1.3 us between them, for a
+// As launches over tiles (ns_gemm.hip) a 128 x 384 matrix is a chain of 16 launches (and two of staging) of 3 us and 1.3 us between them, for a
 // microsecond of matrix-core work each: what bounds it is the chain, not the work.  Here the chain is a sequence of barriers:
 // 128 x 384 in 44 us (staging 7, A = X X^T 2.2, a product of two square matrices 1.4 to 1.8, X' 2.8; LDS reads are 1.3, 0.4 and
 // 1.4 of those), 64 x 1024 in 42, 64 x 128 in 18, where a step is 0.8 us whatever it does.

@@ -145,9 +145,10 @@ def newton_schulz_grouped(
     gram_tail: Optional[bool] = None,
 ) -> Sequence[Tensor]:
     """Orthogonalise several batches of DIFFERENT shapes in one call: every product of the iteration is a
-    single kernel launch over the tiles of all batches (15 GEMM launches in total for five iterations).
+    single kernel launch over the tiles of all batches that share a tile configuration; a call of small matrices only
+    runs the whole iteration in one block per matrix.
     ``inputs[i]`` is ``[..., rows_i, cols_i]`` (bf16 or fp32); ``outs[i]`` (bf16, contiguous, may be the input)
-    receives the result.  All tensors must live on one device."""
+    receives the result; all inputs are read before the first result is written.  All tensors must live on one device."""
     if not inputs:
         return []
     device = inputs[0].device

@@ -127,9 +127,12 @@ int muon_ns_batched_static(const void* in_dev, int in_dtype, int64_t in_batch_st
                            void* stream);
 
 /* The same for several independent batches of different shapes at once (all shape classes of an optimizer
- * step): each product of the iteration is ONE kernel launch over the tiles of every problem, so there are
- * 15 GEMM launches per call whatever the number of shapes, and the tail of one shape's grid is filled by the
- * next.  Replaces the per-parameter task loop of lit_gpt/optim/muon.py:211-333 around the calls above.
+ * step): each product of the iteration is ONE kernel launch over the tiles of every problem that shares a tile
+ * configuration, so the number of launches does not follow the number of shapes (15 for five plain iterations in one
+ * configuration, 18 with the Gram-side tail; up to 16 problems to a launch; leftover tiles that run in a smaller
+ * configuration add one), and the tail of one shape's grid is filled by the next.  A call of nothing but matrices that fit
+ * one compute unit (short side up to 128 with a long side up to 384, up to 64 with up to 1152) runs the whole iteration in one
+ * block per matrix instead: one launch for each of the two sides and for every 24 problems, with the same bits.  Replaces the per-parameter task loop of lit_gpt/optim/muon.py:211-333 around the calls above.
  * problems_host is a HOST array; the workspace is muon_ns_grouped_workspace_bytes(...) bytes. */
 typedef struct muon_ns_problem {
   const void* in; /* device, [batch] rows x cols, dtype in_dtype */
@@ -357,7 +360,7 @@ int muon_spectral_norm(const muon_sn_problem* problems_host, int n_problems, int
  * as in muon_sn_problem (w_ptrs_host: HOST array of `batch` device pointers; dtype, ld, rows, cols as there), sigma as
  * muon_spectral_norm computes it, plus the vectors of the same sequence, UNNORMALISED, in fp32:
  *   u_out_dev [batch][rows]  proportional to W v_steps,   v_out_dev [batch][cols]  proportional to v_steps = (W^T W)^steps 1
- * (the short-side one is the last Gram-side iterate, the long-side one a single pass over the bf16 copy of W).
+ * (the short-side one is the last Gram-side iterate, the long-side one a single pass over W in bf16).
  * Workspace: muon_spectral_norm_workspace_bytes of the same problem. */
 int muon_power_iteration(const void* const* w_ptrs_host, int dtype, int ld, int batch, int rows, int cols, int steps,
                          float* sigma_out_dev, float* u_out_dev, float* v_out_dev, void* workspace_dev,
