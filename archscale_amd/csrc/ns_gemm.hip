@@ -592,19 +592,21 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       land(I0{});
     }
     int kt = 0;
-    auto walk = [&](int end) __attribute__((always_inline)) { for (; kt < end; ++kt) {
-      const int nP = nextP(sP), nQ = nextQ(sQ);
-      // the Q stage before this one in the ring is the one that k-tile kt + SP goes to
-      const int pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
-      const Source src = source(kt + SP);
-      kstep(active, I0{}, sP, sQ, I1{}, No{}, src, 0, pQ);
-      wait_copies<INFLIGHT>();
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      kstep(active, I1{}, nP, nQ, I0{}, Yes{}, src, sP, 0);
-      sP = nP;
-      sQ = nQ;
-    } };
+    auto walk = [&](int end) __attribute__((always_inline)) {   // k-tiles kt .. end - 1
+      for (; kt < end; ++kt) {
+        const int nP = nextP(sP), nQ = nextQ(sQ);
+        // the Q stage before this one in the ring is the one that k-tile kt + SP goes to
+        const int pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
+        const Source src = source(kt + SP);
+        kstep(active, I0{}, sP, sQ, I1{}, No{}, src, 0, pQ);
+        wait_copies<INFLIGHT>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(active, I1{}, nP, nQ, I0{}, Yes{}, src, sP, 0);
+        sP = nP;
+        sQ = nQ;
+      }
+    };
     if constexpr (!SEQUENCE) {
       walk(KT_ALL);
     } else {
