@@ -132,7 +132,8 @@ int muon_ns_batched_static(const void* in_dev, int in_dtype, int64_t in_batch_st
  * configuration, 18 with the Gram-side tail; up to 16 problems to a launch; leftover tiles that run in a smaller
  * configuration add one), and the tail of one shape's grid is filled by the next.  A call of nothing but matrices that fit
  * one compute unit (short side up to 128 with a long side up to 384, up to 64 with up to 1152) runs the whole iteration in one
- * block per matrix instead: one launch for each of the two sides and for every 24 problems, with the same bits.  Replaces the per-parameter task loop of lit_gpt/optim/muon.py:211-333 around the calls above.
+ * block per matrix instead: one launch for each of the two sides and for every 24 problems, with the same bits.
+ * Replaces the per-parameter task loop of lit_gpt/optim/muon.py:211-333 around the calls above.
  * problems_host is a HOST array; the workspace is muon_ns_grouped_workspace_bytes(...) bytes. */
 typedef struct muon_ns_problem {
   const void* in; /* device, [batch] rows x cols, dtype in_dtype */
