@@ -101,6 +101,15 @@ inline int matrix_parts(int tile, long tiles, int kt) {
 // anyway lose nothing (64 of 640 x 8192 267 / 268, 1000 of 128 x 8192 403 / 403).
 inline bool parts_by_blocks(long tiles) { return tiles <= RULE_UNITS / SPLIT_MIN_PARTS; }
 
+// X' = B X in tiles of 256 as a stream (ns_gemm_stream_kernel: one block per unit, its tiles one after the other) where most units have two
+// tiles or more, for reductions of up to STREAM_MAX_K: what it saves is a constant per tile.  tile by tile / as a stream, us: the
+// 64 + 64 expert matrices (K = 512 and 256) 1311 / 1250 a step, the EMA-Muon set of width 1024 1187 / 1163, the depth-16 set (K = 2048 and
+// 512, at the power limit) 21980 / 21660; 4096 x 14336 (K = 4096) 3063 / 3106 a call.  The grid is a multiple of the eight XCDs.
+constexpr int STREAM_MAX_K = 2048;
+inline bool stream_of_tiles(int units, int total, int longest) {
+  return units % 8 == 0 && total >= units + units / 2 && longest <= STREAM_MAX_K;
+}
+
 // X' = B X walks its problems and matrices backwards where the iterates of a call (bf16 bytes) are at most this: it then meets the
 // matrices that X X^T has read last first, and the next X X^T the ones that it has written last, while the memory-side cache
 // (256 MB for X, X' and the square matrices) still holds them.  Iterates of 90 MB: MuonBall step 1519 -> 1494 us, EMA Muon 1216 ->

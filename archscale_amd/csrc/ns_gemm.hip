@@ -175,6 +175,28 @@ __device__ __forceinline__ void lds_tr_read(uint32_t addr, unsigned long long& r
 }
 __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
+// Tile t of a grid of dM x dN tiles that are all computed -> (ti, tj)
+__device__ __forceinline__ void place_in_grid(int t, int dM, int dN, uint32_t inv_line, int& ti, int& tj) {
+  if (dM > 8) {
+    // A wide tile grid in blocks of 4 x 4 tiles, the blocks of one block row (4 row panels of P) one after the other:
+    // the 32 tiles that an XCD works on at a time are two neighbouring blocks, 4 row panels of P and 8 of Q, 12 panels
+    // per k-step.  Whole columns of dM tiles at a time would stream dM + 32 / dM panels (33 for dM = 32, 24 for 22).
+    // The last block row and the last block of a row are as narrow as the grid leaves them (1 to 4 tiles).
+    const int nbi = (dM + 3) >> 2, nbj = (dN + 3) >> 2;
+    int r, bi = divide(t, 4 * dN, inv_line, r);
+    if (bi >= nbi) { r += (bi - (nbi - 1)) * 4 * dN; bi = nbi - 1; }
+    const int h = dM - 4 * bi < 4 ? dM - 4 * bi : 4;
+    int bj = divide_1_to_4(r, h) >> 2;
+    if (bj >= nbj) bj = nbj - 1;
+    const int q = r - bj * 4 * h;
+    const int qc = divide_1_to_4(q, h);
+    ti = 4 * bi + (q - qc * h);
+    tj = 4 * bj + qc;
+  } else {
+    tj = divide(t, dM, inv_line, ti);   // up to 8 row panels: whole columns, 8 x 4 tiles per XCD for dM = 8
+  }
+}
+
 // F16 = 1: the workspace matrices (operands, addend, non-final outputs) are IEEE half instead of bfloat16 (the caller's
 // tensors stay bfloat16); the host keeps them in range with power-of-two factors folded into alpha / beta / out_shift.
 // F16 = 2: bfloat16 operands and addend, IEEE-half output (the step from a bfloat16 iteration to a half one).
@@ -312,23 +334,8 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     int rowlen = dM;
     while (t >= rowlen) { t -= rowlen; ++ti; --rowlen; }
     tj = ti + t;
-  } else if (dM > 8) {
-    // A wide tile grid in blocks of 4 x 4 tiles, the blocks of one block row (4 row panels of P) one after the other:
-    // the 32 tiles that an XCD works on at a time are two neighbouring blocks, 4 row panels of P and 8 of Q, 12 panels
-    // per k-step.  Whole columns of dM tiles at a time would stream dM + 32 / dM panels (33 for dM = 32, 24 for 22).
-    // The last block row and the last block of a row are as narrow as the grid leaves them (1 to 4 tiles).
-    const int nbi = (dM + 3) >> 2, nbj = (dN + 3) >> 2;
-    int r, bi = divide(t, 4 * dN, p.inv_line, r);
-    if (bi >= nbi) { r += (bi - (nbi - 1)) * 4 * dN; bi = nbi - 1; }
-    const int h = dM - 4 * bi < 4 ? dM - 4 * bi : 4;
-    int bj = divide_1_to_4(r, h) >> 2;
-    if (bj >= nbj) bj = nbj - 1;
-    const int q = r - bj * 4 * h;
-    const int qc = divide_1_to_4(q, h);
-    ti = 4 * bi + (q - qc * h);
-    tj = 4 * bj + qc;
   } else {
-    tj = divide(t, dM, p.inv_line, ti);   // up to 8 row panels: whole columns, 8 x 4 tiles per XCD for dM = 8
+    place_in_grid(t, dM, dN, p.inv_line, ti, tj);
   }
   if (quarter) {
     ti = (ti << quarter) + (quadrant >> quarter);
@@ -924,6 +931,273 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
 #endif
 }
 
+// X' = B X in tiles of 256, a block's tiles one after the other: the k-tiles of all of them are ONE stream, the copies run on from the last
+// k-tiles of a tile to the first ones of the next, which arrive during the epilogue, and the epilogue takes no LDS (the stages hold
+// the next tile by then).  What bounds a lone tile of ns_gemm_tile at short reductions is its boundary - set-up, first copies, epilogue
+// and hand-over are 20 of 40 thousand clocks at K = 512, with the matrix cores idle; here 5 are left, the epilogue's.  us per launch,
+// tile by tile / as a stream: 64 x (512 x 2048) + 64 x (256 x 2048) 116 / 102 (with the addend 137 / 127, final 123 / 105; 4.4 TB/s of
+// operands and results are what bounds it then), the EMA-Muon set of width 1024 (K = 1024, 688 tiles) 91 / 86.
+// The arithmetic of an element is that of ns_gemm_tile (same sums, same epilogue roundings): the same bits.
+//   epilogue  A lane has four consecutive rows of one column in every fragment.  Two fragments below one another make eight of them with
+//             one exchange between neighbouring groups of 16 lanes (v_permlane16_swap): 16-byte stores, 64 bytes of each of 16 rows of
+//             X'^T per instruction and 256 by four.  The addend comes the same way, all of it before the first store (loads return
+//             in order behind stores): half of it during the last k-tile, half at the start of the epilogue, when the
+//             fragments of the second k-step are dead.
+//   final     A result wanted in rows (X', not X'^T) is the same computation with the operands' parts exchanged.
+//   waits     The stores of a tile are younger than the copies of the next tile's first two k-tiles and older than the
+//             rest: vector-memory operations complete in order, so the first wait of a tile leaves them outstanding.
+__device__ __forceinline__ void* uniform_ptr(const void* q) {
+  const uint64_t v = (uint64_t)q;
+  return (void*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
+}
+
+template <bool FINAL, bool ADDEND, int F16>
+__global__ void __launch_bounds__(256, 1) ns_gemm_stream_kernel(const GroupedGemmParams gp) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(!(F16 == 2 && FINAL), "the final launch writes the caller's bfloat16");
+  constexpr bool IN16 = F16 == 1, OUT16 = F16 != 0 && !FINAL;
+  constexpr int BT = 256, WT = 128, FR = 8, NC = 8, SP = 2, SQ = 3, OPBYTES = BT * ROW_BYTES, QBASE = SP * OPBYTES;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int wr0 = (wave >> 1) * WT, wc0 = (wave & 1) * WT;
+
+  // this block's tiles: every gridDim-th, from the run of its XCD on
+  const int total = gp.total, backwards = gp.backwards, step = (int)gridDim.x;
+  int index = (int)(blockIdx.x & 7) * (step >> 3) + (int)(blockIdx.x >> 3);
+  if (index >= total) return;
+
+  struct Args {
+    const __bf16 *P, *Q, *E;
+    __bf16* Ct;
+    const float* scale;
+    long strideP, strideQ, strideE, strideCt;
+    int ld, K, tilesM, tilesN, per_mat, lde, ldct, out_shift;
+    uint32_t inv_per_mat, inv_line;
+    float alpha;
+  };
+  int grp = -1;
+  bool rows = false;   // of this problem X' is wanted, not X'^T
+  Args a = {};
+  struct End { char* to; const char* e; int ld, lde; float alpha, factor; };
+  struct Place { const char *P, *Q; int KT; End end; };
+  auto locate = [&](int i) __attribute__((always_inline)) {
+    const int logical = backwards ? total - 1 - i : i;
+    int now = 0;
+#pragma unroll
+    for (int k = 1; k < MAX_GROUPS; ++k) if (logical >= gp.tile_start[k]) now = k;   // (past every tile for k >= n_groups)
+    if (now != grp) {
+      const GemmParams& g = gp.g[now];
+      rows = FINAL && g.C;
+      a = Args{g.P, g.Q, g.E, rows ? g.C : g.Ct, g.scale, g.strideP, g.strideQ, g.strideE, rows ? g.strideC : g.strideCt, g.ldp, g.K, g.tilesM,
+               g.tilesN, g.per_mat, g.lde, rows ? g.ldc : g.ldct, g.out_shift, g.inv_per_mat, g.inv_line, g.alpha};
+      grp = now;
+    }
+    int t, ti, tj;
+    const int b = divide(logical - gp.tile_start[now], a.per_mat, a.inv_per_mat, t);
+    place_in_grid(t, a.tilesM, a.tilesN, a.inv_line, ti, tj);
+    const int R0 = ti * BT, C0 = tj * BT;
+    Place p;
+    const char* const ofB = (const char*)(a.P + (size_t)b * a.strideP + (size_t)R0 * a.ld);
+    const char* const ofX = (const char*)(a.Q + (size_t)b * a.strideQ + (size_t)C0 * a.ld);
+    p.P = rows ? ofX : ofB;
+    p.Q = rows ? ofB : ofX;
+    p.KT = a.K / BK;
+    p.end.to = (char*)(a.Ct + (size_t)b * a.strideCt + (rows ? (size_t)R0 * a.ldct + C0 : (size_t)C0 * a.ldct + R0));
+    p.end.e = ADDEND ? (const char*)(a.E + (size_t)b * a.strideE + (size_t)C0 * a.lde + R0) : nullptr;
+    p.end.ld = a.ldct;
+    p.end.lde = a.lde;
+    p.end.alpha = a.alpha;
+    // (constant memory as far as this launch goes: a scalar load, where a vector one would wait for every copy in flight)
+    p.end.factor = (ADDEND && a.scale ? ((const __attribute__((address_space(4))) float*)(uintptr_t)a.scale)[b] : 1.f) * __builtin_ldexpf(1.f, a.out_shift);
+    return p;
+  };
+
+  Place next = locate(index);
+  // ---- copies (see ns_gemm_tile): the state of what is copied next
+  int off_ld = a.ld;
+  uint32_t off[NC];
+  auto lane_offsets = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int r = (wave * NC + j) * 8 + (lane >> 3);
+      off[j] = (uint32_t)r * (uint32_t)off_ld * 2u + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+    }
+  };
+  lane_offsets();
+  void *cP = uniform_ptr(next.P), *cQ = uniform_ptr(next.Q);
+  int ck = 0, cKT = next.KT, records = -1;
+  struct Source { __amdgpu_buffer_rsrc_t P, Q; uint32_t at; };
+  auto source = [&]() __attribute__((always_inline)) {
+    return Source{__builtin_amdgcn_make_buffer_rsrc(cP, 0, records, 0x00027000), __builtin_amdgcn_make_buffer_rsrc(cQ, 0, records, 0x00027000),
+                  (uint32_t)ck * (uint32_t)ROW_BYTES};
+  };
+  auto copyP = [&](const Source& s, int stage, int j) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.P, (lptr_t)(smem + stage + (wave * NC + j) * 1024), 16, (int)off[j], (int)s.at, 0, 0);
+  };
+  auto copyQ = [&](const Source& s, int stage, int j) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(s.Q, (lptr_t)(smem + stage + (wave * NC + j) * 1024), 16, (int)off[j], (int)s.at, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < SP; ++s) {
+    const Source src = source();
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copyQ(src, QBASE + s * OPBYTES, j);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) copyP(src, s * OPBYTES, j);
+    ++ck;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  f32x4 acc[FR][FR];
+#pragma unroll
+  for (int i = 0; i < FR; ++i)
+#pragma unroll
+    for (int j = 0; j < FR; ++j) { acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; acc_touch<true>(acc[i][j]); }
+
+  u32x4 af[2][FR], bq[2][FR];
+  int rdP[2], rdQ[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    rdP[kk] = lds_chunk_off(wr0 + l16, 4 * kk + lg);
+    rdQ[kk] = lds_chunk_off(wc0 + l16, 4 * kk + lg);
+  }
+  constexpr int NRD = 2 * FR, NMF = FR * FR, RSPAN = NMF * 3 / 4;
+  auto fread = [&](auto buf_, int sP, int sQ, auto kk_, auto r_) __attribute__((always_inline)) {
+    constexpr int buf = decltype(buf_)::value, kk = decltype(kk_)::value, r = decltype(r_)::value;
+    if constexpr (r < FR) bq[buf][r] = *(const u32x4*)(smem + sQ + rdQ[kk] + r * 16 * ROW_BYTES);
+    else af[buf][r - FR] = *(const u32x4*)(smem + sP + rdP[kk] + (r - FR) * 16 * ROW_BYTES);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  // one k-step, as in ns_gemm_tile; the first one copies Q, the second one P
+  auto kstep = [&](auto cbuf_, int rsP, int rsQ, const Source& src, int dst) __attribute__((always_inline)) {
+    constexpr int cbuf = decltype(cbuf_)::value;
+    static_for<NMF>([&](auto q_) __attribute__((always_inline)) {
+      constexpr int q = decltype(q_)::value;
+      mfma16<IN16, true>(acc[q / FR][q % FR], af[cbuf][q / FR], bq[cbuf][q % FR]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (q % (NMF / NC) == 0) {
+        if constexpr (cbuf == 1) copyP(src, dst, q / (NMF / NC));
+        else copyQ(src, dst, q / (NMF / NC));
+      }
+      constexpr int r_lo = q < RSPAN ? (q * NRD + RSPAN - 1) / RSPAN : NRD, r_hi = q + 1 < RSPAN ? ((q + 1) * NRD + RSPAN - 1) / RSPAN : NRD;
+      static_for<r_hi - r_lo>([&](auto d_) __attribute__((always_inline)) {
+        fread(std::integral_constant<int, cbuf ^ 1>{}, rsP, rsQ, std::integral_constant<int, cbuf ^ 1>{}, std::integral_constant<int, r_lo + decltype(d_)::value>{});
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  auto nextP = [](int s) { return s ? 0 : OPBYTES; };
+  auto nextQ = [](int s) { return s == QBASE + (SQ - 1) * OPBYTES ? QBASE : s + OPBYTES; };
+
+  wait_copies<2 * NC>();
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  static_for<NRD>([&](auto r_) __attribute__((always_inline)) { fread(I0{}, 0, QBASE, I0{}, r_); });
+  int sP = 0, sQ = QBASE;
+  constexpr int STORES = FR * FR / 2;   // of a wave and tile
+  bool first = true;
+  for (;;) {
+    const End end = next.end;
+    const int KT = next.KT;
+    const int row = wc0 + l16, col = wr0 + 16 * (lg & 1) + 8 * (lg >> 1);   // of the tile in X'^T: this lane's first 16 bytes
+    u32x4 add[ADDEND ? FR : 1][ADDEND ? FR / 2 : 1];
+    auto fetch_addend = [&](auto j_) __attribute__((always_inline)) {
+      constexpr int j = decltype(j_)::value;
+      const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(end.e), 0, -1, 0x00027000);
+#pragma unroll
+      for (int i = 0; i < FR / 2; ++i)
+        add[j][i] = __builtin_amdgcn_raw_buffer_load_b128(from, (row * end.lde + col) * 2 + i * 64, j * 32 * end.lde, 0);
+    };
+    for (int kt = 0; kt < KT; ++kt) {
+      if (ck == cKT) {   // the next copies are those of the block's next tile, if it has one
+        index += step;
+        records = index < total ? -1 : 0;
+        if (index < total) {
+          next = locate(index);
+          cP = uniform_ptr(next.P);
+          cQ = uniform_ptr(next.Q);
+          cKT = next.KT;
+          if (a.ld != off_ld) { off_ld = a.ld; lane_offsets(); }
+        }
+        ck = 0;
+      }
+      if constexpr (ADDEND) {
+        if (kt == KT - 1) static_for<FR / 2>([&](auto j_) __attribute__((always_inline)) { fetch_addend(j_); });
+      }
+      const Source src = source();
+      ++ck;
+      const int nP = nextP(sP), nQ = nextQ(sQ), pQ = sQ == QBASE ? QBASE + (SQ - 1) * OPBYTES : sQ - OPBYTES;
+      kstep(I0{}, sP, sQ, src, pQ);
+      // the stores of the tile before this one are younger than what the barrier publishes
+      if (kt == 0 && !first) wait_copies<STORES + NC>();
+      else wait_copies<NC>();
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      kstep(I1{}, nP, nQ, src, sP);
+      sP = nP;
+      sQ = nQ;
+    }
+    acc_settle();
+    // ---- epilogue, straight from the registers
+    {
+      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(end.to), 0, -1, 0x00027000);
+      const int at = (row * end.ld + col) * 2;
+      if constexpr (ADDEND) {   // (before the first store: loads return in order behind stores)
+        static_for<FR / 2>([&](auto j_) __attribute__((always_inline)) { fetch_addend(std::integral_constant<int, FR / 2 + decltype(j_)::value>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      static_for<FR>([&](auto j_) __attribute__((always_inline)) {
+        constexpr int j = decltype(j_)::value;
+#pragma unroll
+        for (int i = 0; i < FR; ++i) acc_touch<true>(acc[i][j]);
+        static_for<FR / 2>([&](auto p_) __attribute__((always_inline)) {
+          constexpr int i = 2 * decltype(p_)::value;
+          uint2 half[2], e[2];
+          if constexpr (ADDEND) {   // (the exchange of the result, the other way round)
+            const u32x4 w = add[j][i / 2];
+            const auto x = __builtin_amdgcn_permlane16_swap(w[0], w[2], false, false);
+            const auto y = __builtin_amdgcn_permlane16_swap(w[1], w[3], false, false);
+            e[0] = make_uint2(x[0], y[0]);
+            e[1] = make_uint2(x[1], y[1]);
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = acc[i + h][j][q];
+            if constexpr (ADDEND) {
+              const uint32_t ew[2] = {e[h].x, e[h].y};
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const uint16_t bits = (uint16_t)(ew[q >> 1] >> (16 * (q & 1)));
+                v[q] = fmaf(end.alpha, IN16 ? f16_to_f32(bits) : bf16_to_f32(bits), v[q]);
+              }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] *= end.factor;
+            if constexpr (OUT16) half[h] = make_uint2(f16_pair(v[0], v[1]), f16_pair(v[2], v[3]));
+            else half[h] = make_uint2(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]));
+            acc[i + h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc_touch<true>(acc[i + h][j]);
+          }
+          const auto x = __builtin_amdgcn_permlane16_swap(half[0].x, half[1].x, false, false);
+          const auto y = __builtin_amdgcn_permlane16_swap(half[0].y, half[1].y, false, false);
+          __builtin_amdgcn_raw_buffer_store_b128((u32x4){x[0], y[0], x[1], y[1]}, to, at + i * 32, j * 32 * end.ld, 0);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      acc_settle();
+    }
+    first = false;
+    if (records == 0) break;
+  }
+  wait_copies<0>();
+#endif
+}
+
 // Configurations: block tile, LDS stages of P and Q, blocks that a compute unit holds.
 //   256       all 160 KiB of LDS for one block
 //   128       half of it for each of two blocks
@@ -993,23 +1267,30 @@ long ns_gemm_tiles(int mode, const GemmParams& p) {
   return (long)p.batch * (sym ? (long)p.tilesM * (p.tilesM + 1) / 2 : (long)p.tilesM * p.tilesN);
 }
 
+// The dynamic-LDS limit of a kernel is an attribute of the function on ONE device: set once per device (and kernel, which has one of
+// these; the call is idempotent, so two threads that race on the first launch only repeat it).
+struct LdsLimit {
+  std::atomic<bool> set[64] = {};
+  hipError_t raise(const void* kern, int bytes) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const bool slot = dev >= 0 && dev < 64;
+    if (slot && set[dev].load(std::memory_order_acquire)) return hipSuccess;
+    e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess && slot) set[dev].store(true, std::memory_order_release);
+    return e;
+  }
+};
+
 template <int CFG, int MODE, bool SPLIT, bool FINAL, bool ADDEND = true, int F16 = 0, int CUT = CUT_NONE>
 static hipError_t launch_one(const GroupedGemmParams& gp, hipStream_t stream) {
   constexpr int NT = 256;
   constexpr int SMEM = (Config<CFG>::SP + Config<CFG>::SQ) * Config<CFG>::BT * ROW_BYTES;
   constexpr auto kern = kernel_of<CFG, MODE, SPLIT, FINAL, ADDEND, F16, CUT>();
-  // the dynamic-LDS limit is an attribute of the function on ONE device: set it once per device and instantiation
-  // (the call is idempotent, so two threads that race on the first launch only repeat it)
-  static std::atomic<bool> attr_set[64];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+  static LdsLimit limit;
+  const hipError_t e = limit.raise((const void*)kern, SMEM);
   if (e != hipSuccess) return e;
-  const bool slot = dev >= 0 && dev < 64;
-  if (!slot || !attr_set[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
-    if (e != hipSuccess) return e;
-    if (slot) attr_set[dev].store(true, std::memory_order_release);
-  }
   const long tiles = gp.total;
   if (tiles <= 0) return hipSuccess;
   const long unit = 8L * xcd_run((int)tiles);
@@ -1073,6 +1354,53 @@ static hipError_t launch_sequence(int mode, const GroupedGemmParams& p, hipStrea
   switch (mode) {
     case MODE_SYRK: return launch_one<CFG, MODE_SYRK, false, false, true, 0, CUT_SEQUENCE>(p, s);
     case MODE_SYRK2: return launch_one<CFG, MODE_SYRK2, false, false, true, 0, CUT_SEQUENCE>(p, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+// Whether the tiles of an X' = B X launch may follow one another in a block: whole tiles of 256, nothing that needs the other kernel's
+// bounds checks or unaligned stores, and enough of them (stream_of_tiles).
+static bool stream_takes(const GroupedGemmParams& gp, bool final_, int units) {
+  if (gp.quarter) return false;
+  int longest = 0;
+  for (int i = 0; i < gp.n_groups; ++i) {
+    const GemmParams& g = gp.g[i];
+    longest = g.K > longest ? g.K : longest;
+    if (g.t_first || g.K < 4 * BK || g.ldp != g.ldq || (g.scale && !g.E)) return false;
+    if (!final_) {
+      if (!g.Ct || g.C) return false;
+    } else {
+      const bool rows = g.C != nullptr;
+      const long stride = rows ? g.strideC : g.strideCt;
+      if (g.E || rows == (g.Ct != nullptr) || g.m_valid != g.tilesM * 256 || g.n_valid != g.tilesN * 256) return false;
+      if (((uintptr_t)(rows ? g.C : g.Ct) & 15) || (rows ? g.ldc : g.ldct) % 8 || (g.batch > 1 && stride % 8)) return false;
+    }
+  }
+  return stream_of_tiles(units, gp.total, longest);
+}
+
+template <bool FINAL, bool ADDEND, int F16>
+static hipError_t launch_stream_one(const GroupedGemmParams& gp, hipStream_t stream, int units) {
+  constexpr int SMEM = (Config<CFG_256>::SP + Config<CFG_256>::SQ) * 256 * ROW_BYTES;
+  constexpr auto kern = &ns_gemm_stream_kernel<FINAL, ADDEND, F16>;
+  static LdsLimit limit;
+  const hipError_t e = limit.raise((const void*)kern, SMEM);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)units), dim3(256), SMEM, stream, gp);
+  return hipGetLastError();
+}
+static hipError_t launch_stream(const GroupedGemmParams& gp, bool final_, int f16, hipStream_t s, int units) {
+  const bool addend = gp.g[0].E != nullptr;
+  switch (f16) {
+    case 0:
+      if (final_) return launch_stream_one<true, false, 0>(gp, s, units);
+      return addend ? launch_stream_one<false, true, 0>(gp, s, units) : launch_stream_one<false, false, 0>(gp, s, units);
+    case 1:
+      if (final_) return launch_stream_one<true, false, 1>(gp, s, units);
+      return addend ? launch_stream_one<false, true, 1>(gp, s, units) : launch_stream_one<false, false, 1>(gp, s, units);
+    case 2:
+      if (final_) return hipErrorInvalidValue;
+      return addend ? launch_stream_one<false, true, 2>(gp, s, units) : launch_stream_one<false, false, 2>(gp, s, units);
   }
   return hipErrorInvalidValue;
 }
@@ -1145,6 +1473,7 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
     if (f16 == 0) return launch_cfg<CFG, 0>(mode, split, final_, gp, stream);
     return hipErrorInvalidValue;
   };
+  if (tile == 256 && mode == MODE_BX && !split && stream_takes(gp, final_, units)) return launch_stream(gp, final_, f16, stream, units);
   if (tile == 256) return by_storage(std::integral_constant<int, CFG_256>{});
   if (tile == 128 && deep) return by_storage(std::integral_constant<int, CFG_128_DEEP>{});
   if (tile == 128) return by_storage(std::integral_constant<int, CFG_128>{});

@@ -165,3 +165,18 @@ int main() { int u, t, n, k; while (scanf("%d %d %d %d", &u, &t, &n, &k) == 4) p
     text = "".join("%d %d %d %d\n" % w for w in want)
     out = subprocess.run([str(tmp_path / "fine")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in out] == list(want.values())
+
+
+def test_lines_of_the_stream_of_tiles(tmp_path):
+    """(units, tiles, longest reduction) -> one block for all tiles of a unit or not."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "stream.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int u, t, k; while (scanf("%d %d %d", &u, &t, &k) == 3) printf("%d\n", (int)archscale::stream_of_tiles(u, t, k)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "stream.cpp"), "-o", str(tmp_path / "stream")], check=True)
+    want = {(256, 384, 2048): 1, (256, 383, 2048): 0, (256, 384, 2112): 0, (256, 4096, 256): 1, (304, 456, 512): 1, (304, 455, 512): 0, (38, 400, 512): 0}
+    text = "".join("%d %d %d\n" % w for w in want)
+    out = subprocess.run([str(tmp_path / "stream")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())

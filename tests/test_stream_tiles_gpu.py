@@ -1,0 +1,52 @@
+"""X' = B X with the tiles of a block one after the other: a matrix gives the bits that it gives alone (where launches are too small for
+that form), whatever the number of tiles per block, the mix of classes, the orientation of the result and the storage."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ns, stacks, prec, coeffs):
+    outs = [torch.empty_like(x) for x in stacks]
+    ns.newton_schulz_grouped(stacks, coeffs, 1e-7, prec=prec, outs=outs)
+    for x, o in zip(stacks, outs):
+        for i in {0, x.shape[0] // 2, x.shape[0] - 1}:
+            assert torch.equal(ns.newton_schulz(x[i], coeffs, 1e-7, prec=prec), o[i]), (tuple(x.shape), i)
+
+
+# tiles of X': 384 (one and a half per unit), 416, 1280, 1536; one k-tile count each from the shortest (K = 256) to the longest (2048);
+# more than eight tile rows; extents that are padded, whose final launch needs bounds checks
+@pytest.mark.parametrize("batch,m,n", [(96, 256, 1024), (52, 512, 1024), (160, 256, 2048), (64, 768, 2048), (6, 2048, 2304), (12, 1536, 2304),
+                                       (5, 2048, 2560), (96, 250, 1000)])
+@pytest.mark.parametrize("prec", ["bf16", "f16"])
+def test_stacks_of_one_shape(gpu_device, batch, m, n, prec):
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator(device=gpu_device).manual_seed(batch + m + n)
+    x = (torch.randn(batch, m, n, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
+    for t in (x, x.mT.contiguous()):
+        _check(ns, [t], prec, ns.QUINTIC_SCHEDULE)
+
+
+@pytest.mark.parametrize("prec", ["bf16", "f16"])
+def test_classes_of_different_reductions_and_orientations(gpu_device, prec):
+    """Blocks go from tiles of one problem to those of another: other strides, reductions, results in rows and in columns; iterates below
+    and above the size from which X' = B X walks forwards."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    for scale in (1, 3):
+        shapes = [(10 * scale, 512, 2048), (9 * scale, 2048, 256), (5 * scale, 1024, 1024), (4 * scale, 2816, 1024), (7 * scale, 256, 3072)]
+        stacks = [(torch.randn(*s, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16) for s in shapes]
+        _check(ns, stacks, prec, ns.QUINTIC_SCHEDULE)
+
+
+def test_results_that_are_not_aligned(gpu_device):
+    """A result that is not 16-byte aligned leaves the form for the final launch: the same bits, nothing beside it is touched."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    g = torch.Generator(device=gpu_device).manual_seed(4)
+    x = (torch.randn(96, 256, 1024, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
+    want = torch.empty_like(x)
+    ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[want])
+    flat = torch.full((want.numel() + 8,), 7.0, dtype=torch.bfloat16, device=gpu_device)
+    ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[flat[1:1 + want.numel()].view(want.shape)])
+    assert torch.equal(flat[1:1 + want.numel()].view(want.shape), want)
+    assert bool((flat[:1] == 7.0).all()) and bool((flat[1 + want.numel():] == 7.0).all())
