@@ -68,6 +68,27 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   return {full, tail, 0};
 }
 
+// Symmetric products in tiles of 256 that make less than a round and run as tiles of 128 of the same matrices instead, each matrix in the
+// order of its own smaller tiles (the quadrants of launch_split hold an empty block per diagonal tile and end with a scattered last
+// round).  These are
+// - every launch that launch_split quarters as a whole, and those that it cuts into quarters and sixteenths if two smaller tiles to a
+//   unit hold them (`smaller` of them): 14 x (1024 x 4096) 1106 / 981 us a call; not 4 x (2048 x 4096) (544 of them), 1140 / 1214;
+// - launches up to a full round where reductions are at most HALVED_SHORT_K: the results of a round of large tiles all leave at its
+//   end, 10 of 30 to 40 us with the matrix cores idle, while two smaller blocks to a unit store and multiply at the same time.
+//   180 x (256 x 1024) 518 / 495, 58 x (512 x 1024) 504 / 486, 42 x (768 x 768) 580 / 566, 64 experts of 512 x 2048 784 / 768;
+// - the same up to HALVED_MAX_K where the last round of smaller tiles is neither nearly empty nor more than half of one: 20 x (1024 x
+//   1024) 584 / 554, the EMA-Muon set of width 1024 1128 / 1090; not 160 tiles (16 x (1024 x 2816), power iteration, 235 / 240) nor
+//   240 (24 x (1024 x 2816), 1183 / 1190).
+// At longer reductions they lose: X X^T of 64 + 64 experts (K = 2048), 1214 / 1278 a step.
+constexpr int HALVED_MAX_K = 1024, HALVED_SHORT_K = 768;
+constexpr double HALVED_LEAST = 0.7, HALVED_MOST = 0.85;   // of a round of tiles of 256
+inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller, double longest, const LaunchSplit& cut) {
+  if (tile != 256 || pair) return false;
+  if (cut.whole == 0) return cut.sixteenths == 0 || smaller <= 2L * units;
+  if (cut.whole != total || total > units || longest > HALVED_MAX_K) return false;
+  return longest <= HALVED_SHORT_K || (total >= HALVED_LEAST * units && total <= HALVED_MOST * units);
+}
+
 // Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 (`tiles` of one
 // matrix) with at most one block to a unit.  The cut fixes the order of the sums, so callers ask for RULE_UNITS units and one
 // matrix: a matrix has the same bits alone, in a stack and on any device.  Few tiles walk a long reduction on few units; a part costs 64 KiB of traffic each way and the call a

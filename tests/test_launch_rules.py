@@ -180,3 +180,36 @@ int main() { int u, t, k; while (scanf("%d %d %d", &u, &t, &k) == 3) printf("%d\
     text = "".join("%d %d %d\n" % w for w in want)
     out = subprocess.run([str(tmp_path / "stream")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in out] == list(want.values())
+
+
+def test_lines_of_halved_tiles(tmp_path):
+    """(tile, pair, tiles of 256, tiles of 128 of the same matrices, all k-values, longest) on 256 units -> in tiles of 128 or not."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "halved.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() {
+  int t, p, n, s; double a, l;
+  while (scanf("%d %d %d %d %lf %lf", &t, &p, &n, &s, &a, &l) == 6)
+    printf("%d\n", (int)archscale::halved_tiles(256, t, p != 0, n, s, l, archscale::launch_split(256, t, p != 0, n, a, l)));
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "halved.cpp"), "-o", str(tmp_path / "halved")], check=True)
+    want = {
+        (256, 0, 100, 360, 100 * 4096.0, 4096.0): 1,     # quartered as a whole
+        (256, 0, 140, 504, 140 * 4096.0, 4096.0): 1,     # quarters and sixteenths, two smaller tiles to a unit hold it
+        (256, 0, 144, 544, 144 * 4096.0, 4096.0): 0,     # they do not
+        (256, 0, 208, 744, 208 * 590.0, 1000.0): 1,
+        (256, 0, 256, 832, 256 * 768.0, 768.0): 1,       # a full round, short reductions
+        (256, 0, 257, 840, 257 * 768.0, 768.0): 0,
+        (256, 0, 160, 576, 160 * 1024.0, 1024.0): 0,
+        (256, 0, 180, 648, 180 * 1024.0, 1024.0): 1,
+        (256, 0, 217, 780, 217 * 1024.0, 1024.0): 1,
+        (256, 0, 218, 784, 218 * 1024.0, 1024.0): 0,
+        (256, 0, 217, 780, 217 * 1088.0, 1088.0): 0,     # longer reductions stay
+        (256, 1, 217, 780, 217 * 1024.0, 1024.0): 0,     # hi+lo pairs stay
+        (128, 0, 217, 780, 217 * 1024.0, 1024.0): 0,
+    }
+    text = "".join("%d %d %d %d %.17g %.17g\n" % w for w in want)
+    out = subprocess.run([str(tmp_path / "halved")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())
