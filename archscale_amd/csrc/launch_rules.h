@@ -44,7 +44,9 @@ struct LaunchSplit { int whole, quarters, sixteenths; };
 // The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
 // left beside whole rounds of either kind become sixteen tiles of 64 each, one block per unit at most.  The 136 triangle tiles of
 // a short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
-// 14336 3353 -> 3255; more than 16 tiles so: no further gain.
+// 14336 3353 -> 3255; more than 16 tiles so: no further gain.  A launch of nothing but so few (single
+// symmetric products; one tile of 64 to a unit instead of one of 128 to a fourth of the units): 1024 x 3072 22.4 -> 13.1 us, 1024 x
+// 1024 11.6 -> 7.3, 512 x 2048 16.3 -> 9.6, 512 x 512 7.9 -> 5.5.
 constexpr int RULE_UNITS = 256;   // the device of the figures
 constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
 constexpr int SIXTEENTH_MAX = 16;
@@ -63,7 +65,7 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   const int full = total / units * units, tail = total - full;
   if (tail == 0 || (full > 0 ? tail > scaled(QUARTER_MAX_TAIL) : all > QUARTER_LOAD * units * longest)) return as_is;
   const int half = units / 2, few = scaled(SIXTEENTH_MAX);   // half: one round of quadrants
-  if (!pair && full > 0 && tail <= few) return {full, 0, tail};
+  if (!pair && tail <= few) return {full, 0, tail};   // (full: none or whole rounds)
   if (!pair && tail > half && tail - half <= few) return {full, half, tail - half};
   return {full, tail, 0};
 }
