@@ -91,6 +91,12 @@ inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller
   return longest <= HALVED_SHORT_K || (total >= HALVED_LEAST * units && total <= HALVED_MOST * units);
 }
 
+// Tiles of 128 beyond launch_split's lines whose quadrants still find room in one round, two to a unit: quartered whatever their reductions.
+// us a call, as tiles of 128 / of 64: 3 x (1000 x 2000) (108 tiles) 243 / 235, 1900 x 1900 (120) 282 / 262, 1800 x 2500 361 / 340, 12 x (500 x
+// 2000) 226 / 217, 6 x (700 x 1300) (126) 228 / 216, the fp32 decoder of width 384 (128, reductions of 384 and 1152) 252 / 237; with a second
+// round they lose: 13 x (512 x 1500) (130) 260 / 270, 2048 x 2048 (136) 288 / 342.
+inline bool one_round_of_quadrants(int units, int tile, bool pair, int total) { return tile == 128 && !pair && 2L * total <= units; }
+
 // Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 (`tiles` of one
 // matrix) with at most one block to a unit.  The cut fixes the order of the sums, so callers ask for RULE_UNITS units and one
 // matrix: a matrix has the same bits alone, in a stack and on any device.  Few tiles walk a long reduction on few units; a part costs 64 KiB of traffic each way and the call a

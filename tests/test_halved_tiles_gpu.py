@@ -22,6 +22,14 @@ def test_bits_of_a_matrix_alone(gpu_device, shapes, prec):
             assert torch.equal(ns.newton_schulz(x[i], ns.QUINTIC_SCHEDULE, 1e-7, prec=prec), o[i]), (tuple(x.shape), i)
 
 
+# 108, 120, 126 and 128 tiles of 128: one round of quadrants; 130: not
+@pytest.mark.parametrize("shapes", [[(3, 1000, 2000)], [(12, 500, 1100)], [(6, 700, 1300)], [(8, 384, 384), (8, 96, 384), (12, 1032, 384)],
+                                    [(13, 512, 1500)]])
+@pytest.mark.parametrize("prec", ["bf16", "f16"])
+def test_quadrants_of_one_round(gpu_device, shapes, prec):
+    test_bits_of_a_matrix_alone(gpu_device, shapes, prec)
+
+
 @pytest.mark.parametrize("batch,n,k", [(20, 1024, 1024), (40, 512, 512), (70, 768, 256)])
 def test_stacks_of_single_products(gpu_device, batch, n, k):
     import archscale_amd.optim.newton_schulz_hip as ns

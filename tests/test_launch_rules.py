@@ -221,3 +221,18 @@ def test_few_large_tiles_alone_become_sixteenths(rules):
     got = rules([(u, 256, 0, n, n * 1e3, 1e3, 1, 64) for u, n in want])
     assert [g[:3] for g in got] == list(want.values())
     assert rules([(256, 256, 1, 16, 16e3, 1e3, 1, 64)])[0][:3] == (0, 16, 0)
+
+
+def test_lines_of_one_round_of_quadrants(tmp_path):
+    """(units, tile, pair, tiles) -> quartered because two quadrants to a unit hold them all."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "round.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int u, t, p, n; while (scanf("%d %d %d %d", &u, &t, &p, &n) == 4) printf("%d\n", (int)archscale::one_round_of_quadrants(u, t, p != 0, n)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "round.cpp"), "-o", str(tmp_path / "round")], check=True)
+    want = {(256, 128, 0, 128): 1, (256, 128, 0, 129): 0, (256, 128, 1, 100): 0, (256, 256, 0, 100): 0, (38, 128, 0, 19): 1, (38, 128, 0, 20): 0}
+    text = "".join("%d %d %d %d\n" % w for w in want)
+    out = subprocess.run([str(tmp_path / "round")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())
