@@ -701,27 +701,22 @@ muonh_coef_kernel(const int32_t* __restrict__ prefix, const float* __restrict__ 
   }
 }
 
-template <int WD, bool HAS_COEF>
+// One run of eight elements per thread, EW_TRIPS blocks to a chunk (there is nothing to add up): a block has all its loads in flight and
+// leaves as soon as they are stored, and small launches fill the chip.  A chunk per block, all its loads before the first store /
+// a trip per block: steps of the fp32 decoder of width 384 247.6 / 245.3 us, of the EMA-Muon set of width 1024 1133 / 1125, of the
+// 64 + 64 experts 1275 / 1264.
+template <int WD>
 __device__ __forceinline__ void post_apply_range(const PostItem& it, long begin, long end, float lrwd, int cautious,
                                                  bool vec_ok, float alpha, float beta) {
   if (vec_ok) {
-    float x[EW_TRIPS][8], u[EW_TRIPS][8];   // all loads of the chunk before the first store (see momentum_range)
+    const long i = begin + (long)threadIdx.x * EW_VEC;
+    if (i < end) {
+      float x[8], u[8];
+      Elem<WD>::load8(it.w, i, x);
+      Elem<DT_BF16>::load8(it.u, i, u);
 #pragma unroll
-    for (int t = 0; t < EW_TRIPS; ++t) {
-      const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
-        Elem<WD>::load8(it.w, i, x[t]);
-        Elem<DT_BF16>::load8(it.u, i, u[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < EW_TRIPS; ++t) {
-      const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) x[t][k] = alpha * decayed(x[t][k], u[t][k], lrwd, cautious) + beta * u[t][k];
-        Elem<WD>::store8(it.w, i, x[t]);
-      }
+      for (int k = 0; k < 8; ++k) x[k] = alpha * decayed(x[k], u[k], lrwd, cautious) + beta * u[k];
+      Elem<WD>::store8(it.w, i, x);
     }
   } else {
     for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
@@ -736,24 +731,30 @@ post_apply_kernel(const PostItem* __restrict__ items, const int32_t* __restrict_
                   float lr, float lrwd, int cautious, const float2* __restrict__ coef,
                   const ScalarHyper* __restrict__ hdev) {
   if (hdev) { lr = hdev->lr; lrwd = hdev->lr_wd; cautious = hdev->cautious; }
-  const int chunk = blockIdx.x;
+  const int chunk = blockIdx.x / EW_TRIPS, trip = blockIdx.x % EW_TRIPS;
   const int ii = find_item(prefix, n_items, chunk);
   const PostItem it = items[ii];
-  const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
-  const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
+  const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS + trip * (EW_THREADS * EW_VEC);
+  const long end = begin + EW_THREADS * EW_VEC < it.numel ? begin + EW_THREADS * EW_VEC : it.numel;
   const bool vec_ok = aligned16(it.w) && aligned16(it.u) && (it.numel % EW_VEC == 0);
   float alpha = 1.f, beta = -lr * it.lr_ratio;
   if (coef) { const float2 c = coef[ii]; alpha = c.x; beta = c.y; }
-  if (it.w_dtype == DT_BF16) post_apply_range<DT_BF16, true>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
-  else post_apply_range<DT_F32, true>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
+  if (it.w_dtype == DT_BF16) post_apply_range<DT_BF16>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
+  else post_apply_range<DT_F32>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
+}
+
+static hipError_t launch_post_apply(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks, float lr, float lrwd,
+                                    int cautious, const float2* coef, hipStream_t stream, const ScalarHyper* hdev) {
+  if (total_chunks > 0x7fffffff / EW_TRIPS) return hipErrorInvalidValue;   // (2^42 elements)
+  hipLaunchKernelGGL(post_apply_kernel, dim3(total_chunks * EW_TRIPS), dim3(EW_THREADS), 0, stream, items, prefix, n_items, lr, lrwd,
+                     cautious, coef, hdev);
+  return hipGetLastError();
 }
 
 hipError_t launch_post_plain(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks,
                              float lr, float lrwd, int cautious, hipStream_t stream, const ScalarHyper* hdev) {
   if (total_chunks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(post_apply_kernel, dim3(total_chunks), dim3(EW_THREADS), 0, stream, items, prefix, n_items,
-                     lr, lrwd, cautious, (const float2*)nullptr, hdev);
-  return hipGetLastError();
+  return launch_post_apply(items, prefix, n_items, total_chunks, lr, lrwd, cautious, nullptr, stream, hdev);
 }
 
 hipError_t launch_post_muonh(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks,
@@ -765,9 +766,7 @@ hipError_t launch_post_muonh(const PostItem* items, const int32_t* prefix, int n
   hipLaunchKernelGGL(post_reduce_kernel, dim3(total_chunks), dim3(EW_THREADS), 0, stream, items, prefix, n_items,
                      lrwd, cautious, partial, hdev);
   hipLaunchKernelGGL(muonh_coef_kernel, dim3(n_items), dim3(EW_THREADS), 0, stream, prefix, partial, lr, eps, coef, hdev);
-  hipLaunchKernelGGL(post_apply_kernel, dim3(total_chunks), dim3(EW_THREADS), 0, stream, items, prefix, n_items,
-                     lr, lrwd, cautious, (const float2*)coef, hdev);
-  return hipGetLastError();
+  return launch_post_apply(items, prefix, n_items, total_chunks, lr, lrwd, cautious, coef, stream, hdev);
 }
 
 // ---------------------------------------------------------------------------
