@@ -29,6 +29,9 @@ __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int
   return __builtin_amdgcn_readfirstlane(lo + __popcll(__ballot(owns)) - 1);
 }
 
+// end of the whole runs of eight elements of [begin, end); at most seven elements are left, at the end of an item
+__device__ __forceinline__ long whole_runs(long begin, long end) { return begin + (end - begin) / EW_VEC * EW_VEC; }
+
 // ---------------------------------------------------------------------------
 // 1. momentum:  M <- c_mm*M + c_mg*G ;  U <- c_um*M + c_ug*G   (G optionally += l2*W first)
 //    lit_gpt: (mu, 1, mu|1, 1|0)  (muon.py:665-679);  emerging: (b, 1-b, b|1, 1-b|0)
@@ -36,17 +39,17 @@ __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int
 // ---------------------------------------------------------------------------
 // SS: also accumulate the sum of squares of the update as stored (rounded to U's dtype) into `ss`
 template <int GD, int MD, int UD, bool SS = false>
-__device__ __forceinline__ void momentum_range(const PreItem& it, long begin, long end, const MomentumCoef c, bool vec_ok,
-                                               float* ss = nullptr) {
+__device__ __forceinline__ void momentum_range(const PreItem& it, long begin, long end, const MomentumCoef c, float* ss = nullptr) {
   const void* g = it.g; void* m = it.m; void* u = it.u;
-  if (vec_ok) {
+  const long full = whole_runs(begin, end);
+  {
     // every load of the chunk first, then the arithmetic and the stores: the stores may alias the loads as far as the
     // compiler knows, and a load that waits for the previous trip's stores leaves the memory pipeline half empty
     float gv[EW_TRIPS][8], mv[EW_TRIPS][8];
 #pragma unroll
     for (int t = 0; t < EW_TRIPS; ++t) {
       const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
+      if (i < full) {
         Elem<GD>::load8(g, i, gv[t]);
         Elem<MD>::load8(m, i, mv[t]);
       }
@@ -54,7 +57,7 @@ __device__ __forceinline__ void momentum_range(const PreItem& it, long begin, lo
 #pragma unroll
     for (int t = 0; t < EW_TRIPS; ++t) {
       const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
+      if (i < full) {
         float uv[8];
         if (c.l2 != 0.f) {
           float wv[8];
@@ -75,8 +78,9 @@ __device__ __forceinline__ void momentum_range(const PreItem& it, long begin, lo
         Elem<UD>::keep8(u, i, uv);
       }
     }
-  } else {
-    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
+  }
+  if (full < end) {   // fewer than eight elements
+    for (long i = full + threadIdx.x; i < end; i += EW_THREADS) {
       float gv = Elem<GD>::load1(g, i);
       if (c.l2 != 0.f) {
         const float wv = it.w_dtype == DT_BF16 ? Elem<DT_BF16>::load1(it.w, i) : Elem<DT_F32>::load1(it.w, i);
@@ -100,18 +104,16 @@ momentum_kernel(const PreItem* __restrict__ items, const int32_t* __restrict__ p
   const PreItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
-  const bool vec_ok = aligned16(it.g) && aligned16(it.m) && aligned16(it.u) && (c.l2 == 0.f || aligned16(it.w)) &&
-                      (it.numel % EW_VEC == 0);
   const int key = (it.g_dtype << 2) | (it.m_dtype << 1) | it.u_dtype;
   switch (key) {
-    case 0: momentum_range<DT_BF16, DT_BF16, DT_BF16>(it, begin, end, c, vec_ok); break;
-    case 1: momentum_range<DT_BF16, DT_BF16, DT_F32>(it, begin, end, c, vec_ok); break;
-    case 2: momentum_range<DT_BF16, DT_F32, DT_BF16>(it, begin, end, c, vec_ok); break;
-    case 3: momentum_range<DT_BF16, DT_F32, DT_F32>(it, begin, end, c, vec_ok); break;
-    case 4: momentum_range<DT_F32, DT_BF16, DT_BF16>(it, begin, end, c, vec_ok); break;
-    case 5: momentum_range<DT_F32, DT_BF16, DT_F32>(it, begin, end, c, vec_ok); break;
-    case 6: momentum_range<DT_F32, DT_F32, DT_BF16>(it, begin, end, c, vec_ok); break;
-    default: momentum_range<DT_F32, DT_F32, DT_F32>(it, begin, end, c, vec_ok); break;
+    case 0: momentum_range<DT_BF16, DT_BF16, DT_BF16>(it, begin, end, c); break;
+    case 1: momentum_range<DT_BF16, DT_BF16, DT_F32>(it, begin, end, c); break;
+    case 2: momentum_range<DT_BF16, DT_F32, DT_BF16>(it, begin, end, c); break;
+    case 3: momentum_range<DT_BF16, DT_F32, DT_F32>(it, begin, end, c); break;
+    case 4: momentum_range<DT_F32, DT_BF16, DT_BF16>(it, begin, end, c); break;
+    case 5: momentum_range<DT_F32, DT_BF16, DT_F32>(it, begin, end, c); break;
+    case 6: momentum_range<DT_F32, DT_F32, DT_BF16>(it, begin, end, c); break;
+    default: momentum_range<DT_F32, DT_F32, DT_F32>(it, begin, end, c); break;
   }
 }
 
@@ -136,7 +138,7 @@ stage_sumsq_kernel(const StageParams sp) {
   const int b = local / q.cpm, chunk = local - b * q.cpm;
   const int rows = q.rows, cols = q.cols, ld = q.ld;
   const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
-  float s[1] = {dense_sumsq_ok(base, rows, cols, ld) ? thread_sumsq_dense<DT>(base, (long)rows * cols, chunk, threadIdx.x, CAST_FIRST)
+  float s[1] = {dense_sumsq_ok(rows, cols, ld) ? thread_sumsq_dense<DT>(base, (long)rows * cols, chunk, threadIdx.x, CAST_FIRST)
                                                      : thread_sumsq_strided<DT>(base, rows, cols, ld, chunk, threadIdx.x, CAST_FIRST)};
   block_reduce<1>(s, red);
   if (threadIdx.x == 0) q.partial[(size_t)b * q.cpm + chunk] = s[0];
@@ -149,7 +151,7 @@ stage_sumsq_kernel(const StageParams sp) {
 // ---------------------------------------------------------------------------
 // one 64x64 tile (row tile ty, column tile tx) by one block; d_rows / d_cols are the padded extents (multiples of 64)
 template <int DT, bool CAST_FIRST>
-__device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, int ty, int tx, int rows, int cols, int ld, float s,
+__device__ __forceinline__ void layout_tile(const char* base, int ty, int tx, int rows, int cols, int ld, float s,
                                             uint16_t* D, int ldd, int d_rows, int d_cols, uint16_t* T, int ldt, int out_f16,
                                             int out_shift, float* tile_sumsq) {
   __shared__ uint16_t tile[64][66];
@@ -159,12 +161,11 @@ __device__ __forceinline__ void layout_tile(const char* base, bool stride_ok, in
   const float fs = __builtin_ldexpf(1.f, out_shift);
   const int tr = threadIdx.x >> 3;        // 0..31
   const int tc = (threadIdx.x & 7) * 8;   // 0..56
-  const bool vec = aligned16(base) && (ld % 8 == 0) && stride_ok;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int r = r0 + tr + h * 32, c = c0 + tc;
     float v[8];
-    if (r < rows && c + 7 < cols && vec) {
+    if (r < rows && c + 7 < cols) {
       Elem<DT>::load8(base, (long)r * ld + c, v);
     } else {
 #pragma unroll
@@ -216,7 +217,7 @@ layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstrid
   const int b = blockIdx.z;
   // the matrices of the batch: equally spaced from `in`, or (in == null) separate allocations listed in `ptrs`
   const char* base = in ? (const char*)in + (size_t)b * in_bstride * sizeof(typename Elem<DT>::T) : (const char*)ptrs.p[b];
-  layout_tile<DT, false>(base, !in || in_bstride % 8 == 0, blockIdx.y, blockIdx.x, rows, cols, ld, 1.f,
+  layout_tile<DT, false>(base, blockIdx.y, blockIdx.x, rows, cols, ld, 1.f,
                          D ? D + (size_t)b * bstride : nullptr, ldd, d_rows, d_cols, T ? T + (size_t)b * bstride : nullptr, ldt,
                          0, 0, tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr);
 }
@@ -258,7 +259,7 @@ stage_layout_kernel(const StageParams sp) {
   }
   const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
   uint16_t* dst = q.dst + (size_t)b * q.d_bstride;
-  layout_tile<DT, CAST_FIRST>(base, q.in_bstride % 8 == 0, ty, tx, q.rows, q.cols, q.ld, s, q.transpose ? nullptr : dst, q.ldd,
+  layout_tile<DT, CAST_FIRST>(base, ty, tx, q.rows, q.cols, q.ld, s, q.transpose ? nullptr : dst, q.ldd,
                               q.d_rows, q.d_cols, q.transpose ? dst : nullptr, q.ldd, q.out_f16, q.out_shift, nullptr);
 }
 
@@ -335,8 +336,9 @@ __device__ __forceinline__ void momlay_tile(const MomMat& p, int r0, int c0,
   const void* w = p.w;
   const int tr = threadIdx.x / MOMLAY_TPR, tc = (threadIdx.x % MOMLAY_TPR) * 8;
   const int c = c0 + tc;
-  const bool vec = aligned16(g) && aligned16(m) && (p.cols % 8 == 0) && (p.c.l2 == 0.f || aligned16(w));
-  const bool cols_in = vec && c + 7 < p.cols;
+  // whole runs of eight elements, and the run at the end of a row of odd width one by one
+  const bool whole = c + 7 < p.cols;
+  auto in = [&](int k) { return c + k < p.cols; };
 #pragma unroll
   for (int hb = 0; hb < MOMLAY_PASSES; hb += MOMLAY_BATCH) {
     // all loads of the batch first: the stores below may alias them as far as the compiler knows
@@ -344,59 +346,55 @@ __device__ __forceinline__ void momlay_tile(const MomMat& p, int r0, int c0,
 #pragma unroll
     for (int j = 0; j < MOMLAY_BATCH; ++j) {
       const int r = r0 + tr + (hb + j) * MOMLAY_RPP;
-      if (r < p.rows && cols_in) {
-        const long i = (long)r * p.cols + c;
+      const long i = (long)r * p.cols + c;
+      if (r < p.rows && whole) {
         Elem<GD>::load8(g, i, gv[j]);
         Elem<MD>::load8(m, i, mv[j]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const bool on = r < p.rows && in(k);
+          gv[j][k] = on ? Elem<GD>::load1(g, i + k) : 0.f;
+          mv[j][k] = on ? Elem<MD>::load1(m, i + k) : 0.f;
+        }
       }
     }
 #pragma unroll
     for (int j = 0; j < MOMLAY_BATCH; ++j) {
       const int r = r0 + tr + (hb + j) * MOMLAY_RPP;
-      float uv[8];
-      if (r < p.rows && cols_in) {
-        const long i = (long)r * p.cols + c;
-        if (p.c.l2 != 0.f) {
-          float wv[8];
+      const long i = (long)r * p.cols + c;
+      const bool row_in = r < p.rows;
+      if (p.c.l2 != 0.f && row_in) {
+        float wv[8];
+        if (whole) {
           if (p.w_dtype == DT_BF16) Elem<DT_BF16>::load8(w, i, wv); else Elem<DT_F32>::load8(w, i, wv);
+        } else {
 #pragma unroll
-          for (int k = 0; k < 8; ++k) gv[j][k] = Elem<GD>::round(gv[j][k] + p.c.l2 * wv[k]);
-          Elem<GD>::store8(const_cast<char*>(g), i, gv[j]);
+          for (int k = 0; k < 8; ++k) wv[k] = !in(k) ? 0.f : (p.w_dtype == DT_BF16 ? Elem<DT_BF16>::load1(w, i + k) : Elem<DT_F32>::load1(w, i + k));
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float gm = Elem<MD>::round(gv[j][k]);
-          const float mn = Elem<MD>::round(fmaf(p.c.mm, mv[j][k], p.c.mg * gm));
-          mv[j][k] = mn;
-          uv[k] = fmaf(p.c.um, mn, p.c.ug * gm);
-        }
-        Elem<MD>::store8(m, i, mv[j]);
-      } else {
+        for (int k = 0; k < 8; ++k) gv[j][k] = Elem<GD>::round(gv[j][k] + p.c.l2 * wv[k]);
+        if (whole) Elem<GD>::store8(const_cast<char*>(g), i, gv[j]);
+        else {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          uv[k] = 0.f;
-          if (r < p.rows && c + k < p.cols) {
-            const long i = (long)r * p.cols + c + k;
-            float gs = Elem<GD>::load1(g, i);
-            if (p.c.l2 != 0.f) {
-              const float wv = p.w_dtype == DT_BF16 ? Elem<DT_BF16>::load1(w, i) : Elem<DT_F32>::load1(w, i);
-              gs = Elem<GD>::round(gs + p.c.l2 * wv);
-              Elem<GD>::store1(const_cast<char*>(g), i, gs);
-            }
-            const float gm = Elem<MD>::round(gs);
-            const float mn = Elem<MD>::round(fmaf(p.c.mm, Elem<MD>::load1(m, i), p.c.mg * gm));
-            Elem<MD>::store1(m, i, mn);
-            uv[k] = fmaf(p.c.um, mn, p.c.ug * gm);
-          }
+          for (int k = 0; k < 8; ++k) if (in(k)) Elem<GD>::store1(const_cast<char*>(g), i + k, gv[j][k]);
         }
       }
       uint16_t o[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        o[k] = f2bf(uv[k]);
+        const float gm = Elem<MD>::round(gv[j][k]);
+        const float mn = Elem<MD>::round(fmaf(p.c.mm, mv[j][k], p.c.mg * gm));
+        mv[j][k] = mn;
+        o[k] = f2bf(row_in && in(k) ? fmaf(p.c.um, mn, p.c.ug * gm) : 0.f);
         const float x = bf2f(o[k]);
         sumsq += x * x;
         tile[tr + (hb + j) * MOMLAY_RPP][tc + k] = o[k];
+      }
+      if (row_in && whole) Elem<MD>::store8(m, i, mv[j]);
+      else if (row_in) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) if (in(k)) Elem<MD>::store1(m, i + k, mv[j][k]);
       }
       if (!p.transpose) {
         u32x4 pk;
@@ -470,14 +468,12 @@ momentum_linear_kernel(const MomGroupParams p) {
   it.g_dtype = p.g_dtype; it.m_dtype = p.m_dtype; it.u_dtype = DT_BF16; it.w_dtype = p.w_dtype;
   const long begin = (long)chunk * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
-  const bool vec_ok = aligned16(it.g) && aligned16(it.m) && aligned16(it.u) && (p.c.l2 == 0.f || aligned16(it.w)) &&
-                      (it.numel % EW_VEC == 0);
   float s[1] = {0.f};
   switch ((p.g_dtype << 1) | p.m_dtype) {
-    case 0: momentum_range<DT_BF16, DT_BF16, DT_BF16, true>(it, begin, end, p.c, vec_ok, &s[0]); break;
-    case 1: momentum_range<DT_BF16, DT_F32, DT_BF16, true>(it, begin, end, p.c, vec_ok, &s[0]); break;
-    case 2: momentum_range<DT_F32, DT_BF16, DT_BF16, true>(it, begin, end, p.c, vec_ok, &s[0]); break;
-    default: momentum_range<DT_F32, DT_F32, DT_BF16, true>(it, begin, end, p.c, vec_ok, &s[0]); break;
+    case 0: momentum_range<DT_BF16, DT_BF16, DT_BF16, true>(it, begin, end, p.c, &s[0]); break;
+    case 1: momentum_range<DT_BF16, DT_F32, DT_BF16, true>(it, begin, end, p.c, &s[0]); break;
+    case 2: momentum_range<DT_F32, DT_BF16, DT_BF16, true>(it, begin, end, p.c, &s[0]); break;
+    default: momentum_range<DT_F32, DT_F32, DT_BF16, true>(it, begin, end, p.c, &s[0]); break;
   }
   block_reduce<1>(s, red);
   if (threadIdx.x == 0) k.partial[(size_t)idx * k.blocks_per_mat + chunk] = s[0];
@@ -616,29 +612,26 @@ __device__ __forceinline__ float decayed(float x, float u, float lrwd, int cauti
 }
 
 template <int WD>
-__device__ __forceinline__ void post_reduce_range(const PostItem& it, long begin, long end, float lrwd, int cautious,
-                                                  bool vec_ok, float (&s)[3]) {
-  if (vec_ok) {
+__device__ __forceinline__ void post_reduce_range(const PostItem& it, long begin, long end, float lrwd, int cautious, float (&s)[3]) {
+  const long full = whole_runs(begin, end);
 #pragma unroll
-    for (int t = 0; t < EW_TRIPS; ++t) {
-      const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-      if (i < end) {
-        float x[8], u[8];
-        Elem<WD>::load8(it.w, i, x);
-        Elem<DT_BF16>::load8(it.u, i, u);
+  for (int t = 0; t < EW_TRIPS; ++t) {
+    const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
+    if (i < full) {
+      float x[8], u[8];
+      Elem<WD>::load8(it.w, i, x);
+      Elem<DT_BF16>::load8(it.u, i, u);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float xd = decayed(x[k], u[k], lrwd, cautious);
-          s[0] += xd * xd; s[1] += u[k] * u[k]; s[2] += xd * u[k];
-        }
+      for (int k = 0; k < 8; ++k) {
+        const float xd = decayed(x[k], u[k], lrwd, cautious);
+        s[0] += xd * xd; s[1] += u[k] * u[k]; s[2] += xd * u[k];
       }
     }
-  } else {
-    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
-      const float u = Elem<DT_BF16>::load1(it.u, i);
-      const float xd = decayed(Elem<WD>::load1(it.w, i), u, lrwd, cautious);
-      s[0] += xd * xd; s[1] += u * u; s[2] += xd * u;
-    }
+  }
+  for (long i = full + threadIdx.x; i < end; i += EW_THREADS) {
+    const float u = Elem<DT_BF16>::load1(it.u, i);
+    const float xd = decayed(Elem<WD>::load1(it.w, i), u, lrwd, cautious);
+    s[0] += xd * xd; s[1] += u * u; s[2] += xd * u;
   }
 }
 
@@ -653,10 +646,9 @@ post_reduce_kernel(const PostItem* __restrict__ items, const int32_t* __restrict
   const PostItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
-  const bool vec_ok = aligned16(it.w) && aligned16(it.u) && (it.numel % EW_VEC == 0);
   float s[3] = {0.f, 0.f, 0.f};
-  if (it.w_dtype == DT_BF16) post_reduce_range<DT_BF16>(it, begin, end, lrwd, cautious, vec_ok, s);
-  else post_reduce_range<DT_F32>(it, begin, end, lrwd, cautious, vec_ok, s);
+  if (it.w_dtype == DT_BF16) post_reduce_range<DT_BF16>(it, begin, end, lrwd, cautious, s);
+  else post_reduce_range<DT_F32>(it, begin, end, lrwd, cautious, s);
   block_reduce<3>(s, red);
   if (threadIdx.x == 0) {
     partial[(size_t)chunk * 3 + 0] = s[0];
@@ -706,22 +698,20 @@ muonh_coef_kernel(const int32_t* __restrict__ prefix, const float* __restrict__ 
 // a trip per block: steps of the fp32 decoder of width 384 247.6 / 245.3 us, of the EMA-Muon set of width 1024 1133 / 1125, of the
 // 64 + 64 experts 1275 / 1264.
 template <int WD>
-__device__ __forceinline__ void post_apply_range(const PostItem& it, long begin, long end, float lrwd, int cautious,
-                                                 bool vec_ok, float alpha, float beta) {
-  if (vec_ok) {
-    const long i = begin + (long)threadIdx.x * EW_VEC;
-    if (i < end) {
-      float x[8], u[8];
-      Elem<WD>::load8(it.w, i, x);
-      Elem<DT_BF16>::load8(it.u, i, u);
+__device__ __forceinline__ void post_apply_range(const PostItem& it, long begin, long end, float lrwd, int cautious, float alpha,
+                                                 float beta) {
+  const long i = begin + (long)threadIdx.x * EW_VEC;
+  if (i + EW_VEC <= end) {
+    float x[8], u[8];
+    Elem<WD>::load8(it.w, i, x);
+    Elem<DT_BF16>::load8(it.u, i, u);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) x[k] = alpha * decayed(x[k], u[k], lrwd, cautious) + beta * u[k];
-      Elem<WD>::store8(it.w, i, x);
-    }
+    for (int k = 0; k < 8; ++k) x[k] = alpha * decayed(x[k], u[k], lrwd, cautious) + beta * u[k];
+    Elem<WD>::store8(it.w, i, x);
   } else {
-    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
-      const float u = Elem<DT_BF16>::load1(it.u, i);
-      Elem<WD>::store1(it.w, i, alpha * decayed(Elem<WD>::load1(it.w, i), u, lrwd, cautious) + beta * u);
+    for (long e = i; e < end; ++e) {
+      const float u = Elem<DT_BF16>::load1(it.u, e);
+      Elem<WD>::store1(it.w, e, alpha * decayed(Elem<WD>::load1(it.w, e), u, lrwd, cautious) + beta * u);
     }
   }
 }
@@ -736,11 +726,10 @@ post_apply_kernel(const PostItem* __restrict__ items, const int32_t* __restrict_
   const PostItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS + trip * (EW_THREADS * EW_VEC);
   const long end = begin + EW_THREADS * EW_VEC < it.numel ? begin + EW_THREADS * EW_VEC : it.numel;
-  const bool vec_ok = aligned16(it.w) && aligned16(it.u) && (it.numel % EW_VEC == 0);
   float alpha = 1.f, beta = -lr * it.lr_ratio;
   if (coef) { const float2 c = coef[ii]; alpha = c.x; beta = c.y; }
-  if (it.w_dtype == DT_BF16) post_apply_range<DT_BF16>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
-  else post_apply_range<DT_F32>(it, begin, end, lrwd, cautious, vec_ok, alpha, beta);
+  if (it.w_dtype == DT_BF16) post_apply_range<DT_BF16>(it, begin, end, lrwd, cautious, alpha, beta);
+  else post_apply_range<DT_F32>(it, begin, end, lrwd, cautious, alpha, beta);
 }
 
 static hipError_t launch_post_apply(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks, float lr, float lrwd,
@@ -838,7 +827,7 @@ __device__ __forceinline__ float scalar_elem(float x, float g, float& m, float& 
   return alpha * xd + beta * u;
 }
 
-// one chunk of an item whose arrays are 16-byte aligned: T loads, stores and rounds them (see below)
+// the whole runs of eight of a chunk of an item: T loads, stores and rounds its arrays (see below)
 template <int ALGO, int PHASE, class T>
 __device__ __forceinline__ void scalar_range(const ScalarItem& it, long begin, long end, const ScalarHyper& h, const Direction& dir,
                                              float lr1, float alpha, float beta, float (&s)[3], const T& io) {
@@ -907,27 +896,27 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
   constexpr bool has_v = ALGO == ALGO_ADAMW;
-  const bool vec_ok = aligned16(it.w) && aligned16(it.g) && aligned16(it.m) && (!has_v || aligned16(it.v)) &&
-                      (it.numel % EW_VEC == 0);
+  const long full = whole_runs(begin, end);
   float alpha = 1.f, beta = 0.f;
   if (PHASE == 2) { const float2 c = coef[ii]; alpha = c.x; beta = c.y; }
   const Direction dir = direction_of(h, PHASE != 0);
   const float lr1 = h.lr / h.bias1;
   float s[3] = {0.f, 0.f, 0.f};
-  if (vec_ok) {
+  {
     // Bound by memory once the arithmetic is out of the way: the update of one element was about 100 vector instructions
     // (three IEEE divisions, a branch on the dtype per conversion), four clocks each.  206 million bf16 elements of two
     // vocabulary matrices: phase 1 678 -> 459 us (5.4 TB/s), phase 2 400 -> 280 us (5.9 TB/s).
     const int dt = it.w_dtype;
     const bool one = it.m_dtype == dt && it.g_dtype == dt && (!has_v || it.v_dtype == dt);
-    if (one && dt == DT_BF16) scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, OneDtype<DT_BF16>{});
+    if (one && dt == DT_BF16) scalar_range<ALGO, PHASE>(it, begin, full, h, dir, lr1, alpha, beta, s, OneDtype<DT_BF16>{});
     // (plain AdamW on fp32 arrays is bound by its seven streams and slower with all its loads issued at once: 18 million
     // elements of 20000 x 900 twice, 238 us against 208 us with a branch at each access)
     else if (one && !(ALGO == ALGO_ADAMW && PHASE == 0))
-      scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, OneDtype<DT_F32>{});
-    else scalar_range<ALGO, PHASE>(it, begin, end, h, dir, lr1, alpha, beta, s, MixedDtypes{});
-  } else {
-    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
+      scalar_range<ALGO, PHASE>(it, begin, full, h, dir, lr1, alpha, beta, s, OneDtype<DT_F32>{});
+    else scalar_range<ALGO, PHASE>(it, begin, full, h, dir, lr1, alpha, beta, s, MixedDtypes{});
+  }
+  if (full < end) {   // fewer than eight elements
+    for (long i = full + threadIdx.x; i < end; i += EW_THREADS) {
       float x = load1_rt(it.w, it.w_dtype, i), m = load1_rt(it.m, it.m_dtype, i);
       float g = PHASE != 2 ? load1_rt(it.g, it.g_dtype, i) : 0.f;
       float v = has_v ? load1_rt(it.v, it.v_dtype, i) : 0.f;

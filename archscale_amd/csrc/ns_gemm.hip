@@ -40,6 +40,7 @@ namespace archscale {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));   // a result of the caller's, wherever it starts (16-byte stores of any alignment)
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -851,24 +852,24 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
       const long tbs = SYM ? out.strideC : out.strideCt;
       const int tld = SYM ? out.ldc : out.ldct;
       __bf16* base = Tdst + (size_t)b * tbs;
-      const bool vec_ok = !FINAL || ((tld & 7) == 0 && (tbs & 7) == 0 && (((uintptr_t)Tdst) & 15) == 0);
       const int row = lane / RCH, ch = lane % RCH;   // of a slab of SLAB_ROWS rows of W; W's rows are the tile's columns
-      auto slab = [&](int t) { return *(const uint4*)(W + t * 1024 + row * WROW + ((ch ^ sw(t * SLAB_ROWS + row)) << 4)); };
-      if (!FINAL || (vec_ok && wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
+      auto slab = [&](int t) { return *(const u32x4*)(W + t * 1024 + row * WROW + ((ch ^ sw(t * SLAB_ROWS + row)) << 4)); };
+      using store_t = std::conditional_t<FINAL, u32x4_any, u32x4>;
+      if (!FINAL || (wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
         char* to = (char*)(base + (size_t)(wcol0 + row) * tld + wrow0 + ch * 8);
         static_for<WSLABS>([&](auto t_) __attribute__((always_inline)) {
           constexpr int t = decltype(t_)::value;
-          *(uint4*)(to + (long)(t * SLAB_ROWS * 2) * tld) = slab(t);
+          *(store_t*)(to + (long)(t * SLAB_ROWS * 2) * tld) = slab(t);
           if constexpr (t % 8 == 7) __builtin_amdgcn_sched_barrier(0);
         });
       } else {
 #pragma unroll 4
         for (int t = 0; t < WSLABS; ++t) {
-          const uint4 val = slab(t);
+          const u32x4 val = slab(t);
           const int orow = wcol0 + t * SLAB_ROWS + row, ocol = wrow0 + ch * 8;
           if (orow < out.n_valid) {
-            if (vec_ok && ocol + 7 < out.m_valid) {
-              *(uint4*)(base + (size_t)orow * tld + ocol) = val;
+            if (ocol + 7 < out.m_valid) {
+              *(u32x4_any*)(base + (size_t)orow * tld + ocol) = val;
             } else {
               const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll
@@ -883,7 +884,6 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
     // lane L of the group then holds W[c0 .. c0+3][r0 + L].
     if (SYM || out.C) {
       __bf16* base = Cdst + (size_t)b * out.strideC;
-      const bool vec_ok = !FINAL || ((out.ldc & 7) == 0 && (out.strideC & 7) == 0 && (((uintptr_t)Cdst) & 15) == 0);
       const int s = l16;
       // 16 rows, from row rb * 16 on, of the eight columns from cb * 32 + lg * 8 on
       auto rows16 = [&](int rb, int cb) {
@@ -893,15 +893,16 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
         const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) s16x4*)(W + w_off(c0 + 4 + (s >> 2), rb * 16 + 4 * (s & 3))));
         const uint2 lo = __builtin_bit_cast(uint2, lo4), hi = __builtin_bit_cast(uint2, hi4);
-        return make_uint4(lo.x, lo.y, hi.x, hi.y);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
       };
-      if (!FINAL || (vec_ok && wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
+      using store_t = std::conditional_t<FINAL, u32x4_any, u32x4>;
+      if (!FINAL || (wcol0 + WT <= out.n_valid && wrow0 + WT <= out.m_valid)) {
         char* to = (char*)(base + (size_t)(wrow0 + s) * out.ldc + wcol0 + lg * 8);
         static_for<WT / 16>([&](auto rb_) __attribute__((always_inline)) {
           constexpr int rb = decltype(rb_)::value;
           static_for<WT / 32>([&](auto cb_) __attribute__((always_inline)) {
             constexpr int cb = decltype(cb_)::value;
-            *(uint4*)(to + (long)(rb * 32) * out.ldc + cb * 64) = rows16(rb, cb);
+            *(store_t*)(to + (long)(rb * 32) * out.ldc + cb * 64) = rows16(rb, cb);
           });
           if constexpr (rb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         });
@@ -910,11 +911,11 @@ __device__ __forceinline__ void ns_gemm_tile(const GroupedGemmParams& gp) {
         for (int rb = 0; rb < WT / 16; ++rb)
 #pragma unroll
           for (int cb = 0; cb < WT / 32; ++cb) {
-            const uint4 val = rows16(rb, cb);
+            const u32x4 val = rows16(rb, cb);
             const int orow = wrow0 + rb * 16 + s, ocol = wcol0 + cb * 32 + lg * 8;
             if (orow < out.m_valid) {
-              if (vec_ok && ocol + 7 < out.n_valid) {
-                *(uint4*)(base + (size_t)orow * out.ldc + ocol) = val;
+              if (ocol + 7 < out.n_valid) {
+                *(u32x4_any*)(base + (size_t)orow * out.ldc + ocol) = val;
               } else {
                 const uint32_t w[4] = {val.x, val.y, val.z, val.w};
 #pragma unroll

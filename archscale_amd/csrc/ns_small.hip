@@ -351,7 +351,7 @@ struct Small {
       auto chunk_sums = [&](auto first_, auto count_) __attribute__((always_inline)) {
         constexpr int first = decltype(first_)::value, count = decltype(count_)::value;
         float v[count];
-        if (dense_sumsq_ok(base, p.rows, p.cols, p.in_ld)) {
+        if (dense_sumsq_ok(p.rows, p.cols, p.in_ld)) {
 #pragma unroll
           for (int j = 0; j < count; ++j)
             v[j] = thread_sumsq_dense<DT>(base, (long)m * n, (wave >> 2) + 2 * (first + j), threadIdx.x & 255, sp.cast_first);
@@ -378,7 +378,7 @@ struct Small {
       rest = sp.defer ? f.x : 1.f;
     }
     // whole runs of eight, or element by element (a branch per run would make every load wait for the one before)
-    const bool vec = aligned16(base) && p.in_ld % 8 == 0 && p.in_stride % 8 == 0 && p.cols % 8 == 0;
+    const bool vec = p.cols % 8 == 0;
     const float fs = __builtin_ldexpf(1.f, sp.half ? p.sx : 0);
     // eight elements of a row from column c on, and the eight as they go into the workspace
     auto fetch = [&](auto vec_, int r, int c, float (&v)[8]) __attribute__((always_inline)) {
@@ -507,11 +507,10 @@ __global__ void __launch_bounds__(NT, 1) small_ns_kernel(const SmallNsParams sp)
 
   // the result, out of LDS: rows of X^T as they are for a tall matrix, transpose reads for a wide one
   uint16_t* const out = p.out + (size_t)b * p.out_stride;
-  const bool vec_ok = (p.out_ld & 7) == 0 && (p.out_stride & 7) == 0 && ((uintptr_t)p.out & 15) == 0;
   auto put = [&](int row, int col, int cols, const u32x4& v) __attribute__((always_inline)) {
     uint16_t* to = out + (size_t)row * p.out_ld + col;
-    if (vec_ok && col + 8 <= cols) {
-      *(u32x4*)to = v;
+    if (col + 8 <= cols) {
+      *(u32x4_any*)to = v;
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
