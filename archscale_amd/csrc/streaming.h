@@ -104,32 +104,34 @@ __device__ __forceinline__ void block_reduce(float (&v)[N], float* smem /* N * 4
 // Sum of squares of a 256-thread block's share of a strided matrix: what thread `tid` adds up of the chunk (MUON_CHUNK_ELEMS
 // consecutive elements in row-major order; 0 for a chunk past the end).  Whoever forms the norm of a matrix adds in this order.
 // Dense matrices (dense_sumsq_ok) load a chunk whole before the first sum; the first elements of the matrix stand in past its
-// end and are not counted, and a last run of fewer than eight is fetched one by one.
+// end and are not counted; the elements after the last whole run join at the end.
 __device__ __forceinline__ bool dense_sumsq_ok(int rows, int cols, int ld) { return ld == cols && (long)rows * cols >= EW_VEC; }
 template <int DT>
 __device__ __forceinline__ float thread_sumsq_dense(const char* base, long numel, int chunk, int tid, bool cast_first) {
-  const long first = (long)chunk * MUON_CHUNK_ELEMS + (long)tid * EW_VEC;
+  const long first = (long)chunk * MUON_CHUNK_ELEMS + (long)tid * EW_VEC, full = numel / EW_VEC * EW_VEC;
   float v[EW_TRIPS][EW_VEC], s = 0.f;
 #pragma unroll
   for (int t = 0; t < EW_TRIPS; ++t) {
     const long i = first + (long)t * EW_THREADS * EW_VEC;
-    Elem<DT>::load8(base, i + EW_VEC <= numel ? i : 0, v[t]);
+    Elem<DT>::load8(base, i < full ? i : 0, v[t]);
   }
 #pragma unroll
   for (int t = 0; t < EW_TRIPS; ++t) {
-    const long i = first + (long)t * EW_THREADS * EW_VEC;
-    const bool in = i + EW_VEC <= numel;
-    if (!in && i < numel) {
+    const bool in = first + (long)t * EW_THREADS * EW_VEC < full;
 #pragma unroll
-      for (int k = 0; k < EW_VEC; ++k) v[t][k] = i + k < numel ? Elem<DT>::load1(base, i + k) : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < EW_VEC; ++k) v[t][k] = i < numel ? (DT == DT_F32 && cast_first ? bf2f(f2bf(v[t][k])) : v[t][k]) : 0.f;
+    for (int k = 0; k < EW_VEC; ++k) v[t][k] = in ? (DT == DT_F32 && cast_first ? bf2f(f2bf(v[t][k])) : v[t][k]) : 0.f;
     // (the second square is rounded before the first joins it)
 #pragma unroll
     for (int k = 0; k < EW_VEC; ++k) {
       if (t == 0 && k < 2) s = k == 0 ? v[0][1] * v[0][1] : fmaf(v[0][0], v[0][0], s);
       else s = fmaf(v[t][k], v[t][k], s);
+    }
+  }
+  if (full < numel && full / MUON_CHUNK_ELEMS == chunk && full / EW_VEC % EW_THREADS == tid) {
+    for (long i = full; i < numel; ++i) {
+      float x = Elem<DT>::load1(base, i);
+      if (cast_first) x = bf2f(f2bf(x));
+      s = fmaf(x, x, s);
     }
   }
   return s;
