@@ -3,7 +3,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "launch_rules.h"
+
 namespace archscale {
+
+constexpr int BK = 64;   // elements per k-tile
 
 // MODE_SYRKT: as MODE_SYRK, but P = Q is given K-major ([K][M] row-major, ldp = leading dimension; P == Q required)
 enum { MODE_SYRK = 0, MODE_SYRK2 = 1, MODE_BX = 2, MODE_SYRKT = 3 };
@@ -77,6 +81,30 @@ static_assert(sizeof(GroupedGemmParams) <= 4096, "kernel arguments are limited t
 
 // number of block tiles of one problem
 long ns_gemm_tiles(int mode, const GemmParams& p);
+
+// Whether the tiles of a launch follow one another in a block (ns_gemm_stream_kernel): X' = B X in whole tiles of 256, nothing that needs the
+// other kernel's bounds checks or unaligned stores, no rows of the caller's that lie STREAM_MAX_LD elements apart or more (its stores have one
+// base per tile and signed 32-bit offsets of up to 510 bytes per element of that distance), and enough of them (stream_of_tiles).
+constexpr int STREAM_MAX_LD = 1 << 22;
+inline bool stream_takes(int tile, int mode, bool split, bool final_, const GroupedGemmParams& gp, int units) {
+  if (tile != 256 || mode != MODE_BX || split || gp.quarter) return false;
+  int longest = 0;
+  for (int i = 0; i < gp.n_groups; ++i) {
+    const GemmParams& g = gp.g[i];
+    longest = g.K > longest ? g.K : longest;
+    if (g.t_first || g.K < 4 * BK || g.ldp != g.ldq || (g.scale && !g.E)) return false;
+    if (!final_) {
+      if (!g.Ct || g.C) return false;
+    } else {
+      const bool rows = g.C != nullptr;
+      const long stride = rows ? g.strideC : g.strideCt;
+      if (g.E || rows == (g.Ct != nullptr) || g.m_valid != g.tilesM * 256 || g.n_valid != g.tilesN * 256) return false;
+      const int ld = rows ? g.ldc : g.ldct;
+      if (((uintptr_t)(rows ? g.C : g.Ct) & 15) || ld % 8 || ld >= STREAM_MAX_LD || (g.batch > 1 && stride % 8)) return false;
+    }
+  }
+  return stream_of_tiles(units, gp.tile_start[gp.n_groups], longest);
+}
 
 // tile: side of the block tile, 256, 128, 64 or 32 (four waves each; 64 without the hi+lo pair, 32 for MODE_SYRKT alone)
 // f16: 0 = the workspace matrices of the launch are bfloat16; 1 = IEEE half (see GemmParams::out_shift), not with split;

@@ -45,8 +45,7 @@ typedef u32x4 u32x4_any __attribute__((aligned(2)));   // a result of the caller
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
 
-static constexpr int BK = 64;           // bf16 elements per k-tile: 128 bytes = 8 chunks of 16 B
-static constexpr int ROW_BYTES = BK * 2;
+static constexpr int ROW_BYTES = BK * 2;   // 8 chunks of 16 B
 
 __device__ __forceinline__ uint16_t bf16_bits(float f) {
   __bf16 h = (__bf16)f;  // round to nearest even
@@ -1359,27 +1358,6 @@ static hipError_t launch_sequence(int mode, const GroupedGemmParams& p, hipStrea
   return hipErrorInvalidValue;
 }
 
-// Whether the tiles of an X' = B X launch may follow one another in a block: whole tiles of 256, nothing that needs the other kernel's
-// bounds checks or unaligned stores, and enough of them (stream_of_tiles).
-static bool stream_takes(const GroupedGemmParams& gp, bool final_, int units) {
-  if (gp.quarter) return false;
-  int longest = 0;
-  for (int i = 0; i < gp.n_groups; ++i) {
-    const GemmParams& g = gp.g[i];
-    longest = g.K > longest ? g.K : longest;
-    if (g.t_first || g.K < 4 * BK || g.ldp != g.ldq || (g.scale && !g.E)) return false;
-    if (!final_) {
-      if (!g.Ct || g.C) return false;
-    } else {
-      const bool rows = g.C != nullptr;
-      const long stride = rows ? g.strideC : g.strideCt;
-      if (g.E || rows == (g.Ct != nullptr) || g.m_valid != g.tilesM * 256 || g.n_valid != g.tilesN * 256) return false;
-      if (((uintptr_t)(rows ? g.C : g.Ct) & 15) || (rows ? g.ldc : g.ldct) % 8 || (g.batch > 1 && stride % 8)) return false;
-    }
-  }
-  return stream_of_tiles(units, gp.total, longest);
-}
-
 template <bool FINAL, bool ADDEND, int F16>
 static hipError_t launch_stream_one(const GroupedGemmParams& gp, hipStream_t stream, int units) {
   constexpr int SMEM = (Config<CFG_256>::SP + Config<CFG_256>::SQ) * 256 * ROW_BYTES;
@@ -1474,7 +1452,7 @@ hipError_t launch_ns_gemm_grouped(int tile, int mode, bool split, bool final_, c
     if (f16 == 0) return launch_cfg<CFG, 0>(mode, split, final_, gp, stream);
     return hipErrorInvalidValue;
   };
-  if (tile == 256 && mode == MODE_BX && !split && stream_takes(gp, final_, units)) return launch_stream(gp, final_, f16, stream, units);
+  if (stream_takes(tile, mode, split, final_, gp, units)) return launch_stream(gp, final_, f16, stream, units);
   if (tile == 256) return by_storage(std::integral_constant<int, CFG_256>{});
   if (tile == 128 && deep) return by_storage(std::integral_constant<int, CFG_128_DEEP>{});
   if (tile == 128) return by_storage(std::integral_constant<int, CFG_128>{});

@@ -50,3 +50,29 @@ def test_results_that_are_not_aligned(gpu_device):
     ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[flat[1:1 + want.numel()].view(want.shape)])
     assert torch.equal(flat[1:1 + want.numel()].view(want.shape), want)
     assert bool((flat[:1] == 7.0).all()) and bool((flat[1 + want.numel():] == 7.0).all())
+
+
+# launches that take the form but for their result: extents of whole tiles inside a wider matrix (which they keep), and padded ones; wide and tall
+@pytest.mark.parametrize("batch,m,n", [(160, 256, 2048), (52, 512, 1024), (160, 250, 2000), (52, 500, 1000)])
+@pytest.mark.parametrize("tall", [False, True])
+@pytest.mark.parametrize("left,right", [(8, 24), (3, 0)])
+def test_results_inside_wider_matrices(gpu_device, batch, m, n, tall, left, right):
+    """Results whose rows lie further apart than they are long: the bits of contiguous ones, nothing beside them is touched."""
+    import archscale_amd.optim.newton_schulz_hip as ns
+    from archscale_amd import _lib
+    rows, cols = (n, m) if tall else (m, n)
+    g = torch.Generator(device=gpu_device).manual_seed(batch + m + n)
+    x = (torch.randn(batch, rows, cols, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
+    want = torch.empty_like(x)
+    ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[want])
+    wide = torch.full((batch, rows, left + cols + right), 7.0, dtype=torch.bfloat16, device=gpu_device)
+    view = wide[:, :, left:left + cols]
+    q = (_lib.NsProblem * 1)()
+    q[0].in_ptr, q[0].out_ptr, q[0].in_dtype, q[0].in_ld, q[0].out_ld = x.data_ptr(), view.data_ptr(), _lib.dtype_code(x.dtype), cols, wide.shape[2]
+    q[0].in_batch_stride, q[0].out_batch_stride, q[0].batch, q[0].rows, q[0].cols = rows * cols, rows * wide.shape[2], batch, rows, cols
+    L = _lib.lib()
+    ws = _lib.workspace(gpu_device, L.muon_ns_grouped_workspace_bytes(q, 1, _lib.PREC_BF16))
+    _lib.check(L.muon_ns_grouped(q, 1, _lib.abc_array(ns.QUINTIC_SCHEDULE), 5, 1e-7, 0, _lib.PREC_BF16, _lib.NS_CAST_INPUT_FIRST, ws.data_ptr(),
+                                 ws.numel(), _lib.current_stream_ptr(gpu_device)), "muon_ns_grouped")
+    assert torch.equal(view, want)
+    assert bool((wide[:, :, :left] == 7.0).all()) and bool((wide[:, :, left + cols:] == 7.0).all())
