@@ -723,9 +723,9 @@ __device__ __forceinline__ void post_apply_range(const PostItem& it, long begin,
 __global__ void __launch_bounds__(EW_THREADS)
 post_apply_kernel(const PostItem* __restrict__ items, const int32_t* __restrict__ prefix, int n_items,
                   float lr, float lrwd, int cautious, const float2* __restrict__ coef,
-                  const ScalarHyper* __restrict__ hdev) {
+                  const ScalarHyper* __restrict__ hdev, int first_chunk) {
   if (hdev) { lr = hdev->lr; lrwd = hdev->lr_wd; cautious = hdev->cautious; }
-  const int chunk = blockIdx.x / EW_TRIPS, trip = blockIdx.x % EW_TRIPS;
+  const int chunk = first_chunk + (int)(blockIdx.x / EW_TRIPS), trip = blockIdx.x % EW_TRIPS;
   const int ii = find_item(prefix, n_items, chunk);
   const PostItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS + trip * (EW_THREADS * EW_VEC);
@@ -736,12 +736,18 @@ post_apply_kernel(const PostItem* __restrict__ items, const int32_t* __restrict_
   else post_apply_range<DT_F32>(it, begin, end, lrwd, cautious, alpha, beta);
 }
 
+// A launch holds fewer than 2^32 threads: more chunks than APPLY_MAX_CHUNKS (2^35 elements) take several.
+constexpr int APPLY_MAX_CHUNKS = 0xffffffffu / (EW_THREADS * EW_TRIPS);
 static hipError_t launch_post_apply(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks, float lr, float lrwd,
                                     int cautious, const float2* coef, hipStream_t stream, const ScalarHyper* hdev) {
-  if (total_chunks > 0x7fffffff / EW_TRIPS) return hipErrorInvalidValue;   // (2^42 elements)
-  hipLaunchKernelGGL(post_apply_kernel, dim3(total_chunks * EW_TRIPS), dim3(EW_THREADS), 0, stream, items, prefix, n_items, lr, lrwd,
-                     cautious, coef, hdev);
-  return hipGetLastError();
+  for (int first = 0, count; first < total_chunks; first += count) {
+    count = total_chunks - first < APPLY_MAX_CHUNKS ? total_chunks - first : APPLY_MAX_CHUNKS;
+    hipLaunchKernelGGL(post_apply_kernel, dim3(count * EW_TRIPS), dim3(EW_THREADS), 0, stream, items, prefix, n_items, lr, lrwd, cautious,
+                       coef, hdev, first);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_post_plain(const PostItem* items, const int32_t* prefix, int n_items, int total_chunks,
