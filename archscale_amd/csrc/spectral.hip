@@ -561,46 +561,49 @@ __device__ __forceinline__ int find_item_(const int32_t* __restrict__ prefix, in
   return lo;
 }
 
-// Runs of eight elements in row-major order, 16-byte accesses wherever they start.  Blocks whose rows follow one another (most: whole
-// matrices and groups of their rows) are one row.  Elsewhere a run that crosses the end of a row, and at the end of a block a run of fewer than
-// eight, is taken one by one.  fp32, 17 million elements in widths of 983 and 2257: 47.7 us element by element, 34.7 so.
+// eight elements from any place on (plain accesses: the update was written by the launch before)
+template <int WD>
+__device__ __forceinline__ void ball_load8(const void* p, long i, float (&v)[8]) {
+  if constexpr (WD == DT_BF16) {
+    const u32x4 r = *(const u32x4_any*)((const uint16_t*)p + i);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(r[k] & 0xffff); v[2 * k + 1] = bf2f(r[k] >> 16); }
+  } else {
+    const f32x4 a = *(const f32x4_any*)((const float*)p + i), b = *(const f32x4_any*)((const float*)p + i + 4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { v[k] = a[k]; v[4 + k] = b[k]; }
+  }
+}
+
+// Bound by memory.  Runs of eight elements, 16-byte accesses wherever they start, where rows follow one another (most: whole matrices and
+// groups of their rows, one row as far as this goes) or are whole runs; one element per thread where a run would cross the end of a row
+// inside a wider matrix.  us for 17.8 million elements, bfloat16 / fp32: dense, any width 17.2 / 27.5 (element by element 31.2 / 36.9, with
+// accesses past the caches 19.5 / 33.8); width 1000 in 1005 18.1 / 28.1 (30.4 / 37.3 element by element); width 1001 in 1006 29.6 / 37.4
+// (45.0 / 51.8 in runs that are split at the end of a row, 57 / 97 and 180 / 321 for a width of 3).
 template <int WD>
 __device__ __forceinline__ void ball_range(const muon_ball_item& it, long begin, long end, float fw, float fp) {
   const bool dense = it.ld_w == it.cols && it.ld_phi == it.cols;
-  const long cols = dense ? (long)it.rows * it.cols : it.cols, ld_w = dense ? cols : it.ld_w, ld_phi = dense ? cols : it.ld_phi;
-  float x[EW_TRIPS][8], u[EW_TRIPS][8];
-  long at_w[EW_TRIPS], c[EW_TRIPS];
-  // element k of a run: past the end of its row it is in the next (a run that ends in a row of fewer than eight: in a later one)
-  auto place = [&](long k, long first, long col, long ld) {
-    while (col + k >= cols) { k -= cols; first += ld; }
-    return first + k;
-  };
+  if (dense || it.cols % EW_VEC == 0) {
+    for (long i = begin + (long)threadIdx.x * EW_VEC; i < end; i += EW_THREADS * EW_VEC) {
+      const long r = dense ? 0 : i / it.cols, c = dense ? i : i - r * it.cols;
+      const long w = r * it.ld_w + c, phi = r * it.ld_phi + c;
+      if (i + EW_VEC <= end) {
+        float x[8], u[8];
+        ball_load8<DT_BF16>(it.phi, phi, u);
+        ball_load8<WD>(it.w, w, x);
 #pragma unroll
-  for (int t = 0; t < EW_TRIPS; ++t) {   // all loads before the first store (they may alias as far as the compiler knows)
-    const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-    if (i < end) {
-      const long r = dense ? 0 : ((long)it.rows * it.cols <= 0x7fffffffL ? (long)((uint32_t)i / (uint32_t)it.cols) : i / it.cols);
-      c[t] = i - r * cols;
-      at_w[t] = r * ld_w + c[t];
-      const long at_u = r * ld_phi + c[t];
-      if (i + EW_VEC <= end && c[t] + EW_VEC <= cols) {
-        Elem<WD>::load8(it.w, at_w[t], x[t]);
-        Elem<DT_BF16>::load8(it.phi, at_u, u[t]);
-      } else {
-        for (int k = 0; k < EW_VEC && i + k < end; ++k) {
-          const long a = place(k, at_w[t], c[t], ld_w);
-          Elem<WD>::store1(it.w, a, fw * Elem<WD>::load1(it.w, a) - fp * Elem<DT_BF16>::load1(it.phi, place(k, at_u, c[t], ld_phi)));
-        }
+        for (int k = 0; k < 8; ++k) x[k] = fw * x[k] - fp * u[k];
+        Elem<WD>::keep8(it.w, w, x);
+      } else {   // the last elements of a dense block
+        for (long e = i; e < end; ++e)
+          Elem<WD>::store1(it.w, e, fw * Elem<WD>::load1(it.w, e) - fp * Elem<DT_BF16>::load1(it.phi, e));
       }
     }
-  }
-#pragma unroll
-  for (int t = 0; t < EW_TRIPS; ++t) {
-    const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
-    if (i + EW_VEC <= end && c[t] + EW_VEC <= cols) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) x[t][k] = fw * x[t][k] - fp * u[t][k];
-      Elem<WD>::store8(it.w, at_w[t], x[t]);
+  } else {
+    for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
+      const long r = i / it.cols, c = i - r * it.cols;
+      const float u = Elem<DT_BF16>::load1(it.phi, r * it.ld_phi + c);
+      Elem<WD>::store1(it.w, r * it.ld_w + c, fw * Elem<WD>::load1(it.w, r * it.ld_w + c) - fp * u);
     }
   }
 }

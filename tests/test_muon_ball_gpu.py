@@ -79,7 +79,7 @@ def test_spectral_norm_batches_dtypes_strides_and_zero(gpu_device):
 def test_ball_apply_strided_blocks(gpu_device, w_dt, mode):
     from archscale_amd import _lib
     g = torch.Generator().manual_seed(3)
-    # blocks of two "parameters": whole matrix, a column block (ld > cols), a row block, an odd-sized block (scalar path)
+    # blocks of two "parameters": whole matrix, a column block (ld > cols), a row block, odd-sized blocks
     P1 = (torch.randn(96, 160, generator=g) * 0.05).to(w_dt)
     P2 = (torch.randn(37, 53, generator=g) * 0.05).to(w_dt)
     F1 = torch.randn(96, 160, generator=g).to(torch.bfloat16)
