@@ -29,10 +29,6 @@ __device__ __forceinline__ int find_item(const int32_t* __restrict__ prefix, int
   return __builtin_amdgcn_readfirstlane(lo + __popcll(__ballot(owns)) - 1);
 }
 
-// The second of two passes over the same arrays starts where the first one ended: what that read and wrote last is still in the
-// memory-side cache (256 MB), what it read first has left it.
-__device__ __forceinline__ int backwards(int block) { return (int)gridDim.x - 1 - block; }
-
 // end of the whole runs of eight elements of [begin, end); at most seven elements are left, at the end of an item
 __device__ __forceinline__ long whole_runs(long begin, long end) { return begin + (end - begin) / EW_VEC * EW_VEC; }
 
@@ -645,7 +641,7 @@ post_reduce_kernel(const PostItem* __restrict__ items, const int32_t* __restrict
                    const ScalarHyper* __restrict__ hdev) {
   __shared__ float red[12];
   if (hdev) { lrwd = hdev->lr_wd; cautious = hdev->cautious; }   // hyper-parameters from device memory
-  const int chunk = backwards(blockIdx.x);
+  const int chunk = blockIdx.x;
   const int ii = find_item(prefix, n_items, chunk);
   const PostItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
@@ -900,7 +896,7 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
                      const ScalarHyper* __restrict__ hdev) {
   __shared__ float red[12];
   if (hdev) h = *hdev;   // hyper-parameters from device memory
-  const int chunk = PHASE == 2 ? backwards(blockIdx.x) : (int)blockIdx.x;
+  const int chunk = blockIdx.x;
   const int ii = find_item(prefix, n_items, chunk);
   const ScalarItem it = items[ii];
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
