@@ -561,7 +561,37 @@ __device__ __forceinline__ int find_item_(const int32_t* __restrict__ prefix, in
   return lo;
 }
 
-// eight elements from any place on (plain accesses: the update was written by the launch before)
+// Bound by memory.  Blocks whose rows follow one another (most: whole matrices and groups of their rows) are one row: runs of eight elements in
+// 16-byte accesses past the caches, wherever they start, all loads of a chunk before the first store (they may alias as far as the
+// compiler knows).  us for 268 million elements, bfloat16 / fp32: 250 / 486 at any width, 300 / 482 through the caches run by run, 417 / 535
+// element by element; 17.8 million that are not in the caches 20 / 35, 24 / 38, 46 / 53.  (Repeated calls that find everything in
+// the caches: 17.8 million 19.5 / 33.8, 17.2 / 27.5 through them; steps do not.)
+template <int WD>
+__device__ __forceinline__ void ball_dense(const muon_ball_item& it, long begin, long end, float fw, float fp) {
+  float x[EW_TRIPS][8], u[EW_TRIPS][8];
+#pragma unroll
+  for (int t = 0; t < EW_TRIPS; ++t) {
+    const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
+    if (i + EW_VEC <= end) {
+      Elem<WD>::load8(it.w, i, x[t]);
+      Elem<DT_BF16>::load8(it.phi, i, u[t]);
+    } else {   // the last elements of a block
+      for (long e = i; e < end; ++e)
+        Elem<WD>::store1(it.w, e, fw * Elem<WD>::load1(it.w, e) - fp * Elem<DT_BF16>::load1(it.phi, e));
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < EW_TRIPS; ++t) {
+    const long i = begin + ((long)t * EW_THREADS + threadIdx.x) * EW_VEC;
+    if (i + EW_VEC <= end) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[t][k] = fw * x[t][k] - fp * u[t][k];
+      Elem<WD>::store8(it.w, i, x[t]);
+    }
+  }
+}
+
+// eight elements from any place on, through the caches
 template <int WD>
 __device__ __forceinline__ void ball_load8(const void* p, long i, float (&v)[8]) {
   if constexpr (WD == DT_BF16) {
@@ -575,29 +605,21 @@ __device__ __forceinline__ void ball_load8(const void* p, long i, float (&v)[8])
   }
 }
 
-// Bound by memory.  Runs of eight elements, 16-byte accesses wherever they start, where rows follow one another (most: whole matrices and
-// groups of their rows, one row as far as this goes) or are whole runs; one element per thread where a run would cross the end of a row
-// inside a wider matrix.  us for 17.8 million elements, bfloat16 / fp32: dense, any width 17.2 / 27.5 (element by element 31.2 / 36.9, with
-// accesses past the caches 19.5 / 33.8); width 1000 in 1005 18.1 / 28.1 (30.4 / 37.3 element by element); width 1001 in 1006 29.6 / 37.4
-// (45.0 / 51.8 in runs that are split at the end of a row, 57 / 97 and 180 / 321 for a width of 3).
+// Blocks inside wider matrices, whose rows share lines with their neighbours: through the caches, runs of eight where rows are whole runs and
+// one element per thread where a run would cross the end of a row.  us for 17.8 million elements, so / as dense blocks with the runs split
+// at the ends of rows, bfloat16 and fp32: 24 columns in 32 32 / 34 and 53 / 74, 9 in 17 62 / 136 and 86 / 240, 1001 in 1009 46 / 46 and 58 / 54
+// (30 / 45 and 37 / 52 where the caches hold everything).
 template <int WD>
-__device__ __forceinline__ void ball_range(const muon_ball_item& it, long begin, long end, float fw, float fp) {
-  const bool dense = it.ld_w == it.cols && it.ld_phi == it.cols;
-  if (dense || it.cols % EW_VEC == 0) {
+__device__ __forceinline__ void ball_strided(const muon_ball_item& it, long begin, long end, float fw, float fp) {
+  if (it.cols % EW_VEC == 0) {
     for (long i = begin + (long)threadIdx.x * EW_VEC; i < end; i += EW_THREADS * EW_VEC) {
-      const long r = dense ? 0 : i / it.cols, c = dense ? i : i - r * it.cols;
-      const long w = r * it.ld_w + c, phi = r * it.ld_phi + c;
-      if (i + EW_VEC <= end) {
-        float x[8], u[8];
-        ball_load8<DT_BF16>(it.phi, phi, u);
-        ball_load8<WD>(it.w, w, x);
+      const long r = i / it.cols, c = i - r * it.cols, w = r * it.ld_w + c;
+      float x[8], u[8];
+      ball_load8<DT_BF16>(it.phi, r * it.ld_phi + c, u);
+      ball_load8<WD>(it.w, w, x);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) x[k] = fw * x[k] - fp * u[k];
-        Elem<WD>::keep8(it.w, w, x);
-      } else {   // the last elements of a dense block
-        for (long e = i; e < end; ++e)
-          Elem<WD>::store1(it.w, e, fw * Elem<WD>::load1(it.w, e) - fp * Elem<DT_BF16>::load1(it.phi, e));
-      }
+      for (int k = 0; k < 8; ++k) x[k] = fw * x[k] - fp * u[k];
+      Elem<WD>::keep8(it.w, w, x);
     }
   } else {
     for (long i = begin + threadIdx.x; i < end; i += EW_THREADS) {
@@ -606,6 +628,12 @@ __device__ __forceinline__ void ball_range(const muon_ball_item& it, long begin,
       Elem<WD>::store1(it.w, r * it.ld_w + c, fw * Elem<WD>::load1(it.w, r * it.ld_w + c) - fp * u);
     }
   }
+}
+
+template <int WD>
+__device__ __forceinline__ void ball_range(const muon_ball_item& it, long begin, long end, float fw, float fp) {
+  if (it.ld_w == it.cols && it.ld_phi == it.cols) ball_dense<WD>(it, begin, end, fw, fp);
+  else ball_strided<WD>(it, begin, end, fw, fp);
 }
 
 }  // namespace
