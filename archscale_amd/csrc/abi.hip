@@ -219,7 +219,6 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
   if (env_switches().quarter)
     cut = mode == MODE_SYRKT && !split && fine_tiles(units, tile, total, longest) ? LaunchSplit{0, 0, total}
                                                                                    : launch_split(units, tile, split, total, all, longest);
-  if (env_switches().quarter && cut.whole == total && one_round_of_quadrants(units, tile, split, total)) cut = {0, total, 0};
   // a symmetric product that the rules hand to tiles of 128 as a whole: in the order of those tiles, without the empty lower quadrants
   if (mode != MODE_BX && tile == 256 && env_switches().quarter) {
     GroupedGemmParams q = gp;

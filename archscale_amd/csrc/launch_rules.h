@@ -37,10 +37,7 @@ struct LaunchSplit { int whole, quarters, sixteenths; };
 // (208 tiles of 2816 and 1024 k-values, X X^T of that EMA-Muon set) a product takes 56 us quartered, 66 as it is; at 0.625
 // (160 equal tiles, power iteration over 16 x 1024 x 2816) the call takes 259 against 250 us.
 //
-// Tiles of 128: up to QUARTER_MAX_128 are quartered (up to QUARTER_MAX_128_SHORT where no reduction is longer than 1024: what
-// a tile costs beside its k-tiles then weighs more).  One 512 x 2048 matrix 203 -> 133 us, 768 x 768 173 -> 118, 3001 x
-// 1023 286 -> 198, 1500 x 2000 (78 tiles) 268 -> 241; 136 tiles: the fp32 decoder of width 384 284 -> 262, but 2048 x 8192
-// 709 -> 747; 192 tiles: 3001 x 1023 198 -> 208.
+// Tiles of 128: quartered where two quadrants to a unit hold them all (one_round_of_quadrants).
 // The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
 // left beside whole rounds of either kind become sixteen tiles of 64 each, one block per unit at most.  The 136 triangle tiles of
 // a short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
@@ -48,19 +45,23 @@ struct LaunchSplit { int whole, quarters, sixteenths; };
 // symmetric products; one tile of 64 to a unit instead of one of 128 to a fourth of the units): 1024 x 3072 22.4 -> 13.1 us, 1024 x
 // 1024 11.6 -> 7.3, 512 x 2048 16.3 -> 9.6, 512 x 512 7.9 -> 5.5.
 constexpr int RULE_UNITS = 256;   // the device of the figures
-constexpr int QUARTER_MAX_TAIL = 128, QUARTER_MAX_128 = 100, QUARTER_MAX_128_SHORT = 140;
+constexpr int QUARTER_MAX_TAIL = 128;
 constexpr int SIXTEENTH_MAX = 16;
 constexpr double QUARTER_LOAD = 0.6;
+
+// Tiles of 128 whose quadrants find room in one round, two to a unit: quartered whatever their reductions.  us a call, as tiles of 128 / of 64:
+// one 512 x 2048 matrix 203 / 133, 3001 x 1023 286 / 198, 1500 x 2000 (78 tiles) 268 / 241, 3 x (1000 x 2000) (108) 252 / 243, 1700 x 3000 (105)
+// 368 / 340, 1900 x 1900 (120) 284 / 269, 12 x (500 x 4000) (120) 375 / 354, 6 x (700 x 1300) (126) 222 / 210, single products of 1792 x
+// 4096 27.9 / 25.2, 3 x (1000 x 960) 25.4 / 24.8.  With a second round they lose: 13 x (512 x 1000) (130) 198 / 212, 9 x (640 x 640) (135) 169 / 191,
+// 5 x (896 x 1024) (140) 225 / 260, a product of 1826 x 960 (136) 28.0 / 28.9, 2048 x 2048 (136) 288 / 342.
+inline bool one_round_of_quadrants(int units, int tile, bool pair, int total) { return tile == 128 && !pair && 2L * total <= units; }
 
 // total: tiles of the launch; all, longest: k-values of all its tiles and of the longest one; pair: products of a hi+lo pair
 // (there is no configuration of 64 for them)
 inline LaunchSplit launch_split(int units, int tile, bool pair, int total, double all, double longest) {
   auto scaled = [&](int tiles) { return (int)((long)tiles * units / RULE_UNITS); };
   const LaunchSplit as_is = {total, 0, 0};
-  if (tile == 128) {
-    const int most = scaled(longest > 1024.0 ? QUARTER_MAX_128 : QUARTER_MAX_128_SHORT);
-    return pair || total > most ? as_is : LaunchSplit{0, total, 0};
-  }
+  if (one_round_of_quadrants(units, tile, pair, total)) return {0, total, 0};
   if (tile != 256) return as_is;
   const int full = total / units * units, tail = total - full;
   if (tail == 0 || (full > 0 ? tail > scaled(QUARTER_MAX_TAIL) : all > QUARTER_LOAD * units * longest)) return as_is;
@@ -90,12 +91,6 @@ inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller
   if (cut.whole != total || total > units || longest > HALVED_MAX_K) return false;
   return longest <= HALVED_SHORT_K || (total >= HALVED_LEAST * units && total <= HALVED_MOST * units);
 }
-
-// Tiles of 128 beyond launch_split's lines whose quadrants still find room in one round, two to a unit: quartered whatever their reductions.
-// us a call, as tiles of 128 / of 64: 3 x (1000 x 2000) (108 tiles) 243 / 235, 1900 x 1900 (120) 282 / 262, 1800 x 2500 361 / 340, 12 x (500 x
-// 2000) 226 / 217, 6 x (700 x 1300) (126) 228 / 216, the fp32 decoder of width 384 (128, reductions of 384 and 1152) 252 / 237; with a second
-// round they lose: 13 x (512 x 1500) (130) 260 / 270, 2048 x 2048 (136) 288 / 342.
-inline bool one_round_of_quadrants(int units, int tile, bool pair, int total) { return tile == 128 && !pair && 2L * total <= units; }
 
 // Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 (`tiles` of one
 // matrix) with at most one block to a unit.  The cut fixes the order of the sums, so callers ask for RULE_UNITS units and one

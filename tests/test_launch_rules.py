@@ -48,10 +48,11 @@ def test_lines_on_256_units(rules):
         (256, 0, 145, 145e3, 1e3): (0, 145, 0),
         (256, 0, 160, 160e3, 1e3): (160, 0, 0),
         (256, 0, 208, 208 * 590.0, 1e3): (0, 208, 0),
-        (128, 0, 100, 1.0, 1088.0): (0, 100, 0),
-        (128, 0, 101, 1.0, 1088.0): (101, 0, 0),
-        (128, 0, 140, 1.0, 1024.0): (0, 140, 0),
-        (128, 0, 141, 1.0, 1024.0): (141, 0, 0),
+        # (one round of quadrants, two to a unit, whatever the reductions)
+        (128, 0, 128, 1.0, 1088.0): (0, 128, 0),
+        (128, 0, 129, 1.0, 1088.0): (129, 0, 0),
+        (128, 0, 128, 1.0, 256.0): (0, 128, 0),
+        (128, 0, 129, 1.0, 256.0): (129, 0, 0),
         (128, 1, 10, 1.0, 1024.0): (10, 0, 0),
     }
     got = rules([(256, *k, 1, 64) for k in want])
