@@ -221,18 +221,21 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
                                                                                    : launch_split(units, tile, split, total, all, longest);
   // a symmetric product that the rules hand to tiles of 128 as a whole: in the order of those tiles, without the empty lower quadrants
   if (mode != MODE_BX && tile == 256 && env_switches().quarter) {
-    GroupedGemmParams q = gp;
     long smaller = 0;
     bool whole_matrices = true;
     for (int i = 0; i < gp.n_groups; ++i) {
-      q.g[i].tilesM *= 2;
-      q.g[i].tilesN *= 2;
-      smaller += ns_gemm_tiles(mode, q.g[i]);
-      q.tile_start[i + 1] = (int)smaller;   // (not used where it does not fit: four times less than a round)
+      smaller += (long)gp.g[i].batch * sym_tiles(2 * gp.g[i].tilesM);
       whole_matrices = whole_matrices && !gp.g[i].t_count;
     }
-    if (whole_matrices && halved_tiles(units, tile, split, total, smaller, longest, cut))
+    if (whole_matrices && halved_tiles(units, tile, split, total, smaller, longest, cut)) {
+      GroupedGemmParams q = gp;
+      for (int i = 0; i < gp.n_groups; ++i) {
+        q.g[i].tilesM *= 2;
+        q.g[i].tilesN *= 2;
+        q.tile_start[i + 1] = q.tile_start[i] + (int)ns_gemm_tiles(mode, q.g[i]);
+      }
       return launch_rounds(128, mode, split, final_, q, stream, units, work, f16);
+    }
   }
   if (cut.whole == total) return launch(tile, gp, 1.0);
   // tiles [begin, end) of the launch as (2^level)^2 tiles each of the configuration that is `level` smaller (level 0: as they are)

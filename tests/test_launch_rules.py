@@ -201,15 +201,29 @@ int main() {
         (256, 0, 140, 504, 140 * 4096.0, 4096.0): 1,     # quarters and sixteenths, two smaller tiles to a unit hold it
         (256, 0, 144, 544, 144 * 4096.0, 4096.0): 0,     # they do not
         (256, 0, 208, 744, 208 * 590.0, 1000.0): 1,
-        (256, 0, 256, 832, 256 * 768.0, 768.0): 1,       # a full round, short reductions
-        (256, 0, 257, 840, 257 * 768.0, 768.0): 0,
+        # the second round of smaller tiles: up to half of it; not where it is nearly empty and the reductions are long
+        (256, 0, 216, 768, 216 * 768.0, 768.0): 1,
+        (256, 0, 216, 769, 216 * 768.0, 768.0): 0,
+        (256, 0, 216, 768, 216 * 1024.0, 1024.0): 1,
+        (256, 0, 216, 769, 216 * 1024.0, 1024.0): 0,
+        (256, 0, 170, 597, 170 * 832.0, 832.0): 0,
+        (256, 0, 170, 598, 170 * 832.0, 832.0): 1,
+        (256, 0, 170, 570, 170 * 768.0, 768.0): 1,
         (256, 0, 160, 576, 160 * 1024.0, 1024.0): 0,
-        (256, 0, 180, 648, 180 * 1024.0, 1024.0): 1,
-        (256, 0, 217, 780, 217 * 1024.0, 1024.0): 1,
-        (256, 0, 218, 784, 218 * 1024.0, 1024.0): 0,
-        (256, 0, 217, 780, 217 * 1088.0, 1088.0): 0,     # longer reductions stay
-        (256, 1, 217, 780, 217 * 1024.0, 1024.0): 0,     # hi+lo pairs stay
-        (128, 0, 217, 780, 217 * 1024.0, 1024.0): 0,
+        # short reductions whatever it holds, up to a full round of tiles of 256
+        (256, 0, 256, 968, 256 * 256.0, 256.0): 1,
+        (256, 0, 257, 972, 257 * 256.0, 256.0): 0,
+        (256, 0, 256, 968, 256 * 320.0, 320.0): 0,
+        # matrices of one tile a side (three smaller tiles for one)
+        (256, 0, 181, 543, 181 * 1024.0, 1024.0): 1,
+        (256, 0, 182, 546, 182 * 1024.0, 1024.0): 0,
+        (256, 0, 202, 606, 202 * 512.0, 512.0): 1,
+        (256, 0, 203, 609, 203 * 512.0, 512.0): 0,
+        (256, 0, 256, 768, 256 * 256.0, 256.0): 1,
+        (256, 0, 256, 768, 256 * 768.0, 768.0): 0,
+        (256, 0, 208, 744, 208 * 1088.0, 1088.0): 0,     # longer reductions stay
+        (256, 1, 208, 744, 208 * 1024.0, 1024.0): 0,     # hi+lo pairs stay
+        (128, 0, 208, 744, 208 * 1024.0, 1024.0): 0,
     }
     text = "".join("%d %d %d %d %.17g %.17g\n" % w for w in want)
     out = subprocess.run([str(tmp_path / "halved")], input=text, capture_output=True, text=True, check=True).stdout.split()
