@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include "elementwise.h"
+#include "launch_rules.h"
 #include "streaming.h"
 
 namespace archscale {
@@ -902,7 +903,11 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
   const long begin = (long)(chunk - prefix[ii]) * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < it.numel ? begin + MUON_CHUNK_ELEMS : it.numel;
   constexpr bool has_v = ALGO == ALGO_ADAMW;
-  const long full = whole_runs(begin, end);
+  bool runs = true;
+  if (PHASE == 0)
+    runs = update_in_runs(has_v, it.w_dtype == DT_F32, it.g_dtype == DT_F32, it.m_dtype == DT_F32, has_v && it.v_dtype == DT_F32,
+                          it.numel % EW_VEC == 0 && aligned16(it.w) && aligned16(it.g) && aligned16(it.m) && (!has_v || aligned16(it.v)));
+  const long full = runs ? whole_runs(begin, end) : begin;
   float alpha = 1.f, beta = 0.f;
   if (PHASE == 2) { const float2 c = coef[ii]; alpha = c.x; beta = c.y; }
   const Direction dir = direction_of(h, PHASE != 0);
@@ -921,7 +926,7 @@ scalar_update_kernel(const ScalarItem* __restrict__ items, const int32_t* __rest
       scalar_range<ALGO, PHASE>(it, begin, full, h, dir, lr1, alpha, beta, s, OneDtype<DT_F32>{});
     else scalar_range<ALGO, PHASE>(it, begin, full, h, dir, lr1, alpha, beta, s, MixedDtypes{});
   }
-  if (full < end) {   // fewer than eight elements
+  if (full < end) {   // fewer than eight elements, or all of them
     for (long i = full + threadIdx.x; i < end; i += EW_THREADS) {
       float x = load1_rt(it.w, it.w_dtype, i), m = load1_rt(it.m, it.m_dtype, i);
       float g = PHASE != 2 ? load1_rt(it.g, it.g_dtype, i) : 0.f;

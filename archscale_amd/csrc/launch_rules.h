@@ -162,6 +162,16 @@ inline bool deep_pipeline(int units, int tile, int blocks, int shortest_k) {
   return tile == 128 && blocks <= units && shortest_k >= 1024;
 }
 
+// Plain AdamW and Lion, by which of their arrays are in fp32 (weights, gradient, momentum, variance): in runs of eight elements, or one element
+// per thread where the number of elements is no multiple of eight or an array is not 16-byte aligned and most accesses are fp32 (a run is
+// then two accesses per lane that share lines with the neighbours').  us, in runs / element by element: all fp32, 34117 x 1641 twice, AdamW 638 /
+// 614, Lion 453 / 426; 15916 x 1335 twice 245 / 235 and 174 / 170; 21.2 million elements, AdamW: state alone in fp32 99 / 91, all but the gradient
+// 119 / 128, all but the weights 107 / 123, all in bfloat16 59 / 100; Lion: weights and momentum in fp32 80 / 63, gradient and momentum 67 / 62,
+// momentum alone 59 / 73, all in bfloat16 40 / 74.
+constexpr bool update_in_runs(bool adamw, bool w, bool g, bool m, bool v, bool whole_and_aligned) {
+  return whole_and_aligned || !(adamw ? m && v && w == g : w + g + m >= 2);
+}
+
 // Blocks that sum the squares of one matrix of the power iteration that is read in place and needs no row sums (a tall one), each
 // eight 16-byte runs per thread at a time: as many as the matrix has loads for, whatever its short side (`strips`, which the start
 // vector is written by), up to two rounds of the chip, which keep the memory busy.

@@ -81,6 +81,8 @@ template <> struct Elem<DT_F32> {
   static __device__ __forceinline__ float round(float v) { return v; }
 };
 
+__device__ __forceinline__ bool aligned16(const void* p) { return (((uintptr_t)p) & 15) == 0; }
+
 // ordered block reduction of up to 3 values; result valid in thread 0
 template <int N>
 __device__ __forceinline__ void block_reduce(float (&v)[N], float* smem /* N * 4 floats */) {

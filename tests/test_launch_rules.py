@@ -251,3 +251,22 @@ int main() { int u, t, p, n; while (scanf("%d %d %d %d", &u, &t, &p, &n) == 4) p
     text = "".join("%d %d %d %d\n" % w for w in want)
     out = subprocess.run([str(tmp_path / "round")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in out] == list(want.values())
+
+
+def test_which_plain_updates_go_in_runs_of_eight(tmp_path):
+    """(AdamW, weights, gradient, momentum, variance in fp32, whole runs at aligned places) -> in runs, or element by element."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "runs.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() {
+  int a, w, g, m, v, o;
+  while (scanf("%d %d %d %d %d %d", &a, &w, &g, &m, &v, &o) == 6) printf("%d\n", (int)archscale::update_in_runs(a, w, g, m, v, o));
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "runs.cpp"), "-o", str(tmp_path / "runs")], check=True)
+    by_element = {(1, 1, 1, 1, 1, 0), (1, 0, 0, 1, 1, 0), (0, 1, 1, 1, 0, 0), (0, 1, 0, 1, 0, 0), (0, 0, 1, 1, 0, 0), (0, 1, 1, 0, 0, 0)}
+    every = [tuple(i >> k & 1 for k in range(6)) for i in range(64) if i & 1 or not i & 16]
+    text = "".join("%d %d %d %d %d %d\n" % w for w in every)
+    out = subprocess.run([str(tmp_path / "runs")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert {w for w, o in zip(every, out) if o == "0"} == by_element and len(out) == 48
