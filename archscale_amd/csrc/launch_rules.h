@@ -172,6 +172,16 @@ constexpr bool update_in_runs(bool adamw, bool w, bool g, bool m, bool v, bool w
   return whole_and_aligned || !(adamw ? m && v && w == g : w + g + m >= 2);
 }
 
+// Whether the sum of squares of a matrix goes over its elements in runs of eight (thread_sumsq_dense): rows that follow one another, and whole
+// runs or more than one chunk of `chunk` elements, whose blocks then load all they have at once.  An odd matrix of one chunk is over sooner one
+// element per thread, whole small calls in bfloat16 / fp32, in runs / so: 8 x (67 x 33) 22.0 / 19.8 and 21.0 / 19.5 us, 16 x (101 x 51) 21.3 / 19.4 and
+// 20.2 / 19.3, 3 x (61 x 95) 21.7 / 20.7 and 20.8 / 20.1; of two chunks and more 95 x 121 34.9 / 34.3 and 34.3 / 34.1 (before / in runs), 127 x 381 70.1 /
+// 62.3 and 68.9 / 62.1.
+constexpr bool sums_in_runs(int rows, int cols, int ld, int chunk) {
+  const long n = (long)rows * cols;
+  return ld == cols && (n % 8 == 0 || n > chunk);
+}
+
 // Blocks that sum the squares of one matrix of the power iteration that is read in place and needs no row sums (a tall one), each
 // eight 16-byte runs per thread at a time: as many as the matrix has loads for, whatever its short side (`strips`, which the start
 // vector is written by), up to two rounds of the chip, which keep the memory busy.

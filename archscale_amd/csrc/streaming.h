@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "elementwise.h"
+#include "launch_rules.h"
 
 namespace archscale {
 
@@ -107,7 +108,7 @@ __device__ __forceinline__ void block_reduce(float (&v)[N], float* smem /* N * 4
 // consecutive elements in row-major order; 0 for a chunk past the end).  Whoever forms the norm of a matrix adds in this order.
 // Dense matrices (dense_sumsq_ok) load a chunk whole before the first sum; the first elements of the matrix stand in past its
 // end and are not counted; the elements after the last whole run join at the end.
-__device__ __forceinline__ bool dense_sumsq_ok(int rows, int cols, int ld) { return ld == cols && (long)rows * cols >= EW_VEC; }
+__device__ __forceinline__ bool dense_sumsq_ok(int rows, int cols, int ld) { return sums_in_runs(rows, cols, ld, MUON_CHUNK_ELEMS); }
 template <int DT>
 __device__ __forceinline__ float thread_sumsq_dense(const char* base, long numel, int chunk, int tid, bool cast_first) {
   const long first = (long)chunk * MUON_CHUNK_ELEMS + (long)tid * EW_VEC, full = numel / EW_VEC * EW_VEC;
@@ -143,6 +144,15 @@ __device__ __forceinline__ float thread_sumsq_strided(const char* base, int rows
   const long numel = (long)rows * cols, begin = (long)chunk * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < numel ? begin + MUON_CHUNK_ELEMS : numel;
   float s = 0.f;
+  if (ld == cols) {   // nothing to divide, eight loads in flight
+#pragma unroll 8
+    for (long i = begin + tid; i < end; i += EW_THREADS) {
+      float x = Elem<DT>::load1(base, i);
+      if (cast_first) x = bf2f(f2bf(x));
+      s = fmaf(x, x, s);
+    }
+    return s;
+  }
   for (long i = begin + tid; i < end; i += EW_THREADS) {
     const long r = i / cols, cc = i - r * cols;
     float x = Elem<DT>::load1(base, r * ld + cc);

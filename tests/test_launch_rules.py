@@ -270,3 +270,19 @@ int main() {
     text = "".join("%d %d %d %d %d %d\n" % w for w in every)
     out = subprocess.run([str(tmp_path / "runs")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert {w for w, o in zip(every, out) if o == "0"} == by_element and len(out) == 48
+
+
+def test_which_sums_of_squares_go_in_runs_of_eight(tmp_path):
+    """(rows, columns, leading dimension), chunks of 8192 -> in runs; never a matrix of fewer than eight elements, which has no run."""
+    from archscale_amd.build import CSRC
+    (tmp_path / "sums.cpp").write_text(r"""
+#include <cstdio>
+#include "launch_rules.h"
+int main() { int r, c, l; while (scanf("%d %d %d", &r, &c, &l) == 3) printf("%d\n", (int)archscale::sums_in_runs(r, c, l, 8192)); }
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "sums.cpp"), "-o", str(tmp_path / "sums")], check=True)
+    want = {(1, 8, 8): 1, (2, 4, 4): 1, (67, 33, 33): 0, (64, 128, 128): 1, (8193, 1, 1): 1, (8191, 1, 1): 0, (95, 121, 121): 1, (64, 64, 72): 0,
+            (95, 121, 128): 0, (65536, 65537, 65537): 1, **{(1, n, n): 0 for n in range(1, 8)}}
+    text = "".join("%d %d %d\n" % w for w in want)
+    out = subprocess.run([str(tmp_path / "sums")], input=text, capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in out] == list(want.values())
