@@ -591,20 +591,6 @@ __device__ __forceinline__ void ball_dense(const muon_ball_item& it, long begin,
   }
 }
 
-// eight elements from any place on, through the caches
-template <int WD>
-__device__ __forceinline__ void ball_load8(const void* p, long i, float (&v)[8]) {
-  if constexpr (WD == DT_BF16) {
-    const u32x4 r = *(const u32x4_any*)((const uint16_t*)p + i);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(r[k] & 0xffff); v[2 * k + 1] = bf2f(r[k] >> 16); }
-  } else {
-    const f32x4 a = *(const f32x4_any*)((const float*)p + i), b = *(const f32x4_any*)((const float*)p + i + 4);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { v[k] = a[k]; v[4 + k] = b[k]; }
-  }
-}
-
 // Blocks inside wider matrices, whose rows share lines with their neighbours: through the caches, runs of eight where rows are whole runs and
 // one element per thread where a run would cross the end of a row.  us for 17.8 million elements, so / as dense blocks with the runs split
 // at the ends of rows, bfloat16 and fp32: 24 columns in 32 32 / 34 and 53 / 74, 9 in 17 62 / 136 and 86 / 240, 1001 in 1009 46 / 46 and 58 / 54
@@ -615,8 +601,8 @@ __device__ __forceinline__ void ball_strided(const muon_ball_item& it, long begi
     for (long i = begin + (long)threadIdx.x * EW_VEC; i < end; i += EW_THREADS * EW_VEC) {
       const long r = i / it.cols, c = i - r * it.cols, w = r * it.ld_w + c;
       float x[8], u[8];
-      ball_load8<DT_BF16>(it.phi, r * it.ld_phi + c, u);
-      ball_load8<WD>(it.w, w, x);
+      Elem<DT_BF16>::fetch8(it.phi, r * it.ld_phi + c, u);
+      Elem<WD>::fetch8(it.w, w, x);
 #pragma unroll
       for (int k = 0; k < 8; ++k) x[k] = fw * x[k] - fp * u[k];
       Elem<WD>::keep8(it.w, w, x);

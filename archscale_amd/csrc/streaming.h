@@ -52,6 +52,12 @@ template <> struct Elem<DT_BF16> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(w[k] & 0xffff); v[2 * k + 1] = bf2f(w[k] >> 16); }
   }
+  // the same through the caches, for lines that other accesses share
+  static __device__ __forceinline__ void fetch8(const void* p, long i, float (&v)[8]) {
+    const u32x4 r = *(const u32x4_any*)((const uint16_t*)p + i);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { v[2 * k] = bf2f(r[k] & 0xffff); v[2 * k + 1] = bf2f(r[k] >> 16); }
+  }
   static __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
     return u32x4{f2bf_pair(v[0], v[1]), f2bf_pair(v[2], v[3]), f2bf_pair(v[4], v[5]), f2bf_pair(v[6], v[7])};
   }
@@ -67,6 +73,11 @@ template <> struct Elem<DT_F32> {
     const f32x4 a = __builtin_nontemporal_load((const f32x4_any*)((const float*)p + i));
     const f32x4 b = __builtin_nontemporal_load((const f32x4_any*)((const float*)p + i + 4));
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+  static __device__ __forceinline__ void fetch8(const void* p, long i, float (&v)[8]) {
+    const f32x4 a = *(const f32x4_any*)((const float*)p + i), b = *(const f32x4_any*)((const float*)p + i + 4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { v[k] = a[k]; v[4 + k] = b[k]; }
   }
   static __device__ __forceinline__ void store8(void* p, long i, const float (&v)[8]) {
     const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
