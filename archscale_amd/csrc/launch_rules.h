@@ -41,9 +41,7 @@ struct LaunchSplit { int whole, quarters, sixteenths; };
 // The same again one level down: 128 tiles of 256 are exactly one round of quadrants (two to a unit); up to SIXTEENTH_MAX tiles
 // left beside whole rounds of either kind become sixteen tiles of 64 each, one block per unit at most.  The 136 triangle tiles of
 // a short side of 4096: 97 -> 78 us per product; 4096 x 4096 1466 -> 1376 us, 4000 x 4100 (half storage) 1683 -> 1538, 4096 x
-// 14336 3353 -> 3255; more than 16 tiles so: no further gain.  A launch of nothing but so few (single
-// symmetric products; one tile of 64 to a unit instead of one of 128 to a fourth of the units): 1024 x 3072 22.4 -> 13.1 us, 1024 x
-// 1024 11.6 -> 7.3, 512 x 2048 16.3 -> 9.6, 512 x 512 7.9 -> 5.5.
+// 14336 3353 -> 3255; more than 16 tiles so: no further gain.
 constexpr int RULE_UNITS = 256;   // the device of the figures
 constexpr int QUARTER_MAX_TAIL = 128;
 constexpr int SIXTEENTH_MAX = 16;
@@ -51,8 +49,8 @@ constexpr double QUARTER_LOAD = 0.6;
 
 // Tiles of 128 whose quadrants find room in one round, two to a unit: quartered whatever their reductions.  us a call, as tiles of 128 / of 64:
 // one 512 x 2048 matrix 203 / 133, 3001 x 1023 286 / 198, 1500 x 2000 (78 tiles) 268 / 241, 3 x (1000 x 2000) (108) 252 / 243, 1700 x 3000 (105)
-// 368 / 340, 1900 x 1900 (120) 284 / 269, 12 x (500 x 4000) (120) 375 / 354, 6 x (700 x 1300) (126) 222 / 210, single products of 1792 x
-// 4096 27.9 / 25.2, 3 x (1000 x 960) 25.4 / 24.8.  With a second round they lose: 13 x (512 x 1000) (130) 198 / 212, 9 x (640 x 640) (135) 169 / 191,
+// 368 / 340, 1900 x 1900 (120) 284 / 269, 12 x (500 x 4000) (120) 375 / 354, 6 x (700 x 1300) (126) 222 / 210, single products of 1024
+// x 3072 (36) 22.4 / 13.1, 512 x 512 (10) 7.9 / 5.5, 1792 x 4096 (105) 27.9 / 25.2, 3 x (1000 x 960) 25.4 / 24.8.  With a second round they lose: 13 x (512 x 1000) (130) 198 / 212, 9 x (640 x 640) (135) 169 / 191,
 // 5 x (896 x 1024) (140) 225 / 260, a product of 1826 x 960 (136) 28.0 / 28.9, 2048 x 2048 (136) 288 / 342.
 inline bool one_round_of_quadrants(int units, int tile, bool pair, int total) { return tile == 128 && !pair && 2L * total <= units; }
 
@@ -66,7 +64,7 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
   const int full = total / units * units, tail = total - full;
   if (tail == 0 || (full > 0 ? tail > scaled(QUARTER_MAX_TAIL) : all > QUARTER_LOAD * units * longest)) return as_is;
   const int half = units / 2, few = scaled(SIXTEENTH_MAX);   // half: one round of quadrants
-  if (!pair && tail <= few) return {full, 0, tail};   // (full: none or whole rounds)
+  if (!pair && full > 0 && tail <= few) return {full, 0, tail};
   if (!pair && tail > half && tail - half <= few) return {full, half, tail - half};
   return {full, tail, 0};
 }

@@ -230,14 +230,6 @@ int main() {
     assert [int(v) for v in out] == list(want.values())
 
 
-def test_few_large_tiles_alone_become_sixteenths(rules):
-    """(units, tiles of 256) -> all of them as sixteen tiles of 64, up to one block to a unit; hi+lo pairs have no such tiles."""
-    want = {(256, 1): (0, 0, 1), (256, 16): (0, 0, 16), (256, 17): (0, 17, 0), (128, 8): (0, 0, 8), (128, 9): (0, 9, 0), (15, 1): (0, 1, 0)}
-    got = rules([(u, 256, 0, n, n * 1e3, 1e3, 1, 64) for u, n in want])
-    assert [g[:3] for g in got] == list(want.values())
-    assert rules([(256, 256, 1, 16, 16e3, 1e3, 1, 64)])[0][:3] == (0, 16, 0)
-
-
 def test_lines_of_one_round_of_quadrants(tmp_path):
     """(units, tile, pair, tiles) -> quartered because two quadrants to a unit hold them all."""
     from archscale_amd.build import CSRC
