@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "elementwise.h"
 #include "launch_rules.h"
 #include "streaming.h"
@@ -162,37 +164,40 @@ __device__ __forceinline__ void layout_tile(const char* base, int ty, int tx, in
   const float fs = __builtin_ldexpf(1.f, out_shift);
   const int tr = threadIdx.x >> 3;        // 0..31
   const int tc = (threadIdx.x & 7) * 8;   // 0..56
-  // Runs that start at multiples of 16 bytes go past the caches; elsewhere a line belongs to several, and a second one finds it in the
-  // caches (us a call, past them / through them: power iteration over 3 x (1408 x 3903) 124.7 / 115.0 in fp32 and 122.9 / 115.5 in bfloat16, the
-  // hook on 3001 x 1023 in fp32 176.0 / 172.6, a product of 3001 x 3001 with an addend 83.5 / 77.5).
-  const bool apart = aligned16(base) && ld % 8 == 0;
+  auto rows_in = [&](auto apart_) __attribute__((always_inline)) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = r0 + tr + h * 32, c = c0 + tc;
-    float v[8];
-    if (r < rows && c + 7 < cols) {
-      if (apart) Elem<DT>::load8(base, (long)r * ld + c, v);
-      else Elem<DT>::fetch8(base, (long)r * ld + c, v);
-    } else {
+    for (int h = 0; h < 2; ++h) {
+      const int r = r0 + tr + h * 32, c = c0 + tc;
+      float v[8];
+      if (r < rows && c + 7 < cols) {
+        if constexpr (decltype(apart_)::value) Elem<DT>::load8(base, (long)r * ld + c, v);
+        else Elem<DT>::fetch8(base, (long)r * ld + c, v);
+      } else {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = (r < rows && c + k < cols) ? Elem<DT>::load1(base, (long)r * ld + c + k) : 0.f;
-    }
-    uint16_t o[8];
+        for (int k = 0; k < 8; ++k) v[k] = (r < rows && c + k < cols) ? Elem<DT>::load1(base, (long)r * ld + c + k) : 0.f;
+      }
+      uint16_t o[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float x = CAST_FIRST ? bf2f(f2bf(v[k])) : v[k];
-      // half output: times 2^out_shift, which keeps the normalised entries in the normal range of the format
-      o[k] = out_f16 ? __builtin_bit_cast(uint16_t, (_Float16)(x * s * fs)) : f2bf(x * s);
-      tile[tr + h * 32][tc + k] = o[k];
-      if (tile_sumsq) { const float w = out_f16 ? x * s : bf2f(o[k]); ss[0] += w * w; }
+      for (int k = 0; k < 8; ++k) {
+        const float x = CAST_FIRST ? bf2f(f2bf(v[k])) : v[k];
+        // half output: times 2^out_shift, which keeps the normalised entries in the normal range of the format
+        o[k] = out_f16 ? __builtin_bit_cast(uint16_t, (_Float16)(x * s * fs)) : f2bf(x * s);
+        tile[tr + h * 32][tc + k] = o[k];
+        if (tile_sumsq) { const float w = out_f16 ? x * s : bf2f(o[k]); ss[0] += w * w; }
+      }
+      if (D && r < d_rows && c < d_cols) {
+        u32x4 pk;
+        pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
+        pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
+        *(u32x4*)(D + (size_t)r * ldd + c) = pk;
+      }
     }
-    if (D && r < d_rows && c < d_cols) {
-      u32x4 pk;
-      pk.x = o[0] | ((uint32_t)o[1] << 16); pk.y = o[2] | ((uint32_t)o[3] << 16);
-      pk.z = o[4] | ((uint32_t)o[5] << 16); pk.w = o[6] | ((uint32_t)o[7] << 16);
-      *(u32x4*)(D + (size_t)r * ldd + c) = pk;
-    }
-  }
+  };
+  // Runs go past the caches, but for fp32 rows that do not start at multiples of 16 bytes: a line of theirs belongs to several accesses, and
+  // the later ones find it in the caches.  us a call, past them / through them: power iteration over 3 x (1408 x 3903) 125.4 / 116.9, 13 x (1182 x
+  // 3009) 207.6 / 196.3, the hook on 3001 x 1023 175.6 / 173.9.  (Two bodies: of a choice at each load the compiler makes one load through the caches.)
+  if (DT == DT_BF16 || (aligned16(base) && ld % 8 == 0)) rows_in(std::true_type{});
+  else rows_in(std::false_type{});
   if (tile_sumsq) {   // sum of squares of what this block wrote (every block of the grid: one value per 64x64 tile)
     block_reduce<1>(ss, red);
     if (threadIdx.x == 0) *tile_sumsq = ss[0];
