@@ -153,10 +153,15 @@ stage_sumsq_kernel(const StageParams sp) {
 //    X/(norm+eps), .mT and .contiguous() of newton_schulz_triton.py:358-366).
 // ---------------------------------------------------------------------------
 // one 64x64 tile (row tile ty, column tile tx) by one block; d_rows / d_cols are the padded extents (multiples of 64)
+// apart: rows that do not start at multiples of 16 bytes go past the caches too.  A line of theirs belongs to several accesses, and the later ones
+// find it in the caches, but what comes after may miss what the matrix has pushed out.  us a call, past them / through them: in fp32 the power
+// iteration over 3 x (1408 x 3903) 125.4 / 116.9, 13 x (1182 x 3009) 207.6 / 196.3, the hook on 3001 x 1023 175.6 / 173.9; in bfloat16 operands of single
+// products 2240 x 1847 with an addend 44.5 / 42.6, 3000 x 4001 83.6 / 80.9, but the power iteration over 13 x (1182 x 3009), 50 rounds, 355.1 / 358.0
+// and over 30 x (1001 x 1003) 383.5 / 386.3: so past them where bfloat16 goes to the power iteration or to Newton-Schulz.
 template <int DT, bool CAST_FIRST>
 __device__ __forceinline__ void layout_tile(const char* base, int ty, int tx, int rows, int cols, int ld, float s,
                                             uint16_t* D, int ldd, int d_rows, int d_cols, uint16_t* T, int ldt, int out_f16,
-                                            int out_shift, float* tile_sumsq) {
+                                            int out_shift, float* tile_sumsq, bool apart) {
   __shared__ uint16_t tile[64][66];
   __shared__ float red[4];
   float ss[1] = {0.f};
@@ -193,10 +198,9 @@ __device__ __forceinline__ void layout_tile(const char* base, int ty, int tx, in
       }
     }
   };
-  // Runs go past the caches, but for fp32 rows that do not start at multiples of 16 bytes: a line of theirs belongs to several accesses, and
-  // the later ones find it in the caches.  us a call, past them / through them: power iteration over 3 x (1408 x 3903) 125.4 / 116.9, 13 x (1182 x
-  // 3009) 207.6 / 196.3, the hook on 3001 x 1023 175.6 / 173.9.  (Two bodies: of a choice at each load the compiler makes one load through the caches.)
-  if (DT == DT_BF16 || (aligned16(base) && ld % 8 == 0)) rows_in(std::true_type{});
+  // Runs go past the caches where they start at multiples of 16 bytes, and if `apart` says so elsewhere too.  (Two bodies: of a choice at each load
+  // the compiler makes one load through the caches.)
+  if (apart || (aligned16(base) && ld % 8 == 0)) rows_in(std::true_type{});
   else rows_in(std::false_type{});
   if (tile_sumsq) {   // sum of squares of what this block wrote (every block of the grid: one value per 64x64 tile)
     block_reduce<1>(ss, red);
@@ -230,7 +234,8 @@ layout_kernel(const void* __restrict__ in, const LayoutPtrs ptrs, long in_bstrid
   const char* base = in ? (const char*)in + (size_t)b * in_bstride * sizeof(typename Elem<DT>::T) : (const char*)ptrs.p[b];
   layout_tile<DT, false>(base, blockIdx.y, blockIdx.x, rows, cols, ld, 1.f,
                          D ? D + (size_t)b * bstride : nullptr, ldd, d_rows, d_cols, T ? T + (size_t)b * bstride : nullptr, ldt,
-                         0, 0, tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr);
+                         0, 0, tile_sumsq ? tile_sumsq + ((size_t)b * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x : nullptr,
+                         DT == DT_BF16 && tile_sumsq);   // (no sums of squares: an operand of a single product)
 }
 
 // The copies of a staging launch.  Launch bound for all but the largest calls, hence one launch over all matrices and no
@@ -271,7 +276,7 @@ stage_layout_kernel(const StageParams sp) {
   const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
   uint16_t* dst = q.dst + (size_t)b * q.d_bstride;
   layout_tile<DT, CAST_FIRST>(base, ty, tx, q.rows, q.cols, q.ld, s, q.transpose ? nullptr : dst, q.ldd,
-                              q.d_rows, q.d_cols, q.transpose ? dst : nullptr, q.ldd, q.out_f16, q.out_shift, nullptr);
+                              q.d_rows, q.d_cols, q.transpose ? dst : nullptr, q.ldd, q.out_f16, q.out_shift, nullptr, DT == DT_BF16);
 }
 
 bool stage_blocks(const StageProblem& p, long* sum_blocks, long* tiles) {
