@@ -223,11 +223,14 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
   if (mode != MODE_BX && tile == 256 && env_switches().quarter) {
     long smaller = 0;
     bool whole_matrices = true;
+    double second_load = 0.0;
     for (int i = 0; i < gp.n_groups; ++i) {
+      const long before = std::max(smaller, 2L * units);
       smaller += (long)gp.g[i].batch * sym_tiles(2 * gp.g[i].tilesM);
+      second_load += (double)std::max(smaller - before, 0L) * gp.g[i].K;
       whole_matrices = whole_matrices && !gp.g[i].t_count;
     }
-    if (whole_matrices && halved_tiles(units, tile, split, total, smaller, longest, cut)) {
+    if (whole_matrices && halved_tiles(units, tile, split, total, smaller, second_load, longest, cut)) {
       GroupedGemmParams q = gp;
       for (int i = 0; i < gp.n_groups; ++i) {
         q.g[i].tilesM *= 2;

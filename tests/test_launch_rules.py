@@ -184,15 +184,16 @@ int main() { int u, t, k; while (scanf("%d %d %d", &u, &t, &k) == 3) printf("%d\
 
 
 def test_lines_of_halved_tiles(tmp_path):
-    """(tile, pair, tiles of 256, tiles of 128 of the same matrices, all k-values, longest) on 256 units -> in tiles of 128 or not."""
+    """(tile, pair, tiles of 256, tiles of 128 of the same matrices, all k-values, longest; the k-values of those of 128 beyond two to a unit where
+    they are not all of the longest) on 256 units -> in tiles of 128 or not."""
     from archscale_amd.build import CSRC
     (tmp_path / "halved.cpp").write_text(r"""
 #include <cstdio>
 #include "launch_rules.h"
 int main() {
-  int t, p, n, s; double a, l;
-  while (scanf("%d %d %d %d %lf %lf", &t, &p, &n, &s, &a, &l) == 6)
-    printf("%d\n", (int)archscale::halved_tiles(256, t, p != 0, n, s, l, archscale::launch_split(256, t, p != 0, n, a, l)));
+  int t, p, n, s; double a, l, m;
+  while (scanf("%d %d %d %d %lf %lf %lf", &t, &p, &n, &s, &a, &l, &m) == 7)
+    printf("%d\n", (int)archscale::halved_tiles(256, t, p != 0, n, s, m < 0 ? (s - 512) * l : m, l, archscale::launch_split(256, t, p != 0, n, a, l)));
 }
 """)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "halved.cpp"), "-o", str(tmp_path / "halved")], check=True)
@@ -221,11 +222,16 @@ int main() {
         (256, 0, 203, 609, 203 * 512.0, 512.0): 0,
         (256, 0, 256, 768, 256 * 256.0, 256.0): 1,
         (256, 0, 256, 768, 256 * 768.0, 768.0): 0,
+        # a second round whose tiles are not all of the longest reduction: 128 of 512 and 192 of 256 k-values; up to half a round of 512
+        (256, 0, 256, 832, 256 * 448.0, 512.0, 128 * 512.0 + 192 * 256.0): 1,
+        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * 512.0): 1,
+        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * 512.0 + 64.0): 0,
+        (256, 0, 256, 832, 256 * 512.0, 512.0): 0,
         (256, 0, 208, 744, 208 * 1088.0, 1088.0): 0,     # longer reductions stay
         (256, 1, 208, 744, 208 * 1024.0, 1024.0): 0,     # hi+lo pairs stay
         (128, 0, 208, 744, 208 * 1024.0, 1024.0): 0,
     }
-    text = "".join("%d %d %d %d %.17g %.17g\n" % w for w in want)
+    text = "".join("%d %d %d %d %.17g %.17g %.17g\n" % (w if len(w) == 7 else (*w, -1.0)) for w in want)
     out = subprocess.run([str(tmp_path / "halved")], input=text, capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in out] == list(want.values())
 
