@@ -31,6 +31,7 @@ CHUNK_ELEMS = 8192
 NS_STATIC_SCRATCH_BYTES = 64 << 20
 STREAM_COPY, STREAM_READ, STREAM_MIX = 0, 1, 2
 E_STATIC_LIMIT = -4
+PROF_KEY_STREAM = 30000
 PROF_KEY_MOMENTUM_LAYOUT = 90000
 PROF_KEY_SMALL_NS = 91000
 ABI_VERSION = 3
@@ -304,8 +305,8 @@ def profile_begin() -> None:
 
 def profile_collect(capacity: int = 4096):
     """Per-launch records of the Newton-Schulz GEMMs since profile_begin():
-    list of dicts {kind="gemm", ms, tile, mode, split, final, folded, flops_algorithmic, flops_issued} (``folded`` marks
-    the X' = (B + aI) X launches that read no addend), {kind="momentum_layout", ms, bytes} for the fused momentum
+    list of dicts {kind="gemm", ms, tile, mode, split, final, folded, stream, flops_algorithmic, flops_issued} (``folded`` marks
+    the X' = (B + aI) X launches that read no addend, ``stream`` those whose blocks take many tiles one after the other), {kind="momentum_layout", ms, bytes} for the fused momentum
     launches (``bytes`` = algorithmic HBM bytes of the launch) and {kind="small", ms, side, flops_algorithmic, flops_issued}
     for launches that run the whole iteration of small matrices (short side up to ``side``), a block each."""
     ms = (ctypes.c_float * capacity)()
@@ -324,6 +325,8 @@ def profile_collect(capacity: int = 4096):
         if k > PROF_KEY_SMALL_NS:
             out.append(dict(kind="small", ms=ms[i], side=k - PROF_KEY_SMALL_NS, flops_algorithmic=fa[i], flops_issued=fi[i]))
             continue
-        out.append(dict(kind="gemm", ms=ms[i], tile=k // 100, mode=(k // 10) % 10, split=bool((k % 10) & 2),
+        stream = k >= PROF_KEY_STREAM
+        k -= PROF_KEY_STREAM if stream else 0
+        out.append(dict(kind="gemm", ms=ms[i], stream=stream, tile=k // 100, mode=(k // 10) % 10, split=bool((k % 10) & 2),
                         final=bool((k % 10) & 1), folded=bool((k % 10) & 4), flops_algorithmic=fa[i], flops_issued=fi[i]))
     return out

@@ -165,13 +165,13 @@ int compute_units() {
 // pool that muon_profile_begin creates, so a timed call creates nothing; launches beyond the pool run untimed.
 // Profiling is a single-threaded debugging mode: every timed launch takes one process-wide lock.
 struct ProfRec {
-  // tile*100 + mode*10 + 4*(BX without addend) + split*2 + final; PROF_KEY_MOMENTUM_LAYOUT for the fused momentum; PROF_KEY_SMALL_NS + 64
+  // tile*100 + mode*10 + 4*(BX without addend) + split*2 + final, and PROF_KEY_STREAM for a launch of ns_gemm_stream_kernel; PROF_KEY_MOMENTUM_LAYOUT for the fused momentum; PROF_KEY_SMALL_NS + 64
   // or 128 for the whole iteration of small matrices
   int key;
   double work_algorithmic, work_issued;   // FLOPs of a GEMM launch; bytes of a momentum launch
 };
 constexpr int PROF_POOL = 1024;
-constexpr int PROF_KEY_MOMENTUM_LAYOUT = 90000, PROF_KEY_SMALL_NS = 91000;
+constexpr int PROF_KEY_STREAM = 30000, PROF_KEY_MOMENTUM_LAYOUT = 90000, PROF_KEY_SMALL_NS = 91000;
 std::mutex g_prof_mutex;
 std::vector<hipEvent_t> g_prof_start, g_prof_stop;   // the pool
 std::vector<ProfRec> g_prof;                         // g_prof[i] used events i
@@ -195,7 +195,7 @@ hipError_t timed_launch(int key, double work_algorithmic, double work_issued, hi
 hipError_t timed_gemm(int tile, int mode, bool split, bool final_, const GroupedGemmParams& g, hipStream_t stream,
                       int units, double flops_algorithmic, double flops_issued, int f16 = 0) {
   const int key = tile * 100 + mode * 10 + ((mode == MODE_BX && !g.g[0].E) ? 4 : 0) + (split ? 2 : 0) + (final_ ? 1 : 0);
-  return timed_launch(key, flops_algorithmic, flops_issued, stream,
+  return timed_launch(stream_takes(tile, mode, split, final_, g, units) ? PROF_KEY_STREAM + key : key, flops_algorithmic, flops_issued, stream,
                       [&] { return launch_ns_gemm_grouped(tile, mode, split, final_, g, stream, units, f16); });
 }
 
@@ -223,8 +223,11 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
   if (mode != MODE_BX && tile == 256 && env_switches().quarter) {
     long smaller = 0;
     bool whole_matrices = true;
-    double second_load = 0.0;
+    double second_load = 0.0, issued[2] = {0.0, 0.0};   // (matrix-core work as it is and in smaller tiles)
     for (int i = 0; i < gp.n_groups; ++i) {
+      const double k = (double)gp.g[i].batch * gp.g[i].K;
+      issued[0] += 4.0 * k * sym_tiles_issued(gp.g[i].tilesM);
+      issued[1] += k * sym_tiles_issued(2 * gp.g[i].tilesM);
       const long before = std::max(smaller, 2L * units);
       smaller += (long)gp.g[i].batch * sym_tiles(2 * gp.g[i].tilesM);
       second_load += (double)std::max(smaller - before, 0L) * gp.g[i].K;
@@ -237,7 +240,9 @@ hipError_t launch_rounds(int tile, int mode, bool split, bool final_, const Grou
         q.g[i].tilesN *= 2;
         q.tile_start[i + 1] = q.tile_start[i] + (int)ns_gemm_tiles(mode, q.g[i]);
       }
-      return launch_rounds(128, mode, split, final_, q, stream, units, work, f16);
+      LaunchWork less = {};
+      if (work) less = {work->algorithmic, work->issued * issued[1] / issued[0]};
+      return launch_rounds(128, mode, split, final_, q, stream, units, work ? &less : nullptr, f16);
     }
   }
   if (cut.whole == total) return launch(tile, gp, 1.0);

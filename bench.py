@@ -350,17 +350,18 @@ def main():
 
     # dominant kernel: the X' = aX + BX product in its main (non-final) instantiation
     by_kernel = {}
+    launch_kind = lambda r: (r["tile"], r["mode"], r["split"], r["final"], r["folded"], r["stream"])
     mom = [r for r in recs if r["kind"] == "momentum_layout"]
     recs = [r for r in recs if r["kind"] == "gemm"]
     for r in recs:
-        k = (r["tile"], r["mode"], r["split"], r["final"], r["folded"])
+        k = launch_kind(r)
         d = by_kernel.setdefault(k, dict(n=0, ms=0.0, fa=0.0, fi=0.0))
         d["n"] += 1; d["ms"] += r["ms"]; d["fa"] += r["flops_algorithmic"]; d["fi"] += r["flops_issued"]
     names = {0: "symprod", 1: "syrk2", 2: "bx", 3: "syrkt"}   # symprod: the m x m products of the Gram-side tail
     kernels = []
-    for (tile, mode, split, final, folded), d in sorted(by_kernel.items(), key=lambda kv: -kv[1]["ms"]):
+    for (tile, mode, split, final, folded, stream), d in sorted(by_kernel.items(), key=lambda kv: -kv[1]["ms"]):
         kernels.append({
-            "kernel": f"ns_gemm<{tile},{names[mode]}{',split' if split else ''}{',final' if final else ''}>",
+            "kernel": f"ns_gemm{'_stream' if stream else ''}<{tile},{names[mode]}{',split' if split else ''}{',final' if final else ''}>",
             "addend": (not folded) if mode == 2 else None,
             "launches_per_step": d["n"], "avg_ms": round(d["ms"] / d["n"], 4),
             "algorithmic_tflops": round(d["fa"] / d["ms"] / 1e9, 1), "issued_tflops": round(d["fi"] / d["ms"] / 1e9, 1),
@@ -374,7 +375,7 @@ def main():
     dom_key = max((k for k in by_kernel if k[1] == dom_mode), key=lambda k: by_kernel[k]["ms"])
     # the roofline line is per launch: of the dominant kernel's launches take those that cover every matrix (with the
     # Gram-side tail one launch of the last-but-one iteration covers only the classes that do not take it)
-    dom_recs = [r for r in recs if (r["tile"], r["mode"], r["split"], r["final"], r["folded"]) == dom_key]
+    dom_recs = [r for r in recs if launch_kind(r) == dom_key]
     full = max(r["flops_algorithmic"] for r in dom_recs)
     dom_recs = [r for r in dom_recs if r["flops_algorithmic"] >= 0.999 * full]
     dom = dict(n=len(dom_recs), ms=sum(r["ms"] for r in dom_recs), fa=sum(r["flops_algorithmic"] for r in dom_recs),
@@ -383,7 +384,7 @@ def main():
     roofline = {
         "bound": "mfma", "achieved": round(achieved, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
         "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": None,
-        "kernel": f"ns_gemm_kernel<{dom_key[0]},{names[dom_key[1]]}{',split' if dom_key[2] else ''}"
+        "kernel": f"ns_gemm{'_stream' if dom_key[5] else ''}_kernel<{dom_key[0]},{names[dom_key[1]]}{',split' if dom_key[2] else ''}"
                   f"{',final' if dom_key[3] else ''}>",
         "algorithmic_bytes_per_launch": None,
         "launches": dom["n"], "avg_launch_ms": round(dom["ms"] / dom["n"], 4),

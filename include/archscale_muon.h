@@ -174,7 +174,8 @@ void muon_ns_ksplit_info(int rows, int cols, int* info);
  * records to the HOST arrays (any may be NULL) and returns the number of launches recorded (< 0 on error):
  *   ms                elapsed milliseconds of the launch
  *   key               tile*100 + mode*10 + 4*noaddend + split*2 + final  (mode 0 = X X^T, 1 = cAA+bA, 2 = aX + BX,
- *                     3 = X X^T from the transposed iterate; noaddend: an X' = (B + aI) X launch); 91000 + side (64 or
+ *                     3 = X X^T from the transposed iterate; noaddend: an X' = (B + aI) X launch), plus 30000 for a
+ *                     launch of a block per compute unit, each with many tiles one after the other; 91000 + side (64 or
  *                     128) for a launch that runs the whole iteration of matrices with at most that short side, staging
  *                     included; 90000 for a fused momentum launch, whose work fields carry bytes
  *   flops_algorithmic minimum FLOPs of the product (symmetric products counted once)

@@ -6,25 +6,42 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _check(ns, stacks, prec, coeffs):
+def _streamed(call):
+    """(launches of X' = B X between iterations, final ones) of a call that took the form, or None where the lines are those of another device."""
+    from archscale_amd import _lib
+    _lib.profile_begin()
+    call()
+    torch.cuda.synchronize()
+    recs = [r for r in _lib.profile_collect() if r["kind"] == "gemm" and r["stream"]]
+    assert all(r["mode"] == 2 and r["tile"] == 256 for r in recs)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        return None
+    return sum(not r["final"] for r in recs), sum(r["final"] for r in recs)
+
+
+def _check(ns, stacks, prec, coeffs, final=True):
     outs = [torch.empty_like(x) for x in stacks]
-    ns.newton_schulz_grouped(stacks, coeffs, 1e-7, prec=prec, outs=outs)
+    took = _streamed(lambda: ns.newton_schulz_grouped(stacks, coeffs, 1e-7, prec=prec, outs=outs))
+    assert took is None or (took[0] > 0 and (took[1] > 0) == final), took
     for x, o in zip(stacks, outs):
         for i in {0, x.shape[0] // 2, x.shape[0] - 1}:
-            assert torch.equal(ns.newton_schulz(x[i], coeffs, 1e-7, prec=prec), o[i]), (tuple(x.shape), i)
+            alone = torch.empty_like(x[i])
+            took = _streamed(lambda: ns.newton_schulz_grouped([x[i]], coeffs, 1e-7, prec=prec, outs=[alone]))
+            assert took is None or took == (0, 0)
+            assert torch.equal(alone, o[i]), (tuple(x.shape), i)
 
 
-# tiles of X': 384 (one and a half per unit), 416, 1280, 1536; one k-tile count each from the shortest (K = 256) to the longest (2048);
-# more than eight tile rows; extents that are padded, whose final launch needs bounds checks
-@pytest.mark.parametrize("batch,m,n", [(96, 256, 1024), (52, 512, 1024), (160, 256, 2048), (64, 768, 2048), (6, 2048, 2304), (12, 1536, 2304),
-                                       (5, 2048, 2560), (96, 250, 1000)])
+# tiles of X' on 256 units: 400, 416, 432 and 480 (most units one, some two), 648, 1280 and 1536, 640 of which 128 go in quadrants; reductions
+# from the shortest (K = 256) to the longest (2048); more than eight tile rows; extents that are padded, whose final launch needs bounds checks
+@pytest.mark.parametrize("batch,m,n", [(160, 256, 2048), (128, 256, 1280), (52, 512, 1024), (48, 512, 1280), (64, 768, 2048), (6, 2048, 2304),
+                                       (12, 1536, 2304), (5, 2048, 2560), (160, 250, 2000), (52, 500, 1000)])
 @pytest.mark.parametrize("prec", ["bf16", "f16"])
 def test_stacks_of_one_shape(gpu_device, batch, m, n, prec):
     import archscale_amd.optim.newton_schulz_hip as ns
     g = torch.Generator(device=gpu_device).manual_seed(batch + m + n)
     x = (torch.randn(batch, m, n, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
     for t in (x, x.mT.contiguous()):
-        _check(ns, [t], prec, ns.QUINTIC_SCHEDULE)
+        _check(ns, [t], prec, ns.QUINTIC_SCHEDULE, final=m % 256 == 0 and n % 256 == 0)
 
 
 @pytest.mark.parametrize("prec", ["bf16", "f16"])
@@ -43,11 +60,13 @@ def test_results_that_are_not_aligned(gpu_device):
     """A result that is not 16-byte aligned leaves the form for the final launch: the same bits, nothing beside it is touched."""
     import archscale_amd.optim.newton_schulz_hip as ns
     g = torch.Generator(device=gpu_device).manual_seed(4)
-    x = (torch.randn(96, 256, 1024, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
+    x = (torch.randn(160, 256, 2048, generator=g, device=gpu_device) * 1e-3).to(torch.bfloat16)
     want = torch.empty_like(x)
-    ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[want])
+    took = _streamed(lambda: ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[want]))
+    assert took is None or (took[0] > 0 and took[1] == 1)
     flat = torch.full((want.numel() + 8,), 7.0, dtype=torch.bfloat16, device=gpu_device)
-    ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[flat[1:1 + want.numel()].view(want.shape)])
+    took = _streamed(lambda: ns.newton_schulz_grouped([x], ns.QUINTIC_SCHEDULE, 1e-7, outs=[flat[1:1 + want.numel()].view(want.shape)]))
+    assert took is None or (took[0] > 0 and took[1] == 0)
     assert torch.equal(flat[1:1 + want.numel()].view(want.shape), want)
     assert bool((flat[:1] == 7.0).all()) and bool((flat[1 + want.numel():] == 7.0).all())
 
@@ -72,7 +91,9 @@ def test_results_inside_wider_matrices(gpu_device, batch, m, n, tall, left, righ
     q[0].in_batch_stride, q[0].out_batch_stride, q[0].batch, q[0].rows, q[0].cols = rows * cols, rows * wide.shape[2], batch, rows, cols
     L = _lib.lib()
     ws = _lib.workspace(gpu_device, L.muon_ns_grouped_workspace_bytes(q, 1, _lib.PREC_BF16))
-    _lib.check(L.muon_ns_grouped(q, 1, _lib.abc_array(ns.QUINTIC_SCHEDULE), 5, 1e-7, 0, _lib.PREC_BF16, _lib.NS_CAST_INPUT_FIRST, ws.data_ptr(),
-                                 ws.numel(), _lib.current_stream_ptr(gpu_device)), "muon_ns_grouped")
+    took = _streamed(lambda: _lib.check(L.muon_ns_grouped(
+        q, 1, _lib.abc_array(ns.QUINTIC_SCHEDULE), 5, 1e-7, _lib.EPS_ADD, _lib.PREC_BF16, _lib.NS_CAST_INPUT_FIRST, ws.data_ptr(), ws.numel(),
+        _lib.current_stream_ptr(gpu_device)), "muon_ns_grouped"))
+    assert took is None or (took[0] > 0 and took[1] == (1 if m % 256 == 0 and left == 8 else 0)), took
     assert torch.equal(view, want)
     assert bool((wide[:, :, :left] == 7.0).all()) and bool((wide[:, :, left + cols:] == 7.0).all())
