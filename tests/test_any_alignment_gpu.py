@@ -100,3 +100,12 @@ def test_orthogonalisation_of_views(gpu_device, shape, dtype):
         assert torch.equal(o.views[0], want), shift
         a.check_guards()
         o.check_guards()
+    # rows inside wider matrices: those of a leading dimension that is a multiple of eight at an aligned place, and odd ones anywhere
+    cols = shape[-1]
+    aligned = torch.full((*shape[:-1], (cols + 15) // 8 * 8), GUARD, dtype=dtype, device=gpu_device)
+    aligned[..., :cols] = x
+    want = ns.newton_schulz(aligned[..., :cols])
+    for left, right in ((3, 2), (1, 4), (8, 0)):
+        wide = torch.full((*shape[:-1], left + cols + right), GUARD, dtype=dtype, device=gpu_device)
+        wide[..., left:left + cols] = x
+        assert torch.equal(ns.newton_schulz(wide[..., left:left + cols]), want), (left, right)
