@@ -6,9 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# short reductions up to a full round (192 and 256 tiles of 256), longer ones (200), launches quartered as a whole with long reductions (128 and
+# short reductions up to a full round (192 and 256 tiles of 256), longer ones (200), launches quartered as a whole with long reductions (144 and
 # 150 tiles), one that would end in sixteenths (140), one tile a side in one round of smaller tiles (160), a mix of classes, extents that are padded
-HALVED = [[(64, 512, 640)], [(64, 512, 700), (64, 250, 700)], [(20, 1024, 1024)], [(128, 256, 4096)], [(15, 1000, 4096)], [(14, 1024, 4096)],
+HALVED = [[(64, 512, 640)], [(64, 512, 700), (64, 250, 700)], [(20, 1024, 1024)], [(144, 256, 4096)], [(15, 1000, 4096)], [(14, 1024, 4096)],
           [(160, 250, 1000)], [(20, 1020, 1030)], [(8, 1024, 1024), (12, 1024, 2816), (8, 256, 1024)]]
 
 
@@ -54,8 +54,9 @@ def test_quadrants_of_one_round(gpu_device, shapes, prec):
 
 
 # 200, 156, 240, 160 and 216 tiles of 256: up to half a second round of smaller tiles, all of it with a short reduction, one round of smaller ones of one
-# tile a side, and one that stays in tiles of 256
-@pytest.mark.parametrize("batch,n,k", [(20, 1024, 1024), (52, 512, 512), (40, 768, 256), (160, 256, 1024), (6, 2048, 768)])
+# tile a side, and one that stays in tiles of 256; 128, 90 and 84 tiles: quadrants from a third to half a round, smaller tiles below
+@pytest.mark.parametrize("batch,n,k", [(20, 1024, 1024), (52, 512, 512), (40, 768, 256), (160, 256, 1024), (6, 2048, 768), (128, 256, 1024),
+                                       (9, 1000, 700), (28, 512, 256)])
 def test_stacks_of_single_products(gpu_device, batch, n, k):
     import archscale_amd.optim.newton_schulz_hip as ns
     g = torch.Generator(device=gpu_device).manual_seed(n + k)

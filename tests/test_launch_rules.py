@@ -198,7 +198,11 @@ int main() {
 """)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "halved.cpp"), "-o", str(tmp_path / "halved")], check=True)
     want = {
-        (256, 0, 100, 360, 100 * 4096.0, 4096.0): 1,     # quartered as a whole
+        # quartered as a whole: up to a third of a round, and beyond half of it
+        (256, 0, 85, 306, 85 * 4096.0, 4096.0): 1,
+        (256, 0, 86, 310, 86 * 4096.0, 4096.0): 0,
+        (256, 0, 128, 460, 128 * 4096.0, 4096.0): 0,
+        (256, 0, 129, 464, 129 * 4096.0, 4096.0): 1,
         (256, 0, 140, 504, 140 * 4096.0, 4096.0): 1,     # quarters and sixteenths, two smaller tiles to a unit hold it
         (256, 0, 144, 544, 144 * 4096.0, 4096.0): 0,     # they do not
         (256, 0, 208, 744, 208 * 590.0, 1000.0): 1,
