@@ -80,7 +80,8 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
 //   but 8 x (1024 x 2816) (80) 37.3 / 35.7, 2 x (2048 x 1024) (72) 17.7 / 17.0, 25 x (512 x 2048) (75), whose smaller tiles are one to a unit, 26.4 / 18.2;
 // - launches up to a full round with reductions of up to HALVED_MAX_K: the results of a round of large tiles all leave at its end, 10 of 30 to
 //   40 us with the matrix cores idle, while two smaller blocks to a unit store and multiply at the same time.  What decides is the
-//   second round of smaller tiles, those beyond two to a unit (second_load: their k-values).  As it is / so, us of a single product:
+//   second round of smaller tiles, those beyond two to a unit (second_load: their k-values; HALVED_TILE_K more for what a tile costs
+//   beside them).  As it is / so, us of a single product:
 //   up to half of it, in tiles of the longest reduction: 60 x (512 x 768) (600 smaller tiles) 26.5 / 25.0, 36 x (768 x 768) (756) 27.7 / 26.9, 5 x (2048 x 768) (680) 27.6 / 26.2, 21 x
 //     (1024 x 1024) (756) 31.9 / 30.5; more of it: 38 x (768 x 768) (798) 28.4 / 29.6, 6 x (2048 x 1024) (816) 33.5 / 36.2, 83 x (512 x 768) (830) 29.4 / 31.0;
 //   beyond HALVED_LONG_K not where it is nearly empty: 16 x (1024 x 2816) (576), power iteration, 235 / 247 a call;
@@ -88,9 +89,10 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
 //   matrices of one tile a side (3 smaller tiles for one, not 3.3 and more) only where it holds next to nothing: 170 x (256 x 768) (510)
 //     24.8 / 17.6, 180 (540) 24.9 / 24.6, but 190 (570) 25.1 / 26.3, 217 (651) 25.7 / 28.3; of 512 k-values 200 (600) 21.0 / 20.9, 210 (630) 21.2 / 21.6.
 //   Whole steps: the EMA-Muon set of width 1024 (744) 1128 / 1090; 64 + 64 experts, whose short products are 640 tiles of 512 k-values and then 192 of
-//   256 (0.44 of a second round) 1231 / 1220.
+//   256 (320 in the second round) 1231 / 1220; a MuonH set of width 1001, whose products of the tail are 756 tiles of 1024 and then 42 of 256 (286),
+//   37.7 / 43.6 us a product, 1713 / 1727 a step: with a HALVED_TILE_K of 52 to 256 it stays large and the experts do not.
 // At longer reductions they lose: X X^T of 64 + 64 experts (K = 2048), 1214 / 1278 a step.
-constexpr int HALVED_MAX_K = 1024, HALVED_LONG_K = 768, HALVED_ONE_K = 512, HALVED_SHORT_K = 256;
+constexpr int HALVED_MAX_K = 1024, HALVED_LONG_K = 768, HALVED_ONE_K = 512, HALVED_SHORT_K = 256, HALVED_TILE_K = 160;
 inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller, double second_load, double longest, const LaunchSplit& cut) {
   if (tile != 256 || pair) return false;
   if (cut.whole == 0) return (3L * total < units || 2L * total > units) && (cut.sixteenths == 0 || smaller <= 2L * units);
@@ -98,7 +100,7 @@ inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller
   const long second = smaller - 2L * units;   // tiles of the second round
   if (longest <= HALVED_SHORT_K) return true;
   if (5 * smaller < 16L * total) return 8 * second <= (longest <= HALVED_ONE_K ? 3L : 1L) * units;   // (mostly one tile a side)
-  return second_load <= units * longest && (longest <= HALVED_LONG_K || 3 * second >= units);
+  return second_load + (double)HALVED_TILE_K * second <= units * (longest + HALVED_TILE_K) && (longest <= HALVED_LONG_K || 3 * second >= units);
 }
 
 // Parts that the reduction of a single symmetric product (not of a Newton-Schulz call) is cut into, as tiles of 128 (`tiles` of one

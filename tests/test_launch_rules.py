@@ -226,10 +226,11 @@ int main() {
         (256, 0, 203, 609, 203 * 512.0, 512.0): 0,
         (256, 0, 256, 768, 256 * 256.0, 256.0): 1,
         (256, 0, 256, 768, 256 * 768.0, 768.0): 0,
-        # a second round whose tiles are not all of the longest reduction: 128 of 512 and 192 of 256 k-values; up to half a round of 512
+        # a second round whose tiles are not all of the longest reduction: 128 of 512 and 192 of 256 k-values; up to half a round of 512, 160 more for every tile
         (256, 0, 256, 832, 256 * 448.0, 512.0, 128 * 512.0 + 192 * 256.0): 1,
-        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * 512.0): 1,
-        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * 512.0 + 64.0): 0,
+        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * (512.0 + 160) - 320 * 160): 1,
+        (256, 0, 256, 832, 256 * 448.0, 512.0, 256 * (512.0 + 160) - 320 * 160 + 64): 0,
+        (256, 0, 224, 798, 210 * 1024.0 + 14 * 256.0, 1024.0, 244 * 1024.0 + 42 * 256.0): 0,   # (half a round by k-values alone)
         (256, 0, 256, 832, 256 * 512.0, 512.0): 0,
         (256, 0, 208, 744, 208 * 1088.0, 1088.0): 0,     # longer reductions stay
         (256, 1, 208, 744, 208 * 1024.0, 1024.0): 0,     # hi+lo pairs stay
