@@ -142,7 +142,8 @@ stage_sumsq_kernel(const StageParams sp) {
   const int rows = q.rows, cols = q.cols, ld = q.ld;
   const char* base = (const char*)q.in + (size_t)b * q.in_bstride * sizeof(typename Elem<DT>::T);
   float s[1] = {dense_sumsq_ok(rows, cols, ld) ? thread_sumsq_dense<DT>(base, (long)rows * cols, chunk, threadIdx.x, CAST_FIRST)
-                                                     : thread_sumsq_strided<DT>(base, rows, cols, ld, chunk, threadIdx.x, CAST_FIRST)};
+                : ld == cols                   ? thread_sumsq_one_chunk<DT>(base, rows * cols, threadIdx.x, CAST_FIRST)   // (sums_in_runs)
+                                               : thread_sumsq_strided<DT>(base, rows, cols, ld, chunk, threadIdx.x, CAST_FIRST)};
   block_reduce<1>(s, red);
   if (threadIdx.x == 0) q.partial[(size_t)b * q.cpm + chunk] = s[0];
 }

@@ -355,6 +355,10 @@ struct Small {
 #pragma unroll
           for (int j = 0; j < count; ++j)
             v[j] = thread_sumsq_dense<DT>(base, (long)m * n, (wave >> 2) + 2 * (first + j), threadIdx.x & 255, sp.cast_first);
+        } else if (first == 0 && p.in_ld == p.cols) {   // (one chunk: sums_in_runs)
+#pragma unroll
+          for (int j = 1; j < count; ++j) v[j] = 0.f;
+          v[0] = wave >> 2 ? 0.f : thread_sumsq_one_chunk<DT>(base, m * n, threadIdx.x & 255, sp.cast_first);
         } else {
 #pragma unroll
           for (int j = 0; j < count; ++j)

@@ -150,20 +150,24 @@ __device__ __forceinline__ float thread_sumsq_dense(const char* base, long numel
   }
   return s;
 }
+// (a dense matrix of one chunk that does not go in runs: nothing to divide, eight loads in flight.  Apart from the strided sums, which the kernel of
+// small matrices holds three times: with it inside them 3 x (1083 x 33), which takes neither, 56.1 against 55.6 us, in fp32 53.6 / 52.9)
+template <int DT>
+__device__ __forceinline__ float thread_sumsq_one_chunk(const char* base, int numel, int tid, bool cast_first) {
+  float s = 0.f;
+#pragma unroll 8
+  for (int i = tid; i < numel; i += EW_THREADS) {
+    float x = Elem<DT>::load1(base, i);
+    if (cast_first) x = bf2f(f2bf(x));
+    s = fmaf(x, x, s);
+  }
+  return s;
+}
 template <int DT>
 __device__ __forceinline__ float thread_sumsq_strided(const char* base, int rows, int cols, int ld, int chunk, int tid, bool cast_first) {
   const long numel = (long)rows * cols, begin = (long)chunk * MUON_CHUNK_ELEMS;
   const long end = begin + MUON_CHUNK_ELEMS < numel ? begin + MUON_CHUNK_ELEMS : numel;
   float s = 0.f;
-  if (ld == cols) {   // nothing to divide, eight loads in flight
-#pragma unroll 8
-    for (long i = begin + tid; i < end; i += EW_THREADS) {
-      float x = Elem<DT>::load1(base, i);
-      if (cast_first) x = bf2f(f2bf(x));
-      s = fmaf(x, x, s);
-    }
-    return s;
-  }
   for (long i = begin + tid; i < end; i += EW_THREADS) {
     const long r = i / cols, cc = i - r * cols;
     float x = Elem<DT>::load1(base, r * ld + cc);
