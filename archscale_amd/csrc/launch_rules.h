@@ -73,11 +73,14 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
 // matrix in the order of its own smaller tiles (the quadrants of launch_split hold an empty block per diagonal tile and end with a
 // scattered last round).  These are
 // - every launch that launch_split quarters as a whole, and those that it cuts into quarters and sixteenths if two smaller tiles to a
-//   unit hold them: 14 x (1024 x 4096) 1106 / 981 us a call; not 4 x (2048 x 4096) (544 of them), 1140 / 1214.  Not from a third to half
-//   a round, though: two quadrants to a unit hold it too, four neighbours share their rows of the operands, and an empty one leaves its
-//   unit to the other.  us of a stack of single products as quadrants / so: 12 x (1024 x 2816) (120 tiles) 46.4 / 48.9, 9 of them (90)
-//   37.7 / 40.1, 128 x (256 x 1024) 18.1 / 20.0, 32 x (512 x 1024) (96) 18.2 / 18.6, 17 x (768 x 2816) (102) 38.5 / 40.0, 3 x (2048 x 2048) (108) 30.9 / 31.7;
-//   but 8 x (1024 x 2816) (80) 37.3 / 35.7, 2 x (2048 x 1024) (72) 17.7 / 17.0, 25 x (512 x 2048) (75), whose smaller tiles are one to a unit, 26.4 / 18.2;
+//   unit hold them: 14 x (1024 x 4096) 1106 / 981 us a call; not 4 x (2048 x 4096) (544 of them), 1140 / 1214.  Up to half a round, where
+//   two quadrants to a unit hold it too, four neighbours share their rows of the operands and an empty one leaves its unit to the other, only
+//   what is less than a third of a round with at most nine smaller tiles to eight units, most of them alone on theirs.  us of a stack of
+//   single products as quadrants / so: 12 x (1024 x 2816) (120 large, 432 smaller tiles) 46.4 / 48.9, 9 x (1024 x 2816) (90, 324) 37.7 / 40.1,
+//   128 x (256 x 1024) (128, 384) 18.1 / 20.0, 32 x (512 x 1024) (96, 320) 18.2 / 18.6, 17 x (768 x 2816) (102, 357) 38.5 / 40.0, 3 x (2048 x 2048)
+//   (108, 408) 30.9 / 31.7, 14 x (768 x 1024) (84, 294) 18.2 / 18.4, 4 x (1521 x 416) (84, 312) 34.8 / 35.4, 96 x (256 x 1024) (96, 288) 17.7 / 18.1;
+//   but 8 x (1024 x 2816) (80, 288) 37.3 / 35.7, 28 x (512 x 1024) (84, 280) 18.0 / 17.8, 2 x (2048 x 1024) (72, 272) 17.7 / 17.0, 25 x (512 x 2048)
+//   (75, 250) 26.4 / 18.2;
 // - launches up to a full round with reductions of up to HALVED_MAX_K: the results of a round of large tiles all leave at its end, 10 of 30 to
 //   40 us with the matrix cores idle, while two smaller blocks to a unit store and multiply at the same time.  What decides is the
 //   second round of smaller tiles, those beyond two to a unit (second_load: their k-values; HALVED_TILE_K more for what a tile costs
@@ -95,7 +98,7 @@ inline LaunchSplit launch_split(int units, int tile, bool pair, int total, doubl
 constexpr int HALVED_MAX_K = 1024, HALVED_LONG_K = 768, HALVED_ONE_K = 512, HALVED_SHORT_K = 256, HALVED_TILE_K = 160;
 inline bool halved_tiles(int units, int tile, bool pair, int total, long smaller, double second_load, double longest, const LaunchSplit& cut) {
   if (tile != 256 || pair) return false;
-  if (cut.whole == 0) return (3L * total < units || 2L * total > units) && (cut.sixteenths == 0 || smaller <= 2L * units);
+  if (cut.whole == 0) return (2L * total > units || (3L * total < units && 8 * smaller <= 9L * units)) && (cut.sixteenths == 0 || smaller <= 2L * units);
   if (cut.whole != total || total > units || longest > HALVED_MAX_K) return false;
   const long second = smaller - 2L * units;   // tiles of the second round
   if (longest <= HALVED_SHORT_K) return true;

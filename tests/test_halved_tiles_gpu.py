@@ -54,7 +54,8 @@ def test_quadrants_of_one_round(gpu_device, shapes, prec):
 
 
 # 200, 156, 240, 160 and 216 tiles of 256: up to half a second round of smaller tiles, all of it with a short reduction, one round of smaller ones of one
-# tile a side, and one that stays in tiles of 256; 128, 90 and 84 tiles: quadrants from a third to half a round, smaller tiles below
+# tile a side, and one that stays in tiles of 256; 128, 90 and 84 tiles: quadrants from a third to half a round, smaller tiles
+# below if they are little more than one to a unit
 @pytest.mark.parametrize("batch,n,k", [(20, 1024, 1024), (52, 512, 512), (40, 768, 256), (160, 256, 1024), (6, 2048, 768), (128, 256, 1024),
                                        (9, 1000, 700), (28, 512, 256)])
 def test_stacks_of_single_products(gpu_device, batch, n, k):

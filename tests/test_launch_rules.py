@@ -198,9 +198,11 @@ int main() {
 """)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "halved.cpp"), "-o", str(tmp_path / "halved")], check=True)
     want = {
-        # quartered as a whole: up to a third of a round, and beyond half of it
-        (256, 0, 85, 306, 85 * 4096.0, 4096.0): 1,
-        (256, 0, 86, 310, 86 * 4096.0, 4096.0): 0,
+        # quartered as a whole: little more than one smaller tile to a unit and less than a third of a round; and beyond half of it
+        (256, 0, 80, 288, 80 * 4096.0, 4096.0): 1,
+        (256, 0, 80, 289, 80 * 4096.0, 4096.0): 0,
+        (256, 0, 85, 255, 85 * 4096.0, 4096.0): 1,
+        (256, 0, 86, 258, 86 * 4096.0, 4096.0): 0,
         (256, 0, 128, 460, 128 * 4096.0, 4096.0): 0,
         (256, 0, 129, 464, 129 * 4096.0, 4096.0): 1,
         (256, 0, 140, 504, 140 * 4096.0, 4096.0): 1,     # quarters and sixteenths, two smaller tiles to a unit hold it
