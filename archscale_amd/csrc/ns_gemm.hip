@@ -211,7 +211,8 @@ __device__ __forceinline__ void place_in_grid(int t, int dM, int dN, uint32_t in
 // 128 x 64 read 192 KB, which with the 64 KB of copies is 2048 clk of LDS time per 2048 clk of matrix-core time.
 // Measured on 16 x (2048 x 5632 x 2048), Gaussian operands: 1145 TFLOP/s with eight waves and 32x32x16 MFMAs, 1215 to 1240
 // with four waves and 16x16x32 MFMAs, 1280 to 1300 with a third LDS stage for Q (zero operands, where power does not
-// limit: 1320 / 1330 / 1525).  A persistent form whose copies run on into the next tile measured the same (1300).
+// limit: 1320 / 1330 / 1525).  What a tile costs beside its k-tiles weighs little at this reduction of 2048 and at the power limit; where
+// reductions are short X' = B X goes to ns_gemm_stream_kernel, whose copies run on into the next tile.
 //
 // LDS: SP stages of the P tile and SQ = SP + 1 of the Q tile.  The 256 configuration has room for 2 + 3: the
 // operand that streams from memory (Q = X^T) gets two k-tiles of time to arrive, P, which the caches hold, gets one.
