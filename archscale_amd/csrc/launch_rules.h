@@ -139,10 +139,11 @@ inline int matrix_parts(int tile, long tiles, int kt) {
 // anyway lose nothing (64 of 640 x 8192 267 / 268, 1000 of 128 x 8192 403 / 403).
 inline bool parts_by_blocks(long tiles) { return tiles <= RULE_UNITS / SPLIT_MIN_PARTS; }
 
-// X' = B X in tiles of 256 as a stream (ns_gemm_stream_kernel: one block per unit, its tiles one after the other) where most units have two
-// tiles or more, for reductions of up to STREAM_MAX_K: what it saves is a constant per tile.  tile by tile / as a stream, us: the
-// 64 + 64 expert matrices (K = 512 and 256) 1311 / 1250 a step, the EMA-Muon set of width 1024 1187 / 1163, the depth-16 set (K = 2048 and
-// 512, at the power limit) 21980 / 21660; 4096 x 14336 (K = 4096) 3063 / 3106 a call.  The grid is a multiple of the eight XCDs.
+// X' = B X in tiles of 256 as a stream (ns_gemm_stream_kernel: one block per unit, its tiles one after the other) where units have two tiles
+// or more (launch_split leaves a round and less or more than one and a half), for reductions of up to STREAM_MAX_K: what it saves
+// is a constant per tile.  tile by tile / as a stream, us: the 64 + 64 expert matrices (K = 512 and 256) 1311 / 1250 a step, the EMA-Muon set
+// of width 1024 1187 / 1163, the depth-16 set (K = 2048 and 512, at the power limit) 21980 / 21660; 4096 x 14336 (K = 4096) 3063 / 3106 a
+// call.  The grid is a multiple of the eight XCDs.
 constexpr int STREAM_MAX_K = 2048;
 inline bool stream_of_tiles(int units, int total, int longest) {
   return units % 8 == 0 && total >= units + units / 2 && longest <= STREAM_MAX_K;
