@@ -159,6 +159,8 @@ stage_sumsq_kernel(const StageParams sp) {
 // iteration over 3 x (1408 x 3903) 125.4 / 116.9, 13 x (1182 x 3009) 207.6 / 196.3, the hook on 3001 x 1023 175.6 / 173.9; in bfloat16 operands of single
 // products 2240 x 1847 with an addend 44.5 / 42.6, 3000 x 4001 83.6 / 80.9, but the power iteration over 13 x (1182 x 3009), 50 rounds, 355.1 / 358.0
 // and over 30 x (1001 x 1003) 383.5 / 386.3: so past them where bfloat16 goes to the power iteration or to Newton-Schulz.
+// The two bodies cost the smallest copies 0.3 us beside one element at a time (2984 x 85 5.1 / 5.4, its product 31.3 / 31.8); with the choice around the
+// loads alone and one conversion for both they are slower again (5.7, 3642 x 1928 9.2 / 9.7).
 template <int DT, bool CAST_FIRST>
 __device__ __forceinline__ void layout_tile(const char* base, int ty, int tx, int rows, int cols, int ld, float s,
                                             uint16_t* D, int ldd, int d_rows, int d_cols, uint16_t* T, int ldt, int out_f16,
